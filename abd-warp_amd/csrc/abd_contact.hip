@@ -24,6 +24,7 @@
 #include <cstring>
 
 #include "abd_block.h"
+#include "abd_dense.h"
 #include "abd_device.h"
 #include "abd_inertia.h"
 #include "abd_internal.h"
@@ -148,127 +149,6 @@ __device__ bool contact_terms(int kind, const d3 v[4], const d3 r[4], double d2h
     return true;
 }
 
-// The dense 24x24 block J^T Hx J and gradient gscale J^T gx of one contact (out[0..575]
-// row-major, bodies [I | J]; out[576..599]): vertex t of body half h(t) maps through
-// [1, r_t^T] (x) I3; PT has one vertex on body I, EE two.
-constexpr int kDenseStride = 600;
-constexpr int kDenseGOff = 576;
-__device__ void dense_body_map(int kind, const d3 r[4], const double gx[12], double gscale, const double Hx[144],
-                               double* __restrict__ out) {
-    const int nI = kind == 0 ? 1 : 2;
-    for (int i = 0; i < 24; ++i) {
-        const int hi = i / 12, ai = (i % 12) / 3, ki = i % 3;
-        double gacc = 0.0;
-        for (int t = 0; t < 4; ++t) {
-            if ((t < nI ? 0 : 1) != hi) continue;
-            const double Ji = ai == 0 ? 1.0 : comp(r[t], ai - 1);
-            gacc += Ji * gx[3 * t + ki];
-        }
-        out[kDenseGOff + i] = gscale * gacc;
-        for (int j = 0; j < 24; ++j) {
-            const int hj = j / 12, aj = (j % 12) / 3, kj = j % 3;
-            double acc = 0.0;
-            for (int t = 0; t < 4; ++t) {
-                if ((t < nI ? 0 : 1) != hi) continue;
-                const double Ji = ai == 0 ? 1.0 : comp(r[t], ai - 1);
-                for (int q = 0; q < 4; ++q) {
-                    if ((q < nI ? 0 : 1) != hj) continue;
-                    const double Jj = aj == 0 ? 1.0 : comp(r[q], aj - 1);
-                    acc += Ji * Jj * Hx[12 * (3 * t + ki) + 3 * q + kj];
-                }
-            }
-            out[24 * i + j] = acc;
-        }
-    }
-}
-
-// Exact mode (psd = 2, beyond the reference): the dense 24x24 block
-// J^T (b' d2s/dx2 + b'' ds/dx ds/dx^T) J and the gradient b' J^T ds/dx of one
-// contact, written as out[0..575] (row-major, bodies [I | J]) and out[576..599].
-__device__ bool contact_terms_exact(int kind, const d3 v[4], const d3 r[4], double d2hat, double kappa,
-                                    double* __restrict__ out) {
-    CMap c = kind == 0 ? cmap_pt(v[0], v[1], v[2], v[3]) : cmap_ee(v[0], v[1], v[2], v[3]);
-    bool valid = kind == 0 ? valid_pt(c.beta, c.gamma) : valid_ee(c.beta, c.gamma);
-    double l = signed_distance(c.e0, c.e1p, c.e2p);
-    double s = kind == 0 ? l * l : dot(c.e2p, c.e2p);
-    if (!(s < d2hat && valid)) return false;
-    const double b1 = barrier_d1(s, d2hat, kappa);
-    const double b2 = barrier_d2(s, d2hat, kappa);
-    // (u, v, w) = L x over the contact's vertices (the edge vectors of cmap_pt / cmap_ee)
-    const double Lpt[12] = {0, 1, -1, 0, 0, 0, -1, 1, 1, 0, -1, 0};
-    const double Lee[12] = {-1, 1, 0, 0, 0, 0, -1, 1, -1, 0, 1, 0};
-    const double* L = kind == 0 ? Lpt : Lee;
-    const d3 u = kind == 0 ? v[1] - v[2] : v[1] - v[0];
-    const d3 vv = v[3] - v[2];
-    const d3 w = kind == 0 ? v[0] - v[2] : v[2] - v[0];
-    double ge[9], He[81];
-    plane_dist2_derivs(u, vv, w, ge, He);
-    double gx[12], Hx[144];
-    for (int a = 0; a < 4; ++a)
-        for (int k = 0; k < 3; ++k) {
-            double acc = 0.0;
-            for (int e = 0; e < 3; ++e) acc += L[4 * e + a] * ge[3 * e + k];
-            gx[3 * a + k] = acc;
-        }
-    for (int a = 0; a < 4; ++a)
-        for (int k = 0; k < 3; ++k)
-            for (int b = 0; b < 4; ++b)
-                for (int m = 0; m < 3; ++m) {
-                    double acc = 0.0;
-                    for (int e = 0; e < 3; ++e)
-                        for (int f = 0; f < 3; ++f) acc += L[4 * e + a] * L[4 * f + b] * He[9 * (3 * e + k) + 3 * f + m];
-                    Hx[12 * (3 * a + k) + 3 * b + m] = acc * b1 + (gx[3 * a + k] * gx[3 * b + m]) * b2;
-                }
-    dense_body_map(kind, r, gx, b1, Hx, out);
-    return true;
-}
-
-// Full-IPC mode (psd = 3, beyond the reference): the barrier of the squared distance to the
-// closest feature pair (no validity gate), times the edge-edge mollifier for EE; the 12x12
-// Hessian in the points' coordinates projected onto the PSD cone, then mapped to the two
-// bodies like contact_terms_exact (same storage).
-__device__ bool contact_terms_full(int kind, const d3 v[4], const d3 r[4], double d2hat, double kappa,
-                                   double* __restrict__ out) {
-    const Feat f = kind == 0 ? pt_feature(v) : ee_feature(v);
-    double gs[12], Hx[144];
-    const double s = feature_dist2(kind, f, v, gs, Hx);
-    if (!(s < d2hat)) return false;
-    const double b0 = barrier(s, d2hat, kappa), b1 = barrier_d1(s, d2hat, kappa), b2 = barrier_d2(s, d2hat, kappa);
-    // mollifier m(c), c = |u x v|^2, u = x1 - x0, v = x3 - x2 (EE below eps only)
-    double m = 1.0, m1 = 0.0, m2 = 0.0, gc6[6], Hc6[36];
-    const double eps = kind == 1 ? ee_mollifier_eps(r) : 0.0;
-    const double c = kind == 1 ? cross2_derivs(v[1] - v[0], v[3] - v[2], gc6, Hc6) : 0.0;
-    const bool moll = kind == 1 && c < eps;
-    if (moll) {
-        m = mollifier(c, eps);
-        m1 = (2.0 - 2.0 * c / eps) / eps;
-        m2 = -2.0 / (eps * eps);
-    }
-    // point coefficients of u (points 0, 1) and v (points 2, 3)
-    const double Lc[2][4] = {{-1.0, 1.0, 0.0, 0.0}, {0.0, 0.0, -1.0, 1.0}};
-    double gx[12], gc[12];
-    for (int a = 0; a < 4; ++a)
-        for (int k = 0; k < 3; ++k) {
-            gc[3 * a + k] = moll ? Lc[0][a] * gc6[k] + Lc[1][a] * gc6[3 + k] : 0.0;
-            gx[3 * a + k] = m * b1 * gs[3 * a + k] + b0 * m1 * gc[3 * a + k];
-        }
-    for (int i = 0; i < 12; ++i)
-        for (int j = 0; j < 12; ++j) {
-            double h = m * (b1 * Hx[12 * i + j] + b2 * (gs[i] * gs[j]));
-            if (moll) {
-                const int a = i / 3, k = i % 3, bq = j / 3, mm = j % 3;
-                double hc = 0.0;
-                for (int e = 0; e < 2; ++e)
-                    for (int f2 = 0; f2 < 2; ++f2) hc += Lc[e][a] * Lc[f2][bq] * Hc6[6 * (3 * e + k) + 3 * f2 + mm];
-                h += b0 * (m2 * (gc[i] * gc[j]) + m1 * hc) + b1 * m1 * (gs[i] * gc[j] + gc[i] * gs[j]);
-            }
-            Hx[12 * i + j] = h;
-        }
-    psd_project12(Hx);
-    dense_body_map(kind, r, gx, 1.0, Hx, out);
-    return true;
-}
-
 // stage A: active flags over [PT | EE], plus ordering checks.
 // dn (nullable): the list sizes on the device, [nij, nij, npt, nee, nvg] (the arguments are
 // then upper bounds that only size the launch)
@@ -357,20 +237,45 @@ __device__ __forceinline__ int64_t active_key(const int32_t* __restrict__ pt, in
     return ((int64_t)(is_ee ? 1 : 0) << 32) | (int64_t)t5[2];
 }
 
-// stage C: one thread per active contact.  MODE: 1 the contact-space terms (psd 0 and 1),
-// 2 the exact Hessian, 3 full IPC; one kernel per mode, so that the contact-space path does
-// not carry the dense modes' register and stack footprint.
-template <int MODE>
+// Where stage C leaves what stage D needs of the active contacts, beside their terms.
+struct ContactOut {
+    double* __restrict__ cbuf;
+    uint8_t* __restrict__ swap;
+    uint8_t* __restrict__ hl_pt;
+    uint8_t* __restrict__ hl_ee;
+    uint8_t* __restrict__ pflag;
+    int64_t nij;
+    int64_t* __restrict__ pseg;
+};
+
+// The pair's flags and run of active contact e = candidate i, tuple t5.
+__device__ __forceinline__ void contact_bookkeeping(const ContactOut& O, const int32_t* __restrict__ pt, int64_t npt,
+                                                    const int32_t* __restrict__ ee,
+                                                    const int32_t* __restrict__ act, int64_t nact, int64_t e,
+                                                    bool is_ee, const int32_t* __restrict__ t5) {
+    const int64_t key = ((int64_t)(is_ee ? 1 : 0) << 32) | (int64_t)t5[2];
+    O.pflag[t5[2]] = 1;  // the body pair has an active contact (every writer stores 1)
+    // the run of this key in the sorted active list: [begin, end) of (type, pair) from
+    // the neighbours' keys (recomputed here from the lists)
+    const int64_t kprev = e > 0 ? active_key(pt, npt, ee, act[e - 1]) : -1;
+    const int64_t knext = e + 1 < nact ? active_key(pt, npt, ee, act[e + 1]) : -1;
+    int64_t* ps = O.pseg + 2 * ((is_ee ? O.nij : 0) + t5[2]);
+    if (kprev != key) ps[0] = e;
+    if (knext != key) ps[1] = e + 1;
+    O.swap[e] = t5[0] > t5[1] ? 1 : 0;  // body I is ij1 (PT second order)
+    if (is_ee)
+        O.hl_ee[t5[1]] = 1;
+    else
+        O.hl_pt[t5[1]] = 1;
+}
+
+// stage C: one thread per active contact (the contact-space terms, psd 0 and 1).
 __global__ __launch_bounds__(kBlock) void contact_kernel(AbdScene sc, AbdParams P, const double* __restrict__ x,
                                                           const int32_t* __restrict__ pt, int64_t npt,
                                                           const int32_t* __restrict__ ee,
                                                           const int32_t* __restrict__ act, int64_t nact,
                                                           const int64_t* __restrict__ dnact,
-                                                          const int64_t* __restrict__ dn,
-                                                          double* __restrict__ cbuf, int64_t* __restrict__ ckey,
-                                                          uint8_t* __restrict__ swap, uint8_t* __restrict__ hl_pt,
-                                                          uint8_t* __restrict__ hl_ee, uint8_t* __restrict__ pflag,
-                                                          int64_t nij, int64_t* __restrict__ pseg) {
+                                                          const int64_t* __restrict__ dn, ContactOut O) {
     const SceneView S = view_of(sc);
     if (dnact) nact = *dnact;
     if (dn) npt = dn[2];
@@ -386,29 +291,48 @@ __global__ __launch_bounds__(kBlock) void contact_kernel(AbdScene sc, AbdParams 
         d3 v[4], r[4];
         load4(x, vi, v);
         load4(sc.x0, vi, r);
-        if (MODE == 3)
-            contact_terms_full(is_ee ? 1 : 0, v, r, P.d2hat, P.kappa, cbuf + e * kDenseStride);
-        else if (MODE == 2)
-            contact_terms_exact(is_ee ? 1 : 0, v, r, P.d2hat, P.kappa, cbuf + e * kDenseStride);
-        else
-            contact_terms(is_ee ? 1 : 0, v, r, P.d2hat, P.kappa, P.psd, cbuf + e * kContactStride);
-        const int64_t key = ((int64_t)(is_ee ? 1 : 0) << 32) | (int64_t)t5[2];
-        ckey[e] = key;
-        pflag[t5[2]] = 1;  // the body pair has an active contact (every writer stores 1)
-        // the run of this key in the sorted active list: [begin, end) of (type, pair) from
-        // the neighbours' keys (recomputed here from the lists, not read from ckey)
-        const int64_t kprev = e > 0 ? active_key(pt, npt, ee, act[e - 1]) : -1;
-        const int64_t knext = e + 1 < nact ? active_key(pt, npt, ee, act[e + 1]) : -1;
-        int64_t* ps = pseg + 2 * ((is_ee ? nij : 0) + t5[2]);
-        if (kprev != key) ps[0] = e;
-        if (knext != key) ps[1] = e + 1;
-        swap[e] = t5[0] > t5[1] ? 1 : 0;  // body I is ij1 (PT second order)
-        if (is_ee)
-            hl_ee[t5[1]] = 1;
-        else
-            hl_pt[t5[1]] = 1;
+        contact_terms(is_ee ? 1 : 0, v, r, P.d2hat, P.kappa, P.psd, O.cbuf + e * kContactStride);
+        contact_bookkeeping(O, pt, npt, ee, act, nact, e, is_ee, t5);
     }
 }
+
+// stage C of the dense modes (MODE 2 the exact Hessian, 3 full IPC): one wave per active
+// contact (grid-stride), see abd_dense.h.
+template <int MODE>
+__global__ __launch_bounds__(kWave) void contact_dense_kernel(AbdScene sc, AbdParams P, const double* __restrict__ x,
+                                                              const int32_t* __restrict__ pt, int64_t npt,
+                                                              const int32_t* __restrict__ ee,
+                                                              const int32_t* __restrict__ act, int64_t nact,
+                                                              const int64_t* __restrict__ dnact,
+                                                              const int64_t* __restrict__ dn, ContactOut O) {
+    __shared__ DenseLds D;
+    const SceneView S = view_of(sc);
+    if (dnact) nact = *dnact;
+    if (dn) npt = dn[2];
+    const int lane = threadIdx.x;
+    for (int64_t e = blockIdx.x; e < nact; e += gridDim.x) {  // uniform over the wave
+        const int64_t i = act[e];
+        const bool is_ee = i >= npt;
+        const int32_t* t5 = is_ee ? ee + 5 * (i - npt) : pt + 5 * i;
+        int64_t vi[4];
+        if (is_ee)
+            fetch_ee_idx(S, t5, vi);
+        else
+            fetch_pt_idx(S, t5, vi);
+        d3 v[4], r[4];
+        load4(x, vi, v);
+        load4(sc.x0, vi, r);
+        if (MODE == 3)
+            wave_contact_full(lane, is_ee ? 1 : 0, v, r, P.d2hat, P.kappa, D, O.cbuf + e * kDenseStride);
+        else
+            wave_contact_exact(lane, is_ee ? 1 : 0, v, r, P.d2hat, P.kappa, D, O.cbuf + e * kDenseStride);
+        if (lane == 0) contact_bookkeeping(O, pt, npt, ee, act, nact, e, is_ee, t5);
+    }
+}
+
+// workgroups of the dense modes' stage C, at most: one wave each, at 8 KB of LDS the 16 or so
+// a CU holds at once fill the device's 256 CUs
+constexpr int64_t kDenseGrid = 4096;
 
 constexpr int kPairThreads = 576;  // one thread per entry of the 24x24 body-pair block
 constexpr int kPairBufStride = 2 * 144 + 24;  // diag(ij0), diag(ij1), g(ij0), g(ij1)
@@ -470,7 +394,7 @@ __global__ __launch_bounds__(kBlock) void pair_items_kernel(int64_t nij, const i
 
 // stage D2: one work item per workgroup (grid-stride over the *total items): the sums, in
 // contact order, of one chunk's contacts into part[item] (24x24 block in the pair's body
-// order [ij0 | ij1], then g), for contacts stored whole by contact_terms_exact / _full.
+// order [ij0 | ij1], then g), for contacts stored whole by contact_dense_kernel.
 __global__ __launch_bounds__(kPairThreads) void pair_partial_dense_kernel(const double* __restrict__ cbuf,
                                                                            const uint8_t* __restrict__ swap,
                                                                            const int64_t* __restrict__ idesc,
@@ -831,17 +755,6 @@ __global__ __launch_bounds__(kBlock) void pair_gh_kernel(int kind, AbdParams P, 
             v[k] = ld3(x4 + 12 * i + 3 * k);
             r[k] = ld3(r4 + 12 * i + 3 * k);
         }
-        if (P.psd >= 2) {
-            double* buf = scratch + i * kDenseStride;
-            bool act = P.psd == 3 ? contact_terms_full(kind, v, r, P.d2hat, P.kappa, buf)
-                                  : contact_terms_exact(kind, v, r, P.d2hat, P.kappa, buf);
-            active[i] = act ? 1 : 0;
-            for (int a = 0; a < 24; ++a) {
-                g24[24 * i + a] = act ? buf[kDenseGOff + a] : 0.0;
-                for (int c = 0; c < 24; ++c) H24[576 * i + 24 * a + c] = act ? buf[24 * a + c] : 0.0;
-            }
-            continue;
-        }
         double* buf = scratch + i * kContactStride;
         bool act = contact_terms(kind, v, r, P.d2hat, P.kappa, P.psd, buf);
         active[i] = act ? 1 : 0;
@@ -856,6 +769,36 @@ __global__ __launch_bounds__(kBlock) void pair_gh_kernel(int kind, AbdParams P, 
                     }
                 H24[576 * i + 24 * a + c] = h;
             }
+        }
+    }
+}
+
+// The same in the dense modes, one wave per contact.
+__global__ __launch_bounds__(kWave) void pair_gh_dense_kernel(int kind, AbdParams P, const double* __restrict__ x4,
+                                                              const double* __restrict__ r4, int64_t n,
+                                                              uint8_t* __restrict__ active, double* __restrict__ g24,
+                                                              double* __restrict__ H24,
+                                                              double* __restrict__ scratch) {
+    __shared__ DenseLds D;
+    const int lane = threadIdx.x;
+    for (int64_t i = blockIdx.x; i < n; i += gridDim.x) {
+        d3 v[4], r[4];
+        for (int k = 0; k < 4; ++k) {
+            v[k] = ld3(x4 + 12 * i + 3 * k);
+            r[k] = ld3(r4 + 12 * i + 3 * k);
+        }
+        double* buf = scratch + i * kDenseStride;
+        const bool act = P.psd == 3 ? wave_contact_full(lane, kind, v, r, P.d2hat, P.kappa, D, buf)
+                                    : wave_contact_exact(lane, kind, v, r, P.d2hat, P.kappa, D, buf);
+        dense_sync();
+        if (lane == 0) active[i] = act ? 1 : 0;
+        // every lane reads back what it wrote (entry q of the block and gradient is lane q % 64's)
+        for (int q = lane; q < kDenseStride; q += kWave) {
+            const double h = act ? buf[q] : 0.0;
+            if (q < kDenseGOff)
+                H24[576 * i + q] = h;
+            else
+                g24[24 * i + q - kDenseGOff] = h;
         }
     }
 }
@@ -1085,26 +1028,25 @@ int contact_gh(hipStream_t s, const AbdScene* sc, const AbdParams* P, const doub
     }
     if (nact > 0) {
         double* cbuf;
-        int64_t* ckey;
         uint8_t* swp;
-        if ((rc = arena_get(kSlotContact, (sizeof(double) * stride + sizeof(int64_t) + 1) * (size_t)nact,
-                            (void**)&cbuf)))
-            return rc;
-        ckey = reinterpret_cast<int64_t*>(cbuf + stride * nact);
-        swp = reinterpret_cast<uint8_t*>(ckey + nact);
+        if ((rc = arena_get(kSlotContact, (sizeof(double) * stride + 1) * (size_t)nact, (void**)&cbuf))) return rc;
+        swp = reinterpret_cast<uint8_t*>(cbuf + stride * nact);
         const double cbytes = 4.0 + 20 + 16 + 192 + 8.0 * stride + 9;
         int ph = prof_start(kProfContact, s, dn ? 1.0 : cbytes * nact);
         const int64_t* dnact = dn ? dev_nact : nullptr;
-        const dim3 cgrid(grid_for(nact, kBlock, 65535));
-        if (P->psd == 3)
-            hipLaunchKernelGGL(contact_kernel<3>, cgrid, dim3(kBlock), 0, s, *sc, *P, x, pt, npt, ee,
-                               (const int32_t*)act, nact, dnact, dn, cbuf, ckey, swp, hl_pt, hl_ee, pflag, nij, pseg);
-        else if (P->psd == 2)
-            hipLaunchKernelGGL(contact_kernel<2>, cgrid, dim3(kBlock), 0, s, *sc, *P, x, pt, npt, ee,
-                               (const int32_t*)act, nact, dnact, dn, cbuf, ckey, swp, hl_pt, hl_ee, pflag, nij, pseg);
-        else
-            hipLaunchKernelGGL(contact_kernel<1>, cgrid, dim3(kBlock), 0, s, *sc, *P, x, pt, npt, ee,
-                               (const int32_t*)act, nact, dnact, dn, cbuf, ckey, swp, hl_pt, hl_ee, pflag, nij, pseg);
+        const ContactOut O{cbuf, swp, hl_pt, hl_ee, pflag, nij, pseg};
+        if (dense) {
+            const dim3 dgrid((unsigned)std::min<int64_t>(nact, kDenseGrid));
+            if (P->psd == 3)
+                hipLaunchKernelGGL(contact_dense_kernel<3>, dgrid, dim3(kWave), 0, s, *sc, *P, x, pt, npt, ee,
+                                   (const int32_t*)act, nact, dnact, dn, O);
+            else
+                hipLaunchKernelGGL(contact_dense_kernel<2>, dgrid, dim3(kWave), 0, s, *sc, *P, x, pt, npt, ee,
+                                   (const int32_t*)act, nact, dnact, dn, O);
+        } else {
+            hipLaunchKernelGGL(contact_kernel, dim3(grid_for(nact, kBlock, 65535)), dim3(kBlock), 0, s, *sc, *P, x,
+                               pt, npt, ee, (const int32_t*)act, nact, dnact, dn, O);
+        }
         ABD_CHECK_LAUNCH();
         prof_stop(ph, s);
         if ((rc = prof_count_bytes(ph, s, dnact, cbytes, 0.0, 0.0, 0.0, true))) return rc;
@@ -1187,8 +1129,12 @@ int abd_pair_gh(abd_stream_t stream, int32_t kind, const AbdParams* P, const dou
     const int stride = P->psd >= 2 ? kDenseStride : kContactStride;
     int rc = arena_get(kSlotContact, sizeof(double) * stride * (size_t)n, (void**)&scratch);
     if (rc) return rc;
-    hipLaunchKernelGGL(pair_gh_kernel, dim3(grid_for(n)), dim3(kBlock), 0, to_stream(stream), kind, *P, x4, r4, n,
-                       active, g24, H24, scratch);
+    if (P->psd >= 2)
+        hipLaunchKernelGGL(pair_gh_dense_kernel, dim3((unsigned)std::min<int64_t>(n, kDenseGrid)), dim3(kWave), 0,
+                           to_stream(stream), kind, *P, x4, r4, n, active, g24, H24, scratch);
+    else
+        hipLaunchKernelGGL(pair_gh_kernel, dim3(grid_for(n)), dim3(kBlock), 0, to_stream(stream), kind, *P, x4, r4, n,
+                           active, g24, H24, scratch);
     ABD_CHECK_LAUNCH();
     return ABD_OK;
 }
