@@ -732,11 +732,14 @@ __global__ __launch_bounds__(kBlock) void body_finalize_kernel(AbdScene sc, AbdP
 }
 
 // the gh stage's flags and counters: the ordering flag, n8 bytes at a8, n64 int64 at a64
+// (nact_dev, nullable: an active count that no later stage writes)
 __global__ void gh_zero_kernel(int* __restrict__ err, uint8_t* __restrict__ a8, int64_t n8,
-                               int64_t* __restrict__ a64, int64_t n64, int64_t* __restrict__ b64, int64_t nb64) {
+                               int64_t* __restrict__ a64, int64_t n64, int64_t* __restrict__ b64, int64_t nb64,
+                               int64_t* __restrict__ nact_dev) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < nb64) b64[i] = 0;
     if (i == 0) {
+        if (nact_dev) *nact_dev = 0;
         err[0] = 0;
         err[1] = err[2] = 0;  // stage D's counters of full and partial chunks
     }
@@ -966,7 +969,7 @@ int contact_gh(hipStream_t s, const AbdScene* sc, const AbdParams* P, const doub
         const int64_t n8 = 2 * (int64_t)nb + nij, n64 = 4 * nij;
         const int64_t nz = std::max(std::max(n8, n64), nblk);
         hipLaunchKernelGGL(gh_zero_kernel, dim3(grid_for(nz, kBlock, INT32_MAX)), dim3(kBlock), 0, s, err, hl_pt, n8,
-                           pseg, n64, bcnt, nblk);
+                           pseg, n64, bcnt, nblk, n > 0 ? nullptr : n_active_dev);
         ABD_CHECK_LAUNCH();
     }
     int64_t nact = 0;
@@ -990,7 +993,6 @@ int contact_gh(hipStream_t s, const AbdScene* sc, const AbdParams* P, const doub
             dev_nact = boff + nblk;
         }
     }
-    if (!dev_nact && n_active_dev && (rc = zero_fill(s, n_active_dev, sizeof(int64_t)))) return rc;
     const bool dense = P->psd >= 2;
     const int stride = dense ? kDenseStride : kContactStride;
     if (dn) {

@@ -971,19 +971,15 @@ int keep_from_superset(hipStream_t s, const AbdScene* sc, const KeepInput& in, c
         hipLaunchKernelGGL(keep_count_kernel, dim3((unsigned)nall), dim3(kBlock), 0, s, A);
         ABD_CHECK_LAUNCH();
     }
-    ScanSeg sg[kKeepLists];
-    int nseg = 0;
+    ScanSeg sg[kKeepLists];  // an empty list's scan only writes its total, 0
     for (int k = 0; k < kKeepLists; ++k)
-        if (n[k] > 0) sg[nseg++] = ScanSeg{A.bcnt[k], A.boff[k], nblk[k], A.boff[k] + nblk[k], dcount + k};
-    if ((rc = scan_exclusive_i64_multi(s, sg, nseg))) return rc;
+        sg[k] = ScanSeg{A.bcnt[k], A.boff[k], nblk[k], A.boff[k] + nblk[k], dcount + k};
+    if ((rc = scan_exclusive_i64_multi(s, sg, kKeepLists))) return rc;
     if (nall > 0) {
         hipLaunchKernelGGL(keep_write_kernel, dim3((unsigned)nall), dim3(kBlock), 0, s, A, 0, kKeepLists);
         ABD_CHECK_LAUNCH();
     }
     prof_stop(ph, s);
-    // an empty list's total is 0 (its scan segment is skipped)
-    for (int k = 0; k < kKeepLists; ++k)
-        if (n[k] == 0 && (rc = zero_fill(s, dcount + k, sizeof(int64_t)))) return rc;
     if (hcount) {
         ABD_CHECK(hipMemcpyAsync(hcount, dcount, kKeepLists * sizeof(int64_t), hipMemcpyDeviceToHost, s));
         if (sync) ABD_CHECK(hipStreamSynchronize(s));

@@ -426,7 +426,7 @@ __global__ void update_q_scenes_kernel(int nb, const int32_t* __restrict__ body_
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= 12 * nb) return;
     const int b = i / 12, r = i % 12;
-    const double al = alpha[body_scene[b]];
+    const double al = alpha[body_scene ? body_scene[b] : 0];
     // a scene that does not move keeps its state bit for bit, whatever dq holds
     double* out = r < 3 ? p_out + 3 * b + r : A_out + 9 * b + r - 3;
     double* out2 = r < 3 ? (p_out2 ? p_out2 + 3 * b + r : nullptr) : (A_out2 ? A_out2 + 9 * b + r - 3 : nullptr);
@@ -477,7 +477,7 @@ int update_q_scenes_dual(hipStream_t s, const AbdScene* sc, const double* A, con
     const int nb = sc->n_bodies;
     if (nb == 0) return ABD_OK;
     hipLaunchKernelGGL(update_q_scenes_kernel, dim3(grid_for(12 * (int64_t)nb)), dim3(kBlock), 0, s, nb,
-                       sc->body_scene, A, p, dq, alpha, A_out, p_out, A_out2, p_out2);
+                       sc->n_scenes > 1 ? sc->body_scene : nullptr, A, p, dq, alpha, A_out, p_out, A_out2, p_out2);
     ABD_CHECK_LAUNCH();
     return ABD_OK;
 }

@@ -155,7 +155,7 @@ int reduce_plan(hipStream_t s, const AbdScene* sc, const AbdParams* P, int S, co
                 const int64_t* dn = nullptr);
 // Per-scene TOI (abd_scene_toi; S = 1: the whole system as one scene) with an optional plan;
 // active (nullable, [S]): scenes whose TOI is wanted, the others report 1 unevaluated.
-// Per-scene dot products a.b and c.d (seg_dot2_kernel's) that the TOI's final per-scene pass computes
+// Per-scene dot products a.b and c.d (each seg_dot_kernel's) that the TOI's final per-scene pass computes
 // after the scene's TOI when out1 is set (the driver's q.g and g.g, one launch less).
 struct SceneDots {
     const int32_t* sboff = nullptr;
@@ -176,9 +176,6 @@ __host__ __device__ inline double first_step_length(double t) {
     if (t < 1.0) t *= 0.9;
     return t;
 }
-// out1 = a . b and out2 = c . d per scene (S = 1: over all 12 nb rows), one launch
-int dots(hipStream_t s, const AbdScene* sc, int S, const double* a, const double* b, const double* c,
-         const double* d, double* out1, double* out2);
 // The end of a step: x_out = x(q - alpha dq), the arithmetic of update_q + project_vertices
 // with alpha_host (alpha_dev, active null), or of update_q_scenes + project_vertices with
 // alpha_dev [n_scenes] or alpha_host for the scenes with active[s] (0 for the others).  With
@@ -194,6 +191,8 @@ int contact_energy(hipStream_t s, const AbdScene* sc, const AbdParams* P, int S,
 // A_out2, p_out2 are given).
 int update_q_dual(hipStream_t s, int nb, const double* A, const double* p, const double* dq, double alpha,
                   double* A_out, double* p_out, double* A_out2, double* p_out2);
+// Whether abd_bsr_solve of nb bodies waits for the device between its launches.
+bool solve_waits(int32_t method, int nb);
 int update_q_scenes_dual(hipStream_t s, const AbdScene* sc, const double* A, const double* p, const double* dq,
                          const double* alpha, double* A_out, double* p_out, double* A_out2, double* p_out2);
 // Collision set from a superset of it (keep_from_superset, abd_cull.hip): the superset's

@@ -412,7 +412,7 @@ __global__ __launch_bounds__(kRedThreads) void toi_final_kernel(const int64_t* _
         out[s] = r;
         if (alpha) alpha[s] = !active || active[s] ? first_step_length(r) : -1.0;
     }
-    if (D.out1) {  // uniform: seg_dot2_kernel's sums of this scene
+    if (D.out1) {  // uniform: seg_dot_kernel's sums of this scene
         const int64_t i0 = D.sboff ? 12 * (int64_t)D.sboff[s] : 0, i1 = D.sboff ? 12 * (int64_t)D.sboff[s + 1] : D.n;
         double acc1 = 0.0, acc2 = 0.0;
         for (int64_t i = i0 + threadIdx.x; i < i1; i += blockDim.x) {
@@ -439,29 +439,6 @@ __global__ __launch_bounds__(kRedThreads) void seg_dot_kernel(const int32_t* __r
     for (int64_t i = i0 + threadIdx.x; i < i1; i += blockDim.x) acc += a[i] * b[i];
     const double r = block_sum_fast(acc, sh);
     if (threadIdx.x == 0) out[s] = r;
-}
-
-// out1[s] = a . b and out2[s] = c . d over the rows of scene s, each bit-identical to its
-// seg_dot_kernel
-__global__ __launch_bounds__(kRedThreads) void seg_dot2_kernel(const int32_t* __restrict__ sboff, int64_t n,
-                                                               const double* __restrict__ a,
-                                                               const double* __restrict__ b,
-                                                               const double* __restrict__ c,
-                                                               const double* __restrict__ d,
-                                                               double* __restrict__ out1, double* __restrict__ out2) {
-    __shared__ double sh[34];
-    const int s = blockIdx.x;
-    const int64_t i0 = sboff ? 12 * (int64_t)sboff[s] : 0, i1 = sboff ? 12 * (int64_t)sboff[s + 1] : n;
-    double acc1 = 0.0, acc2 = 0.0;
-    for (int64_t i = i0 + threadIdx.x; i < i1; i += blockDim.x) {
-        acc1 += a[i] * b[i];
-        acc2 += c[i] * d[i];
-    }
-    block_sum2_fast(acc1, acc2, sh);
-    if (threadIdx.x == 0) {
-        out1[s] = acc1;
-        out2[s] = acc2;
-    }
 }
 
 // orthogonal_energy.py:25-51 summed over the bodies of each scene (one workgroup per scene)
@@ -757,14 +734,6 @@ int scene_toi(hipStream_t s, const AbdScene* sc, const AbdParams* P, int S, cons
     if ((npt && !pt) || (nee && !ee) || (nvg && !vg)) return ABD_ERR_ARG;
     const Lists L = contact_lists(*P, pt, npt, ee, nee, vg, nvg, dn, vids);  // abd.py:288-299
     return toi_reduce(s, *sc, *P, S, x_t0, x_t1, L, plan, toi, active, nullptr, first_alpha, dots);
-}
-
-int dots(hipStream_t s, const AbdScene* sc, int S, const double* a, const double* b, const double* c,
-         const double* d, double* out1, double* out2) {
-    hipLaunchKernelGGL(seg_dot2_kernel, dim3(S), dim3(kRedThreads), 0, s, S > 1 ? sc->scene_boff : nullptr,
-                       12 * (int64_t)sc->n_bodies, a, b, c, d, out1, out2);
-    ABD_CHECK_LAUNCH();
-    return ABD_OK;
 }
 
 // ------------------------------------------------- allocation-free TOI scratch

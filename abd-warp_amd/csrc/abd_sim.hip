@@ -1,11 +1,10 @@
 // abd_sim.hip — native frame driver: AffineBodySimulator.step (abd.py:212-276)
 // run from C++ over the stage entry points of this library.  The candidate lists a
 // Newton iteration filters from the candidate superset keep their sizes on the device
-// (every launch sized by the superset's, which bound them), so an iteration waits for
-// the device once: the plain driver for the scalars its line search and convergence
-// test branch on (time of impact, q.g, g.g, the first trial's energies), the batched
-// driver, whose line searches and convergence tests run on the device, for the lists'
-// sizes and the number of scenes still iterating.  The arithmetic is the same sequence
+// (every launch sized by the superset's, which bound them), and line searches and
+// convergence tests run on the device, so an iteration is one recorded graph (or its
+// launches) and one wait, for the lists' sizes and the number of scenes still iterating.
+// One scene is a batch of one: the same iteration.  The arithmetic is the same sequence
 // of kernels as the Python mirror, so both give identical states.
 #include <hip/hip_runtime.h>
 
@@ -98,6 +97,9 @@ struct CandSet {
     }
 };
 
+// words of a recorded iteration's key (graph_key)
+constexpr int kKeyWords = 5;
+
 struct Sim {
     Arena arena;  // the stages' scratch during this simulator's calls
     AbdScene sc;
@@ -120,40 +122,37 @@ struct Sim {
     bool col_fresh = false;  // col (with its structure) is the collision set at the current x
     DevBuf<int32_t> row_ptr, cols, slots;
     DevBuf<double> blocks;
-    DevBuf<double> scal;  // [0] E contact, [1] E inertia, [2] toi, [3] dot, [4] resid
+    DevBuf<double> scal;        // the residual of hessian_solve
     DevBuf<int32_t> iters;
     DevBuf<int64_t> dcount;     // culling totals gathered for one read-back
     DevBuf<int64_t> cnt;        // device sizes of the filtered sets (kCnt*), read back per iteration
     int64_t* hcnt = nullptr;    // pinned copy of cnt
-    int64_t gen = 0;            // the current step's number: the range test's flag value
-    double* host = nullptr;     // pinned scalars
     int64_t* hcount = nullptr;  // pinned list counts
     int64_t stats[10] = {};
-    // independent scenes (n_scenes > 1): per-scene device values and pinned host copies
+    // per-scene device values (one scene: a batch of one)
     int ns = 1, max_scene_bodies = 0;
     DevBuf<double> sv;          // [kSv][ns]
-    // the batched driver's Newton / line-search state on the device (ls_decide_kernel): rows
+    // the Newton / line-search state of every scene on the device (ls_decide_kernel): rows
     // of the current iteration (lcur) and of the next, so that a step redone from a
     // recomputed swept set repeats the same decisions
     DevBuf<uint8_t> lsflag;     // [kLfRows][ns]
     DevBuf<double> lsval;       // [kLvRows][ns]
     DevBuf<int32_t> lsit;       // [2][ns] Newton iterations of each scene in this frame
-    // the batched Newton iteration recorded as a HIP graph and replayed while the launches it
+    // the Newton iteration recorded as a HIP graph and replayed while the launches it
     // holds stay valid (GraphKey); a key met for the first time runs eagerly, the second
     // time it is recorded
     bool graphs = true;
+    bool solve_waits = false;  // the solver reads back between its launches: never recorded
     int64_t gcount[3] = {};  // iterations replayed, recorded (then replayed), launched eagerly
     hipGraphExec_t gexec = nullptr;
     hipStream_t cap_stream = nullptr;  // the recording stream (the caller's may be the null stream)
-    uint64_t gkey[4] = {}, gseen[4] = {}, gfailed[4] = {};
-    int64_t sup_gen = 0;  // advanced whenever the candidate superset is culled anew
+    uint64_t gkey[kKeyWords] = {}, gseen[kKeyWords] = {}, gfailed[kKeyWords] = {};
     int32_t* hiters = nullptr;  // pinned [ns]: the iteration counts read back at a frame's end
     std::vector<int32_t> scene_it;  // Newton iterations of each scene in the last frame
     // line-search candidates evaluated together: states, vertices and per-candidate scalars
     DevBuf<double> cand_E;          // [kLsSpec][2 ns] trial energies
     DevBuf<double> cand_alpha;      // [kLsSpec][ns]
     DevBuf<int64_t> plan;           // reduction plan of the swept candidate set (CCD + line search)
-    double* hcand = nullptr;        // pinned [kLsSpec][ns] alphas, then [kLsSpec][2 ns] energies
 };
 
 // Step lengths evaluated per line-search pass after the first: the trials alpha,
@@ -181,7 +180,8 @@ enum { kSvEc = 0, kSvEi, kSvToi, kSvQtg, kSvGtg, kSvAlpha, kSv };
 // stage, the flag of a step leaving the superset's ranges, the batched line search's
 // outputs (scenes iterating after this iteration, scenes still searching, trials of the
 // second pass and of the next, the solver's iterations summed over the iterating scenes);
-// the host's copy holds a staging row for the exact sizes of a culled collision set after it
+// the host's copy holds staging rows for the exact sizes of a culled collision set and of
+// the superset after it
 enum {
     kCntCol = 0,
     kCntSw = 8,
@@ -192,7 +192,8 @@ enum {
     kCntK1 = 20,
     kCntK2 = 21,
     kCntSolver = 22,
-    kCntLen = 24
+    kCntSup = 24,  // the candidate superset's sizes
+    kCntLen = 32
 };
 // rows of Sim::lsflag (iterating: the current and the next iteration's; searching) and of
 // Sim::lsval (E0: the current and the next; the accepted trial's energy); the next
@@ -200,12 +201,6 @@ enum {
 // (ls_commit_kernel)
 enum { kLfNewton = 0, kLfSearch = 2, kLfRows };
 enum { kLvE0 = 0, kLvE1 = 2, kLvRows };
-
-int get_scalars(hipStream_t s, Sim& S, int first, int count) {
-    ABD_CHECK(hipMemcpyAsync(S.host + first, S.scal.p + first, sizeof(double) * count, hipMemcpyDeviceToHost, s));
-    ABD_CHECK(hipStreamSynchronize(s));
-    return ABD_OK;
-}
 
 // The EE, PT and VG candidate lists of one set of boxes (culling.py:32-76), culled side
 // by side so that their counts come back in two host synchronizations instead of five;
@@ -378,6 +373,15 @@ constexpr double kSkinOverDhat = 30.0;
 // the step's end (step_end).
 int swept_set_launch(hipStream_t s, Sim& S);
 
+// n rounded up to a multiple of an eighth of its power of two (at least 64; 0 stays 0: an
+// empty list is launched over nothing).
+int64_t size_bound(int64_t n) {
+    if (n <= 64) return n > 0 ? 64 : 0;
+    int64_t step = 8;
+    while (step * 16 <= n) step *= 2;
+    return (n + step - 1) / step * step;
+}
+
 // The superset culled anew around the current step (its ends widened by the skin; host
 // synchronizations for the culling counts), then the swept set filtered from it.
 int swept_set_recull(hipStream_t s, Sim& S) {
@@ -386,7 +390,6 @@ int swept_set_recull(hipStream_t s, Sim& S) {
     const int64_t n3 = 3 * (int64_t)S.nv;
     int rc;
     S.sup_valid = false;
-    ++S.sup_gen;
     if ((rc = vertex_ranges(s, n3, st.x, st.xk, kSkinOverDhat * S.P.dhat, S.vlo.p, S.vhi.p))) return rc;
     if ((rc = swept_boxes(s, &S.sc, -1, S.vlo.p, S.vhi.p, dh, S.sbody.lo.p, S.sbody.hi.p))) return rc;
     // with the (j, i) order: the swept set (and the collision sets after it) keep it
@@ -395,7 +398,6 @@ int swept_set_recull(hipStream_t s, Sim& S) {
     if ((rc = swept_boxes(s, &S.sc, ABD_KIND_EDGE, S.vlo.p, S.vhi.p, dh, S.sedge.lo.p, S.sedge.hi.p))) return rc;
     if ((rc = swept_boxes(s, &S.sc, ABD_KIND_POINT, S.vlo.p, S.vhi.p, S.P.dhat, S.spt.lo.p, S.spt.hi.p))) return rc;
     if ((rc = cull_lists(s, S, S.sup, S.sbody, S.spt, S.stri, S.sedge))) return rc;
-    S.sup.exact = true;
     // the tuples' vertex ids, read by the filters and, carried into the swept set, by the CCD
     // and the line search (the superset serves many steps)
     if ((rc = S.sup.ptv.reserve(4 * (size_t)S.sup.npt + 4))) return rc;
@@ -403,6 +405,21 @@ int swept_set_recull(hipStream_t s, Sim& S) {
     if ((rc = cand_vertex_ids(s, &S.sc, 0, S.sup.ptl.p, S.sup.npt, S.sup.ptv.p))) return rc;
     if ((rc = cand_vertex_ids(s, &S.sc, 1, S.sup.eel.p, S.sup.nee, S.sup.eev.p))) return rc;
     S.sup.vids = true;
+    // its exact sizes to the device; from here the counts are bounds in steps of an eighth,
+    // which size the launches and buffers of the sets filtered from it, so that an iteration
+    // recorded for one superset replays for the next of about its size
+    int64_t* h = S.hcnt + kCntLen + 8;  // rewritten only after the next recull's synchronizations
+    h[0] = h[1] = S.sup.nij;
+    h[2] = S.sup.npt;
+    h[3] = S.sup.nee;
+    h[4] = S.sup.nvg;
+    ABD_CHECK(hipMemcpyAsync(S.cnt.p + kCntSup, h, 5 * sizeof(int64_t), hipMemcpyHostToDevice, s));
+    S.sup.nij = size_bound(S.sup.nij);
+    S.sup.npt = size_bound(S.sup.npt);
+    S.sup.nee = size_bound(S.sup.nee);
+    S.sup.nvg = size_bound(S.sup.nvg);
+    S.sup.dn = S.cnt.p + kCntSup;
+    S.sup.exact = false;
     S.sup_valid = true;
     return swept_set_launch(s, S);
 }
@@ -441,20 +458,6 @@ int swept_set_launch(hipStream_t s, Sim& S) {
     return ABD_OK;
 }
 
-// The end of the step (xk = x(q - dq) for the scenes in `active`, or every scene), with the
-// range test of both ends against the superset's ranges when there is a superset.
-int step_end(hipStream_t s, Sim& S, const uint8_t* active) {
-    const AbdSimState& st = S.st;
-    ++S.gen;
-    return project_step(s, &S.sc, st.A, st.p, st.dq, nullptr, 1.0, active, st.xk, st.x,
-                        S.sup_valid ? S.vlo.p : nullptr, S.sup_valid ? S.vhi.p : nullptr, S.cnt.p + kCntRange,
-                        S.gen);
-}
-
-// After the iteration's synchronization: true when the step left the superset's ranges, so
-// that the swept set must be recomputed.
-bool swept_left_ranges(const Sim& S) { return S.hcnt[kCntRange] == S.gen; }
-
 // The lists' sizes for the statistics (after the iteration's synchronization).
 void count_stats(Sim& S) {
     const int64_t* h = S.hcnt;
@@ -466,173 +469,14 @@ void count_stats(Sim& S) {
     S.stats[9] += h[kCntSw + 3];
 }
 
-// abd.py:133-141 at a frame's start (alpha = 0: xk = x), which also gives the first Newton
-// iteration's collision set with its structure
-int compute_energy(hipStream_t s, Sim& S, double alpha, double* E) {
-    int rc;
-    const AbdSimState& st = S.st;
-    if ((rc = abd_update_q(s, S.nb, st.A, st.p, st.dq, alpha, st.Ak, st.pk))) return rc;
-    if ((rc = abd_project_vertices(s, &S.sc, st.Ak, st.pk, st.xk))) return rc;
-    if ((rc = collision_at_frame_start(s, S, st.xk))) return rc;
-    S.col_fresh = alpha == 0.0;
-    const CandSet& C = S.col;
-    if ((rc = contact_energy(s, &S.sc, &S.P, 1, st.xk, C.ptl.p, C.npt, C.eel.p, C.nee, C.vgl.p, C.nvg, C.counts(),
-                             S.scal.p)))
-        return rc;
-    if ((rc = abd_inertia_energy(s, &S.sc, &S.P, st.Ak, st.pk, st.A0, st.p0, st.Adot, st.pdot, S.scal.p + 1)))
-        return rc;
-    if ((rc = get_scalars(s, S, 0, 2))) return rc;
-    S.stats[5] += 1;
-    *E = S.host[0] + S.host[1];
-    return ABD_OK;
-}
-
-// abd.py:133-141 inside the line search, for K trial step lengths at once (energies to
-// E[K], one host round trip): the energy at q - alpha dq over the swept candidate set of
-// this iteration (swept_set_launch), without re-culling
-int line_energy_multi(hipStream_t s, Sim& S, const double* alphas, int K, double* E) {
-    int rc;
-    const AbdSimState& st = S.st;
-    double* ha = S.hcand;
-    double* he = S.hcand + kLsSpec;
-    for (int k = 0; k < K; ++k) ha[k] = alphas[k];
-    ABD_CHECK(hipMemcpyAsync(S.cand_alpha.p, ha, sizeof(double) * K, hipMemcpyHostToDevice, s));
-    if ((rc = line_trials(s, &S.sc, &S.P, 1, K, S.cand_alpha.p, st.A, st.p, st.dq, st.A0, st.p0, st.Adot, st.pdot,
-                          S.sw.ptl.p, S.sw.npt, S.sw.eel.p, S.sw.nee, S.sw.vgl.p, S.sw.nvg, S.plan.p, S.cand_E.p,
-                          S.sw.counts(), S.sw.vertex_ids())))
-        return rc;
-    ABD_CHECK(hipMemcpyAsync(he, S.cand_E.p, sizeof(double) * 2 * K, hipMemcpyDeviceToHost, s));
-    ABD_CHECK(hipStreamSynchronize(s));
-    for (int k = 0; k < K; ++k) E[k] = he[2 * k] + he[2 * k + 1];
-    S.stats[5] += K;
-    return ABD_OK;
-}
-
-// abd.py:278-303 and the line search's first trial, launched only, then one read-back: the
-// step's swept set (ccd: xk = the end of the full step), its reduction plan, the TOI into
-// scal[2], q.g and g.g, the first trial's energies (its step length from the TOI, on the
-// device), the solver's iteration count and the sets' sizes.  A step that left the
-// superset's ranges is recomputed from a superset culled around it.
-int ccd_and_first_trial(hipStream_t s, Sim& S) {
-    int rc;
-    const AbdSimState& st = S.st;
-    const int nb = S.nb;
-    for (int attempt = 0;; ++attempt) {
-        if ((rc = attempt == 0 ? swept_set_launch(s, S) : swept_set_recull(s, S))) return rc;
-        const CandSet& W = S.sw;
-        // one reduction plan of the swept set serves the TOI and every line-search trial
-        if ((rc = reduce_plan(s, &S.sc, &S.P, 1, W.ptl.p, W.npt, W.eel.p, W.nee, W.vgl.p, W.nvg, S.plan.p,
-                              W.counts())))
-            return rc;
-        // the TOI, and from it on the device the first trial's step length
-        if ((rc = scene_toi(s, &S.sc, &S.P, 1, st.x, st.xk, W.ptl.p, W.npt, W.eel.p, W.nee, W.vgl.p, W.nvg,
-                            S.plan.p, S.scal.p + 2, nullptr, W.counts(), S.cand_alpha.p, W.vertex_ids())))
-            return rc;
-        // q.g (abd.py:148) and g.g (abd.py:265): g and dq are final here
-        if ((rc = dots(s, &S.sc, 1, st.dq, st.g, st.g, st.g, S.scal.p + 3, S.scal.p + 5))) return rc;
-        if ((rc = line_trials(s, &S.sc, &S.P, 1, 1, S.cand_alpha.p, st.A, st.p, st.dq, st.A0, st.p0, st.Adot,
-                              st.pdot, W.ptl.p, W.npt, W.eel.p, W.nee, W.vgl.p, W.nvg, S.plan.p, S.cand_E.p,
-                              W.counts(), W.vertex_ids())))
-            return rc;
-        ABD_CHECK(hipMemcpyAsync(S.hcand + kLsSpec, S.cand_E.p, sizeof(double) * 2, hipMemcpyDeviceToHost, s));
-        ABD_CHECK(hipMemcpyAsync(S.host + 6, S.iters.p, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-        ABD_CHECK(hipMemcpyAsync(S.hcnt, S.cnt.p, kCntLen * sizeof(int64_t), hipMemcpyDeviceToHost, s));
-        if ((rc = get_scalars(s, S, 2, 4))) return rc;
-        // a recomputed swept set lies inside the superset culled around this very step
-        if (attempt > 0 || !swept_left_ranges(S)) return ABD_OK;
-    }
-}
-
-int step(hipStream_t s, Sim& S) {
-    const AbdSimState& st = S.st;
-    const AbdParams& P = S.P;
-    const int nb = S.nb;
-    int rc;
-    // q_gets_q0 (abd.py:124-128)
-    ABD_CHECK(hipMemcpyAsync(st.A, st.A0, 72 * (size_t)nb, hipMemcpyDeviceToDevice, s));
-    ABD_CHECK(hipMemcpyAsync(st.p, st.p0, 24 * (size_t)nb, hipMemcpyDeviceToDevice, s));
-    ABD_CHECK(hipMemcpyAsync(st.Ak, st.A0, 72 * (size_t)nb, hipMemcpyDeviceToDevice, s));
-    ABD_CHECK(hipMemcpyAsync(st.pk, st.p0, 24 * (size_t)nb, hipMemcpyDeviceToDevice, s));
-    double E0;
-    S.sw_valid = false;  // a frame starts from the state the caller holds
-    if ((rc = compute_energy(s, S, 0.0, &E0))) return rc;
-    int it = 0;
-    for (;;) {
-        // (Ak, pk) = (A, p) here: the collision set is culled on x
-        if ((rc = abd_project_vertices(s, &S.sc, st.A, st.p, st.x))) return rc;
-        if (S.col_fresh)
-            S.col_fresh = false;  // the frame-start energy's set: the same positions
-        else if ((rc = S.sw_valid ? collision_from_swept(s, S, st.x) : collision_at_frame_start(s, S, st.x)))
-            return rc;
-        const size_t nslot = nb + 2 * (size_t)S.col.nij;
-        if ((rc = S.blocks.reserve(nslot * 16 * 9))) return rc;
-        ABD_CHECK(hipMemsetAsync(S.blocks.p, 0, sizeof(double) * nslot * 16 * 9, s));
-        // g: overwritten by the inertia gradient (abd.py:236-237 zeroes it first)
-        if ((rc = inertia_gh(s, &S.sc, &P, st.A, st.p, st.A0, st.p0, st.Adot, st.pdot, st.g, S.blocks.p)))
-            return rc;
-        const CandSet& C = S.col;
-        const GhLists L{C.ptl.p, C.npt, C.eel.p, C.nee, C.vgl.p, C.nvg, C.nij, C.counts()};
-        if ((rc = contact_gh(s, &S.sc, &P, st.x, L, S.row_ptr.p, S.slots.p, st.g, S.blocks.p, nullptr, nullptr,
-                             S.cnt.p + kCntNact)))
-            return rc;
-        if ((rc = abd_bsr_solve(s, P.solver, nb, S.row_ptr.p, S.cols.p, S.slots.p, S.blocks.p, st.g, st.dq,
-                                P.solver_tol, P.solver_maxiter, 10, S.iters.p, nullptr)))
-            return rc;
-        // CCD over the full step (xk = its end) and the first trial (abd.py:278-303)
-        if ((rc = step_end(s, S, nullptr))) return rc;
-        if ((rc = ccd_and_first_trial(s, S))) return rc;
-        count_stats(S);
-        S.stats[5] += 1;
-        const double qTg = S.host[3], gTg = S.host[5];
-        int32_t sit;
-        memcpy(&sit, S.host + 6, sizeof(int32_t));
-        S.stats[6] += sit;
-        // abd.py:146-160 line search (Armijo test as written)
-        double alpha = first_step_length(S.host[2]), E1 = 0.0;
-        for (int pass = 0;; ++pass) {
-            // the first trial alone (usually accepted), then the rest down to alpha_min
-            const int K = pass == 0 ? 1 : trials_to_floor(alpha, P.alpha_min);
-            double trial[kLsSpec], Ek[kLsSpec];
-            for (int k = 0; k < K; ++k) trial[k] = k == 0 ? alpha : trial[k - 1] * 0.5;
-            if (pass == 0)
-                Ek[0] = S.hcand[kLsSpec] + S.hcand[kLsSpec + 1];
-            else if ((rc = line_energy_multi(s, S, trial, K, Ek)))
-                return rc;
-            int acc = -1;
-            for (int k = 0; k < K && acc < 0; ++k) {
-                const bool wolfe = Ek[k] < E0 + P.c1 * trial[k] * qTg;
-                if (wolfe || trial[k] < P.alpha_min) acc = k;
-            }
-            if (acc >= 0) {
-                alpha = trial[acc];
-                E1 = Ek[acc];
-                break;
-            }
-            alpha = trial[K - 1] * 0.5;
-        }
-        E0 = E1;
-        // q and (Ak, pk) = q - alpha dq, the accepted trial
-        if ((rc = update_q_dual(s, nb, st.A, st.p, st.dq, alpha, st.A, st.p, st.Ak, st.pk))) return rc;
-        ++it;
-        if (gTg < P.tol || it >= P.max_iter) break;
-    }
-    if ((rc = abd_update_q0qdot(s, nb, P.dt, st.A, st.p, st.A0, st.p0, st.Adot, st.pdot))) return rc;
-    if ((rc = abd_project_vertices(s, &S.sc, st.A0, st.p0, st.x_view))) return rc;
-    S.stats[0] += it;
-    S.stats[7] += 1;
-    S.scene_it.assign(1, it);
-    return ABD_OK;
-}
-
 // ---------------------------------------------------------------- batched
-// Many independent scenes advanced together: one launch per stage covers every
-// scene, and each scene keeps its own Newton loop, step length and stopping
-// test, exactly the per-scene sequence of step() above.  A scene that has
-// converged is masked out of the solve and takes zero-length steps.  The line
-// searches and the stopping tests run on the device (ls_decide_kernel), so an
-// iteration waits for the device once.
+// The independent scenes of a batch (or the one scene) advanced together: one launch per
+// stage covers every scene, and each scene keeps its own Newton loop, step length and
+// stopping test (abd.py:212-276).  A scene that has converged is masked out of the solve
+// and takes zero-length steps.  The line searches and the stopping tests run on the
+// device (ls_decide_kernel), so an iteration waits for the device once.
 
-// The device rows of the batched Newton / line-search state for the current iteration.
+// The device rows of the Newton / line-search state for the current iteration.
 struct LsDev {
     int ns;
     const uint8_t* newton;  // scenes iterating (the solver's mask of this iteration)
@@ -694,8 +538,7 @@ __device__ __forceinline__ int64_t ls_block_reduce(int64_t v, bool take_max, int
 // still searching: a, a/2, ... from half the last rejected trial down to the first below
 // alpha_min (trials_to_floor), -1 elsewhere.  When no scene is searching any more, the
 // stopping test of every iterating scene (abd.py:265-268: g.g < tol or the iteration cap)
-// writes the next iteration's rows.  One workgroup; the host's step() makes the same
-// decisions with the same arithmetic.
+// writes the next iteration's rows.  One workgroup.
 __global__ __launch_bounds__(kLsThreads) void ls_decide_kernel(LsDev L, double c1, double alpha_min, double tol,
                                                                 int max_iter, int first, int K,
                                                                 double* __restrict__ alpha,
@@ -799,24 +642,41 @@ __global__ __launch_bounds__(kLsThreads) void ls_commit_kernel(int ns, uint8_t* 
     if (blockIdx.x == 0 && threadIdx.x == 0) *range_flag = 0;
 }
 
-// per-scene energies at q = q_base - alpha_s dq (abd.py:133-141): sv rows Ec, Ei
-int compute_energy_scenes(hipStream_t s, Sim& S, const double* dalpha) {
+// q_gets_q0 (abd.py:124-128): q = (Ak, pk) = q0, and the accepted step lengths 0.
+__global__ __launch_bounds__(kLsThreads) void frame_state_kernel(int nb, int ns, const double* __restrict__ A0,
+                                                                  const double* __restrict__ p0,
+                                                                  double* __restrict__ A, double* __restrict__ p,
+                                                                  double* __restrict__ Ak, double* __restrict__ pk,
+                                                                  double* __restrict__ dalpha) {
+    const int i = blockIdx.x * kLsThreads + threadIdx.x;
+    if (i < 9 * nb) A[i] = Ak[i] = A0[i];
+    if (i < 3 * nb) p[i] = pk[i] = p0[i];
+    if (i < ns) dalpha[i] = 0.0;
+}
+
+// A frame's start: q = q0 and the energies there (abd.py:224-225), sv rows Ec, Ei
+int frame_start_scenes(hipStream_t s, Sim& S) {
     int rc;
     const AbdSimState& st = S.st;
     const int ns = S.ns;
-    if ((rc = abd_update_q_scenes(s, &S.sc, st.A, st.p, st.dq, dalpha, st.Ak, st.pk))) return rc;
+    hipLaunchKernelGGL(frame_state_kernel, dim3(grid_for(std::max(9 * (int64_t)S.nb, (int64_t)ns), kLsThreads, INT32_MAX)),
+                       dim3(kLsThreads), 0, s, S.nb, ns, st.A0, st.p0, st.A, st.p, st.Ak, st.pk,
+                       S.sv.p + kSvAlpha * ns);
+    ABD_CHECK_LAUNCH();
     if ((rc = abd_project_vertices(s, &S.sc, st.Ak, st.pk, st.xk))) return rc;
-    // at a frame's start (every alpha 0: zero-length steps are exact copies, xk = x): the
-    // first Newton iteration's collision set too, with its structure
+    // xk = x: the first Newton iteration's collision set too, with its structure
     if ((rc = collision_at_frame_start(s, S, st.xk))) return rc;
     S.col_fresh = true;
     const CandSet& C = S.col;
     if ((rc = contact_energy(s, &S.sc, &S.P, ns, st.xk, C.ptl.p, C.npt, C.eel.p, C.nee, C.vgl.p, C.nvg, C.counts(),
                              S.sv.p + kSvEc * ns)))
         return rc;
-    if ((rc = abd_scene_inertia_energy(s, &S.sc, &S.P, st.Ak, st.pk, st.A0, st.p0, st.Adot, st.pdot,
-                                       S.sv.p + kSvEi * ns)))
-        return rc;
+    if (ns > 1)
+        rc = abd_scene_inertia_energy(s, &S.sc, &S.P, st.Ak, st.pk, st.A0, st.p0, st.Adot, st.pdot,
+                                      S.sv.p + kSvEi * ns);
+    else
+        rc = abd_inertia_energy(s, &S.sc, &S.P, st.Ak, st.pk, st.A0, st.p0, st.Adot, st.pdot, S.sv.p + kSvEi);
+    if (rc) return rc;
     S.stats[5] += 1;
     return ABD_OK;
 }
@@ -843,7 +703,8 @@ int read_counts(hipStream_t s, Sim& S) {
     return ABD_OK;
 }
 
-// The range test of the batched step's end (a vertex outside the superset's ranges writes 1
+// The end of the step (xk = x(q - dq) for the scenes in `active`) with the range test of both
+// ends against the superset's ranges when there is a superset (a vertex outside the superset's ranges writes 1
 // over the 0 of ls_commit_kernel).
 int step_end_scenes(hipStream_t s, Sim& S, const uint8_t* active) {
     const AbdSimState& st = S.st;
@@ -886,7 +747,7 @@ int ccd_and_search_scenes(hipStream_t s, Sim& S, const LsDev& L) {
     return ABD_OK;
 }
 
-// One batched Newton iteration up to the read-back of its counts (abd.py:224-271): the last
+// One Newton iteration of every scene up to the read-back of its counts (abd.py:224-271): the last
 // iteration's accepted steps applied, then collision set, gradient and Hessian, solve, step
 // end with the range test, swept set, TOI and line search.  With no host branch on device
 // values, the same launches every time for the same sizes: the form a HIP graph records.
@@ -917,26 +778,33 @@ int iteration_scenes(hipStream_t s, Sim& S) {
     if ((rc = contact_gh(s, &S.sc, &P, st.x, GL, S.row_ptr.p, S.slots.p, st.g, S.blocks.p, nullptr, nullptr,
                          S.cnt.p + kCntNact)))
         return rc;
-    if ((rc = abd_bsr_solve_scenes(s, P.solver, &S.sc, S.max_scene_bodies, S.row_ptr.p, S.cols.p, S.slots.p,
-                                   S.blocks.p, st.g, st.dq, P.solver_tol, P.solver_maxiter, 10, L.newton, S.iters.p,
-                                   nullptr)))
-        return rc;
+    if (ns > 1)
+        rc = abd_bsr_solve_scenes(s, P.solver, &S.sc, S.max_scene_bodies, S.row_ptr.p, S.cols.p, S.slots.p,
+                                  S.blocks.p, st.g, st.dq, P.solver_tol, P.solver_maxiter, 10, L.newton, S.iters.p,
+                                  nullptr);
+    else
+        rc = abd_bsr_solve(s, P.solver, nb, S.row_ptr.p, S.cols.p, S.slots.p, S.blocks.p, st.g, st.dq, P.solver_tol,
+                           P.solver_maxiter, 10, S.iters.p, nullptr);
+    if (rc) return rc;
     // CCD over the full steps of the scenes still iterating (abd.py:278-303)
     if ((rc = step_end_scenes(s, S, L.newton))) return rc;
     if ((rc = swept_set_launch(s, S))) return rc;
     return ccd_and_search_scenes(s, S, L);
 }
 
-// What a recorded iteration depends on besides device values: the candidate superset (its
-// sizes bound every launch), the scratch pointers and the culling tiles.
-void graph_key(const Sim& S, uint64_t key[4]) {
+// What a recorded iteration depends on besides device values: the candidate superset's
+// size bounds (they size every launch), the scratch pointers and the culling tiles.
+void graph_key(const Sim& S, uint64_t key[kKeyWords]) {
     const AbdTuning t = tuning();
-    key[0] = (uint64_t)S.sup_gen + 1;
-    key[1] = alloc_generation();
-    key[2] = ((uint64_t)(uint32_t)t.cull_chunk << 32) | (uint32_t)t.cull_grid;
-    key[3] = (uint64_t)S.sup.nij ^ ((uint64_t)S.sup.npt << 20) ^ ((uint64_t)S.sup.nee << 40) ^ (uint64_t)S.sup.nvg;
+    key[0] = (uint64_t)S.sup.nij << 32 | (uint64_t)S.sup.nvg;
+    key[1] = (uint64_t)S.sup.npt;
+    key[2] = (uint64_t)S.sup.nee;
+    key[3] = alloc_generation();
+    key[4] = ((uint64_t)(uint32_t)t.cull_chunk << 32) | (uint32_t)t.cull_grid;
 }
-bool same_key(const uint64_t a[4], const uint64_t b[4]) { return !memcmp(a, b, 4 * sizeof(uint64_t)); }
+bool same_key(const uint64_t a[kKeyWords], const uint64_t b[kKeyWords]) {
+    return !memcmp(a, b, kKeyWords * sizeof(uint64_t));
+}
 
 // Records iteration_scenes into S.gexec (updated in place when the topology allows), on a
 // stream of the simulator's own (the legacy null stream cannot record); nothing runs.  A
@@ -992,13 +860,8 @@ int step_scenes(hipStream_t s, Sim& S) {
     const int nb = S.nb, ns = S.ns;
     int rc;
     double* dalpha = S.sv.p + kSvAlpha * ns;
-    ABD_CHECK(hipMemcpyAsync(st.A, st.A0, 72 * (size_t)nb, hipMemcpyDeviceToDevice, s));
-    ABD_CHECK(hipMemcpyAsync(st.p, st.p0, 24 * (size_t)nb, hipMemcpyDeviceToDevice, s));
-    ABD_CHECK(hipMemcpyAsync(st.Ak, st.A0, 72 * (size_t)nb, hipMemcpyDeviceToDevice, s));
-    ABD_CHECK(hipMemcpyAsync(st.pk, st.p0, 24 * (size_t)nb, hipMemcpyDeviceToDevice, s));
-    if ((rc = zero_fill(s, dalpha, sizeof(double) * ns))) return rc;
     S.sw_valid = false;  // a frame starts from the state the caller holds
-    if ((rc = compute_energy_scenes(s, S, dalpha))) return rc;
+    if ((rc = frame_start_scenes(s, S))) return rc;
     {
         // the first iteration's rows, taken over by its ls_commit_kernel
         const LsDev L = ls_dev(S);
@@ -1013,8 +876,9 @@ int step_scenes(hipStream_t s, Sim& S) {
         // a steady iteration (collision set from the last swept set, superset kept) replays
         // its recorded graph; the first time a key is met the iteration runs eagerly, the
         // second time it is recorded (every buffer then holds its size for these launches)
-        const bool steady = S.graphs && S.sw_valid && !S.col_fresh && S.sup_valid && !prof_enabled();
-        uint64_t key[4];
+        const bool steady =
+            S.graphs && !S.solve_waits && S.sw_valid && !S.col_fresh && S.sup_valid && !prof_enabled();
+        uint64_t key[kKeyWords];
         graph_key(S, key);
         bool ran = false;
         if (steady && S.gexec && same_key(key, S.gkey)) {
@@ -1116,9 +980,7 @@ int abd_sim_create(const AbdScene* scene, const AbdParams* params, const AbdSimS
     if (!rc) rc = S->cols.reserve(nb + 512);
     if (!rc) rc = S->slots.reserve(nb + 512);
     if (!rc) rc = S->blocks.reserve((nb + 512) * 144);
-    if (!rc) rc = S->scal.reserve(8);
-    if (!rc) rc = S->iters.reserve(4);
-    if (!rc && hipHostMalloc((void**)&S->host, 8 * sizeof(double), hipHostMallocDefault) != hipSuccess) rc = ABD_ERR_ARG;
+    if (!rc) rc = S->scal.reserve(1);
     if (!rc && hipHostMalloc((void**)&S->hcount, 8 * sizeof(int64_t), hipHostMallocDefault) != hipSuccess)
         rc = ABD_ERR_ARG;
     {
@@ -1131,8 +993,12 @@ int abd_sim_create(const AbdScene* scene, const AbdParams* params, const AbdSimS
         if (!rc && hipMemset(S->cnt.p, 0, sizeof(int64_t) * S->cnt.cap) != hipSuccess) rc = ABD_ERR_ARG;
         if (!rc && hipHostMalloc((void**)&S->hcnt, 2 * kCntLen * sizeof(int64_t), hipHostMallocDefault) != hipSuccess)
             rc = ABD_ERR_ARG;
-        if (!rc && hipHostMalloc((void**)&S->hcand, sizeof(double) * 3 * nsc * kLsSpec, hipHostMallocDefault) !=
-                       hipSuccess)
+        if (!rc) rc = S->sv.reserve((size_t)kSv * nsc);
+        if (!rc) rc = S->lsflag.reserve((size_t)kLfRows * nsc);
+        if (!rc) rc = S->lsval.reserve((size_t)kLvRows * nsc);
+        if (!rc) rc = S->lsit.reserve(2 * (size_t)nsc);
+        if (!rc) rc = S->iters.reserve(nsc);
+        if (!rc && hipHostMalloc((void**)&S->hiters, sizeof(int32_t) * nsc, hipHostMallocDefault) != hipSuccess)
             rc = ABD_ERR_ARG;
     }
     if (!rc && scene->n_scenes > 1) {
@@ -1148,15 +1014,8 @@ int abd_sim_create(const AbdScene* scene, const AbdParams* params, const AbdSimS
         }
         if (!rc && (sb[0] != 0 || sb[ns] != scene->n_bodies)) rc = ABD_ERR_ARG;
         S->ns = ns;
-        if (!rc) rc = S->sv.reserve((size_t)kSv * ns);
-        if (!rc) rc = S->lsflag.reserve((size_t)kLfRows * ns);
-        if (!rc) rc = S->lsval.reserve((size_t)kLvRows * ns);
-        if (!rc) rc = S->lsit.reserve(2 * (size_t)ns);
-        if (!rc) rc = S->iters.reserve(ns);
-        if (!rc) rc = S->scal.reserve(8 + (size_t)ns);
-        if (!rc && hipHostMalloc((void**)&S->hiters, sizeof(int32_t) * ns, hipHostMallocDefault) != hipSuccess)
-            rc = ABD_ERR_ARG;
     }
+    S->solve_waits = S->ns == 1 && solve_waits(params->solver, scene->n_bodies);
     if (rc) {
         abd_sim_destroy(S);
         return rc;
@@ -1169,7 +1028,7 @@ int abd_sim_step(void* sim, abd_stream_t stream, int64_t* stats) {
     if (!sim) return ABD_ERR_ARG;
     Sim& S = *static_cast<Sim*>(sim);
     ArenaScope scope(&S.arena);
-    int rc = S.ns > 1 ? step_scenes(to_stream(stream), S) : step(to_stream(stream), S);
+    const int rc = step_scenes(to_stream(stream), S);
     if (stats)
         for (int k = 0; k < 10; ++k) stats[k] = S.stats[k];
     return rc;
@@ -1200,10 +1059,10 @@ int abd_sim_hessian_solve(void* sim, abd_stream_t stream, int32_t method, double
         return rc;
     ABD_CHECK(hipMemsetAsync(y, 0, sizeof(double) * 12 * S.nb, s));
     if ((rc = abd_bsr_solve(s, method, S.nb, S.row_ptr.p, S.cols.p, S.slots.p, S.blocks.p, rhs, y, tol, maxiter, 10,
-                            S.iters.p, S.scal.p + 4)))
+                            S.iters.p, S.scal.p)))
         return rc;
     if (iters) ABD_CHECK(hipMemcpyAsync(iters, S.iters.p, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-    if (resid) ABD_CHECK(hipMemcpyAsync(resid, S.scal.p + 4, sizeof(double), hipMemcpyDeviceToHost, s));
+    if (resid) ABD_CHECK(hipMemcpyAsync(resid, S.scal.p, sizeof(double), hipMemcpyDeviceToHost, s));
     ABD_CHECK(hipStreamSynchronize(s));
     return ABD_OK;
 }
@@ -1347,8 +1206,7 @@ int abd_sim_destroy(void* sim) {
     S->plan.release();
     S->dcount.release();
     S->cnt.release();
-    if (S->hcand) (void)hipHostFree(S->hcand);
-    for (void* h : {(void*)S->host, (void*)S->hcount, (void*)S->hcnt, (void*)S->hiters})
+    for (void* h : {(void*)S->hcount, (void*)S->hcnt, (void*)S->hiters})
         if (h) (void)hipHostFree(h);
     delete S;
     return ABD_OK;

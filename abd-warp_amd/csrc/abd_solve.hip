@@ -1235,6 +1235,10 @@ __global__ void mw_finish_kernel(int n, MwState W, double* __restrict__ xg, int3
     }
 }
 
+bool solve_waits(int32_t method, int nb) {
+    return nb > kLargeBodies && method != ABD_SOLVER_BICGSTAB;  // solve_cg_multi
+}
+
 }  // namespace abd
 
 using namespace abd;
