@@ -694,6 +694,8 @@ struct KeepArgs {
     const int32_t *tris, *edges;
     float pdil;
     double edil, tdil;
+    const double* alpha;  // KeepAtX: entries apart at their scene's step length are dropped
+    const int32_t* body_scene;
 };
 
 // point_boxes_kernel's box of vertex v at x, or with x1 set swept_point_boxes_kernel's
@@ -755,6 +757,12 @@ __device__ __forceinline__ void prim_box_at(const double* __restrict__ x, const 
     prim_box_of<NV>(x, x1, vi, dil, lo, hi);
 }
 
+// an entry of body b apart at the step length its scene has taken: the boxes there do not
+// overlap, and neither they nor the vertices need to be read
+__device__ __forceinline__ bool keep_apart(const KeepArgs& A, int b, float apart) {
+    return A.alpha[A.body_scene ? A.body_scene[b] : 0] < (double)apart;
+}
+
 __device__ __forceinline__ bool keep_pred(const KeepArgs& A, int k, int64_t i) {
     const KeepBoxes& B = A.bx;
     if (k <= 1) {
@@ -765,6 +773,7 @@ __device__ __forceinline__ bool keep_pred(const KeepArgs& A, int k, int64_t i) {
     if (k <= 3) {  // (I, J, ii, a, b): both bodies' boxes and the two primitives' boxes
         const int32_t* t5 = (k == 2 ? A.in.pt : A.in.ee) + 5 * i;
         const int I = t5[0], J = t5[1];
+        if (A.alpha && keep_apart(A, I, (k == 2 ? A.in.vids.apart_pt : A.in.vids.apart_ee)[i])) return false;
         const int32_t* vid = k == 2 ? A.in.vids.pt : A.in.vids.ee;
         if (A.x && vid) {  // the candidate's vertex ids stored beside the list
             vid += 4 * i;
@@ -805,6 +814,7 @@ __device__ __forceinline__ bool keep_pred(const KeepArgs& A, int k, int64_t i) {
     const float qlo[3] = {-1e3f, -1e3f, -1e3f};
     const float qhi[3] = {1e3f, A.fg, 1e3f};
     const int b = A.in.vg[2 * i];
+    if (A.alpha && keep_apart(A, b, A.in.vids.apart_vg[i])) return false;
     const int64_t v = A.voff[b] + (int64_t)A.in.vg[2 * i + 1];
     if (!((double)B.blo[3 * b + 1] < A.yth)) return false;
     if (A.x) {
@@ -939,6 +949,8 @@ int keep_from_superset(hipStream_t s, const AbdScene* sc, const KeepInput& in, c
     A.pdil = at ? (float)at->pdil : 0.0f;
     A.edil = at ? at->edil : 0.0;
     A.tdil = at ? at->tdil : 0.0;
+    A.alpha = at && in.vids.apart_pt ? at->alpha : nullptr;
+    A.body_scene = at ? at->body_scene : nullptr;
     A.yth = 0.5 * dhat + ground;
     A.fg = (float)ground;
     const int64_t n[kKeepLists] = {in.nij, in.ji ? in.nij : 0, in.npt, in.nee, in.nvg};

@@ -425,6 +425,60 @@ __device__ __forceinline__ bool cand_toi_bracketed(int kind, const SceneView& S,
     coplanar_poly(a, b, coef);
     return cubic_bracket(coef, 0.0, 1.0).kind != CubicBracket::kNone;
 }
+// A lower bound of the step lengths at which a PT (kind 0) / EE (kind 1) candidate can be
+// active on the step a -> b of its vertices: below it some axis separates the two
+// primitives by more than dhat, so the barrier is zero, and their boxes dilated as the
+// collision set's (FP32 rounding included) do not overlap; above 1 they are apart on the
+// whole step, so its CCD finds no contact either.  Along an axis the gap between the boxes
+// is concave in the step length (a minimum of linear functions minus a maximum), so from a
+// positive gap at the start it stays above the chord to the gap at the end.  The margins:
+// 1e-3 dhat for the rounding of positions on the step, 5e-7 of the coordinates for the
+// boxes' casts (four roundings of 2^-24), the boxes' motion over the tolerance of the CCD's
+// roots.  NaN or infinite coordinates give 0.
+__device__ __forceinline__ float chord_zero(double u0, double u1, float best) {
+    if (!(u0 > 0.0)) return best;
+    const float f0 = (float)u0, f1 = (float)u1;
+    const float t = u1 > 0.0 ? 2.0f : f0 / (f0 - f1);
+    return t > best ? t : best;
+}
+__device__ __forceinline__ float apart_until(int kind, const d3 a[4], const d3 b[4], double dhat) {
+    float best = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        double l[2][2], h[2][2];  // [end][primitive]
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const d3* v = e ? b : a;
+            const double c0 = comp(v[0], k), c1 = comp(v[1], k), c2 = comp(v[2], k), c3 = comp(v[3], k);
+            const double m23 = c2 < c3 ? c2 : c3, x23 = c2 < c3 ? c3 : c2;
+            if (kind == 0) {
+                l[e][0] = h[e][0] = c0;
+                l[e][1] = c1 < m23 ? c1 : m23;
+                h[e][1] = c1 > x23 ? c1 : x23;
+            } else {
+                l[e][0] = c0 < c1 ? c0 : c1;
+                h[e][0] = c0 < c1 ? c1 : c0;
+                l[e][1] = m23;
+                h[e][1] = x23;
+            }
+        }
+        double m = 0.0, move = 0.0;
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            m = fmax(m, fmax(fmax(fabs(l[0][p]), fabs(h[0][p])), fmax(fabs(l[1][p]), fabs(h[1][p]))));
+            move += fmax(fabs(l[1][p] - l[0][p]), fabs(h[1][p] - h[0][p]));
+        }
+        const double d = 1.001 * dhat + 5e-7 * m + 4.0 * kXError * move;
+        best = chord_zero((l[0][1] - h[0][0]) - d, (l[1][1] - h[1][0]) - d, best);
+        best = chord_zero((l[0][0] - h[0][1]) - d, (l[1][0] - h[1][1]) - d, best);
+    }
+    return best * (1.0f - 2e-6f);  // below the chord's zero whatever its roundings
+}
+// The same of a vertex above the ground (its height y0 -> y1).
+__device__ __forceinline__ float apart_until_vg(double y0, double y1, double ground, double dhat) {
+    const double d = 1.001 * dhat + 5e-7 * fmax(fabs(ground), fmax(fabs(y0), fabs(y1)));
+    return chord_zero((y0 - ground) - d, (y1 - ground) - d, 0.0f) * (1.0f - 2e-6f);
+}
 __device__ __forceinline__ double cand_toi_vg(const int32_t* __restrict__ voff, const double* __restrict__ x0,
                                               const double* __restrict__ x1, const int32_t* t2, double ground) {
     const int64_t vid = voff[t2[0]] + t2[1];

@@ -129,30 +129,46 @@ int vertex_ranges(hipStream_t s, int64_t n3, const double* x0, const double* x1,
 // *flag (device, 0 before) becomes 1 when some coordinate of x0 or x1 leaves [lo, hi].
 int within_ranges(hipStream_t s, int64_t n3, const double* x0, const double* x1, const double* lo, const double* hi,
                   int64_t* flag);
-// K line-search trials q - alpha dq at once (alpha [K][S] on the device, S = 1: the
-// whole system as one scene; a negative alpha skips that scene's trial and gives 0):
-// per-scene contact energies to E[2 S k + s] and inertia energies to E[2 S k + S + s].
 // dn (here and below, nullable): the lists' sizes on the device, [nij, nij, npt, nee, nvg],
 // the counts passed then bounding them.
-// The scene vertex ids of each PT / EE candidate of a list (4 per tuple, in the order
-// fetch_pt_idx / fetch_ee_idx give them), stored beside it so that a kernel reads them
-// instead of gathering them through the topology; either may be null.
-struct VertIds {
+// What a candidate set keeps beside its tuples (each nullable): the scene vertex ids of each
+// PT / EE candidate (4 per tuple, in the order fetch_pt_idx / fetch_ee_idx give them), so
+// that a kernel reads them instead of gathering them through the topology; and of each PT /
+// EE / VG candidate the step length below which it stays inactive on the step last passed to
+// scene_toi (apart_until), written there and read by line_chunks and the next filter.
+struct CandSide {
     const int32_t* pt = nullptr;
     const int32_t* ee = nullptr;
+    float* apart_pt = nullptr;
+    float* apart_ee = nullptr;
+    float* apart_vg = nullptr;
 };
-int line_trials(hipStream_t s, const AbdScene* sc, const AbdParams* P, int S, int K, const double* alpha,
-                const double* A, const double* p, const double* dq, const double* A0, const double* p0,
-                const double* Adot, const double* pdot, const int32_t* pt, int64_t npt, const int32_t* ee, int64_t nee,
-                const int32_t* vg, int64_t nvg, const int64_t* plan, double* E, const int64_t* dn = nullptr,
-                VertIds vids = {});
+// Line-search trials q - alpha dq of at most kMaxTrials lengths at once (S = 1: the whole
+// system as one scene).  trial_states: the bodies' states st [K][nb][12] (16-byte aligned)
+// and inertia energies e [K][nb] at alpha [K][S] (device), or with `halve` at alpha[s] / 2^k;
+// a negative length is skipped.  line_chunks: the chunks' contact energies at alpha [K][S]
+// (negative: 0) over a planned set, scene s's at trial k part[stride k + choff[s] ..
+// choff[s + 1]) in the order their sum is taken.
+constexpr int kMaxTrials = 12;
+struct TrialSums {
+    const int64_t* choff;
+    const double* part;
+    int64_t stride;
+};
+int trial_states(hipStream_t s, const AbdScene* sc, const AbdParams* P, int S, int K, const double* alpha, bool halve,
+                 const double* A, const double* p, const double* dq, const double* A0, const double* p0,
+                 const double* Adot, const double* pdot, double* st, double* e);
+int line_chunks(hipStream_t s, const AbdScene* sc, const AbdParams* P, int S, int K, const double* alpha,
+                const double* st, const int32_t* pt, int64_t npt, const int32_t* ee, int64_t nee, const int32_t* vg,
+                int64_t nvg, const int64_t* plan, const int64_t* dn, CandSide vids, TrialSums* out);
 // The per-scene chunk plan of the energy / TOI reductions over one set of candidate lists
 // (plan: reduce_plan_elems(S) int64 on the device), made once and passed as `plan` to every
-// reduction over those lists (nullptr: each makes its own).
+// reduction over those lists (nullptr: each makes its own).  Also readies the CCD's scratch for
+// one scene_toi with the plan, and zeroes nzero (at most 1024) counters of the caller.
 size_t reduce_plan_elems(int S);
 int reduce_plan(hipStream_t s, const AbdScene* sc, const AbdParams* P, int S, const int32_t* pt, int64_t npt,
                 const int32_t* ee, int64_t nee, const int32_t* vg, int64_t nvg, int64_t* plan,
-                const int64_t* dn = nullptr);
+                const int64_t* dn = nullptr, int64_t* zero = nullptr, int nzero = 0);
 // Per-scene TOI (abd_scene_toi; S = 1: the whole system as one scene) with an optional plan;
 // active (nullable, [S]): scenes whose TOI is wanted, the others report 1 unevaluated.
 // Per-scene dot products a.b and c.d (each seg_dot_kernel's) that the TOI's final per-scene pass computes
@@ -166,7 +182,7 @@ struct SceneDots {
 int scene_toi(hipStream_t s, const AbdScene* sc, const AbdParams* P, int S, const double* x_t0, const double* x_t1,
               const int32_t* pt, int64_t npt, const int32_t* ee, int64_t nee, const int32_t* vg, int64_t nvg,
               const int64_t* plan, double* toi, const uint8_t* active, const int64_t* dn = nullptr,
-              double* first_alpha = nullptr, VertIds vids = {}, const SceneDots* dots = nullptr);
+              double* first_alpha = nullptr, CandSide vids = {}, const SceneDots* dots = nullptr);
 // The line search's first step length from a TOI (abd.py:300-302): clamped to [0, 1], x 0.9
 // below 1.  scene_toi's first_alpha (device, nullable) receives it per scene (-1 for the
 // scenes not active).
@@ -206,7 +222,7 @@ struct KeepInput {
     const int32_t *ij, *ji, *pt, *ee, *vg;
     int64_t nij, npt, nee, nvg;
     const int64_t* dn = nullptr;
-    VertIds vids = {};  // the PT / EE tuples' vertex ids (nullable)
+    CandSide vids = {};  // the PT / EE tuples' vertex ids (nullable)
 };
 struct KeepBoxes {
     const float *blo, *bhi, *plo, *phi, *elo, *ehi, *tlo, *thi;
@@ -215,16 +231,21 @@ struct KeepOutput {
     int32_t *ij, *ji, *pt, *ee, *vg;
     int32_t *ptv = nullptr, *eev = nullptr;  // the kept tuples' vertex ids (when the input has them)
 };
-// The vertex ids of n PT (kind 0) or EE (kind 1) tuples into vid [n][4] (VertIds).
+// The vertex ids of n PT (kind 0) or EE (kind 1) tuples into vid [n][4] (CandSide).
 int cand_vertex_ids(hipStream_t s, const AbdScene* sc, int kind, const int32_t* tuples, int64_t n, int32_t* vid);
 // The primitive boxes of the predicates computed per entry from the vertices x instead of
 // read from KeepBoxes (whose point, edge and triangle boxes are then unused): the box
 // kernels' own expressions, points (float)x -+ (float)pdil, edges and triangles the FP64
 // min / max of their vertices -+ edil / tdil, cast to FP32; with x1 set, the swept boxes'
 // (the union of the boxes at x and at x1).
+// alpha (nullable): x is the state at step length alpha[scene] of the step the input's
+// apart_* were written for; an entry apart at its scene's length is dropped unevaluated (its
+// boxes there do not overlap).  body_scene null: one scene.
 struct KeepAtX {
     const double *x, *x1;
     double pdil, edil, tdil;
+    const double* alpha = nullptr;
+    const int32_t* body_scene = nullptr;
 };
 // sync false: the totals reach hcount with the stream's next synchronization (the caller's);
 // hcount null: they stay on the device.

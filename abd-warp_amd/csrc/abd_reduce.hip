@@ -33,6 +33,7 @@ struct ListRef {
     int64_t n;
     int kind;                   // kListPT / kListEE / kListVG
     const int32_t* v = nullptr;  // PT / EE: the candidates' scene vertex ids, 4 per tuple (nullable)
+    float* apart = nullptr;      // the candidates' apart_until (nullable)
 };
 __device__ __forceinline__ const int32_t* vids_of(const ListRef& r, int64_t i) { return r.v ? r.v + 4 * i : nullptr; }
 // dn (nullable): the lists' sizes on the device, [nij, nij, npt, nee, nvg] (the keep
@@ -72,9 +73,24 @@ __device__ __forceinline__ int64_t n_chunks(int64_t len) { return (len + kChunkI
 // thread (scene s ends where scene s + 1 begins), then the chunk counts of the scenes in
 // tiles of blockDim with a running offset.
 constexpr int kPlanThreads = 1024;
+constexpr unsigned long long kBitsOne = 0x3FF0000000000000ull;  // 1.0
+// What the plan's kernel also sets for the CCD that follows it (nullable): the scene slots to
+// 1, the queue count and nzero counters of the caller to 0.
+struct ToiInit {
+    unsigned long long* slots = nullptr;
+    int32_t* qcount = nullptr;
+    int64_t* zero = nullptr;
+    int nzero = 0;
+};
 __global__ __launch_bounds__(kPlanThreads) void plan_kernel(int S, const int32_t* __restrict__ body_scene, Lists L,
-                                                            int64_t* __restrict__ seg, int64_t* __restrict__ choff) {
+                                                            int64_t* __restrict__ seg, int64_t* __restrict__ choff,
+                                                            ToiInit I) {
     __shared__ int64_t sh[kPlanThreads];
+    if (I.slots) {
+        for (int s = threadIdx.x; s < S; s += blockDim.x) I.slots[s] = kBitsOne;
+        if (threadIdx.x == 0) *I.qcount = 0;
+    }
+    if (I.zero && threadIdx.x < I.nzero) I.zero[threadIdx.x] = 0;
     __shared__ int64_t tile_total;
     for (int idx = threadIdx.x; idx < kLists * (S + 1); idx += blockDim.x) {
         const int l = idx / (S + 1), s = idx % (S + 1);
@@ -118,66 +134,79 @@ __device__ __forceinline__ int scene_of_chunk(const int64_t* __restrict__ choff,
     return lo;
 }
 
-// Vertex positions at the line-search trial state q - alpha dq of one scene, computed on
-// the fly with the arithmetic of abd_update_q + abd_project_vertices (abd.py:305-353), so
-// that they equal the projected vertices of the updated state bit for bit.
+// Vertex positions at a line-search trial state, placed on the fly from the bodies' trial
+// states st ([nb][12], A then p: trial_states_kernel) with the arithmetic of
+// abd_update_q + abd_project_vertices (abd.py:305-353), so that they equal the projected
+// vertices of the updated state bit for bit.
 struct VertsTrial {
-    const double *xr, *A, *p, *dq;  // rest positions, state, step
-    double alpha;
-    __device__ __forceinline__ static d3 place(const double (&Ab)[9], const double (&pb)[3],
-                                               const double* __restrict__ r) {
+    const double *xr, *st;  // rest positions, trial states (16-byte aligned)
+    __device__ __forceinline__ void state(int b, double (&q)[12]) const {
+        typedef double v2 __attribute__((ext_vector_type(2)));
+        const v2* p = reinterpret_cast<const v2*>(st + 12 * (int64_t)b);
+#pragma unroll
+        for (int i = 0; i < 6; ++i) {
+            const v2 v = p[i];
+            q[2 * i] = v.x;
+            q[2 * i + 1] = v.y;
+        }
+    }
+    __device__ __forceinline__ static d3 place(const double (&q)[12], const double* __restrict__ r) {
         double x[3];
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
-            double v = pb[c] + r[0] * Ab[c];
-            v = v + r[1] * Ab[3 + c];
-            v = v + r[2] * Ab[6 + c];
+            double v = q[9 + c] + r[0] * q[c];
+            v = v + r[1] * q[3 + c];
+            v = v + r[2] * q[6 + c];
             x[c] = v;
         }
         return mk(x[0], x[1], x[2]);
     }
     __device__ __forceinline__ void load4(int I, int J, const int64_t vi[4], int nI, d3 v[4]) const {
-        double AI[9], pI[3], AJ[9], pJ[3];
-        trial_state(I, alpha, A, p, dq, AI, pI);
-        trial_state(J, alpha, A, p, dq, AJ, pJ);
-        for (int k = 0; k < 4; ++k)
-            v[k] = k < nI ? place(AI, pI, xr + 3 * vi[k]) : place(AJ, pJ, xr + 3 * vi[k]);
+        double qI[12], qJ[12];
+        state(I, qI);
+        state(J, qJ);
+        for (int k = 0; k < 4; ++k) v[k] = k < nI ? place(qI, xr + 3 * vi[k]) : place(qJ, xr + 3 * vi[k]);
     }
     __device__ __forceinline__ double y(int b, int64_t vid) const {
-        double Ab[9], pb[3];
-        trial_state(b, alpha, A, p, dq, Ab, pb);
-        return place(Ab, pb, xr + 3 * vid).y;
+        double q[12];
+        state(b, q);
+        return place(q, xr + 3 * vid).y;
     }
 };
 
-// VertsTrial with the trial states of the bodies [b0, b0 + n) computed once per workgroup
-// into LDS (st: 12 doubles per body, A then p).
-struct VertsTrialLds {
-    const double* xr;
-    const double* st;
-    int b0;
-    __device__ __forceinline__ void state(int b, double (&Ab)[9], double (&pb)[3]) const {
-        const double* q = st + 12 * (b - b0);
+// The bodies' trial states q - alpha dq (st [K][nb][12]) and inertia energies there (e
+// [K][nb]) of K trials.  halve: trial k has the length alpha[scene] / 2^k (the halvings of a
+// line search are known with its first length), else alpha[k][scene]; a negative length
+// leaves its trial unwritten.  One thread per (body, trial): the energies' kernels and
+// every candidate evaluated then read 96 bytes of a body instead of forming its state.
+__global__ __launch_bounds__(kRedThreads) void trial_states_kernel(AbdScene sc, AbdParams P, int S, int K,
+                                                                   const double* __restrict__ alpha, int halve,
+                                                                   const double* __restrict__ A,
+                                                                   const double* __restrict__ p,
+                                                                   const double* __restrict__ dq,
+                                                                   const double* __restrict__ A0,
+                                                                   const double* __restrict__ p0,
+                                                                   const double* __restrict__ Adot,
+                                                                   const double* __restrict__ pdot,
+                                                                   double* __restrict__ st, double* __restrict__ e) {
+    const int64_t i = (int64_t)blockIdx.x * kRedThreads + threadIdx.x;
+    const int nb = sc.n_bodies;
+    if (i >= (int64_t)nb * K) return;
+    const int b = (int)(i % nb), k = (int)(i / nb);
+    const int s = S > 1 ? sc.body_scene[b] : 0;
+    double al = halve ? alpha[s] : alpha[(int64_t)k * S + s];
+    if (al < 0.0) return;
+    if (halve)
+        for (int q = 0; q < k; ++q) al *= 0.5;
+    double Ab[9], pb[3];
+    trial_state(b, al, A, p, dq, Ab, pb);
+    double* o = st + 12 * i;
 #pragma unroll
-        for (int i = 0; i < 9; ++i) Ab[i] = q[i];
+    for (int q = 0; q < 9; ++q) o[q] = Ab[q];
 #pragma unroll
-        for (int i = 0; i < 3; ++i) pb[i] = q[9 + i];
-    }
-    __device__ __forceinline__ void load4(int I, int J, const int64_t vi[4], int nI, d3 v[4]) const {
-        double AI[9], pI[3], AJ[9], pJ[3];
-        state(I, AI, pI);
-        state(J, AJ, pJ);
-        for (int k = 0; k < 4; ++k)
-            v[k] = k < nI ? VertsTrial::place(AI, pI, xr + 3 * vi[k]) : VertsTrial::place(AJ, pJ, xr + 3 * vi[k]);
-    }
-    __device__ __forceinline__ double y(int b, int64_t vid) const {
-        double Ab[9], pb[3];
-        state(b, Ab, pb);
-        return VertsTrial::place(Ab, pb, xr + 3 * vid).y;
-    }
-};
-// bodies of a scene whose trial states a chunk workgroup keeps in LDS
-constexpr int kTrialLdsBodies = 128;
+    for (int q = 0; q < 3; ++q) o[9 + q] = pb[q];
+    e[i] = inertia_energy_q(P, sc.mass, sc.I0, b, Ab, pb, A0, p0, Adot, pdot);
+}
 
 // ipcsk/energy.py:10-48 per candidate
 template <class Src>
@@ -190,87 +219,186 @@ __device__ __forceinline__ double energy_term(int kind, const AbdScene& sc, cons
     return cand_energy_vg(sc.voff, X, t, P.ground, P.d2hat, P.kappa);
 }
 
-// The line-search trials of chunk_kernel<2>: step lengths alpha [trial][S] (a negative
-// length skips that scene's trial: its sums are 0) and the state.
-struct TrialArgs {
-    const double *alpha, *A, *p, *dq;
+// Chunk c of the plan: its scene s, list l (kLists: none) and candidates [start, end).
+struct ChunkRange {
+    int s, l;
+    int64_t start, end;
 };
-
-// One chunk per workgroup.  OP 0 sums energies at positions x0; OP 2 sums energies at the
-// trial state blockIdx.y of T (partials part + part_stride blockIdx.y).
-template <int OP>
-__global__ __launch_bounds__(kRedThreads) void chunk_kernel(AbdScene sc, AbdParams P, const double* __restrict__ x0,
-                                                            const double* __restrict__ x1, TrialArgs T, Lists L,
-                                                            int S, const int64_t* __restrict__ seg,
-                                                            const int64_t* __restrict__ choff,
-                                                            double* __restrict__ part, int64_t part_stride) {
-    __shared__ double sh[kRedThreads];
-    part += part_stride * blockIdx.y;
-    const int64_t c = blockIdx.x;
-    if (c >= choff[S]) return;
-    const int s = scene_of_chunk(choff, S, c);
-    // skipped trials (uniform over the workgroup): the neutral element of the sum
-    if (OP == 2 && T.alpha[(int64_t)S * blockIdx.y + s] < 0.0) {
-        if (threadIdx.x == 0) part[c] = 0.0;
-        return;
-    }
-    int64_t k = c - choff[s];
-    int l = 0;
-    int64_t start = 0, end = 0;
-    for (; l < kLists; ++l) {
-        const int64_t a = seg[2 * (kLists * (int64_t)s + l)], b = seg[2 * (kLists * (int64_t)s + l) + 1];
+__device__ __forceinline__ ChunkRange chunk_range(int S, const int64_t* __restrict__ seg,
+                                                  const int64_t* __restrict__ choff, int64_t c) {
+    ChunkRange r{scene_of_chunk(choff, S, c), 0, 0, 0};
+    int64_t k = c - choff[r.s];
+    for (; r.l < kLists; ++r.l) {
+        const int64_t a = seg[2 * (kLists * (int64_t)r.s + r.l)], b = seg[2 * (kLists * (int64_t)r.s + r.l) + 1];
         const int64_t nch = n_chunks(b - a);
         if (k < nch) {
-            start = a + k * kChunkItems;
-            end = start + kChunkItems < b ? start + kChunkItems : b;
+            r.start = a + k * kChunkItems;
+            r.end = r.start + kChunkItems < b ? r.start + kChunkItems : b;
             break;
         }
         k -= nch;
     }
-    const SceneView V{sc.voff, sc.foff, sc.eoff, sc.tris, sc.edges, sc.x0};
-    const int kind = l < kLists ? L.l[l].kind : 0;
-    const int w = width_of(kind);
-    double acc = 0.0;
-    if (l < kLists) {
-        if (OP == 0) {
-            const Verts X{x0};
-            for (int64_t i = start + threadIdx.x; i < end; i += blockDim.x)
-                acc += energy_term(kind, sc, V, P, X, L.l[l].p + w * i, vids_of(L.l[l], i));
-        } else if (OP == 2) {
-            const double al = T.alpha[(int64_t)S * blockIdx.y + s];
-            const int b0 = S > 1 ? sc.scene_boff[s] : 0, b1 = S > 1 ? sc.scene_boff[s + 1] : sc.n_bodies;
-            if (b1 - b0 <= kTrialLdsBodies) {  // uniform over the workgroup
-                __shared__ double st[12 * kTrialLdsBodies];
-                for (int b = b0 + threadIdx.x; b < b1; b += blockDim.x) {
-                    double Ab[9], pb[3];
-                    trial_state(b, al, T.A, T.p, T.dq, Ab, pb);
-                    double* q = st + 12 * (b - b0);
-                    for (int i = 0; i < 9; ++i) q[i] = Ab[i];
-                    for (int i = 0; i < 3; ++i) q[9 + i] = pb[i];
-                }
-                __syncthreads();
-                const VertsTrialLds X{sc.x0, st, b0};
-                for (int64_t i = start + threadIdx.x; i < end; i += blockDim.x)
-                    acc += energy_term(kind, sc, V, P, X, L.l[l].p + w * i, vids_of(L.l[l], i));
-            } else {
-                const VertsTrial X{sc.x0, T.A, T.p, T.dq, al};
-                for (int64_t i = start + threadIdx.x; i < end; i += blockDim.x)
-                    acc += energy_term(kind, sc, V, P, X, L.l[l].p + w * i, vids_of(L.l[l], i));
-            }
-        }
-    }
-    const double r = block_sum_fast(acc, sh);
-    if (threadIdx.x == 0) part[c] = r;
+    return r;
 }
 
-template <int OP>
+// Energies at positions x0, one chunk per workgroup.
+__global__ __launch_bounds__(kRedThreads) void chunk_kernel(AbdScene sc, AbdParams P, const double* __restrict__ x0,
+                                                            Lists L, int S, const int64_t* __restrict__ seg,
+                                                            const int64_t* __restrict__ choff,
+                                                            double* __restrict__ part) {
+    __shared__ double sh[17];
+    const int64_t c = blockIdx.x;
+    if (c >= choff[S]) return;
+    const ChunkRange r = chunk_range(S, seg, choff, c);
+    double acc = 0.0;
+    if (r.l < kLists) {
+        const SceneView V{sc.voff, sc.foff, sc.eoff, sc.tris, sc.edges, sc.x0};
+        const int kind = L.l[r.l].kind, w = width_of(kind);
+        const Verts X{x0};
+        for (int64_t i = r.start + threadIdx.x; i < r.end; i += kRedThreads)
+            acc += energy_term(kind, sc, V, P, X, L.l[r.l].p + w * i, vids_of(L.l[r.l], i));
+    }
+    acc = block_sum_fast(acc, sh);
+    if (threadIdx.x == 0) part[c] = acc;
+}
+
+// The line-search trials: step lengths alpha [trial][S] (a negative length skips that
+// scene's trial: its sums are 0) and the bodies' states at each ([trial][nb][12]).
+struct TrialArgs {
+    const double *alpha, *st;
+};
+
+// The energies of up to kMaxTrials trials, one chunk per workgroup, the trials dealt over blockIdx.y
+// (partials part + part_stride trial).  Nearly every candidate of a step's set is inactive at
+// a trial (its boxes meet only further along the step, or not at all), so the (trial,
+// candidate) pairs that may be active (apart_until at most the trial's length: 4 bytes read
+// a candidate) are listed in LDS, all trials together, and evaluated side by side; each
+// thread then adds its own candidates' terms in order: the sum of every candidate in turn,
+// whose other terms are zeros.  A pair's place in the list is its trial's and wave's first
+// place plus its rank among the wave's ballots, so that the owner finds it again.  Bound by
+// the latency of a workgroup's few dependent gathers: evaluating every candidate at every
+// trial took 60 us for a pass of one trial and 130 us for one of twelve over 1.3M
+// candidates (256 scenes), this 39 and 74 us (0.35M and 1.1M pairs evaluated).
+constexpr int kTrialItems = kChunkItems / kRedThreads;
+constexpr int kTrialBatch = 1024;  // pairs listed at a time
+__global__ __launch_bounds__(kRedThreads, 4) void trial_chunk_kernel(AbdScene sc, AbdParams P, TrialArgs T, Lists L,
+                                                                     int S, int K, const int64_t* __restrict__ seg,
+                                                                     const int64_t* __restrict__ choff,
+                                                                     double* __restrict__ part, int64_t part_stride) {
+    constexpr int kWaves = kRedThreads / kWave;
+    __shared__ double term[kTrialBatch];
+    __shared__ uint16_t pair[kTrialBatch];  // trial << 11 | candidate of the chunk
+    __shared__ int first[kMaxTrials * kWaves + 1];
+    __shared__ double wsum[kMaxTrials][kWaves];
+    __shared__ double sal[kMaxTrials];
+    static_assert(kChunkItems == 2048 && kMaxTrials <= 32, "a pair fits 16 bits");
+    static_assert(kMaxTrials * kWaves <= kWave, "one lane a (trial, wave)");
+    const int64_t c = blockIdx.x;
+    if (c >= choff[S]) return;
+    const ChunkRange r = chunk_range(S, seg, choff, c);
+    const int t = threadIdx.x, lane = lane_id(), w = wave_id();
+    const int nk = (K - (int)blockIdx.y + (int)gridDim.y - 1) / (int)gridDim.y;  // this workgroup's trials
+    if (t < nk) sal[t] = T.alpha[(int64_t)S * (blockIdx.y + t * gridDim.y) + r.s];
+    __syncthreads();
+    bool any = false;
+    for (int k = 0; k < nk; ++k) any |= !(sal[k] < 0.0);
+    double* const out = part + part_stride * blockIdx.y + c;
+    if (!any) {  // uniform: no trial of the scene is wanted, the neutral element of the sum
+        if (t < nk) out[part_stride * t * gridDim.y] = 0.0;
+        return;
+    }
+    const ListRef& Lr = L.l[r.l < kLists ? r.l : 0];
+    float apart[kTrialItems];
+#pragma unroll
+    for (int u = 0; u < kTrialItems; ++u) {
+        const int64_t i = r.start + u * kRedThreads + t;
+        apart[u] = i < r.end ? (Lr.apart ? Lr.apart[i] : 0.0f) : 4.0f;
+    }
+    // (trial, candidate) pairs of each wave, then their exclusive prefix sum over (trial, wave)
+    for (int k = 0; k < nk; ++k) {
+        const double al = sal[k];
+        int n = 0;
+        if (!(al < 0.0))
+#pragma unroll
+            for (int u = 0; u < kTrialItems; ++u) n += __popcll(__ballot(!(al < (double)apart[u])));
+        if (lane == 0) first[k * kWaves + w] = n;
+    }
+    __syncthreads();
+    if (w == 0) {
+        const int n = lane < nk * kWaves ? first[lane] : 0;
+        int incl = n;
+#pragma unroll
+        for (int off = 1; off < kWave; off <<= 1) {
+            const int y = __shfl_up(incl, off);
+            if (lane >= off) incl += y;
+        }
+        if (lane < nk * kWaves) first[lane] = incl - n;
+        if (lane == kWave - 1) first[nk * kWaves] = incl;
+    }
+    __syncthreads();
+    const SceneView V{sc.voff, sc.foff, sc.eoff, sc.tris, sc.edges, sc.x0};
+    const int width = width_of(Lr.kind);
+    const unsigned long long below = (1ull << lane) - 1ull;
+    // batches of whole trials, or of a part of one trial's pairs (its sums then carried on)
+    double acc = 0.0;
+    for (int k0 = 0, b0 = 0; k0 < nk;) {  // uniform
+        int k1 = k0 + 1;
+        while (k1 < nk && first[(k1 + 1) * kWaves] - b0 <= kTrialBatch) ++k1;
+        const int b1 = min(first[k1 * kWaves], b0 + kTrialBatch);
+        for (int k = k0; k < k1; ++k) {
+            const double al = sal[k];
+            if (al < 0.0) continue;
+            int at = first[k * kWaves + w] - b0;
+#pragma unroll
+            for (int u = 0; u < kTrialItems; ++u) {
+                const bool on = !(al < (double)apart[u]);
+                const unsigned long long m = __ballot(on);
+                const int q = at + __popcll(m & below);
+                if (on && q >= 0 && q < b1 - b0) pair[q] = (uint16_t)((k << 11) | (u * kRedThreads + t));
+                at += __popcll(m);
+            }
+        }
+        __syncthreads();
+        for (int q = t; q < b1 - b0; q += kRedThreads) {
+            const int64_t i = r.start + (pair[q] & 2047);
+            const int64_t k = blockIdx.y + (pair[q] >> 11) * gridDim.y;
+            const VertsTrial X{sc.x0, T.st + 12 * k * sc.n_bodies};
+            term[q] = energy_term(Lr.kind, sc, V, P, X, Lr.p + width * i, vids_of(Lr, i));
+        }
+        __syncthreads();
+        const bool whole = b1 == first[k1 * kWaves];  // the last trial of the batch ends in it
+        for (int k = k0; k < k1; ++k) {
+            const double al = sal[k];
+            if (!(al < 0.0)) {
+                int at = first[k * kWaves + w] - b0;
+#pragma unroll
+                for (int u = 0; u < kTrialItems; ++u) {
+                    const bool on = !(al < (double)apart[u]);
+                    const unsigned long long m = __ballot(on);
+                    const int q = at + __popcll(m & below);
+                    if (on && q >= 0 && q < b1 - b0) acc += term[q];
+                    at += __popcll(m);
+                }
+            }
+            if (whole || k + 1 < k1) {
+                const double v = wave_sum_down(acc);
+                if (lane == 0) wsum[k][w] = v;
+                acc = 0.0;
+            }
+        }
+        __syncthreads();
+        b0 = b1;
+        k0 = whole ? k1 : k1 - 1;
+    }
+    // the trials' sums with block_sum_fast's pairing (four waves of its sixteen: the shuffles
+    // by 8 and 4 add the empty waves' zeros, those by 2 and 1 give (w0 + w2) + (w1 + w3))
+    if (t < nk) out[part_stride * t * gridDim.y] = (wsum[t][0] + wsum[t][2]) + (wsum[t][1] + wsum[t][3]);
+}
+
 __global__ __launch_bounds__(kRedThreads) void scene_final_kernel(const int64_t* __restrict__ choff,
                                                                   const double* __restrict__ part,
-                                                                  double* __restrict__ out, int64_t part_stride,
-                                                                  int64_t out_stride) {
-    __shared__ double sh[kRedThreads];
-    part += part_stride * blockIdx.y;
-    out += out_stride * blockIdx.y;
+                                                                  double* __restrict__ out) {
+    __shared__ double sh[17];
     const int s = blockIdx.x;
     double acc = 0.0;
     for (int64_t i = choff[s] + threadIdx.x; i < choff[s + 1]; i += blockDim.x) acc += part[i];
@@ -281,9 +409,12 @@ __global__ __launch_bounds__(kRedThreads) void scene_final_kernel(const int64_t*
 // ---------------------------------------------------------------- CCD TOI
 // The scene minimum of the TOIs below 1 (ccd.py:9-40, abd.py:284-299) in two passes.
 // toi_scan_kernel: one candidate per thread (kToiSplit workgroups of kRedThreads per chunk
-// of the plan): the vertex-ground TOI directly, and for a PT / EE candidate its
-// coplanarity cubic and bracket test; the few candidates with a bracketed root in [0, 1]
-// go to a queue (one atomic per wave).  toi_solve_kernel: the full collision_time of each
+// of the plan): the vertex-ground TOI directly; a PT / EE candidate whose primitives some
+// axis keeps apart on the whole step (apart_until above 1, also stored for the line search)
+// has no contact, and the others, gathered side by side, take their coplanarity cubic and
+// bracket test; the few candidates with a bracketed root in [0, 1] go to a queue (one
+// atomic per wave).  1.3M candidates of 256 scenes: 74 us with the cubic for every one, 69 us
+// so (0.4M of them near), the gathers of eight vertices each being most of it.  toi_solve_kernel: the full collision_time of each
 // queued candidate (root searches and validity), its TOI below 1 min-ed into its scene's
 // slot (non-negative doubles order like their bit patterns, so an integer atomic min is
 // exact).  toi_final_kernel: per scene the minimum of its chunks' partials and its slot.
@@ -292,13 +423,6 @@ __global__ __launch_bounds__(kRedThreads) void scene_final_kernel(const int64_t*
 constexpr int kToiSplit = kChunkItems / kRedThreads;  // one candidate per thread
 constexpr int kToiSolveThreads = 64;
 constexpr int kToiSolveGrid = 2048;
-constexpr unsigned long long kBitsOne = 0x3FF0000000000000ull;  // 1.0
-
-__global__ void toi_init_kernel(int S, unsigned long long* __restrict__ slots, int32_t* __restrict__ qcount) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s < S) slots[s] = kBitsOne;
-    if (s == 0) *qcount = 0;
-}
 
 __device__ __forceinline__ double wave_min(double v) {
 #pragma unroll
@@ -317,39 +441,57 @@ __global__ __launch_bounds__(kRedThreads, 4) void toi_scan_kernel(AbdScene sc, A
                                                                double* __restrict__ part, int32_t* __restrict__ queue,
                                                                int32_t* __restrict__ qcount) {
     __shared__ double sh[kRedThreads / kWave];
+    __shared__ uint8_t near_id[kRedThreads];
+    __shared__ int near_count;
     const int64_t c = blockIdx.x;
     if (c >= choff[S]) return;  // uniform over the workgroup
-    const int s = scene_of_chunk(choff, S, c);
+    const ChunkRange r = chunk_range(S, seg, choff, c);
+    const bool on = !active || active[r.s];
+    if (threadIdx.x == 0) near_count = 0;
+    __syncthreads();
+    const SceneView V{sc.voff, sc.foff, sc.eoff, sc.tris, sc.edges, sc.x0};
+    const ListRef& Lr = L.l[r.l < kLists ? r.l : 0];
+    const int kind = Lr.kind, ck = kind == kListPT ? 0 : 1;
+    const int64_t i0 = r.start + (int64_t)blockIdx.y * kRedThreads, i = i0 + threadIdx.x;
+    const double dhat = fmax(P.dhat, sqrt(P.d2hat));  // the boxes' dilation, the barrier's range
     double acc = 1.0;
-    bool queued = false;
-    int32_t entry = 0;
-    if (!active || active[s]) {
-        int64_t k = c - choff[s];
-        int l = 0;
-        int64_t start = 0, end = 0;
-        for (; l < kLists; ++l) {
-            const int64_t a = seg[2 * (kLists * (int64_t)s + l)], b = seg[2 * (kLists * (int64_t)s + l) + 1];
-            const int64_t nch = n_chunks(b - a);
-            if (k < nch) {
-                start = a + k * kChunkItems;
-                end = start + kChunkItems < b ? start + kChunkItems : b;
-                break;
-            }
-            k -= nch;
-        }
-        const int64_t i = start + (int64_t)blockIdx.y * kRedThreads + threadIdx.x;
-        if (l < kLists && i < end) {
-            const int kind = L.l[l].kind;
-            const int32_t* t = L.l[l].p + (int64_t)width_of(kind) * i;
+    bool near = false;
+    if (r.l < kLists && i < r.end) {
+        float apart = 0.0f;
+        if (on) {
+            const int32_t* t = Lr.p + (int64_t)width_of(kind) * i;
             if (kind == kListVG) {
+                const int64_t vid = sc.voff[t[0]] + t[1];
+                apart = apart_until_vg(x0[3 * vid + 1], x1[3 * vid + 1], P.ground, dhat);
                 const double tv = cand_toi_vg(sc.voff, x0, x1, t, P.ground);
                 if (tv < 1.0) acc = tv;  // `if t < 1: atomic_min`
             } else {
-                const SceneView V{sc.voff, sc.foff, sc.eoff, sc.tris, sc.edges, sc.x0};
-                queued = cand_toi_bracketed(kind == kListPT ? 0 : 1, V, x0, x1, t, vids_of(L.l[l], i));
-                entry = (int32_t)((i << 1) | (kind == kListEE ? 1 : 0));
+                d3 a[4], b[4];
+                cand_verts(ck, V, x0, x1, t, a, b, vids_of(Lr, i));
+                apart = apart_until(ck, a, b, dhat);
+                near = !(apart > 1.0f);
             }
         }
+        if (Lr.apart) Lr.apart[i] = apart;
+    }
+    // the candidates that come near each other, side by side: the cubic and its bracket test
+    // only for these
+    {
+        const unsigned long long m = __ballot(near);
+        if (m) {
+            int base = 0;
+            if (lane_id() == 0) base = atomicAdd(&near_count, __popcll(m));
+            base = __shfl(base, 0);
+            if (near) near_id[base + __popcll(m & ((1ull << lane_id()) - 1ull))] = (uint8_t)threadIdx.x;
+        }
+    }
+    __syncthreads();
+    bool queued = false;
+    int32_t entry = 0;
+    if (threadIdx.x < near_count) {
+        const int64_t j = i0 + near_id[threadIdx.x];
+        queued = cand_toi_bracketed(ck, V, x0, x1, Lr.p + 5 * j, vids_of(Lr, j));
+        entry = (int32_t)((j << 1) | (kind == kListEE ? 1 : 0));
     }
     // wave-aggregated push of the queued candidates
     const unsigned long long mask = __ballot(queued);
@@ -365,9 +507,9 @@ __global__ __launch_bounds__(kRedThreads, 4) void toi_scan_kernel(AbdScene sc, A
     if (lane_id() == 0) sh[wave_id()] = wm;
     __syncthreads();
     if (threadIdx.x == 0) {
-        double r = sh[0];
-        for (int w = 1; w < kRedThreads / kWave; ++w) r = sh[w] < r ? sh[w] : r;
-        part[c * kToiSplit + blockIdx.y] = r;
+        double m = sh[0];
+        for (int w = 1; w < kRedThreads / kWave; ++w) m = sh[w] < m ? sh[w] : m;
+        part[c * kToiSplit + blockIdx.y] = m;
     }
 }
 
@@ -486,7 +628,7 @@ struct ReduceScratch {
 // The per-scene segments and chunk offsets of the lists: plan_in when given (made by
 // reduce_plan for these lists), else computed into plan_buf (nullable: the arena).
 int get_plan(hipStream_t s, const AbdScene& sc, int S, const Lists& L, const int64_t* plan_in,
-             const int64_t** seg, const int64_t** choff, int64_t* plan_buf = nullptr) {
+             const int64_t** seg, const int64_t** choff, int64_t* plan_buf = nullptr, ToiInit init = {}) {
     if (plan_in) {
         *seg = plan_in;
         *choff = plan_in + 2 * kLists * (size_t)S;
@@ -496,32 +638,36 @@ int get_plan(hipStream_t s, const AbdScene& sc, int S, const Lists& L, const int
     int rc = plan ? ABD_OK : arena_get(kSlotPlan, sizeof(int64_t) * reduce_plan_elems(S), (void**)&plan);
     if (rc) return rc;
     hipLaunchKernelGGL(plan_kernel, dim3(1), dim3(kPlanThreads), 0, s, S, sc.body_scene, L, plan,
-                       plan + 2 * kLists * (size_t)S);
+                       plan + 2 * kLists * (size_t)S, init);
     ABD_CHECK_LAUNCH();
     *seg = plan;
     *choff = plan + 2 * kLists * (size_t)S;
     return ABD_OK;
 }
 
-// Plan + chunks + per-scene sums (OP 0) over the lists; S = 1 treats the lists as one scene.
+// The arena's scene slots and queue count of the CCD.
+int toi_slots(int S, unsigned long long** slots, int32_t** qcount) {
+    const int rc = arena_get(kSlotToiSlots, sizeof(unsigned long long) * (size_t)(S + 1), (void**)slots);
+    if (!rc) *qcount = reinterpret_cast<int32_t*>(*slots + S);
+    return rc;
+}
+
+// Plan + chunks + per-scene energies over the lists at x; S = 1 treats the lists as one scene.
 // Algorithmic bytes: 128 per PT, 132 per EE and 32 per VG candidate.
-template <int OP>
-int seg_reduce(hipStream_t s, const AbdScene& sc, const AbdParams& P, int S, const double* x0, const double* x1,
-               const Lists& L, const int64_t* plan_in, double* out, int prof_id) {
+int seg_reduce(hipStream_t s, const AbdScene& sc, const AbdParams& P, int S, const double* x, const Lists& L,
+               double* out, int prof_id) {
     const int64_t bound = chunk_bound(L, S);
     if (bound > INT32_MAX) return ABD_ERR_ARG;
     const int64_t *seg, *choff;
     double* part = nullptr;
-    int rc = get_plan(s, sc, S, L, plan_in, &seg, &choff);
+    int rc = get_plan(s, sc, S, L, nullptr, &seg, &choff);
     if (!rc) rc = arena_get(kSlotReduce, sizeof(double) * (size_t)bound, (void**)&part);
     if (rc) return rc;
     int ph = prof_start_ext(prof_id, L.dn ? 1.0 : 128.0 * L.l[1].n + 132.0 * L.l[0].n + 32.0 * L.l[2].n);
-    prof_launch(ph, chunk_kernel<OP>, dim3((unsigned)bound), dim3(kRedThreads), 0, s, sc, P, x0, x1,
-                TrialArgs{nullptr, nullptr, nullptr, nullptr}, L, S, seg, choff, part, (int64_t)0);
+    prof_launch(ph, chunk_kernel, dim3((unsigned)bound), dim3(kRedThreads), 0, s, sc, P, x, L, S, seg, choff, part);
     ABD_CHECK_LAUNCH();
     if ((rc = prof_count_bytes(ph, s, L.dn, 128.0, 132.0, 32.0, 0.0))) return rc;
-    hipLaunchKernelGGL(scene_final_kernel<OP>, dim3(S), dim3(kRedThreads), 0, s, choff, part, out, (int64_t)0,
-                       (int64_t)0);
+    hipLaunchKernelGGL(scene_final_kernel, dim3(S), dim3(kRedThreads), 0, s, choff, (const double*)part, out);
     ABD_CHECK_LAUNCH();
     return ABD_OK;
 }
@@ -576,16 +722,12 @@ int toi_reduce(hipStream_t s, const AbdScene& sc, const AbdParams& P, int S, con
         int rc;
         if ((rc = arena_get(kSlotReduce, sizeof(double) * (size_t)(bound * kToiSplit), (void**)&w.part))) return rc;
         if ((rc = arena_get(kSlotToiQueue, sizeof(int32_t) * (size_t)(nq + 1), (void**)&w.queue))) return rc;
-        if ((rc = arena_get(kSlotToiSlots, sizeof(unsigned long long) * (size_t)(S + 1), (void**)&w.slots)))
-            return rc;
-        w.qcount = reinterpret_cast<int32_t*>(w.slots + S);
+        if ((rc = toi_slots(S, &w.slots, &w.qcount))) return rc;
     }
     const int64_t *seg, *choff;
-    int rc = get_plan(s, sc, S, L, plan_in, &seg, &choff, w.plan);
+    // (a plan made by reduce_plan has set the arena's slots)
+    int rc = get_plan(s, sc, S, L, plan_in, &seg, &choff, w.plan, ToiInit{w.slots, w.qcount});
     if (rc) return rc;
-    hipLaunchKernelGGL(toi_init_kernel, dim3((unsigned)ceil_div(S, kRedThreads)), dim3(kRedThreads), 0, s, S,
-                       w.slots, w.qcount);
-    ABD_CHECK_LAUNCH();
     // algorithmic bytes of the scan: tuple, indices and four vertices at both ends per PT / EE
     // candidate (224 / 228 B), tuple, offset and a vertex at both ends per VG candidate (56 B),
     // over the scenes it evaluates (counted on the device)
@@ -610,98 +752,70 @@ int toi_reduce(hipStream_t s, const AbdScene& sc, const AbdParams& P, int S, con
 // sum order of the energy; a minimum does not depend on it).  The switches of
 // const_params.py:42-44 drop a whole list.
 Lists contact_lists(const AbdParams& P, const int32_t* pt, int64_t npt, const int32_t* ee, int64_t nee,
-                    const int32_t* vg, int64_t nvg, const int64_t* dn = nullptr, VertIds vids = {}) {
+                    const int32_t* vg, int64_t nvg, const int64_t* dn = nullptr, CandSide vids = {}) {
     if (!P.pt) npt = 0;
     if (!P.ee) nee = 0;
     if (!P.vg) nvg = 0;
-    return Lists{{{ee, nee, kListEE, vids.ee}, {pt, npt, kListPT, vids.pt}, {vg, nvg, kListVG, nullptr}}, dn};
+    return Lists{{{ee, nee, kListEE, vids.ee, vids.apart_ee},
+                  {pt, npt, kListPT, vids.pt, vids.apart_pt},
+                  {vg, nvg, kListVG, nullptr, vids.apart_vg}},
+                 dn};
 }
 
 size_t reduce_plan_elems(int S) { return 2 * kLists * (size_t)S + (size_t)S + 1; }
 
 int reduce_plan(hipStream_t s, const AbdScene* sc, const AbdParams* P, int S, const int32_t* pt, int64_t npt,
-                const int32_t* ee, int64_t nee, const int32_t* vg, int64_t nvg, int64_t* plan, const int64_t* dn) {
+                const int32_t* ee, int64_t nee, const int32_t* vg, int64_t nvg, int64_t* plan, const int64_t* dn,
+                int64_t* zero, int nzero) {
     const Lists L = contact_lists(*P, pt, npt, ee, nee, vg, nvg, dn);
+    ToiInit init{nullptr, nullptr, zero, nzero};
+    if (int rc = toi_slots(S, &init.slots, &init.qcount)) return rc;
     hipLaunchKernelGGL(plan_kernel, dim3(1), dim3(kPlanThreads), 0, s, S, sc->body_scene, L, plan,
-                       plan + 2 * kLists * (size_t)S);
+                       plan + 2 * kLists * (size_t)S, init);
     ABD_CHECK_LAUNCH();
     return ABD_OK;
 }
 
 // ---------------------------------------------------------- line-search trials
 // K trial states q - alpha dq evaluated together (alpha: [K][S] on the device; S = 1
-// treats the scene as one): per scene the contact energy of every trial over the
-// candidate lists, each candidate's vertices placed at the trial state on the fly
-// (VertsTrial), and the inertia energy of every trial, with one plan of the lists for all.
-// E[2S k + s] is the contact energy and E[2S k + S + s] the inertia energy of scene s
-// at trial k, each bit-identical to the single-state reductions at that state.
+// treats the scene as one): per scene the chunks' contact energies of every trial, each
+// bit-identical to the chunk sums at that state.
 
-// scene_final_kernel<0> and the inertia energy of one (scene, trial) in one workgroup: the
-// contact energy from the trial's chunk partials (E[2 S k + s]) and the inertia energy at the
-// trial state (E[2 S k + S + s]), each with the arithmetic of its own kernel.
-__global__ __launch_bounds__(kRedThreads) void trial_energies_kernel(const int64_t* __restrict__ choff,
-                                                                     const double* __restrict__ part,
-                                                                     int64_t part_stride, int S,
-                                                                     const double* __restrict__ alpha,
-                                                                     const int32_t* __restrict__ sboff, int nb,
-                                                                     AbdParams P, const double* __restrict__ mass,
-                                                                     const double* __restrict__ I0v,
-                                                                     const double* __restrict__ A,
-                                                                     const double* __restrict__ p,
-                                                                     const double* __restrict__ dq,
-                                                                     const double* __restrict__ A0,
-                                                                     const double* __restrict__ p0,
-                                                                     const double* __restrict__ Adot,
-                                                                     const double* __restrict__ pdot,
-                                                                     double* __restrict__ E) {
-    __shared__ double sh[kRedThreads];
-    const int s = blockIdx.x, k = blockIdx.y;
-    part += part_stride * k;
-    double acc = 0.0;
-    for (int64_t i = choff[s] + threadIdx.x; i < choff[s + 1]; i += blockDim.x) acc += part[i];
-    const double rc = block_sum_fast(acc, sh);
-    if (threadIdx.x == 0) E[(int64_t)2 * S * k + s] = rc;
-    const double al = alpha[(int64_t)S * k + s];
-    if (al < 0.0) {  // skipped trial (uniform over the workgroup)
-        if (threadIdx.x == 0) E[(int64_t)2 * S * k + S + s] = 0.0;
-        return;
-    }
-    const int b0 = S > 1 ? sboff[s] : 0, b1 = S > 1 ? sboff[s + 1] : nb;
-    acc = 0.0;
-    for (int b = b0 + threadIdx.x; b < b1; b += blockDim.x) {
-        double Ab[9], pb[3];
-        trial_state(b, al, A, p, dq, Ab, pb);
-        acc += inertia_energy_q(P, mass, I0v, b, Ab, pb, A0, p0, Adot, pdot);
-    }
-    const double ri = block_sum_fast(acc, sh);
-    if (threadIdx.x == 0) E[(int64_t)2 * S * k + S + s] = ri;
+int trial_states(hipStream_t s, const AbdScene* sc, const AbdParams* P, int S, int K, const double* alpha, bool halve,
+                 const double* A, const double* p, const double* dq, const double* A0, const double* p0,
+                 const double* Adot, const double* pdot, double* st, double* e) {
+    const int64_t n = (int64_t)sc->n_bodies * K;
+    if (n <= 0) return ABD_OK;
+    hipLaunchKernelGGL(trial_states_kernel, dim3(grid_for(n, kRedThreads, INT32_MAX)), dim3(kRedThreads), 0, s, *sc,
+                       *P, S, K, alpha, halve ? 1 : 0, A, p, dq, A0, p0, Adot, pdot, st, e);
+    ABD_CHECK_LAUNCH();
+    return ABD_OK;
 }
 
-int line_trials(hipStream_t s, const AbdScene* sc, const AbdParams* P, int S, int K, const double* alpha,
-                const double* A, const double* p, const double* dq, const double* A0, const double* p0,
-                const double* Adot, const double* pdot, const int32_t* pt, int64_t npt, const int32_t* ee, int64_t nee,
-                const int32_t* vg, int64_t nvg, const int64_t* plan_in, double* E, const int64_t* dn, VertIds vids) {
+// workgroups of a line-search pass: twice what the device holds at once (four a CU)
+constexpr int64_t kTrialGrid = 2048;
+int line_chunks(hipStream_t s, const AbdScene* sc, const AbdParams* P, int S, int K, const double* alpha,
+                const double* st, const int32_t* pt, int64_t npt, const int32_t* ee, int64_t nee, const int32_t* vg,
+                int64_t nvg, const int64_t* plan, const int64_t* dn, CandSide vids, TrialSums* out) {
     int rc;
     const Lists L = contact_lists(*P, pt, npt, ee, nee, vg, nvg, dn, vids);
-    npt = L.l[1].n;
-    nee = L.l[0].n;
-    nvg = L.l[2].n;
     const int64_t bound = chunk_bound(L, S);
-    if (bound > INT32_MAX) return ABD_ERR_ARG;
+    if (bound > INT32_MAX || K < 1 || K > kMaxTrials || !plan) return ABD_ERR_ARG;
     const int64_t *seg, *choff;
     double* part;
-    if ((rc = get_plan(s, *sc, S, L, plan_in, &seg, &choff))) return rc;
+    if ((rc = get_plan(s, *sc, S, L, plan, &seg, &choff))) return rc;
     if ((rc = arena_get(kSlotReduce, sizeof(double) * (size_t)bound * K, (void**)&part))) return rc;
     // bytes: those of the (trial, scene) pairs evaluated, counted on the device
     int ph = prof_start_ext(kProfEnergy, 1.0);
-    prof_launch(ph, chunk_kernel<2>, dim3((unsigned)bound, K), dim3(kRedThreads), 0, s, *sc, *P,
-                (const double*)nullptr, (const double*)nullptr, TrialArgs{alpha, A, p, dq}, L, S, seg, choff,
-                part, bound);
+    // a workgroup's trials share its listing and fill its batches; a third of them each, or
+    // as many as leave the device kTrialGrid workgroups
+    const int64_t most = std::max<int64_t>(3, kTrialGrid / bound);
+    const unsigned groups = (unsigned)std::min<int64_t>(K, most);
+    prof_launch(ph, trial_chunk_kernel, dim3((unsigned)bound, groups), dim3(kRedThreads), 0, s, *sc, *P,
+                TrialArgs{alpha, st}, L, S, K, seg, choff, part, bound);
     ABD_CHECK_LAUNCH();
     if ((rc = attach_seg_bytes(ph, s, S, K, alpha, nullptr, seg, 132.0, 128.0, 32.0))) return rc;
-    hipLaunchKernelGGL(trial_energies_kernel, dim3(S, K), dim3(kRedThreads), 0, s, choff, (const double*)part, bound,
-                       S, alpha, sc->scene_boff, sc->n_bodies, *P, sc->mass, sc->I0, A, p, dq, A0, p0, Adot, pdot, E);
-    ABD_CHECK_LAUNCH();
+    *out = TrialSums{choff, part, bound};
     return ABD_OK;
 }
 
@@ -723,13 +837,13 @@ int contact_energy(hipStream_t s, const AbdScene* sc, const AbdParams* P, int S,
                    int64_t npt, const int32_t* ee, int64_t nee, const int32_t* vg, int64_t nvg, const int64_t* dn,
                    double* E) {
     const Lists L = contact_lists(*P, pt, npt, ee, nee, vg, nvg, dn);
-    return seg_reduce<0>(s, *sc, *P, S, xk, nullptr, L, nullptr, E, kProfEnergy);
+    return seg_reduce(s, *sc, *P, S, xk, L, E, kProfEnergy);
 }
 
 int scene_toi(hipStream_t s, const AbdScene* sc, const AbdParams* P, int S, const double* x_t0, const double* x_t1,
               const int32_t* pt, int64_t npt, const int32_t* ee, int64_t nee, const int32_t* vg, int64_t nvg,
               const int64_t* plan, double* toi, const uint8_t* active, const int64_t* dn, double* first_alpha,
-              VertIds vids, const SceneDots* dots) {
+              CandSide vids, const SceneDots* dots) {
     if (!P || !x_t0 || !x_t1 || !toi || npt < 0 || nee < 0 || nvg < 0) return ABD_ERR_ARG;
     if ((npt && !pt) || (nee && !ee) || (nvg && !vg)) return ABD_ERR_ARG;
     const Lists L = contact_lists(*P, pt, npt, ee, nee, vg, nvg, dn, vids);  // abd.py:288-299

@@ -16,6 +16,7 @@
 #include <cstring>
 #include <vector>
 
+#include "abd_block.h"
 #include "abd_internal.h"
 #include "abd_profile.h"
 
@@ -66,16 +67,19 @@ struct BoxBuf {
 // candidate tuples of one set of boxes.  The counts are exact when the set was culled
 // (exact: consumers take them from here); a set filtered on the device has its sizes at dn
 // ([nij, nij, npt, nee, nvg], device) and the counts here bound them.
-// With `vids`, the PT and EE tuples' scene vertex ids (4 each, VertIds) are kept beside them.
+// With `vids`, the PT and EE tuples' scene vertex ids (4 each, CandSide) are kept beside them.
 struct CandSet {
     DevBuf<int32_t> ij, ji, ptl, eel, vgl;
     DevBuf<int32_t> ptv, eev;
+    DevBuf<float> apt, aee, avg;  // the candidates' apart_until (the swept set's)
     int64_t nij = 0, npt = 0, nee = 0, nvg = 0;
     bool exact = true;
     bool vids = false;
     const int64_t* dn = nullptr;
     const int64_t* counts() const { return exact ? nullptr : dn; }
-    VertIds vertex_ids() const { return vids ? VertIds{ptv.p, eev.p} : VertIds{}; }
+    CandSide side() const {
+        return CandSide{vids ? ptv.p : nullptr, vids ? eev.p : nullptr, apt.p, aee.p, avg.p};
+    }
     int reserve_like(const CandSet& o, bool with_vids = false) {
         int rc = ij.reserve(2 * (size_t)o.nij + 2);
         if (!rc) rc = ji.reserve(2 * (size_t)o.nij + 2);
@@ -94,6 +98,9 @@ struct CandSet {
         vgl.release();
         ptv.release();
         eev.release();
+        apt.release();
+        aee.release();
+        avg.release();
     }
 };
 
@@ -132,7 +139,7 @@ struct Sim {
     // per-scene device values (one scene: a batch of one)
     int ns = 1, max_scene_bodies = 0;
     DevBuf<double> sv;          // [kSv][ns]
-    // the Newton / line-search state of every scene on the device (ls_decide_kernel): rows
+    // the Newton / line-search state of every scene on the device (ls_pass_kernel): rows
     // of the current iteration (lcur) and of the next, so that a step redone from a
     // recomputed swept set repeats the same decisions
     DevBuf<uint8_t> lsflag;     // [kLfRows][ns]
@@ -150,8 +157,9 @@ struct Sim {
     int32_t* hiters = nullptr;  // pinned [ns]: the iteration counts read back at a frame's end
     std::vector<int32_t> scene_it;  // Newton iterations of each scene in the last frame
     // line-search candidates evaluated together: states, vertices and per-candidate scalars
-    DevBuf<double> cand_E;          // [kLsSpec][2 ns] trial energies
     DevBuf<double> cand_alpha;      // [kLsSpec][ns]
+    DevBuf<double> trial_st;        // [1 + kLsSpec][nb][12] the bodies' trial states
+    DevBuf<double> trial_e;         // [1 + kLsSpec][nb] and inertia energies
     DevBuf<int64_t> plan;           // reduction plan of the swept candidate set (CCD + line search)
 };
 
@@ -159,7 +167,7 @@ struct Sim {
 // alpha/2, ..., alpha/2^(kLsSpec-1) of the backtracking loop (abd.py:146-160), whose
 // accept test depends only on each trial's own energy, so taking the first accepted
 // trial of a pass gives exactly the sequential loop's step.
-constexpr int kLsSpec = 12;
+constexpr int kLsSpec = kMaxTrials;
 
 // Trials a pass needs from step length a on: a, a/2, ... up to the first one below
 // alpha_min, which the loop accepts whatever its energy (at most kLsSpec; a pass that
@@ -196,11 +204,11 @@ enum {
     kCntLen = 32
 };
 // rows of Sim::lsflag (iterating: the current and the next iteration's; searching) and of
-// Sim::lsval (E0: the current and the next; the accepted trial's energy); the next
+// Sim::lsval (E0: the current and the next); the next
 // iteration's rows are copied over the current ones at the start of every iteration
 // (ls_commit_kernel)
 enum { kLfNewton = 0, kLfSearch = 2, kLfRows };
-enum { kLvE0 = 0, kLvE1 = 2, kLvRows };
+enum { kLvE0 = 0, kLvRows = 2 };
 
 // The EE, PT and VG candidate lists of one set of boxes (culling.py:32-76), culled side
 // by side so that their counts come back in two host synchronizations instead of five;
@@ -318,10 +326,13 @@ int collision_from(hipStream_t s, Sim& S, const CandSet& W, const double* xv) {
     if ((rc = abd_body_boxes(s, &S.sc, xv, dh, S.body.lo.p, S.body.hi.p))) return rc;
     if ((rc = S.col.reserve_like(W))) return rc;
     const KeepInput in{W.ij.p, W.ji.p, W.ptl.p, W.eel.p, W.vgl.p, W.nij, W.npt, W.nee, W.nvg, W.counts(),
-                       W.vertex_ids()};
+                       W.side()};
     const KeepBoxes bx{S.body.lo.p, S.body.hi.p, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
     const KeepOutput out{S.col.ij.p, S.col.ji.p, S.col.ptl.p, S.col.eel.p, S.col.vgl.p};
-    const KeepAtX at{xv, nullptr, S.P.dhat, dh, 0.0};
+    // (the swept set's entries apart at the accepted step length are dropped first)
+    const KeepAtX at{xv,   nullptr, S.P.dhat,
+                     dh,   0.0,     &W == &S.sw ? S.sv.p + kSvAlpha * S.ns : nullptr,
+                     S.ns > 1 ? S.sc.body_scene : nullptr};
     if ((rc = keep_from_superset(s, &S.sc, in, bx, S.P.dhat, S.P.ground, out, S.cnt.p + kCntCol, nullptr, false,
                                  &at)))
         return rc;
@@ -435,9 +446,12 @@ int swept_set_launch(hipStream_t s, Sim& S) {
     if ((rc = swept_boxes(s, &S.sc, -1, st.x, st.xk, dh, S.tbody.lo.p, S.tbody.hi.p, S.body.lo.p, S.body.hi.p)))
         return rc;
     if ((rc = S.sw.reserve_like(S.sup, S.sup.vids))) return rc;
+    if ((rc = S.sw.apt.reserve((size_t)S.sup.npt + 1))) return rc;
+    if ((rc = S.sw.aee.reserve((size_t)S.sup.nee + 1))) return rc;
+    if ((rc = S.sw.avg.reserve((size_t)S.sup.nvg + 1))) return rc;
     const CandSet& W = S.sup;
     const KeepInput in{W.ij.p, W.ji.p, W.ptl.p, W.eel.p, W.vgl.p, W.nij, W.npt, W.nee, W.nvg, W.counts(),
-                       W.vertex_ids()};
+                       W.side()};
     const KeepBoxes bx{S.tbody.lo.p, S.tbody.hi.p, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
     KeepOutput o{S.sw.ij.p, S.sw.ji.p, S.sw.ptl.p, S.sw.eel.p, S.sw.vgl.p};
     if (W.vids) {
@@ -474,7 +488,7 @@ void count_stats(Sim& S) {
 // stage covers every scene, and each scene keeps its own Newton loop, step length and
 // stopping test (abd.py:212-276).  A scene that has converged is masked out of the solve
 // and takes zero-length steps.  The line searches and the stopping tests run on the
-// device (ls_decide_kernel), so an iteration waits for the device once.
+// device (ls_pass_kernel), so an iteration waits for the device once.
 
 // The device rows of the Newton / line-search state for the current iteration.
 struct LsDev {
@@ -484,7 +498,6 @@ struct LsDev {
     uint8_t* search;        // scenes whose line search has not accepted a trial
     const double* E0;       // energy at the iteration's start (abd.py:225)
     double* E0_nxt;
-    double* E1;             // the accepted trial's energy
     double* dalpha;         // the accepted step length (0: a scene not iterating)
     const int32_t* it;      // Newton iterations of the frame so far
     int32_t* it_nxt;
@@ -503,7 +516,6 @@ LsDev ls_dev(Sim& S) {
     L.search = S.lsflag.p + (size_t)kLfSearch * ns;
     L.E0 = S.lsval.p + (size_t)(kLvE0 + c) * ns;
     L.E0_nxt = S.lsval.p + (size_t)(kLvE0 + n) * ns;
-    L.E1 = S.lsval.p + (size_t)kLvE1 * ns;
     L.dalpha = S.sv.p + (size_t)kSvAlpha * ns;
     L.it = S.lsit.p + (size_t)c * ns;
     L.it_nxt = S.lsit.p + (size_t)n * ns;
@@ -516,102 +528,81 @@ LsDev ls_dev(Sim& S) {
 
 constexpr int kLsThreads = 256;
 
-__device__ __forceinline__ int64_t ls_block_reduce(int64_t v, bool take_max, int64_t* sh) {
-    const int t = threadIdx.x;
-    sh[t] = v;
-    __syncthreads();
-    for (int w = kLsThreads / 2; w > 0; w >>= 1) {
-        if (t < w) sh[t] = take_max ? (sh[t] > sh[t + w] ? sh[t] : sh[t + w]) : sh[t] + sh[t + w];
-        __syncthreads();
-    }
-    const int64_t r = sh[0];
-    __syncthreads();
-    return r;
-}
-
-// One pass of every scene's line search (abd.py:146-160; the Armijo test as written, a
-// trial below alpha_min accepted whatever its energy), then the next pass's trials:
-// alpha [K][ns] holds this pass's step lengths (negative: not evaluated) and E [K][2 ns]
-// their contact and inertia energies (line_trials); a scene takes the first trial that
-// passes.  first: the pass of the first trial, over the iterating scenes (the others get
-// step length 0).  Then alpha [kLsSpec][ns] receives the next pass's trials of the scenes
-// still searching: a, a/2, ... from half the last rejected trial down to the first below
-// alpha_min (trials_to_floor), -1 elsewhere.  When no scene is searching any more, the
-// stopping test of every iterating scene (abd.py:265-268: g.g < tol or the iteration cap)
-// writes the next iteration's rows.  One workgroup.
-__global__ __launch_bounds__(kLsThreads) void ls_decide_kernel(LsDev L, double c1, double alpha_min, double tol,
-                                                                int max_iter, int first, int K,
-                                                                double* __restrict__ alpha,
-                                                                const double* __restrict__ E) {
-    __shared__ int64_t sh[kLsThreads];
-    const int ns = L.ns;
-    int64_t nsearch = 0, kmax = 0;
-    for (int s = threadIdx.x; s < ns; s += kLsThreads) {
-        bool searching = first ? L.newton[s] != 0 : L.search[s] != 0;
-        if (first && !searching) L.dalpha[s] = 0.0;
-        double a0 = 0.0;  // the next pass's first trial
-        if (searching) {
-            bool acc = false;
-            double last = 0.0;
-            const double e0 = L.E0[s], qtg = L.qtg[s];
-            for (int k = 0; k < K && !acc; ++k) {
-                const double a = alpha[(int64_t)k * ns + s];
-                if (a < 0.0) break;  // past this scene's trials
-                last = a;
-                const double e1 = E[2 * (int64_t)ns * k + s] + E[2 * (int64_t)ns * k + ns + s];
-                const bool wolfe = e1 < e0 + c1 * a * qtg;
-                if (wolfe || a < alpha_min) {
-                    acc = true;
-                    L.dalpha[s] = a;
-                    L.E1[s] = e1;
-                }
-            }
-            if (acc) {
-                searching = false;
-            } else {
-                a0 = last * 0.5;
+// One pass of a scene's line search (abd.py:146-160; the Armijo test as written, a trial
+// below alpha_min accepted whatever its energy): the energies of this pass's trials alpha
+// [K][ns] (negative: no further trial), one after the other up to the first that passes: the
+// contact energy from the chunks' sums C, the inertia energy from the bodies' e [K][nb],
+// each added as a reduction of its own would.  first: the pass of the first trial, over the
+// iterating scenes (the others get step length 0).  A scene that takes a trial has its
+// stopping test (abd.py:265-268: g.g < tol or the iteration cap) written to the next
+// iteration's rows; one that does not has its next pass's trials written to alpha
+// [kLsSpec][ns]: a, a/2, ... from half the last rejected trial down to the first below
+// alpha_min (trials_to_floor), -1 past them and for the scenes not searching.  One workgroup
+// per scene; the totals over the scenes are integers, added by atomics (zeroed before the
+// first pass).
+__global__ __launch_bounds__(kLsThreads) void ls_pass_kernel(LsDev L, double c1, double alpha_min, double tol,
+                                                              int max_iter, int first, int K,
+                                                              double* __restrict__ alpha, TrialSums C,
+                                                              const double* __restrict__ e,
+                                                              const int32_t* __restrict__ sboff, int nb) {
+    __shared__ double sh[34];
+    const int s = blockIdx.x, ns = L.ns, t = threadIdx.x;
+    const bool searching = first ? L.newton[s] != 0 : L.search[s] != 0;  // uniform
+    if (!searching) {
+        if (first) {
+            if (t < kLsSpec) alpha[(int64_t)t * ns + s] = -1.0;
+            if (t == 0) {
+                L.dalpha[s] = 0.0;
+                L.search[s] = 0;
+                L.E0_nxt[s] = L.E0[s];
+                L.it_nxt[s] = L.it[s];
+                L.newton_nxt[s] = 0;
             }
         }
-        L.search[s] = searching ? 1 : 0;
-        const int need = searching ? trials_to_floor(a0, alpha_min) : 0;
-        double ak = a0;  // a0, a0 / 2, ... in a register (no re-read of what was just written)
-        for (int k = 0; k < kLsSpec; ++k) {
-            alpha[(int64_t)k * ns + s] = k >= need ? -1.0 : ak;
-            ak *= 0.5;
-        }
-        nsearch += searching ? 1 : 0;
-        kmax = need > kmax ? need : kmax;
+        return;
     }
-    nsearch = ls_block_reduce(nsearch, false, sh);
-    kmax = ls_block_reduce(kmax, true, sh);
-    int64_t nact = 0, solver = 0;
-    if (nsearch == 0) {  // uniform: every line search has ended
-        for (int s = threadIdx.x; s < ns; s += kLsThreads) {
-            uint8_t nn = 0;
-            double e0 = L.E0[s];
-            int32_t itn = L.it[s];
-            if (L.newton[s]) {
-                e0 = L.E1[s];
-                itn += 1;
-                solver += L.iters[s] > 0 ? L.iters[s] : 0;
-                nn = (L.gtg[s] < tol || itn >= max_iter) ? 0 : 1;
-            }
-            L.E0_nxt[s] = e0;
-            L.it_nxt[s] = itn;
-            L.newton_nxt[s] = nn;
-            nact += nn;
-        }
-        nact = ls_block_reduce(nact, false, sh);
-        solver = ls_block_reduce(solver, false, sh);
+    const int b0 = sboff ? sboff[s] : 0, b1 = sboff ? sboff[s + 1] : nb;
+    const int64_t c0 = C.choff[s], c1_ = C.choff[s + 1];
+    const double e0 = L.E0[s], qtg = L.qtg[s];
+    double last = 0.0, e1 = 0.0;
+    bool acc = false;
+    for (int k = 0; k < K && !acc; ++k) {
+        const double a = alpha[(int64_t)k * ns + s];
+        if (a < 0.0) break;  // past this scene's trials
+        last = a;
+        double ec = 0.0, ei = 0.0;
+        for (int64_t i = c0 + t; i < c1_; i += kLsThreads) ec += C.part[C.stride * k + i];
+        for (int b = b0 + t; b < b1; b += kLsThreads) ei += e[(int64_t)nb * k + b];
+        block_sum2_fast(ec, ei, sh);
+        e1 = ec + ei;
+        const bool wolfe = e1 < e0 + c1 * a * qtg;
+        acc = wolfe || a < alpha_min;
     }
-    if (threadIdx.x == 0) {
-        L.cnt[kCntSearch] = nsearch;
-        L.cnt[first ? kCntK1 : kCntK2] = kmax;
-        if (nsearch == 0) {
-            L.cnt[kCntNewton] = nact;
-            L.cnt[kCntSolver] = solver;
-        }
+    __syncthreads();  // every thread has read this pass's trials
+    const double a0 = last * 0.5;  // the next pass's first trial
+    const int need = acc ? 0 : trials_to_floor(a0, alpha_min);
+    if (t < kLsSpec) {
+        double ak = a0;
+        for (int k = 0; k < t; ++k) ak *= 0.5;
+        alpha[(int64_t)t * ns + s] = t >= need ? -1.0 : ak;
     }
+    if (t != 0) return;
+    L.search[s] = acc ? 0 : 1;
+    unsigned long long* cnt = reinterpret_cast<unsigned long long*>(L.cnt);
+    if (!acc) {
+        if (first) atomicAdd(cnt + kCntSearch, 1ull);
+        atomicMax(cnt + (first ? kCntK1 : kCntK2), (unsigned long long)need);
+        return;
+    }
+    if (!first) atomicAdd(cnt + kCntSearch, ~0ull);  // one less
+    const int32_t itn = L.it[s] + 1, si = L.iters[s];
+    const uint8_t nn = (L.gtg[s] < tol || itn >= max_iter) ? 0 : 1;
+    L.dalpha[s] = last;
+    L.E0_nxt[s] = e1;
+    L.it_nxt[s] = itn;
+    L.newton_nxt[s] = nn;
+    if (nn) atomicAdd(cnt + kCntNewton, 1ull);
+    if (si > 0) atomicAdd(cnt + kCntSolver, (unsigned long long)si);
 }
 
 // A frame's start: E0 = the energy at q0 (abd.py:224-225), every scene iterating, no
@@ -681,20 +672,29 @@ int frame_start_scenes(hipStream_t s, Sim& S) {
     return ABD_OK;
 }
 
-// One line-search pass over every scene: the energies at q - alpha dq of the trials alpha
-// [K][ns] (device) over the swept candidate set of this iteration, into cand_E [K][2 ns]
-int line_pass(hipStream_t s, Sim& S, int K) {
-    const AbdSimState& st = S.st;
-    return line_trials(s, &S.sc, &S.P, S.ns, K, S.cand_alpha.p, st.A, st.p, st.dq, st.A0, st.p0, st.Adot, st.pdot,
-                       S.sw.ptl.p, S.sw.npt, S.sw.eel.p, S.sw.nee, S.sw.vgl.p, S.sw.nvg, S.plan.p, S.cand_E.p,
-                       S.sw.counts(), S.sw.vertex_ids());
-}
-
-int ls_decide(hipStream_t s, Sim& S, const LsDev& L, bool first, int K) {
-    hipLaunchKernelGGL(ls_decide_kernel, dim3(1), dim3(kLsThreads), 0, s, L, S.P.c1, S.P.alpha_min, S.P.tol,
-                       (int)S.P.max_iter, first ? 1 : 0, K, S.cand_alpha.p, (const double*)S.cand_E.p);
+// One line-search pass over every scene: the energies at q - alpha dq of the K trials (their
+// states from trial k0 of trial_st on) over the swept candidate set of this iteration, and
+// the scenes' decisions
+int line_pass(hipStream_t s, Sim& S, const LsDev& L, bool first, int K, int k0) {
+    int rc;
+    const int64_t nb = S.nb;
+    TrialSums C;
+    if ((rc = line_chunks(s, &S.sc, &S.P, S.ns, K, S.cand_alpha.p, S.trial_st.p + 12 * nb * k0, S.sw.ptl.p, S.sw.npt,
+                          S.sw.eel.p, S.sw.nee, S.sw.vgl.p, S.sw.nvg, S.plan.p, S.sw.counts(), S.sw.side(), &C)))
+        return rc;
+    hipLaunchKernelGGL(ls_pass_kernel, dim3(S.ns), dim3(kLsThreads), 0, s, L, S.P.c1, S.P.alpha_min, S.P.tol,
+                       (int)S.P.max_iter, first ? 1 : 0, K, S.cand_alpha.p, C,
+                       (const double*)(S.trial_e.p + nb * k0), S.ns > 1 ? S.sc.scene_boff : nullptr, S.nb);
     ABD_CHECK_LAUNCH();
     return ABD_OK;
+}
+
+// The trial states of K trials into trial_st from trial k0 on
+int pass_states(hipStream_t s, Sim& S, int K, bool halve, int k0) {
+    const AbdSimState& st = S.st;
+    const int64_t nb = S.nb;
+    return trial_states(s, &S.sc, &S.P, S.ns, K, S.cand_alpha.p, halve, st.A, st.p, st.dq, st.A0, st.p0, st.Adot,
+                        st.pdot, S.trial_st.p + 12 * nb * k0, S.trial_e.p + nb * k0);
 }
 
 int read_counts(hipStream_t s, Sim& S) {
@@ -720,7 +720,8 @@ int ccd_and_search_scenes(hipStream_t s, Sim& S, const LsDev& L) {
     const int ns = S.ns;
     const CandSet& W = S.sw;
     int rc;
-    if ((rc = reduce_plan(s, &S.sc, &P, ns, W.ptl.p, W.npt, W.eel.p, W.nee, W.vgl.p, W.nvg, S.plan.p, W.counts())))
+    if ((rc = reduce_plan(s, &S.sc, &P, ns, W.ptl.p, W.npt, W.eel.p, W.nee, W.vgl.p, W.nvg, S.plan.p, W.counts(),
+                          S.cnt.p + kCntNewton, kCntSolver - kCntNewton + 1)))
         return rc;
     // the TOI of the scenes still iterating and from it the first trial's step lengths; in the
     // same final pass q.g and g.g of the Armijo and stopping tests (abd.py:148,265: g and dq
@@ -735,14 +736,13 @@ int ccd_and_search_scenes(hipStream_t s, Sim& S, const LsDev& L) {
     qg.out1 = S.sv.p + kSvQtg * ns;
     qg.out2 = S.sv.p + kSvGtg * ns;
     if ((rc = scene_toi(s, &S.sc, &P, ns, st.x, st.xk, W.ptl.p, W.npt, W.eel.p, W.nee, W.vgl.p, W.nvg, S.plan.p,
-                        S.sv.p + kSvToi * ns, L.newton, W.counts(), S.cand_alpha.p, W.vertex_ids(), &qg)))
+                        S.sv.p + kSvToi * ns, L.newton, W.counts(), S.cand_alpha.p, W.side(), &qg)))
         return rc;
     // the line search: the first trial, then every remaining halving of the scenes that
     // rejected it, each decided on the device
-    if ((rc = line_pass(s, S, 1))) return rc;
-    if ((rc = ls_decide(s, S, L, true, 1))) return rc;
-    if ((rc = line_pass(s, S, kLsSpec))) return rc;
-    if ((rc = ls_decide(s, S, L, false, kLsSpec))) return rc;
+    if ((rc = pass_states(s, S, 1 + kLsSpec, true, 0))) return rc;
+    if ((rc = line_pass(s, S, L, true, 1, 0))) return rc;
+    if ((rc = line_pass(s, S, L, false, kLsSpec, 1))) return rc;
     ABD_CHECK(hipMemcpyAsync(S.hcnt, S.cnt.p, kCntLen * sizeof(int64_t), hipMemcpyDeviceToHost, s));
     return ABD_OK;
 }
@@ -916,8 +916,9 @@ int step_scenes(hipStream_t s, Sim& S) {
         // further passes: only when alpha_min lies more than kLsSpec halvings below a first trial
         while (S.hcnt[kCntSearch] > 0) {
             const int64_t K = S.hcnt[kCntK2];
-            if ((rc = line_pass(s, S, kLsSpec))) return rc;
-            if ((rc = ls_decide(s, S, L, false, kLsSpec))) return rc;
+            if ((rc = zero_fill(s, S.cnt.p + kCntK2, sizeof(int64_t)))) return rc;
+            if ((rc = pass_states(s, S, kLsSpec, false, 1))) return rc;
+            if ((rc = line_pass(s, S, L, false, kLsSpec, 1))) return rc;
             if ((rc = read_counts(s, S))) return rc;
             S.stats[5] += K;
         }
@@ -985,8 +986,9 @@ int abd_sim_create(const AbdScene* scene, const AbdParams* params, const AbdSimS
         rc = ABD_ERR_ARG;
     {
         const int nsc = scene->n_scenes > 1 ? scene->n_scenes : 1;
-        if (!rc) rc = S->cand_E.reserve(2 * (size_t)nsc * kLsSpec);
         if (!rc) rc = S->cand_alpha.reserve((size_t)nsc * kLsSpec);
+        if (!rc) rc = S->trial_st.reserve(12 * nb * (1 + kLsSpec));
+        if (!rc) rc = S->trial_e.reserve(nb * (1 + kLsSpec));
         if (!rc) rc = S->plan.reserve(reduce_plan_elems(nsc));
         if (!rc) rc = S->dcount.reserve(8);
         if (!rc) rc = S->cnt.reserve(kCntLen);
@@ -1201,7 +1203,8 @@ int abd_sim_destroy(void* sim) {
     S->lsflag.release();
     S->lsval.release();
     S->lsit.release();
-    S->cand_E.release();
+    S->trial_st.release();
+    S->trial_e.release();
     S->cand_alpha.release();
     S->plan.release();
     S->dcount.release();

@@ -49,3 +49,37 @@ def test_dense_contacts_one_wave_each(psd, n):
                 continue
             assert rel_err(g24[i], g) <= 1e-9
             assert rel_err(H24[i], np.block([[Hi, Hij], [Hij.T, Hj]])) <= 1e-9
+
+
+@pytest.mark.parametrize("nb,seed", [(2, 0), (3, 1), (9, 2)])
+def test_line_search_prunes_nothing_active(nb, seed):
+    """Frames whose line searches halve and whose steps are cut short by contacts: iterations
+    and energies of the native driver (which evaluates only the candidates that can be active
+    at a trial) against the oracle's, which evaluates every one.  1e-7, the drivers' bound."""
+    from abd_hip import scenes
+    from abd_hip.abd import AffineBodySimulator
+    from abd_hip.const_params import ContactParams
+    rng = np.random.default_rng(seed)
+    lib = [scenes.cube_mesh(), scenes.icosphere_mesh(1, 0.5), scenes.subdivided_box_mesh(2)]
+    meshes = [lib[k % 3] for k in range(nb)]
+    # columns of three with gaps of 1 to 1.3 dhat, thrown at each other
+    p, y = np.zeros((nb, 3)), {}
+    for b, (V, F) in enumerate(meshes):
+        c = b // 3
+        base = y.get(c, 0.0) + rng.uniform(1.0, 1.3) * 1e-3
+        p[b] = (1.5 * c + rng.uniform(-0.01, 0.01), base - V[:, 1].min(), rng.uniform(-0.01, 0.01))
+        y[c] = base + np.ptp(V[:, 1])
+    pdot = rng.uniform(-0.3, 0.3, (nb, 3))
+    spec = scenes.build_scene(meshes, np.stack([np.eye(3)] * nb), p, np.zeros((nb, 3, 3)), pdot, ground=0.0)
+    cp = ContactParams(ground=0.0, psd=1, solver=3)
+    sim = AffineBodySimulator(spec, cp, native=True)
+    ref = O.OracleSim(spec, cp)
+    for f in range(3):
+        n = sim.step(f)
+        before = int(ref.stats[0])
+        ref.step()
+        assert n == int(ref.stats[0]) - before
+    torch.cuda.synchronize()
+    assert np.abs(sim.states.A.cpu().numpy() - ref.A).max() <= 1e-7
+    assert np.abs(sim.states.p.cpu().numpy() - ref.p).max() <= 1e-7
+    assert sim.stats["energy_evals"] > sim.stats["newton_iters"] + 3  # some search halved
