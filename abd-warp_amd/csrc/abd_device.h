@@ -414,13 +414,10 @@ __device__ __forceinline__ void cand_verts(int kind, const SceneView& S, const d
         b[q] = ld3(x1 + 3 * vi[q]);
     }
 }
-// Whether collision_time of the candidate can be below 1: its coplanarity cubic has a
-// bracketed root in [0, 1] (cubic_bracket); otherwise it has no root and its TOI is 1.
-__device__ __forceinline__ bool cand_toi_bracketed(int kind, const SceneView& S, const double* __restrict__ x0,
-                                                   const double* __restrict__ x1, const int32_t* t,
-                                                   const int32_t* vid = nullptr) {
-    d3 a[4], b[4];
-    cand_verts(kind, S, x0, x1, t, a, b, vid);
+// Whether collision_time of the step a -> b of a candidate's vertices can be below 1: its
+// coplanarity cubic has a bracketed root in [0, 1] (cubic_bracket); otherwise it has no root
+// and its TOI is 1.
+__device__ __forceinline__ bool toi_bracketed(const d3 a[4], const d3 b[4]) {
     double coef[4];
     coplanar_poly(a, b, coef);
     return cubic_bracket(coef, 0.0, 1.0).kind != CubicBracket::kNone;
@@ -429,55 +426,52 @@ __device__ __forceinline__ bool cand_toi_bracketed(int kind, const SceneView& S,
 // active on the step a -> b of its vertices: below it some axis separates the two
 // primitives by more than dhat, so the barrier is zero, and their boxes dilated as the
 // collision set's (FP32 rounding included) do not overlap; above 1 they are apart on the
-// whole step, so its CCD finds no contact either.  Along an axis the gap between the boxes
+// whole step.  Along an axis the gap between the boxes
 // is concave in the step length (a minimum of linear functions minus a maximum), so from a
-// positive gap at the start it stays above the chord to the gap at the end.  The margins:
-// 1e-3 dhat for the rounding of positions on the step, 5e-7 of the coordinates for the
-// boxes' casts (four roundings of 2^-24), the boxes' motion over the tolerance of the CCD's
-// roots.  NaN or infinite coordinates give 0.
-__device__ __forceinline__ float chord_zero(double u0, double u1, float best) {
-    if (!(u0 > 0.0)) return best;
-    const float f0 = (float)u0, f1 = (float)u1;
-    const float t = u1 > 0.0 ? 2.0f : f0 / (f0 - f1);
+// positive gap at the start it stays above the chord to the gap at the end.  In FP32 on the
+// differences to one vertex.  The margins: 1e-3 dhat for the rounding of positions on the
+// step, 1e-6 of the differences for FP32, 5e-7 of the coordinates for the boxes' casts (four
+// roundings of 2^-24).  NaN or infinite coordinates give 0.
+__device__ __forceinline__ float chord_zero(float u0, float u1, float best) {
+    if (!(u0 > 0.0f)) return best;
+    const float t = u1 > 0.0f ? 2.0f : u0 / (u0 - u1);
     return t > best ? t : best;
 }
+constexpr float kApartShrink = 1.0f - 4e-6f;  // below the chord's zero whatever its roundings
 __device__ __forceinline__ float apart_until(int kind, const d3 a[4], const d3 b[4], double dhat) {
     float best = 0.0f;
+    const float dh = 1.001f * (float)dhat;
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-        double l[2][2], h[2][2];  // [end][primitive]
+        const double ref = comp(a[0], k);
+        float l[2][2], h[2][2];  // [end][primitive]
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
             const d3* v = e ? b : a;
-            const double c0 = comp(v[0], k), c1 = comp(v[1], k), c2 = comp(v[2], k), c3 = comp(v[3], k);
-            const double m23 = c2 < c3 ? c2 : c3, x23 = c2 < c3 ? c3 : c2;
-            if (kind == 0) {
-                l[e][0] = h[e][0] = c0;
-                l[e][1] = c1 < m23 ? c1 : m23;
-                h[e][1] = c1 > x23 ? c1 : x23;
-            } else {
-                l[e][0] = c0 < c1 ? c0 : c1;
-                h[e][0] = c0 < c1 ? c1 : c0;
-                l[e][1] = m23;
-                h[e][1] = x23;
-            }
+            const float c0 = (float)(comp(v[0], k) - ref), c1 = (float)(comp(v[1], k) - ref),
+                        c2 = (float)(comp(v[2], k) - ref), c3 = (float)(comp(v[3], k) - ref);
+            const float m23 = fminf(c2, c3), x23 = fmaxf(c2, c3);
+            l[e][0] = kind == 0 ? c0 : fminf(c0, c1);
+            h[e][0] = kind == 0 ? c0 : fmaxf(c0, c1);
+            l[e][1] = kind == 0 ? fminf(c1, m23) : m23;
+            h[e][1] = kind == 0 ? fmaxf(c1, x23) : x23;
         }
-        double m = 0.0, move = 0.0;
+        float m = 0.0f;
 #pragma unroll
-        for (int p = 0; p < 2; ++p) {
-            m = fmax(m, fmax(fmax(fabs(l[0][p]), fabs(h[0][p])), fmax(fabs(l[1][p]), fabs(h[1][p]))));
-            move += fmax(fabs(l[1][p] - l[0][p]), fabs(h[1][p] - h[0][p]));
-        }
-        const double d = 1.001 * dhat + 5e-7 * m + 4.0 * kXError * move;
+        for (int p = 0; p < 2; ++p)
+            m = fmaxf(m, fmaxf(fmaxf(-l[0][p], h[0][p]), fmaxf(-l[1][p], h[1][p])));
+        const float d = dh + 1e-6f * m + 5e-7f * (fabsf((float)ref) + m);
         best = chord_zero((l[0][1] - h[0][0]) - d, (l[1][1] - h[1][0]) - d, best);
         best = chord_zero((l[0][0] - h[0][1]) - d, (l[1][0] - h[1][1]) - d, best);
     }
-    return best * (1.0f - 2e-6f);  // below the chord's zero whatever its roundings
+    return best * kApartShrink;
 }
 // The same of a vertex above the ground (its height y0 -> y1).
 __device__ __forceinline__ float apart_until_vg(double y0, double y1, double ground, double dhat) {
-    const double d = 1.001 * dhat + 5e-7 * fmax(fabs(ground), fmax(fabs(y0), fabs(y1)));
-    return chord_zero((y0 - ground) - d, (y1 - ground) - d, 0.0f) * (1.0f - 2e-6f);
+    const float u0 = (float)(y0 - ground), u1 = (float)(y1 - ground);
+    const float m = fmaxf(fabsf(u0), fabsf(u1));
+    const float d = 1.001f * (float)dhat + 1e-6f * m + 5e-7f * (fabsf((float)ground) + m);
+    return chord_zero(u0 - d, u1 - d, 0.0f) * kApartShrink;
 }
 __device__ __forceinline__ double cand_toi_vg(const int32_t* __restrict__ voff, const double* __restrict__ x0,
                                               const double* __restrict__ x1, const int32_t* t2, double ground) {

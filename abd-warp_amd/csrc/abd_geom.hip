@@ -31,173 +31,6 @@ __global__ __launch_bounds__(kBlock) void project_kernel(const int32_t* __restri
     }
 }
 
-// The end of a step, x = x(q - alpha dq): per vertex the body's state with the arithmetic of
-// update_q_kernel (one alpha_host) or of update_q_scenes_kernel (alpha_dev per scene, or
-// alpha_host for the scenes in `active` and 0 for the others; a scene with alpha 0 keeps its
-// state bit for bit), placed as project_kernel does.  With lo / hi, the range test of
-// within_ranges on this end and on x_other: *flag = gen when some coordinate leaves them.
-__global__ __launch_bounds__(kBlock) void project_step_kernel(const int32_t* __restrict__ vert_body,
-                                                               const int32_t* __restrict__ body_scene,
-                                                               const double* __restrict__ x0,
-                                                               const double* __restrict__ A,
-                                                               const double* __restrict__ p,
-                                                               const double* __restrict__ dq,
-                                                               const double* __restrict__ alpha_dev,
-                                                               double alpha_host,
-                                                               const uint8_t* __restrict__ active,
-                                                               double* __restrict__ x,
-                                                               const double* __restrict__ x_other,
-                                                               const double* __restrict__ lo,
-                                                               const double* __restrict__ hi,
-                                                               int64_t* __restrict__ flag, int64_t gen, int64_t nv) {
-    bool out = false;
-    for (int64_t v = (int64_t)blockIdx.x * kBlock + threadIdx.x; v < nv; v += (int64_t)gridDim.x * kBlock) {
-        const int b = vert_body[v];
-        double pb[3], Ab[9];
-        if (alpha_dev || active) {
-            const int sc = body_scene ? body_scene[b] : 0;
-            const double al = alpha_dev ? alpha_dev[sc] : (active[sc] ? alpha_host : 0.0);
-#pragma unroll
-            for (int r = 0; r < 3; ++r) pb[r] = al == 0.0 ? p[3 * b + r] : p[3 * b + r] - dq[3 * (4 * b) + r] * al;
-#pragma unroll
-            for (int r = 0; r < 9; ++r)
-                Ab[r] = al == 0.0 ? A[9 * b + r] : A[9 * b + r] - dq[3 * (4 * b + 1 + r / 3) + r % 3] * al;
-        } else {
-#pragma unroll
-            for (int r = 0; r < 3; ++r) pb[r] = p[3 * b + r] - dq[3 * (4 * b) + r] * alpha_host;
-#pragma unroll
-            for (int r = 0; r < 9; ++r) Ab[r] = A[9 * b + r] - dq[3 * (4 * b + 1 + r / 3) + r % 3] * alpha_host;
-        }
-        const double r0 = x0[3 * v], r1 = x0[3 * v + 1], r2 = x0[3 * v + 2];
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            double r = pb[k] + r0 * Ab[k];
-            r = r + r1 * Ab[3 + k];
-            r = r + r2 * Ab[6 + k];
-            x[3 * v + k] = r;
-            if (lo) {
-                const double l = lo[3 * v + k], h = hi[3 * v + k], o = x_other[3 * v + k];
-                out |= !(r >= l && r <= h && o >= l && o <= h);  // NaN counts as outside
-            }
-        }
-    }
-    if (lo && __any(out) && lane_id() == 0) *flag = gen;  // every writer stores gen
-}
-
-// The body state of a step's end for project_step2_kernel: project_step_kernel's arithmetic.
-__device__ __forceinline__ void step_end_body(int b, const int32_t* __restrict__ body_scene,
-                                              const double* __restrict__ A, const double* __restrict__ p,
-                                              const double* __restrict__ dq, const double* __restrict__ alpha_dev,
-                                              double alpha_host, const uint8_t* __restrict__ active, double pb[3],
-                                              double Ab[9]) {
-    if (alpha_dev || active) {
-        const int sc = body_scene ? body_scene[b] : 0;
-        const double al = alpha_dev ? alpha_dev[sc] : (active[sc] ? alpha_host : 0.0);
-#pragma unroll
-        for (int r = 0; r < 3; ++r) pb[r] = al == 0.0 ? p[3 * b + r] : p[3 * b + r] - dq[3 * (4 * b) + r] * al;
-#pragma unroll
-        for (int r = 0; r < 9; ++r)
-            Ab[r] = al == 0.0 ? A[9 * b + r] : A[9 * b + r] - dq[3 * (4 * b + 1 + r / 3) + r % 3] * al;
-    } else {
-#pragma unroll
-        for (int r = 0; r < 3; ++r) pb[r] = p[3 * b + r] - dq[3 * (4 * b) + r] * alpha_host;
-#pragma unroll
-        for (int r = 0; r < 9; ++r) Ab[r] = A[9 * b + r] - dq[3 * (4 * b + 1 + r / 3) + r % 3] * alpha_host;
-    }
-}
-
-// project_step_kernel over vertex pairs (2i, 2i + 1): the pair's six coordinates of x0, the ranges,
-// x_other and x as three 16-byte accesses each (the arrays 16-byte aligned), the body state computed
-// again for the second vertex only when it is of another body; an odd last vertex is the last
-// thread's.  Same
-// arithmetic, same results.
-typedef double dvec2 __attribute__((ext_vector_type(2)));
-__global__ __launch_bounds__(kBlock) void project_step2_kernel(const int32_t* __restrict__ vert_body,
-                                                                const int32_t* __restrict__ body_scene,
-                                                                const double* __restrict__ x0,
-                                                                const double* __restrict__ A,
-                                                                const double* __restrict__ p,
-                                                                const double* __restrict__ dq,
-                                                                const double* __restrict__ alpha_dev,
-                                                                double alpha_host,
-                                                                const uint8_t* __restrict__ active,
-                                                                double* __restrict__ x,
-                                                                const double* __restrict__ x_other,
-                                                                const double* __restrict__ lo,
-                                                                const double* __restrict__ hi,
-                                                                int64_t* __restrict__ flag, int64_t gen, int64_t nv) {
-    bool out = false;
-    const int64_t npair = (nv + 1) / 2;
-    for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < npair; i += (int64_t)gridDim.x * kBlock) {
-        const int64_t v0 = 2 * i;
-        const bool two = v0 + 1 < nv;
-        const int b0 = vert_body[v0], b1 = two ? vert_body[v0 + 1] : b0;
-        double c[6], l[6], h[6], o[6], rr[6];
-        if (two) {
-            const dvec2* X0 = reinterpret_cast<const dvec2*>(x0 + 3 * v0);
-#pragma unroll
-            for (int q = 0; q < 3; ++q) {
-                const dvec2 a = X0[q];
-                c[2 * q] = a.x;
-                c[2 * q + 1] = a.y;
-            }
-            if (lo) {
-                const dvec2 *L = reinterpret_cast<const dvec2*>(lo + 3 * v0), *H = reinterpret_cast<const dvec2*>(hi + 3 * v0),
-                            *O = reinterpret_cast<const dvec2*>(x_other + 3 * v0);
-#pragma unroll
-                for (int q = 0; q < 3; ++q) {
-                    const dvec2 a = L[q], b = H[q], e = O[q];
-                    l[2 * q] = a.x;
-                    l[2 * q + 1] = a.y;
-                    h[2 * q] = b.x;
-                    h[2 * q + 1] = b.y;
-                    o[2 * q] = e.x;
-                    o[2 * q + 1] = e.y;
-                }
-            }
-        } else {
-#pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                c[k] = x0[3 * v0 + k];
-                c[3 + k] = 0.0;
-                if (lo) {
-                    l[k] = lo[3 * v0 + k];
-                    h[k] = hi[3 * v0 + k];
-                    o[k] = x_other[3 * v0 + k];
-                }
-            }
-        }
-        // one body state in registers: vertex 1's is computed over vertex 0's when they differ
-        double pb[3], Ab[9];
-        step_end_body(b0, body_scene, A, p, dq, alpha_dev, alpha_host, active, pb, Ab);
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            if (u == 1 && b1 != b0) step_end_body(b1, body_scene, A, p, dq, alpha_dev, alpha_host, active, pb, Ab);
-            const double r0 = c[3 * u], r1 = c[3 * u + 1], r2 = c[3 * u + 2];
-#pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                double r = pb[k] + r0 * Ab[k];
-                r = r + r1 * Ab[3 + k];
-                r = r + r2 * Ab[6 + k];
-                rr[3 * u + k] = r;
-                if (lo && (u == 0 || two)) {
-                    const int j = 3 * u + k;
-                    out |= !(r >= l[j] && r <= h[j] && o[j] >= l[j] && o[j] <= h[j]);  // NaN counts as outside
-                }
-            }
-        }
-        if (two) {
-            dvec2* Xo = reinterpret_cast<dvec2*>(x + 3 * v0);
-#pragma unroll
-            for (int q = 0; q < 3; ++q) Xo[q] = dvec2{rr[2 * q], rr[2 * q + 1]};
-        } else {
-#pragma unroll
-            for (int k = 0; k < 3; ++k) x[3 * v0 + k] = rr[k];
-        }
-    }
-    if (lo && __any(out) && lane_id() == 0) *flag = gen;  // every writer stores gen
-}
-
 // abd.py:337-353
 __global__ void update_q_kernel(int nb, const double* __restrict__ A, const double* __restrict__ p,
                                 const double* __restrict__ dq, double alpha, double* A_out, double* p_out,
@@ -396,25 +229,19 @@ __global__ __launch_bounds__(kBlock) void swept_prim_boxes_kernel(const int32_t*
         }
     }
 }
-// plo / phi (nullable): the body boxes at x0 already computed with the same dilation (the
-// collision set's), read instead of recomputed — the same values.
 __global__ __launch_bounds__(kBlock) void swept_body_boxes_kernel(int nb, const int32_t* __restrict__ voff,
                                                                    const double* __restrict__ x0,
                                                                    const double* __restrict__ x1, double dil,
-                                                                   const float* __restrict__ plo,
-                                                                   const float* __restrict__ phi,
                                                                    float* __restrict__ lo, float* __restrict__ hi) {
     const int b = blockIdx.x * (kBlock / kWave) + wave_id();
     if (b >= nb) return;  // the whole wave (no barrier)
     double mn0[3], mx0[3], mn1[3], mx1[3];
-    if (!plo) wave_extrema(x0, voff[b], voff[b + 1], mn0, mx0);
+    wave_extrema(x0, voff[b], voff[b + 1], mn0, mx0);
     wave_extrema(x1, voff[b], voff[b + 1], mn1, mx1);
     if (lane_id() == 0)
         for (int k = 0; k < 3; ++k) {
-            const float l0 = plo ? plo[3 * b + k] : (float)(mn0[k] - dil);
-            const float h0 = phi ? phi[3 * b + k] : (float)(mx0[k] + dil);
-            lo[3 * b + k] = fminf(l0, (float)(mn1[k] - dil));
-            hi[3 * b + k] = fmaxf(h0, (float)(mx1[k] + dil));
+            lo[3 * b + k] = fminf((float)(mn0[k] - dil), (float)(mn1[k] - dil));
+            hi[3 * b + k] = fmaxf((float)(mx0[k] + dil), (float)(mx1[k] + dil));
         }
 }
 
@@ -439,27 +266,6 @@ __global__ void update_q_scenes_kernel(int nb, const int32_t* __restrict__ body_
     }
     *out = v;
     if (out2) *out2 = v;
-}
-
-int project_step(hipStream_t s, const AbdScene* sc, const double* A, const double* p, const double* dq,
-                 const double* alpha_dev, double alpha_host, const uint8_t* active, double* x_out,
-                 const double* x_other, const double* lo, const double* hi, int64_t* flag, int64_t gen) {
-    if (sc->n_verts == 0) return ABD_OK;
-    // vertex pairs with 16-byte accesses when every array allows them
-    const auto a16 = [](const void* q) { return q == nullptr || ((uintptr_t)q & 15) == 0; };
-    if (a16(sc->x0) && a16(x_out) && a16(x_other) && a16(lo) && a16(hi)) {
-        hipLaunchKernelGGL(project_step2_kernel, dim3(grid_for(((int64_t)sc->n_verts + 1) / 2, kBlock, 1 << 20)),
-                           dim3(kBlock), 0, s, sc->vert_body, sc->n_scenes > 1 ? sc->body_scene : nullptr, sc->x0,
-                           A, p, dq, alpha_dev, alpha_host, active, x_out, x_other, lo, hi, flag, gen,
-                           (int64_t)sc->n_verts);
-        ABD_CHECK_LAUNCH();
-        return ABD_OK;
-    }
-    hipLaunchKernelGGL(project_step_kernel, dim3(grid_for(sc->n_verts, kBlock, 1 << 20)), dim3(kBlock), 0, s,
-                       sc->vert_body, sc->n_scenes > 1 ? sc->body_scene : nullptr, sc->x0, A, p, dq, alpha_dev,
-                       alpha_host, active, x_out, x_other, lo, hi, flag, gen, (int64_t)sc->n_verts);
-    ABD_CHECK_LAUNCH();
-    return ABD_OK;
 }
 
 // q_out = q - alpha dq, also written to (A_out2, p_out2) when they are given
@@ -492,16 +298,15 @@ __global__ __launch_bounds__(kBlock) void vertex_ranges_kernel(int64_t n3, const
     }
 }
 
-__global__ __launch_bounds__(kBlock) void within_ranges_kernel(int64_t n3, const double* __restrict__ x0,
-                                                                const double* __restrict__ x1,
+__global__ __launch_bounds__(kBlock) void within_ranges_kernel(int64_t n3, const double* __restrict__ x,
                                                                 const double* __restrict__ lo,
-                                                                const double* __restrict__ hi,
+                                                                const double* __restrict__ hi, double margin,
+                                                                const double* __restrict__ r,
+                                                                const double* __restrict__ r0,
                                                                 int64_t* __restrict__ flag) {
     bool out = false;
-    for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n3; i += (int64_t)gridDim.x * kBlock) {
-        const double a = x0[i], b = x1[i], l = lo[i], h = hi[i];
-        out |= !(a >= l && a <= h && b >= l && b <= h);  // NaN counts as outside
-    }
+    for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n3; i += (int64_t)gridDim.x * kBlock)
+        out |= !(x[i] - margin >= lo[i] && x[i] + margin <= hi[i] && r[i] == r0[i]);  // NaN: outside
     if (__any(out) && lane_id() == 0) *flag = 1;  // every writer stores 1
 }
 
@@ -513,18 +318,17 @@ int vertex_ranges(hipStream_t s, int64_t n3, const double* x0, const double* x1,
     return ABD_OK;
 }
 
-int within_ranges(hipStream_t s, int64_t n3, const double* x0, const double* x1, const double* lo, const double* hi,
-                  int64_t* flag) {
+int within_ranges(hipStream_t s, int64_t n3, const double* x, const double* lo, const double* hi, double margin,
+                  const double* r, const double* r0, int64_t* flag) {
     if (n3 <= 0) return ABD_OK;
-    hipLaunchKernelGGL(within_ranges_kernel, dim3(grid_for(n3, kBlock, 4096)), dim3(kBlock), 0, s, n3, x0, x1, lo,
-                       hi, flag);
+    hipLaunchKernelGGL(within_ranges_kernel, dim3(grid_for(n3, kBlock, 4096)), dim3(kBlock), 0, s, n3, x, lo, hi,
+                       margin, r, r0, flag);
     ABD_CHECK_LAUNCH();
     return ABD_OK;
 }
 
 int swept_boxes(hipStream_t s, const AbdScene* sc, int kind, const double* x0, const double* x1, double dil,
-                float* lo, float* hi, const float* plo, const float* phi) {
-    if (!plo != !phi || (plo && kind != -1)) return ABD_ERR_ARG;
+                float* lo, float* hi) {
     if (kind == ABD_KIND_POINT) {
         if (!sc->n_verts) return ABD_OK;
         hipLaunchKernelGGL(swept_point_boxes_kernel, dim3(grid_for(3 * (int64_t)sc->n_verts)), dim3(kBlock), 0, s, x0,
@@ -540,7 +344,7 @@ int swept_boxes(hipStream_t s, const AbdScene* sc, int kind, const double* x0, c
     } else if (kind == -1) {
         if (!sc->n_bodies) return ABD_OK;
         hipLaunchKernelGGL(swept_body_boxes_kernel, dim3((unsigned)ceil_div(sc->n_bodies, kBlock / kWave)),
-                           dim3(kBlock), 0, s, sc->n_bodies, sc->voff, x0, x1, dil, plo, phi, lo, hi);
+                           dim3(kBlock), 0, s, sc->n_bodies, sc->voff, x0, x1, dil, lo, hi);
     } else {
         return ABD_ERR_ARG;
     }

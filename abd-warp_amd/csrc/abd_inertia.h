@@ -52,6 +52,51 @@ __device__ __forceinline__ double inertia_energy_body(const AbdParams& P, const 
                                                       const double* __restrict__ pdot) {
     return inertia_energy_q(P, mass, I0v, b, Ak + 9 * b, pk + 3 * b, A0, p0, Adot, pdot);
 }
+// Row e of body b's inertia gradient (orthogonal_energy.py:99-112; e 0: p, 1..3: the rows of
+// A) at its state (A, p), A0 .. pdot of the body.
+__device__ __forceinline__ void inertia_gradient_row(const AbdParams& P, int e, const double* A, const double* p,
+                                                     const double* __restrict__ A0, const double* __restrict__ p0,
+                                                     const double* __restrict__ Adot,
+                                                     const double* __restrict__ pdot, double m, double i0,
+                                                     double g[3]) {
+    double At[9], pt[3];
+    tilde(P, A0, Adot, p0, pdot, At, pt);
+    if (e == 0) {
+        for (int k = 0; k < 3; ++k) g[k] = 0.0 + (p[k] - pt[k]) * m;
+        return;
+    }
+    const int i = e - 1;
+    double gr[3] = {-A[3 * i], -A[3 * i + 1], -A[3 * i + 2]};
+    for (int j = 0; j < 3; ++j) {
+        const double d = row_dot(A, i, j);
+        for (int k = 0; k < 3; ++k) gr[k] += d * A[3 * j + k];
+    }
+    for (int k = 0; k < 3; ++k)
+        g[k] = P.dt * P.dt * (gr[k] * 4.0 * P.stiffness) +
+               (A[3 * i + k] - (A0[3 * i + k] + P.dt * Adot[3 * i + k])) * i0;
+}
+// Sub-block (ii, jj) of a body's inertia Hessian (orthogonal_energy.py:63-96) at its state A.
+__device__ __forceinline__ void inertia_hessian_block(const AbdParams& P, int ii, int jj, const double* A, double m_,
+                                                      double i0, double dh[9]) {
+    const double m = ii == jj ? (ii == 0 ? m_ : i0) : 0.0;
+    for (int k = 0; k < 9; ++k) dh[k] = k % 4 == 0 ? m : 0.0;
+    if (ii == 0 || jj == 0) return;
+    const int i = ii - 1, j = jj - 1;
+    double h[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+    if (i == j) {
+        const double qq = row_dot(A, i, i) - 1.0;
+        for (int k = 0; k < 3; ++k)
+            for (int r = 0; r < 3; ++r)
+                for (int c = 0; c < 3; ++c) h[3 * r + c] += A[3 * k + r] * A[3 * k + c];
+        for (int r = 0; r < 3; ++r)
+            for (int c = 0; c < 3; ++c) h[3 * r + c] += A[3 * i + r] * A[3 * i + c] + (r == c ? qq : 0.0);
+    } else {
+        const double d = row_dot(A, j, i);
+        for (int r = 0; r < 3; ++r)
+            for (int c = 0; c < 3; ++c) h[3 * r + c] = A[3 * j + r] * A[3 * i + c] + (r == c ? d : 0.0);
+    }
+    for (int k = 0; k < 9; ++k) dh[k] += h[k] * 4.0 * P.stiffness * P.dt * P.dt;
+}
 // body b's state q - alpha dq (abd.py:337-353; alpha = 0 keeps q exactly)
 __device__ __forceinline__ void trial_state(int b, double alpha, const double* __restrict__ A,
                                             const double* __restrict__ p, const double* __restrict__ dq, double Ak[9],

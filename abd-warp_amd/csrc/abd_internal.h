@@ -115,20 +115,19 @@ int vg_cull_begin(hipStream_t s, const AbdScene* sc, const float* blo, const flo
 int vg_cull_fill(hipStream_t s, VgCull& C, int32_t* out, int64_t cap, int64_t n);
 
 // Swept boxes dilated at both ends (kind ABD_KIND_*, or -1 for body boxes): the union of
-// the dilated boxes at x0 and at x1.  plo / phi (body boxes only; both or neither): the
-// body boxes at x0 with the same dilation, already computed (read instead of recomputed;
-// the same values).
+// the dilated boxes at x0 and at x1.
 int swept_boxes(hipStream_t s, const AbdScene* sc, int kind, const double* x0, const double* x1, double dil,
-                float* lo, float* hi, const float* plo = nullptr, const float* phi = nullptr);
+                float* lo, float* hi);
 // Vertex ranges of a candidate superset (n3 = 3 * vertices): lo = min(x0, x1) - skin,
 // hi = max(x0, x1) + skin per coordinate.  Boxes of any positions inside these ranges
 // lie inside the swept boxes of (lo, hi) (every box formula is monotone in the
 // positions), so their culling output is a subset of that superset's.
 int vertex_ranges(hipStream_t s, int64_t n3, const double* x0, const double* x1, double skin, double* lo,
                   double* hi);
-// *flag (device, 0 before) becomes 1 when some coordinate of x0 or x1 leaves [lo, hi].
-int within_ranges(hipStream_t s, int64_t n3, const double* x0, const double* x1, const double* lo, const double* hi,
-                  int64_t* flag);
+// *flag (device, 0 before) becomes 1 when some coordinate of x leaves [lo + margin, hi - margin],
+// or of the rest positions r differs from r0.
+int within_ranges(hipStream_t s, int64_t n3, const double* x, const double* lo, const double* hi, double margin,
+                  const double* r, const double* r0, int64_t* flag);
 // dn (here and below, nullable): the lists' sizes on the device, [nij, nij, npt, nee, nvg],
 // the counts passed then bounding them.
 // What a candidate set keeps beside its tuples (each nullable): the scene vertex ids of each
@@ -192,13 +191,49 @@ __host__ __device__ inline double first_step_length(double t) {
     if (t < 1.0) t *= 0.9;
     return t;
 }
-// The end of a step: x_out = x(q - alpha dq), the arithmetic of update_q + project_vertices
-// with alpha_host (alpha_dev, active null), or of update_q_scenes + project_vertices with
-// alpha_dev [n_scenes] or alpha_host for the scenes with active[s] (0 for the others).  With
-// lo / hi, *flag (device) becomes gen when a coordinate of x_out or of x_other leaves them.
-int project_step(hipStream_t s, const AbdScene* sc, const double* A, const double* p, const double* dq,
-                 const double* alpha_dev, double alpha_host, const uint8_t* active, double* x_out,
-                 const double* x_other, const double* lo, const double* hi, int64_t* flag, int64_t gen);
+// The per-body passes of an iteration (abd_body.hip).  body_start: the accepted step lengths
+// alpha [ns] taken (A, p in place, Ak, pk alike), x, the body boxes at x dilated by dil, the
+// inertia gradient and the diagonal Hessian slots (both written), the scenes' rows
+// committed (row 1 of newton, E0, it over row 0), *range_flag and the words zeroed.
+struct BodyStart {
+    const double* alpha;
+    double *A, *p, *Ak, *pk;
+    const double* dq;
+    double* x;
+    double dil;
+    float *lo, *hi;
+    const double *A0, *p0, *Adot, *pdot;
+    double *g, *blocks;
+    double* zero;  // nzero words zeroed
+    int64_t nzero;
+    int ns;
+    uint8_t* newton;
+    double* E0;
+    int32_t* it;
+    int64_t* range_flag;
+};
+int body_start(hipStream_t s, const AbdScene* sc, const AbdParams* P, const BodyStart& U);
+// body_end: x = x(q - dq) of the scenes in active (x(q) of the others), the union (slo, shi)
+// of the body boxes there and blo, bhi; with lo, hi the range test (margin inside them) into
+// *flag, which bodies within skin - margin of qref [2][nb][12] (step_states of the step the
+// ranges were made around) pass by their rest_max [nb][3].
+struct BodyEnd {
+    const double *A, *p, *dq;
+    const uint8_t* active;
+    int ns;
+    double* x;
+    double dil;
+    const float *blo, *bhi;
+    float *slo, *shi;
+    const double *lo, *hi, *qref, *rest_max;
+    double skin, margin;
+    int64_t* flag;
+};
+int body_end(hipStream_t s, const AbdScene* sc, const BodyEnd& U);
+// each body's largest |rest coordinate| per axis (out [nb][3]) and a copy of the rest positions
+int rest_max(hipStream_t s, const AbdScene* sc, double* out, double* copy);
+int step_states(hipStream_t s, const AbdScene* sc, const double* A, const double* p, const double* dq,
+                const uint8_t* active, double* qref);
 // abd_contact_energy (S = 1) / abd_scene_contact_energy with the lists' sizes on the device.
 int contact_energy(hipStream_t s, const AbdScene* sc, const AbdParams* P, int S, const double* xk, const int32_t* pt,
                    int64_t npt, const int32_t* ee, int64_t nee, const int32_t* vg, int64_t nvg, const int64_t* dn,
@@ -271,9 +306,6 @@ struct GhLists {
     int64_t nij;
     const int64_t* dn;
 };
-// The inertia gradient (overwriting g) and Hessian (added into the diagonal slots) in one launch.
-int inertia_gh(hipStream_t s, const AbdScene* sc, const AbdParams* P, const double* A, const double* p,
-               const double* A0, const double* p0, const double* Adot, const double* pdot, double* g, double* blocks);
 int contact_gh(hipStream_t s, const AbdScene* sc, const AbdParams* P, const double* x, const GhLists& L,
                const int32_t* row_ptr, const int32_t* slots, double* g, double* blocks, uint8_t* highlight,
                int64_t* n_active, int64_t* n_active_dev);

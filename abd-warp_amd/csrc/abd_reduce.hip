@@ -409,12 +409,10 @@ __global__ __launch_bounds__(kRedThreads) void scene_final_kernel(const int64_t*
 // ---------------------------------------------------------------- CCD TOI
 // The scene minimum of the TOIs below 1 (ccd.py:9-40, abd.py:284-299) in two passes.
 // toi_scan_kernel: one candidate per thread (kToiSplit workgroups of kRedThreads per chunk
-// of the plan): the vertex-ground TOI directly; a PT / EE candidate whose primitives some
-// axis keeps apart on the whole step (apart_until above 1, also stored for the line search)
-// has no contact, and the others, gathered side by side, take their coplanarity cubic and
-// bracket test; the few candidates with a bracketed root in [0, 1] go to a queue (one
-// atomic per wave).  1.3M candidates of 256 scenes: 74 us with the cubic for every one, 69 us
-// so (0.4M of them near), the gathers of eight vertices each being most of it.  toi_solve_kernel: the full collision_time of each
+// of the plan): the vertex-ground TOI directly, and for a PT / EE candidate its
+// coplanarity cubic and bracket test (with its apart_until, from the same vertices, for the
+// line search); the few candidates with a bracketed root in [0, 1] go to a queue (one
+// atomic per wave).  toi_solve_kernel: the full collision_time of each
 // queued candidate (root searches and validity), its TOI below 1 min-ed into its scene's
 // slot (non-negative doubles order like their bit patterns, so an integer atomic min is
 // exact).  toi_final_kernel: per scene the minimum of its chunks' partials and its slot.
@@ -441,21 +439,18 @@ __global__ __launch_bounds__(kRedThreads, 4) void toi_scan_kernel(AbdScene sc, A
                                                                double* __restrict__ part, int32_t* __restrict__ queue,
                                                                int32_t* __restrict__ qcount) {
     __shared__ double sh[kRedThreads / kWave];
-    __shared__ uint8_t near_id[kRedThreads];
-    __shared__ int near_count;
     const int64_t c = blockIdx.x;
     if (c >= choff[S]) return;  // uniform over the workgroup
     const ChunkRange r = chunk_range(S, seg, choff, c);
     const bool on = !active || active[r.s];
-    if (threadIdx.x == 0) near_count = 0;
-    __syncthreads();
     const SceneView V{sc.voff, sc.foff, sc.eoff, sc.tris, sc.edges, sc.x0};
     const ListRef& Lr = L.l[r.l < kLists ? r.l : 0];
     const int kind = Lr.kind, ck = kind == kListPT ? 0 : 1;
-    const int64_t i0 = r.start + (int64_t)blockIdx.y * kRedThreads, i = i0 + threadIdx.x;
+    const int64_t i = r.start + (int64_t)blockIdx.y * kRedThreads + threadIdx.x;
     const double dhat = fmax(P.dhat, sqrt(P.d2hat));  // the boxes' dilation, the barrier's range
     double acc = 1.0;
-    bool near = false;
+    bool queued = false;
+    int32_t entry = 0;
     if (r.l < kLists && i < r.end) {
         float apart = 0.0f;
         if (on) {
@@ -469,29 +464,11 @@ __global__ __launch_bounds__(kRedThreads, 4) void toi_scan_kernel(AbdScene sc, A
                 d3 a[4], b[4];
                 cand_verts(ck, V, x0, x1, t, a, b, vids_of(Lr, i));
                 apart = apart_until(ck, a, b, dhat);
-                near = !(apart > 1.0f);
+                queued = toi_bracketed(a, b);
+                entry = (int32_t)((i << 1) | (kind == kListEE ? 1 : 0));
             }
         }
         if (Lr.apart) Lr.apart[i] = apart;
-    }
-    // the candidates that come near each other, side by side: the cubic and its bracket test
-    // only for these
-    {
-        const unsigned long long m = __ballot(near);
-        if (m) {
-            int base = 0;
-            if (lane_id() == 0) base = atomicAdd(&near_count, __popcll(m));
-            base = __shfl(base, 0);
-            if (near) near_id[base + __popcll(m & ((1ull << lane_id()) - 1ull))] = (uint8_t)threadIdx.x;
-        }
-    }
-    __syncthreads();
-    bool queued = false;
-    int32_t entry = 0;
-    if (threadIdx.x < near_count) {
-        const int64_t j = i0 + near_id[threadIdx.x];
-        queued = cand_toi_bracketed(ck, V, x0, x1, Lr.p + 5 * j, vids_of(Lr, j));
-        entry = (int32_t)((j << 1) | (kind == kListEE ? 1 : 0));
     }
     // wave-aggregated push of the queued candidates
     const unsigned long long mask = __ballot(queued);

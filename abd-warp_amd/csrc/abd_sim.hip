@@ -125,6 +125,8 @@ struct Sim {
     CandSet sup;
     BoxBuf sbody, stri, sedge, spt;  // the superset's boxes
     DevBuf<double> vlo, vhi;         // its vertex ranges
+    DevBuf<double> qref;             // the states they were made around
+    DevBuf<double> rest_max, rest_ref;  // the bodies' rest extents and the rest positions then
     bool sup_valid = false;
     bool col_fresh = false;  // col (with its structure) is the collision set at the current x
     DevBuf<int32_t> row_ptr, cols, slots;
@@ -206,7 +208,7 @@ enum {
 // rows of Sim::lsflag (iterating: the current and the next iteration's; searching) and of
 // Sim::lsval (E0: the current and the next); the next
 // iteration's rows are copied over the current ones at the start of every iteration
-// (ls_commit_kernel)
+// (body_start)
 enum { kLfNewton = 0, kLfSearch = 2, kLfRows };
 enum { kLvE0 = 0, kLvRows = 2 };
 
@@ -320,10 +322,9 @@ int collision_set(hipStream_t s, Sim& S, bool structure, const double* xv) {
 int collision_from(hipStream_t s, Sim& S, const CandSet& W, const double* xv) {
     const double dh = S.P.dhat * 0.5;
     int rc;
-    // the body boxes at x (also the start half of the next swept body boxes); the primitive
-    // boxes of collision_set's dilations are evaluated per entry of W by the filter: W holds
-    // far fewer entries than the scene has primitives
-    if ((rc = abd_body_boxes(s, &S.sc, xv, dh, S.body.lo.p, S.body.hi.p))) return rc;
+    // S.body: the body boxes at xv; the primitive boxes of collision_set's dilations are
+    // evaluated per entry of W by the filter: W holds far fewer entries than the scene has
+    // primitives
     if ((rc = S.col.reserve_like(W))) return rc;
     const KeepInput in{W.ij.p, W.ji.p, W.ptl.p, W.eel.p, W.vgl.p, W.nij, W.npt, W.nee, W.nvg, W.counts(),
                        W.side()};
@@ -346,6 +347,16 @@ int collision_from(hipStream_t s, Sim& S, const CandSet& W, const double* xv) {
 }
 int collision_from_swept(hipStream_t s, Sim& S, const double* xv) { return collision_from(s, S, S.sw, xv); }
 
+// Skin of the candidate superset's vertex ranges, in units of dhat: wide enough that the
+// later Newton steps of a frame (and of the next frames while the scenes rest) stay inside,
+// so that a batch of scenes, which reuses the superset only when all of them do, skips
+// most cullings; 30 measured best among 2, 10, 30 and 100 on the 256-scene workload.
+constexpr double kSkinOverDhat = 30.0;
+double skin_of(const Sim& S) { return kSkinOverDhat * S.P.dhat; }
+// What the range tests leave of it, far above the rounding of positions: a point of a step
+// whose ends pass them is inside the ranges too.
+double range_margin(const Sim& S) { return 1e-6 * skin_of(S); }
+
 // A frame's first collision set: filtered from the candidate superset when the state lies
 // inside its vertex ranges (boxes at any positions inside them lie inside its boxes, so the
 // culling output is a subset of it), else culled.
@@ -353,19 +364,19 @@ int collision_at_frame_start(hipStream_t s, Sim& S, const double* xv) {
     if (S.sup_valid) {
         int rc;
         ABD_CHECK(hipMemsetAsync(S.dcount.p + 7, 0, sizeof(int64_t), s));
-        if ((rc = within_ranges(s, 3 * (int64_t)S.nv, xv, xv, S.vlo.p, S.vhi.p, S.dcount.p + 7))) return rc;
+        if ((rc = within_ranges(s, 3 * (int64_t)S.nv, xv, S.vlo.p, S.vhi.p, range_margin(S), S.sc.x0, S.rest_ref.p,
+                                S.dcount.p + 7))) return rc;
         ABD_CHECK(hipMemcpyAsync(S.hcount + 7, S.dcount.p + 7, sizeof(int64_t), hipMemcpyDeviceToHost, s));
         ABD_CHECK(hipStreamSynchronize(s));
-        if (S.hcount[7] == 0) return collision_from(s, S, S.sup, xv);
+        if (S.hcount[7] == 0) {
+            if ((rc = abd_body_boxes(s, &S.sc, xv, 0.5 * S.P.dhat, S.body.lo.p, S.body.hi.p))) return rc;
+            return collision_from(s, S, S.sup, xv);
+        }
+        S.sup_valid = false;  // the frame starts outside it (or with another rest shape)
     }
     return collision_set(s, S, true, xv);
 }
 
-// Skin of the candidate superset's vertex ranges, in units of dhat: wide enough that the
-// later Newton steps of a frame (and of the next frames while the scenes rest) stay inside,
-// so that a batch of scenes, which reuses the superset only when all of them do, skips
-// most cullings; 30 measured best among 2, 10, 30 and 100 on the 256-scene workload.
-constexpr double kSkinOverDhat = 30.0;
 
 // abd.py:170-185, with both ends of every box dilated as in collision_set: one candidate
 // set per Newton iteration that holds both the CCD candidates of the step (a pair that
@@ -401,7 +412,9 @@ int swept_set_recull(hipStream_t s, Sim& S) {
     const int64_t n3 = 3 * (int64_t)S.nv;
     int rc;
     S.sup_valid = false;
-    if ((rc = vertex_ranges(s, n3, st.x, st.xk, kSkinOverDhat * S.P.dhat, S.vlo.p, S.vhi.p))) return rc;
+    if ((rc = vertex_ranges(s, n3, st.x, st.xk, skin_of(S), S.vlo.p, S.vhi.p))) return rc;
+    if ((rc = step_states(s, &S.sc, st.A, st.p, st.dq, S.lsflag.p + (size_t)kLfNewton * S.ns, S.qref.p))) return rc;
+    if ((rc = rest_max(s, &S.sc, S.rest_max.p, S.rest_ref.p))) return rc;
     if ((rc = swept_boxes(s, &S.sc, -1, S.vlo.p, S.vhi.p, dh, S.sbody.lo.p, S.sbody.hi.p))) return rc;
     // with the (j, i) order: the swept set (and the collision sets after it) keep it
     if ((rc = body_pairs(s, S, S.sup, S.sbody, true))) return rc;
@@ -440,11 +453,9 @@ int swept_set_launch(hipStream_t s, Sim& S) {
     const AbdSimState& st = S.st;
     int rc;
     if (!S.sup_valid) return swept_set_recull(s, S);
-    // body boxes: the half at x is this iteration's collision set's (same dilation; reading
-    // it beats a second pass over every vertex).  Primitive swept boxes: evaluated by the
-    // filter per entry of the superset from both ends (far fewer entries than primitives)
-    if ((rc = swept_boxes(s, &S.sc, -1, st.x, st.xk, dh, S.tbody.lo.p, S.tbody.hi.p, S.body.lo.p, S.body.hi.p)))
-        return rc;
+    // the swept body boxes come from the step's end (body_end); the primitives' are evaluated
+    // by the filter per entry of the superset from both ends (far fewer entries than
+    // primitives)
     if ((rc = S.sw.reserve_like(S.sup, S.sup.vids))) return rc;
     if ((rc = S.sw.apt.reserve((size_t)S.sup.npt + 1))) return rc;
     if ((rc = S.sw.aee.reserve((size_t)S.sup.nee + 1))) return rc;
@@ -619,20 +630,6 @@ __global__ __launch_bounds__(kLsThreads) void ls_frame_start_kernel(int ns, cons
     }
 }
 
-// The start of a Newton iteration: the rows the last iteration's decisions wrote become the
-// current ones, and the range test's flag is cleared for this step.
-__global__ __launch_bounds__(kLsThreads) void ls_commit_kernel(int ns, uint8_t* __restrict__ flag,
-                                                                double* __restrict__ val,
-                                                                int32_t* __restrict__ it,
-                                                                int64_t* __restrict__ range_flag) {
-    for (int s = blockIdx.x * kLsThreads + threadIdx.x; s < ns; s += gridDim.x * kLsThreads) {
-        flag[(int64_t)kLfNewton * ns + s] = flag[(int64_t)(kLfNewton + 1) * ns + s];
-        val[(int64_t)kLvE0 * ns + s] = val[(int64_t)(kLvE0 + 1) * ns + s];
-        it[s] = it[ns + s];
-    }
-    if (blockIdx.x == 0 && threadIdx.x == 0) *range_flag = 0;
-}
-
 // q_gets_q0 (abd.py:124-128): q = (Ak, pk) = q0, and the accepted step lengths 0.
 __global__ __launch_bounds__(kLsThreads) void frame_state_kernel(int nb, int ns, const double* __restrict__ A0,
                                                                   const double* __restrict__ p0,
@@ -703,13 +700,33 @@ int read_counts(hipStream_t s, Sim& S) {
     return ABD_OK;
 }
 
-// The end of the step (xk = x(q - dq) for the scenes in `active`) with the range test of both
-// ends against the superset's ranges when there is a superset (a vertex outside the superset's ranges writes 1
-// over the 0 of ls_commit_kernel).
+// The end of the step (xk = x(q - dq) for the scenes in `active`), the swept body boxes and
+// the range test against the superset's ranges when there is a superset (a vertex outside
+// writes 1 over the 0 of body_start).
 int step_end_scenes(hipStream_t s, Sim& S, const uint8_t* active) {
     const AbdSimState& st = S.st;
-    return project_step(s, &S.sc, st.A, st.p, st.dq, nullptr, 1.0, active, st.xk, st.x,
-                        S.sup_valid ? S.vlo.p : nullptr, S.sup_valid ? S.vhi.p : nullptr, S.cnt.p + kCntRange, 1);
+    BodyEnd U{};
+    U.A = st.A;
+    U.p = st.p;
+    U.dq = st.dq;
+    U.active = active;
+    U.ns = S.ns;
+    U.x = st.xk;
+    U.dil = 0.5 * S.P.dhat;
+    U.blo = S.body.lo.p;
+    U.bhi = S.body.hi.p;
+    U.slo = S.tbody.lo.p;
+    U.shi = S.tbody.hi.p;
+    if (S.sup_valid) {
+        U.lo = S.vlo.p;
+        U.hi = S.vhi.p;
+        U.qref = S.qref.p;
+        U.rest_max = S.rest_max.p;
+    }
+    U.skin = skin_of(S);
+    U.margin = range_margin(S);
+    U.flag = S.cnt.p + kCntRange;
+    return body_end(s, &S.sc, U);
 }
 
 // The swept set's TOI, q.g and g.g, and both line-search passes with their decisions, then
@@ -757,22 +774,41 @@ int iteration_scenes(hipStream_t s, Sim& S) {
     const int nb = S.nb, ns = S.ns;
     const LsDev L = ls_dev(S);
     int rc;
-    // q and (Ak, pk) = the accepted trial of every scene (step length 0: an exact copy)
-    if ((rc = update_q_scenes_dual(s, &S.sc, st.A, st.p, st.dq, L.dalpha, st.A, st.p, st.Ak, st.pk))) return rc;
-    hipLaunchKernelGGL(ls_commit_kernel, dim3((unsigned)ceil_div(ns, kLsThreads)), dim3(kLsThreads), 0, s, ns,
-                       S.lsflag.p, S.lsval.p, S.lsit.p, S.cnt.p + kCntRange);
-    ABD_CHECK_LAUNCH();
-    // (Ak, pk) = (A, p) here: the collision set is culled on x
-    if ((rc = abd_project_vertices(s, &S.sc, st.A, st.p, st.x))) return rc;
+    // q and (Ak, pk) = the accepted trial of every scene (step length 0: an exact copy), the
+    // rows committed, x and its body boxes, the inertia terms, the off-diagonal slots zeroed
+    const int64_t nij = S.col_fresh ? S.col.nij : S.sw.nij;
+    if ((rc = S.blocks.reserve((nb + 2 * (size_t)nij) * 144))) return rc;
+    BodyStart U;
+    U.alpha = L.dalpha;
+    U.A = st.A;
+    U.p = st.p;
+    U.Ak = st.Ak;
+    U.pk = st.pk;
+    U.dq = st.dq;
+    U.x = st.x;
+    U.dil = 0.5 * P.dhat;
+    U.lo = S.body.lo.p;
+    U.hi = S.body.hi.p;
+    U.A0 = st.A0;
+    U.p0 = st.p0;
+    U.Adot = st.Adot;
+    U.pdot = st.pdot;
+    U.g = st.g;
+    U.blocks = S.blocks.p;
+    U.zero = S.blocks.p + 144 * (int64_t)nb;
+    U.nzero = 2 * 144 * nij;
+    U.ns = ns;
+    U.newton = S.lsflag.p + (size_t)kLfNewton * ns;
+    U.E0 = S.lsval.p + (size_t)kLvE0 * ns;
+    U.it = S.lsit.p;
+    U.range_flag = S.cnt.p + kCntRange;
+    if ((rc = body_start(s, &S.sc, &P, U))) return rc;
+    // the collision set at x: the frame start's (the same positions), else from the last
+    // iteration's swept set
     if (S.col_fresh)
-        S.col_fresh = false;  // the frame-start energy's set: the same positions
-    else if ((rc = S.sw_valid ? collision_from_swept(s, S, st.x) : collision_at_frame_start(s, S, st.x)))
+        S.col_fresh = false;
+    else if ((rc = collision_from_swept(s, S, st.x)))
         return rc;
-    const size_t nslot = nb + 2 * (size_t)S.col.nij;
-    if ((rc = S.blocks.reserve(nslot * 16 * 9))) return rc;
-    if ((rc = zero_fill(s, S.blocks.p, sizeof(double) * nslot * 16 * 9))) return rc;
-    // g: overwritten by the inertia gradient (abd.py:236-237 zeroes it first)
-    if ((rc = inertia_gh(s, &S.sc, &P, st.A, st.p, st.A0, st.p0, st.Adot, st.pdot, st.g, S.blocks.p))) return rc;
     const CandSet& C = S.col;
     const GhLists GL{C.ptl.p, C.npt, C.eel.p, C.nee, C.vgl.p, C.nvg, C.nij, C.counts()};
     if ((rc = contact_gh(s, &S.sc, &P, st.x, GL, S.row_ptr.p, S.slots.p, st.g, S.blocks.p, nullptr, nullptr,
@@ -863,7 +899,7 @@ int step_scenes(hipStream_t s, Sim& S) {
     S.sw_valid = false;  // a frame starts from the state the caller holds
     if ((rc = frame_start_scenes(s, S))) return rc;
     {
-        // the first iteration's rows, taken over by its ls_commit_kernel
+        // the first iteration's rows, taken over by its body_start_kernel
         const LsDev L = ls_dev(S);
         hipLaunchKernelGGL(ls_frame_start_kernel, dim3((unsigned)ceil_div(ns, kLsThreads)), dim3(kLsThreads), 0, s,
                            ns, (const double*)(S.sv.p + kSvEc * ns), (const double*)(S.sv.p + kSvEi * ns), L.E0_nxt,
@@ -970,6 +1006,9 @@ int abd_sim_create(const AbdScene* scene, const AbdParams* params, const AbdSimS
     if (!rc) rc = S->spt.reserve(S->nv);
     if (!rc) rc = S->vlo.reserve(3 * (size_t)S->nv + 3);
     if (!rc) rc = S->vhi.reserve(3 * (size_t)S->nv + 3);
+    if (!rc) rc = S->qref.reserve(24 * nb);
+    if (!rc) rc = S->rest_max.reserve(3 * nb);
+    if (!rc) rc = S->rest_ref.reserve(3 * (size_t)S->nv + 3);
     for (CandSet* C : {&S->col, &S->sw, &S->sup}) {
         if (!rc) rc = C->ij.reserve(2 * 256);
         if (!rc) rc = C->ji.reserve(2 * 256);
@@ -1193,6 +1232,9 @@ int abd_sim_destroy(void* sim) {
     S->sup.release();
     S->vlo.release();
     S->vhi.release();
+    S->qref.release();
+    S->rest_max.release();
+    S->rest_ref.release();
     S->row_ptr.release();
     S->cols.release();
     S->slots.release();

@@ -83,3 +83,36 @@ def test_line_search_prunes_nothing_active(nb, seed):
     assert np.abs(sim.states.A.cpu().numpy() - ref.A).max() <= 1e-7
     assert np.abs(sim.states.p.cpu().numpy() - ref.p).max() <= 1e-7
     assert sim.stats["energy_evals"] > sim.stats["newton_iters"] + 3  # some search halved
+
+
+@pytest.mark.parametrize("mesh", ["cube", "ico2", "ico3"])
+def test_body_passes_by_mesh_size(mesh):
+    """The per-body passes with one wave a body (8 and 162 vertices) and with four (642):
+    the vertices placed by a frame, and a frame after the rest shape was changed in place,
+    against the oracle (1e-7, the drivers' bound)."""
+    from abd_hip import scenes
+    from abd_hip.abd import AffineBodySimulator
+    from abd_hip.const_params import ContactParams
+    m = {"cube": scenes.cube_mesh, "ico2": lambda: scenes.icosphere_mesh(2, 0.5),
+         "ico3": lambda: scenes.icosphere_mesh(3, 0.5)}[mesh]()
+    h = m[0][:, 1].max() - m[0][:, 1].min()
+    p = np.array([[0.0, 5e-4 - m[0][:, 1].min() + k * (h + 1.1e-3), 0.01 * k] for k in range(3)])
+    spec = scenes.build_scene([m] * 3, np.stack([np.eye(3)] * 3), p, np.zeros((3, 3, 3)), np.zeros((3, 3)), ground=0.0)
+    cp = ContactParams(ground=0.0, psd=1, solver=3)
+    sim = AffineBodySimulator(spec, cp, native=True)
+    for scale in (1.0, 0.999):
+        if scale != 1.0:  # another rest shape in the same buffers, the state kept
+            sim.meshes.x0.mul_(scale)
+        st = sim.states
+        sp = scenes.build_scene([(m[0] * scale, m[1])] * 3, *(t.cpu().numpy() for t in (st.A0, st.p0, st.Adot, st.pdot)),
+                                ground=0.0)
+        ref = O.OracleSim(sp, cp)
+        ref.dq[...] = sim.dq.cpu().numpy()
+        sim.step()
+        ref.step()
+        torch.cuda.synchronize()
+        A, q = st.A0.cpu().numpy(), st.p0.cpu().numpy()
+        assert np.abs(A - ref.A).max() <= 1e-7 and np.abs(q - ref.p).max() <= 1e-7
+        body = np.repeat(np.arange(3), np.diff(sp.voff))
+        x = np.einsum("vr,vrk->vk", sp.x0, A[body]) + q[body]
+        assert np.abs(sim.meshes.x_view.cpu().numpy() - x).max() <= 1e-13
