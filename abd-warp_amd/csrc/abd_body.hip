@@ -66,12 +66,18 @@ __global__ __launch_bounds__(T) void body_start_kernel(AbdScene sc, AbdParams P,
     if (b >= nb) {
         const int64_t i0 = (int64_t)(b - nb) * T + t, step = (int64_t)(gridDim.x - nb) * T;
         for (int64_t i = i0; i < U.nzero; i += step) U.zero[i] = 0;
+        for (int64_t i = i0; i < U.nzero32; i += step) U.zero32[i] = 0;
         for (int64_t s = i0; s < U.ns; s += step) {
             U.newton[s] = U.newton[U.ns + s];
             U.E0[s] = U.E0[U.ns + s];
             U.it[s] = U.it[U.ns + s];
+            if (U.slots) U.slots[s] = 0x3FF0000000000000ull;  // 1.0
         }
-        if (i0 == 0) *U.range_flag = 0;
+        if (i0 < U.ncounters) U.counters[i0] = 0;
+        if (i0 == 0) {
+            *U.range_flag = 0;
+            if (U.qcount) *U.qcount = 0;
+        }
         return;
     }
     const double al = U.alpha[U.ns > 1 ? sc.body_scene[b] : 0];
@@ -181,6 +187,7 @@ __global__ __launch_bounds__(T) void body_end_kernel(AbdScene sc, BodyEnd U) {
             U.slo[3 * b + k] = fminf(U.blo[3 * b + k], (float)(mn[k] - U.dil));
             U.shi[3 * b + k] = fmaxf(U.bhi[3 * b + k], (float)(mx[k] + U.dil));
         }
+    if (t == 0) U.on[b] = al != 0.0;
 }
 
 // The largest |rest coordinate| of each body, per axis (one wave per body), and a copy of the
@@ -229,7 +236,7 @@ int body_start(hipStream_t s, const AbdScene* sc, const AbdParams* P, const Body
     const bool small = small_bodies(sc);
     const int T = small ? kWave : kBlock;
     // workgroups for the rows and the fill: about 16 words a thread
-    const int64_t extra = std::min<int64_t>(4096, 1 + ceil_div(std::max<int64_t>(U.nzero, U.ns), 16 * (int64_t)T));
+    const int64_t extra = std::min<int64_t>(4096, 1 + ceil_div(std::max<int64_t>(U.nzero + U.nzero32 / 2, U.ns), 16 * (int64_t)T));
     const dim3 grid((unsigned)(sc->n_bodies + extra));
     if (small)
         hipLaunchKernelGGL(body_start_kernel<kWave>, grid, dim3(T), 0, s, *sc, *P, U);

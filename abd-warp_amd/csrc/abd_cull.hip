@@ -16,6 +16,8 @@
 
 #include <math.h>
 
+#include <algorithm>
+
 #include "abd_block.h"
 #include "abd_device.h"
 #include "abd_internal.h"
@@ -675,6 +677,16 @@ namespace {
 
 // The five lists of a keep pass: 0 ij, 1 ji, 2 PT, 3 EE, 4 VG.
 constexpr int kKeepLists = 5;
+// blocks of a super-block: a block's offset is the sum of the super-blocks' counts before its
+// own (added to by the count pass: integers, any order) and of the blocks' before it inside
+constexpr int kSuper = 64;
+constexpr int kXcds = 8;
+// words between super-block counts: adds to one cache line wait for each other (about 10 ns
+// each: packed, a count pass of 18 k blocks took 108 us instead of 87)
+constexpr int kSuperStride = 8;
+constexpr int kFlagAlign = 16;
+// blocks of PT / EE entries a workgroup of the sweep's write pass takes
+constexpr int kSweepBlocks = 4;  // (a thread's flags are one word)
 struct KeepArgs {
     KeepInput in;
     KeepBoxes bx;
@@ -684,11 +696,15 @@ struct KeepArgs {
     double yth;
     float fg;
     int64_t n[kKeepLists];
-    int64_t blk0[kKeepLists + 1];  // first workgroup (block of kBlock entries) of each list
-    int64_t* bcnt[kKeepLists];
-    int64_t* boff[kKeepLists];
+    int64_t blk0[kKeepLists + 1];  // first workgroup of each list (one per block of kBlock
+                                   // entries, rounded up to a multiple of kXcds)
+    uint32_t* bcnt[kKeepLists];    // kept entries of each block
+    uint32_t* scnt[kKeepLists];    // and of each super-block
+    const int64_t* pair_off;       // the pair blocks' offsets when a scan made them
+    int64_t* dcount;               // the five totals
     uint8_t* flag;                 // each entry's predicate (count pass), read by the write pass
-    int64_t flag0[kKeepLists];     // first flag of each list
+    int64_t flag0[kKeepLists];     // first flag of each list (a multiple of kFlagAlign)
+    int64_t grp0[kKeepLists + 1];  // first workgroup of each list in the sweep's write pass
     // primitive boxes from the vertices when x is set (KeepAtX)
     const double *x, *x1;
     const int32_t *tris, *edges;
@@ -696,6 +712,7 @@ struct KeepArgs {
     double edil, tdil;
     const double* alpha;  // KeepAtX: entries apart at their scene's step length are dropped
     const int32_t* body_scene;
+    KeepSweep W;
 };
 
 // point_boxes_kernel's box of vertex v at x, or with x1 set swept_point_boxes_kernel's
@@ -825,7 +842,8 @@ __device__ __forceinline__ bool keep_pred(const KeepArgs& A, int k, int64_t i) {
     return overlap(B.plo + 3 * v, B.phi + 3 * v, qlo, qhi);
 }
 
-__device__ __forceinline__ void keep_write(const KeepArgs& A, int k, int64_t i, int64_t o) {
+template <class Off>
+__device__ __forceinline__ void keep_write(const KeepArgs& A, const Off& pair_off, int k, int64_t i, int64_t o) {
     if (k <= 1) {
         const int32_t* pr = (k == 0 ? A.in.ij : A.in.ji) + 2 * i;
         int32_t* q = (k == 0 ? A.out.ij : A.out.ji) + 2 * o;
@@ -838,7 +856,7 @@ __device__ __forceinline__ void keep_write(const KeepArgs& A, int k, int64_t i, 
         q[1] = t5[1];
         // the pair's index in the kept ij: its block's offset + its rank in the block (the
         // tuple is kept only if its pair's body boxes overlap, so the pair is kept)
-        q[2] = (int32_t)(A.boff[0][t5[2] / kBlock] + A.remap[t5[2]]);
+        q[2] = (int32_t)(pair_off[t5[2] / kBlock] + A.remap[t5[2]]);
         q[3] = t5[3];
         q[4] = t5[4];
         const int32_t* vin = k == 2 ? A.in.vids.pt : A.in.vids.ee;
@@ -864,53 +882,277 @@ __device__ __forceinline__ int64_t keep_n(const KeepArgs& A, int k) {
     return A.in.dn ? (k == 1 && !A.in.ji ? 0 : A.in.dn[k]) : A.n[k];
 }
 
+// Which of n blocks the workgroup `loc` of a list takes (-1: none): the workgroups of one XCD
+// (they are dealt to the XCDs in turn) take a contiguous run of blocks, whose entries share
+// vertices in its L2.  n: the blocks in use, of a launch over at least as many rounded up.
+__device__ __forceinline__ int64_t xcd_block(int64_t loc, int64_t n) {
+    const int64_t run = (n + kXcds - 1) / kXcds, y = loc / kXcds, b = loc % kXcds * run + y;
+    return y < run && b < n ? b : -1;
+}
+__device__ __forceinline__ int64_t blocks_of(int64_t n) { return (n + kBlock - 1) / kBlock; }
+
 __global__ __launch_bounds__(kBlock) void keep_count_kernel(KeepArgs A) {
     __shared__ int shw[kBlock / kWave];
     const int64_t g = blockIdx.x;
     int k = 0;
     while (k + 1 < kKeepLists && g >= A.blk0[k + 1]) ++k;
-    const int64_t blk = g - A.blk0[k];
+    const int64_t nk = keep_n(A, k), blk = xcd_block(g - A.blk0[k], blocks_of(nk));
+    if (blk < 0) return;  // uniform
     const int64_t i = blk * kBlock + threadIdx.x;
-    bool pred = false;
-    const bool in_list = i < keep_n(A, k);
-    if (in_list) {
-        pred = keep_pred(A, k, i);
-        A.flag[A.flag0[k] + i] = pred ? 1 : 0;
-    }
-    if (k == 0) {  // uniform over the workgroup
-        int tot;
-        const int r = block_rank(pred, shw, &tot);
-        if (in_list) A.remap[i] = pred ? r : -1;
-        if (threadIdx.x == 0) A.bcnt[k][blk] = tot;
-        return;
-    }
-    const int c = __popcll(__ballot(pred ? 1 : 0));
-    if (lane_id() == 0) shw[wave_id()] = c;
-    __syncthreads();
+    const bool in_list = i < nk;
+    const bool pred = in_list && keep_pred(A, k, i);
+    if (in_list) A.flag[A.flag0[k] + i] = pred ? 1 : 0;
+    int tot;
+    const int r = block_rank(pred, shw, &tot);
+    if (k == 0 && in_list) A.remap[i] = pred ? r : -1;
     if (threadIdx.x == 0) {
-        int t = 0;
-        for (int w = 0; w < kBlock / kWave; ++w) t += shw[w];
-        A.bcnt[k][blk] = t;
+        A.bcnt[k][blk] = (uint32_t)tot;
+        if (tot) atomicAdd(A.scnt[k] + kSuperStride * (blk / kSuper), (uint32_t)tot);
     }
 }
 
-// The write pass over lists [k0, k1), one entry per thread: the kept entries at their
-// ordered ranks (the block's scanned offset + the rank in the block).
-__global__ __launch_bounds__(kBlock) void keep_write_kernel(KeepArgs A, int k0, int k1) {
+// The kept entries before block blk of list k: whole super-blocks, then the blocks of its own.
+__device__ __forceinline__ int64_t block_offset(const KeepArgs& A, int k, int64_t blk, int64_t* sh) {
+    const int64_t sb = blk / kSuper;
+    int64_t v = 0;
+    for (int64_t q = threadIdx.x; q < sb; q += kBlock) v += A.scnt[k][kSuperStride * q];
+    const int64_t b = sb * kSuper + threadIdx.x;
+    if (b < blk) v += A.bcnt[k][b];
+#pragma unroll
+    for (int off = kWave / 2; off > 0; off >>= 1) v += __shfl_xor(v, off);
+    if (lane_id() == 0) sh[wave_id()] = v;
+    __syncthreads();
+    v = 0;
+    for (int w = 0; w < kBlock / kWave; ++w) v += sh[w];
+    __syncthreads();
+    return v;
+}
+
+// The pair blocks' offsets, which place the tuples' pair indices: summed in LDS where there
+// are at most kBlock of them (65536 pairs), else scanned before.
+__device__ __forceinline__ void pair_offsets(const KeepArgs& A, int64_t* poff, int64_t* sh) {
+    if (A.pair_off) return;
+    const int t = threadIdx.x;
+    poff[t] = block_exclusive_scan_i64(t < blocks_of(keep_n(A, 0)) ? (int64_t)A.bcnt[0][t] : 0, sh);
+    __syncthreads();
+}
+__device__ __forceinline__ void write_entry(const KeepArgs& A, const int64_t* poff, int k, int64_t i, int64_t o) {
+    if (A.pair_off)
+        keep_write(A, A.pair_off, k, i, o);
+    else
+        keep_write(A, poff, k, i, o);
+}
+
+// The write pass, one entry per thread: the kept entries at their ordered ranks (the block's
+// offset + the rank in the block), the totals by each list's last block.
+__global__ __launch_bounds__(kBlock) void keep_write_kernel(KeepArgs A) {
     __shared__ int shw[kBlock / kWave];
-    const int64_t g = (int64_t)blockIdx.x + A.blk0[k0];
-    int k = k0;
-    while (k + 1 < k1 && g >= A.blk0[k + 1]) ++k;
-    const int64_t blk = g - A.blk0[k];
-    const int64_t i = blk * kBlock + threadIdx.x;
-    const int64_t nk = keep_n(A, k);
+    __shared__ int64_t sh[kBlock / kWave];
+    __shared__ int64_t poff[kBlock];
+    const int64_t g = blockIdx.x;
+    const int t = threadIdx.x;
+    if (g == 0 && t < kKeepLists && A.blk0[t] == A.blk0[t + 1]) A.dcount[t] = 0;  // an empty list
+    if (g >= A.blk0[kKeepLists]) return;
+    int k = 0;
+    while (k + 1 < kKeepLists && g >= A.blk0[k + 1]) ++k;
+    const int64_t nk = keep_n(A, k), nblk = blocks_of(nk), blk = xcd_block(g - A.blk0[k], nblk);
+    if (nk == 0 && g == A.blk0[k] && t == 0) A.dcount[k] = 0;
+    if (blk < 0) return;  // uniform
+    const bool last = blk + 1 == nblk;
+    const uint32_t mine = A.bcnt[k][blk];
+    if (mine == 0 && !last) return;  // uniform: nothing kept
+    const int64_t off = block_offset(A, k, blk, sh);
+    if (last && t == 0) A.dcount[k] = off + mine;
+    if (mine == 0) return;
+    if (k == 2 || k == 3) pair_offsets(A, poff, sh);
+    const int64_t i = blk * kBlock + t;
     const bool pred = i < nk && A.flag[A.flag0[k] + i] != 0;
     int tot;
-    const int64_t r = A.boff[k][blk] + block_rank(pred, shw, &tot);
-    if (pred) keep_write(A, k, i, r);
+    const int64_t r = off + block_rank(pred, shw, &tot);
+    if (pred) write_entry(A, poff, k, i, r);
+}
+
+// The scenes of the lanes with `kept` counted in list l (EE, PT, VG): one add a wave, or one a
+// lane where a wave holds entries of several scenes.
+__device__ __forceinline__ void count_scene(const KeepSweep& W, int l, bool kept, int s) {
+    const unsigned long long m = __ballot(kept);
+    if (W.S == 1 || !m) return;
+    const int leader = __ffsll((long long)m) - 1;
+    const int s0 = __shfl(s, leader);
+    uint32_t* c = W.scnt + (int64_t)l * W.S;
+    if (__ballot(kept && s != s0) == 0) {
+        if (lane_id() == leader) atomicAdd(c + s0, (uint32_t)__popcll(m));
+    } else if (kept) {
+        atomicAdd(c + s, 1u);
+    }
+}
+
+// The write pass of a swept set with its CCD (KeepSweep).  PT / EE entries: kSweepBlocks
+// blocks a workgroup, whose kept entries are listed in LDS, so that the lanes are full where a
+// third of the superset is kept; each then has its tuple written and, from one gather of its
+// eight vertices, its apart_until and cubic taken.  The gathers' latency bounds it (3/4 of the
+// wave cycles wait, the address units are busy a third of the time).  1.3 M kept of 4.5 M:
+// 119 us, against 46 (write) + 121 (scan of the written lists) + 19 (plan) as passes of their
+// own.  What it cost on the way: one counter for the queue and every wave adding to it 40 us
+// more (hence one add a workgroup); blocks dealt to the XCDs in turn 11-24 us more (hence
+// xcd_block); four waves a SIMD, with 25 registers spilled, 20 us more than three; all in the
+// count pass, whose waves then hold the CCD's registers, 55 us more.
+__global__ __launch_bounds__(kBlock, 3) void sweep_write_kernel(KeepArgs A) {
+    constexpr int kWaves = kBlock / kWave;
+    __shared__ int64_t woff[kWaves];
+    __shared__ int wcnt[kWaves], wpair[kWaves], qn, qbase;
+    __shared__ int64_t poff[kBlock];
+    __shared__ uint16_t list[kSweepBlocks * kBlock], qlist[kSweepBlocks * kBlock];
+    const int64_t g = blockIdx.x;
+    const int t = threadIdx.x;
+    const KeepSweep& W = A.W;
+    if (g == 0 && t < kKeepLists && A.blk0[t] == A.blk0[t + 1]) A.dcount[t] = 0;  // an empty list
+    if (g >= A.grp0[kKeepLists]) return;
+    int k = 0;
+    while (k + 1 < kKeepLists && g >= A.grp0[k + 1]) ++k;
+    const bool tuples = k == 2 || k == 3;
+    const int64_t nk = keep_n(A, k), nblk = blocks_of(nk);
+    const int64_t ngrp = tuples ? (nblk + kSweepBlocks - 1) / kSweepBlocks : nblk;
+    const int64_t grp = xcd_block(g - A.grp0[k], ngrp);
+    if (nk == 0 && g == A.grp0[k] && t == 0) A.dcount[k] = 0;
+    if (grp < 0) return;  // uniform
+    const int64_t blk = tuples ? grp * kSweepBlocks : grp;
+    const bool last = grp + 1 == ngrp;
+    const int64_t i0 = blk * kBlock;
+    // the kept entries before the workgroup's (block_offset's), its own, and the pair
+    // blocks' offsets (pair_offsets'), their loads in flight together and one scan for all
+    uint32_t word = 0;
+    if (tuples) {
+        const int64_t i = i0 + kSweepBlocks * t;
+        if (i < nk) word = *reinterpret_cast<const uint32_t*>(A.flag + A.flag0[k] + i);
+        for (int j = 0; j < kSweepBlocks; ++j)
+            if (i + j >= nk || (word >> (8 * j) & 0xff) == 0) word &= ~(0xffu << (8 * j));
+    } else if (i0 + t < nk) {
+        word = A.flag[A.flag0[k] + i0 + t];
+    }
+    const int64_t sb = blk / kSuper;
+    int64_t before = 0;
+    for (int64_t q = t; q < sb; q += kBlock) before += A.scnt[k][kSuperStride * q];
+    if (sb * kSuper + t < blk) before += A.bcnt[k][sb * kSuper + t];
+    const int pairs = tuples && !A.pair_off && t < blocks_of(keep_n(A, 0)) ? (int)A.bcnt[0][t] : 0;
+    int c = 0;
+#pragma unroll
+    for (int j = 0; j < kSweepBlocks; ++j) c += (word >> (8 * j) & 0xff) != 0;
+    int ci = c, pi = pairs;
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+        const int u = __shfl_up(ci, o), v = __shfl_up(pi, o);
+        if (lane_id() >= o) {
+            ci += u;
+            pi += v;
+        }
+        before += __shfl_xor(before, o);
+    }
+    if (lane_id() == kWave - 1) {
+        woff[wave_id()] = before;
+        wcnt[wave_id()] = ci;
+        wpair[wave_id()] = pi;
+    }
+    if (t == 0) qn = 0;
+    __syncthreads();
+    int64_t off = 0;
+    int mine = 0;
+    for (int w = 0; w < kWaves; ++w) {
+        if (w < wave_id()) {
+            ci += wcnt[w];
+            pi += wpair[w];
+        }
+        off += woff[w];
+        mine += wcnt[w];
+    }
+    if (last && t == 0) A.dcount[k] = off + mine;
+    if (mine == 0) return;  // uniform: nothing kept
+    if (!tuples) {
+        const bool pred = c != 0;
+        const int64_t i = i0 + t, r = off + ci - c;
+        if (pred) write_entry(A, poff, k, i, r);
+        if (k < 4) return;  // uniform
+        int s = 0;
+        if (pred) {
+            const int32_t* tu = A.in.vg + 2 * i;
+            s = W.S > 1 ? W.body_scene[tu[0]] : 0;
+            float apart = 0.0f;
+            if (W.body_on[tu[0]]) {
+                const int64_t v = A.voff[tu[0]] + (int64_t)tu[1];
+                apart = apart_until_vg(A.x[3 * v + 1], A.x1[3 * v + 1], W.ground, W.dhat);
+                const double tv = cand_toi_vg(A.voff, A.x, A.x1, tu, W.ground);
+                // a TOI below 0 gives the first length that 0 gives
+                if (tv < 1.0 && W.use_vg)
+                    atomicMin(W.slots + s, (unsigned long long)__double_as_longlong(tv > 0.0 ? tv : 0.0));
+            }
+            W.avg[r] = apart;
+        }
+        count_scene(W, 2, pred, s);
+        return;
+    }
+    poff[t] = pi - pairs;
+    {
+        int r = ci - c;
+#pragma unroll
+        for (int j = 0; j < kSweepBlocks; ++j)
+            if (word >> (8 * j) & 0xff) list[r++] = (uint16_t)(kSweepBlocks * t + j);
+    }
+    __syncthreads();
+    const SceneView V{A.voff, A.foff, A.eoff, A.tris, A.edges, nullptr};
+    const int32_t* tuple = k == 2 ? A.in.pt : A.in.ee;
+    const int32_t* vids = k == 2 ? A.in.vids.pt : A.in.vids.ee;
+    float* out = k == 2 ? W.apt : W.aee;
+    const bool use = k == 2 ? W.use_pt : W.use_ee;
+    for (int j0 = wave_id() * kWave; j0 < mine; j0 += kBlock) {
+        const int j = j0 + lane_id();
+        const bool in = j < mine;
+        bool queued = false;
+        int s = 0;
+        if (in) {
+            const int64_t i = i0 + list[j], o = off + j;
+            const int32_t* tu = tuple + 5 * i;
+            s = W.S > 1 ? W.body_scene[tu[0]] : 0;
+            write_entry(A, poff, k, i, o);
+            float apart = 0.0f;
+            if (W.body_on[tu[0]]) {
+                d3 a[4], b[4];
+                cand_verts(k == 2 ? 0 : 1, V, A.x, A.x1, tu, a, b, vids ? vids + 4 * i : nullptr);
+                apart = apart_until(k == 2 ? 0 : 1, a, b, W.dhat);
+                queued = use && toi_bracketed(a, b);
+            }
+            out[o] = apart;
+        }
+        count_scene(W, k == 3 ? 0 : 1, in, s);
+        const unsigned long long mq = __ballot(queued);
+        if (mq) {
+            const int leader = __ffsll((long long)mq) - 1;
+            int32_t base = 0;
+            if (lane_id() == leader) base = atomicAdd(&qn, (int)__popcll(mq));
+            base = __shfl(base, leader);
+            if (queued) qlist[base + __popcll(mq & ((1ull << lane_id()) - 1ull))] = (uint16_t)j;
+        }
+    }
+    __syncthreads();
+    if (qn == 0) return;  // uniform
+    if (t == 0) qbase = atomicAdd(W.qcount, qn);
+    __syncthreads();
+    for (int q = t; q < qn; q += kBlock)
+        W.queue[qbase + q] = (int32_t)(((off + qlist[q]) << 1) | (k == 3 ? 1 : 0));
+}
+
+// The pair blocks' offsets of more than kBlock blocks.
+__global__ __launch_bounds__(kScanThreads) void keep_pair_scan_kernel(const uint32_t* __restrict__ cnt, int64_t n,
+                                                                      int64_t* __restrict__ off) {
+    scan_block_exclusive_by([cnt](int64_t i) { return (int64_t)cnt[i]; }, off, n, nullptr, nullptr);
 }
 
 }  // namespace
+
+size_t keep_counters(int64_t nij, int64_t npt, int64_t nee, int64_t nvg) {
+    size_t n = 0;
+    for (int64_t m : {nij, nij, npt, nee, nvg}) n += (size_t)ceil_div(ceil_div(m, (int64_t)kBlock), kSuper);
+    return kSuperStride * n;
+}
 
 namespace {
 __global__ __launch_bounds__(kBlock) void cand_vid_kernel(SceneView V, int kind, const int32_t* __restrict__ tuples,
@@ -934,8 +1176,8 @@ int cand_vertex_ids(hipStream_t s, const AbdScene* sc, int kind, const int32_t* 
 
 int keep_from_superset(hipStream_t s, const AbdScene* sc, const KeepInput& in, const KeepBoxes& bx, double dhat,
                        double ground, const KeepOutput& out, int64_t* dcount, int64_t* hcount, bool sync,
-                       const KeepAtX* at) {
-    KeepArgs A;
+                       const KeepAtX* at, uint32_t* counters, const KeepSweep* sweep) {
+    KeepArgs A{};
     A.in = in;
     A.bx = bx;
     A.out = out;
@@ -953,29 +1195,47 @@ int keep_from_superset(hipStream_t s, const AbdScene* sc, const KeepInput& in, c
     A.body_scene = at ? at->body_scene : nullptr;
     A.yth = 0.5 * dhat + ground;
     A.fg = (float)ground;
+    A.dcount = dcount;
+    if (sweep) A.W = *sweep;
     const int64_t n[kKeepLists] = {in.nij, in.ji ? in.nij : 0, in.npt, in.nee, in.nvg};
-    int64_t nblk[kKeepLists], total = 0, nflag = 0;
+    int64_t nblk[kKeepLists], total = 0, nflag = 0, nsup = 0;
     A.blk0[0] = 0;
     for (int k = 0; k < kKeepLists; ++k) {
         A.flag0[k] = nflag;
-        nflag += n[k];
+        nflag += ceil_div(n[k], (int64_t)kFlagAlign) * kFlagAlign;
         A.n[k] = n[k];
         nblk[k] = ceil_div(n[k], (int64_t)kBlock);
-        A.blk0[k + 1] = A.blk0[k] + nblk[k];
-        total += 2 * (nblk[k] + 1);
+        A.blk0[k + 1] = A.blk0[k] + ceil_div(nblk[k], (int64_t)kXcds) * kXcds;
+        total += nblk[k];
+        nsup += ceil_div(nblk[k], kSuper);
     }
-    if (A.blk0[kKeepLists] > INT32_MAX) return ABD_ERR_ARG;
-    int64_t* buf;
+    if (A.blk0[kKeepLists] >= INT32_MAX) return ABD_ERR_ARG;
+    if (sweep && in.npt + in.nee > (int64_t)INT32_MAX / 2) return ABD_ERR_ARG;  // the queue's indices
+    // more pair blocks than the write pass sums in LDS: scanned, their offsets beside the counts
+    const bool scan = nblk[0] > kBlock;
+    uint32_t* buf;
     int rc;
-    if ((rc = arena_get(kSlotKeep, sizeof(int64_t) * (size_t)total, (void**)&buf))) return rc;
+    const size_t own = counters ? 0 : keep_counters(in.nij, in.npt, in.nee, in.nvg);
+    const size_t even = ((size_t)total + own + 1) & ~(size_t)1;
+    if ((rc = arena_get(kSlotKeep, sizeof(uint32_t) * even + (scan ? sizeof(int64_t) * (size_t)nblk[0] : 0),
+                        (void**)&buf)))
+        return rc;
     if ((rc = arena_get(kSlotKeepMap, sizeof(int32_t) * ((size_t)in.nij + 1), (void**)&A.remap))) return rc;
+    int64_t* pair_off = scan ? reinterpret_cast<int64_t*>(buf + even) : nullptr;
+    A.pair_off = pair_off;
+    if (!counters) {
+        counters = buf;
+        buf += own;
+        if ((rc = zero_fill(s, counters, sizeof(uint32_t) * own))) return rc;
+    }
     for (int k = 0; k < kKeepLists; ++k) {
         A.bcnt[k] = buf;
-        A.boff[k] = buf + nblk[k] + 1;
-        buf += 2 * (nblk[k] + 1);
+        buf += nblk[k];
+        A.scnt[k] = counters;
+        counters += kSuperStride * ceil_div(nblk[k], kSuper);
     }
     // counts of all five lists in one launch (with the kept pairs' ranks in their
-    // workgroups), their scans (totals to dcount), then every list written in one launch
+    // workgroups), then every list written in one launch, with the totals to dcount
     const int64_t nall = A.blk0[kKeepLists];
     if ((rc = arena_get(kSlotKeepFlags, (size_t)nflag + 1, (void**)&A.flag))) return rc;
     const int ph = prof_start(kProfKeep, s, 0.0);
@@ -983,15 +1243,30 @@ int keep_from_superset(hipStream_t s, const AbdScene* sc, const KeepInput& in, c
         hipLaunchKernelGGL(keep_count_kernel, dim3((unsigned)nall), dim3(kBlock), 0, s, A);
         ABD_CHECK_LAUNCH();
     }
-    ScanSeg sg[kKeepLists];  // an empty list's scan only writes its total, 0
-    for (int k = 0; k < kKeepLists; ++k)
-        sg[k] = ScanSeg{A.bcnt[k], A.boff[k], nblk[k], A.boff[k] + nblk[k], dcount + k};
-    if ((rc = scan_exclusive_i64_multi(s, sg, kKeepLists))) return rc;
-    if (nall > 0) {
-        hipLaunchKernelGGL(keep_write_kernel, dim3((unsigned)nall), dim3(kBlock), 0, s, A, 0, kKeepLists);
+    if (scan) {
+        hipLaunchKernelGGL(keep_pair_scan_kernel, dim3(1), dim3(kScanThreads), 0, s, (const uint32_t*)A.bcnt[0],
+                           nblk[0], pair_off);
         ABD_CHECK_LAUNCH();
     }
     prof_stop(ph, s);
+    if (sweep) {
+        A.grp0[0] = 0;
+        for (int k = 0; k < kKeepLists; ++k)
+            A.grp0[k + 1] = A.grp0[k] +
+                            ceil_div(nblk[k], (int64_t)kXcds * (k == 2 || k == 3 ? kSweepBlocks : 1)) * kXcds;
+        // bytes: per superset entry (an upper bound of the kept ones) the CCD's tuple, ids and
+        // vertices at both ends
+        const int phw = prof_start(kProfToi, s, 228.0 * in.nee + 224.0 * in.npt + 56.0 * in.nvg);
+        hipLaunchKernelGGL(sweep_write_kernel, dim3((unsigned)std::max<int64_t>(A.grp0[kKeepLists], 1)),
+                           dim3(kBlock), 0, s, A);
+        ABD_CHECK_LAUNCH();
+        prof_stop(phw, s);
+    } else {
+        const int phw = prof_start(kProfKeep, s, 0.0);
+        hipLaunchKernelGGL(keep_write_kernel, dim3((unsigned)std::max<int64_t>(nall, 1)), dim3(kBlock), 0, s, A);
+        ABD_CHECK_LAUNCH();
+        prof_stop(phw, s);
+    }
     if (hcount) {
         ABD_CHECK(hipMemcpyAsync(hcount, dcount, kKeepLists * sizeof(int64_t), hipMemcpyDeviceToHost, s));
         if (sync) ABD_CHECK(hipStreamSynchronize(s));

@@ -134,7 +134,7 @@ int within_ranges(hipStream_t s, int64_t n3, const double* x, const double* lo, 
 // PT / EE candidate (4 per tuple, in the order fetch_pt_idx / fetch_ee_idx give them), so
 // that a kernel reads them instead of gathering them through the topology; and of each PT /
 // EE / VG candidate the step length below which it stays inactive on the step last passed to
-// scene_toi (apart_until), written there and read by line_chunks and the next filter.
+// whose CCD was taken (apart_until), written by the filter (KeepSweep) and read by line_chunks and the next filter.
 struct CandSide {
     const int32_t* pt = nullptr;
     const int32_t* ee = nullptr;
@@ -160,30 +160,19 @@ int trial_states(hipStream_t s, const AbdScene* sc, const AbdParams* P, int S, i
 int line_chunks(hipStream_t s, const AbdScene* sc, const AbdParams* P, int S, int K, const double* alpha,
                 const double* st, const int32_t* pt, int64_t npt, const int32_t* ee, int64_t nee, const int32_t* vg,
                 int64_t nvg, const int64_t* plan, const int64_t* dn, CandSide vids, TrialSums* out);
-// The per-scene chunk plan of the energy / TOI reductions over one set of candidate lists
-// (plan: reduce_plan_elems(S) int64 on the device), made once and passed as `plan` to every
-// reduction over those lists (nullptr: each makes its own).  Also readies the CCD's scratch for
-// one scene_toi with the plan, and zeroes nzero (at most 1024) counters of the caller.
+// The per-scene chunk plan of the energy reductions over one set of candidate lists: its size
+// (int64); the swept set's is made by its filter (KeepSweep).
 size_t reduce_plan_elems(int S);
-int reduce_plan(hipStream_t s, const AbdScene* sc, const AbdParams* P, int S, const int32_t* pt, int64_t npt,
-                const int32_t* ee, int64_t nee, const int32_t* vg, int64_t nvg, int64_t* plan,
-                const int64_t* dn = nullptr, int64_t* zero = nullptr, int nzero = 0);
-// Per-scene TOI (abd_scene_toi; S = 1: the whole system as one scene) with an optional plan;
-// active (nullable, [S]): scenes whose TOI is wanted, the others report 1 unevaluated.
-// Per-scene dot products a.b and c.d (each seg_dot_kernel's) that the TOI's final per-scene pass computes
-// after the scene's TOI when out1 is set (the driver's q.g and g.g, one launch less).
+// Per-scene dot products a.b and c.d (each seg_dot_kernel's) that the TOI's final per-scene
+// pass computes after the scene's TOI when out1 is set (the driver's q.g and g.g).
 struct SceneDots {
     const int32_t* sboff = nullptr;
     int64_t n = 0;
     const double *a = nullptr, *b = nullptr, *c = nullptr, *d = nullptr;
     double *out1 = nullptr, *out2 = nullptr;
 };
-int scene_toi(hipStream_t s, const AbdScene* sc, const AbdParams* P, int S, const double* x_t0, const double* x_t1,
-              const int32_t* pt, int64_t npt, const int32_t* ee, int64_t nee, const int32_t* vg, int64_t nvg,
-              const int64_t* plan, double* toi, const uint8_t* active, const int64_t* dn = nullptr,
-              double* first_alpha = nullptr, CandSide vids = {}, const SceneDots* dots = nullptr);
 // The line search's first step length from a TOI (abd.py:300-302): clamped to [0, 1], x 0.9
-// below 1.  scene_toi's first_alpha (device, nullable) receives it per scene (-1 for the
+// below 1.  sweep_toi's first_alpha (device, nullable) receives it per scene (-1 for the
 // scenes not active).
 __host__ __device__ inline double first_step_length(double t) {
     t = t < 1.0 ? t : 1.0;  // std::min(1.0, t)
@@ -206,6 +195,12 @@ struct BodyStart {
     double *g, *blocks;
     double* zero;  // nzero words zeroed
     int64_t nzero;
+    uint32_t* zero32;  // nzero32 more, of 4 bytes
+    int64_t nzero32;
+    unsigned long long* slots;  // [ns] set to 1.0
+    int32_t* qcount;            // set to 0
+    int64_t* counters;          // ncounters set to 0
+    int ncounters;
     int ns;
     uint8_t* newton;
     double* E0;
@@ -228,6 +223,7 @@ struct BodyEnd {
     const double *lo, *hi, *qref, *rest_max;
     double skin, margin;
     int64_t* flag;
+    uint8_t* on;  // [nb] active of the body's scene
 };
 int body_end(hipStream_t s, const AbdScene* sc, const BodyEnd& U);
 // each body's largest |rest coordinate| per axis (out [nb][3]) and a copy of the rest positions
@@ -282,11 +278,41 @@ struct KeepAtX {
     const double* alpha = nullptr;
     const int32_t* body_scene = nullptr;
 };
+// The CCD of a step taken while its swept set is written (x, x1: the step's ends), over the
+// scenes with active[s]: each kept PT / EE / VG entry's apart_until, the PT / EE entries whose
+// cubic has a bracketed root queued as (output index << 1 | is EE), the VG entries' TOI min-ed
+// into their scene's slot, and the kept entries per list (EE, PT, VG) and scene counted
+// (S > 1), from which sweep_toi makes the reduction plan of the output lists.
+constexpr int kSweepLists = 3;
+struct KeepSweep {
+    int S;
+    const uint8_t* active;   // [S]
+    const uint8_t* body_on;  // [nb], a body's scene's
+    const int32_t* body_scene;
+    double ground, dhat;
+    int32_t* queue;
+    int32_t* qcount;            // 0 before
+    unsigned long long* slots;  // 1.0 before
+    float *apt, *aee, *avg;     // apart_until beside the output lists
+    uint32_t* scnt;             // [kSweepLists][S], 0 before
+    int use_pt, use_ee, use_vg;  // a list switched off has no TOI
+};
+// Counters of a filter of lists of these sizes (uint32, an even number of them, 0 before it).
+size_t keep_counters(int64_t nij, int64_t npt, int64_t nee, int64_t nvg);
+// The arena's CCD scratch of a set of nq PT and EE candidates over S scenes.
+int toi_scratch(int S, int64_t nq, unsigned long long** slots, int32_t** qcount, int32_t** queue);
+// The reduction plan (int64 [reduce_plan_elems(S)]) of the lists a sweep wrote (dn: their
+// sizes on the device in the keep layout; npt, nee bound them), the scene minima from the
+// queued candidates, the first step lengths and the scenes' dots.
+int sweep_toi(hipStream_t s, const AbdScene* sc, const AbdParams* P, int S, const double* x_t0, const double* x_t1,
+              const int32_t* pt, int64_t npt, const int32_t* ee, int64_t nee, const int64_t* dn, CandSide side,
+              const KeepSweep& W, int64_t* plan, double* toi, double* first_alpha, const SceneDots& dots);
 // sync false: the totals reach hcount with the stream's next synchronization (the caller's);
 // hcount null: they stay on the device.
+// counters (nullable): keep_counters words zeroed before (else the call zeroes its own).
 int keep_from_superset(hipStream_t s, const AbdScene* sc, const KeepInput& in, const KeepBoxes& bx, double dhat,
                        double ground, const KeepOutput& out, int64_t* dcount, int64_t* hcount, bool sync = true,
-                       const KeepAtX* at = nullptr);
+                       const KeepAtX* at = nullptr, uint32_t* counters = nullptr, const KeepSweep* sweep = nullptr);
 // abd_bsr_structure; dnij (nullable): the pair count on the device (nij bounds it; cols and
 // slots hold nb + 2 nij entries).
 int bsr_structure(hipStream_t s, int nb, const int32_t* ij, const int32_t* ji, int64_t nij, const int64_t* dnij,

@@ -75,12 +75,10 @@ __device__ __forceinline__ int64_t n_chunks(int64_t len) { return (len + kChunkI
 constexpr int kPlanThreads = 1024;
 constexpr unsigned long long kBitsOne = 0x3FF0000000000000ull;  // 1.0
 // What the plan's kernel also sets for the CCD that follows it (nullable): the scene slots to
-// 1, the queue count and nzero counters of the caller to 0.
+// 1, the queue count to 0.
 struct ToiInit {
     unsigned long long* slots = nullptr;
     int32_t* qcount = nullptr;
-    int64_t* zero = nullptr;
-    int nzero = 0;
 };
 __global__ __launch_bounds__(kPlanThreads) void plan_kernel(int S, const int32_t* __restrict__ body_scene, Lists L,
                                                             int64_t* __restrict__ seg, int64_t* __restrict__ choff,
@@ -90,7 +88,6 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(int S, const int32_t
         for (int s = threadIdx.x; s < S; s += blockDim.x) I.slots[s] = kBitsOne;
         if (threadIdx.x == 0) *I.qcount = 0;
     }
-    if (I.zero && threadIdx.x < I.nzero) I.zero[threadIdx.x] = 0;
     __shared__ int64_t tile_total;
     for (int idx = threadIdx.x; idx < kLists * (S + 1); idx += blockDim.x) {
         const int l = idx / (S + 1), s = idx % (S + 1);
@@ -410,9 +407,9 @@ __global__ __launch_bounds__(kRedThreads) void scene_final_kernel(const int64_t*
 // The scene minimum of the TOIs below 1 (ccd.py:9-40, abd.py:284-299) in two passes.
 // toi_scan_kernel: one candidate per thread (kToiSplit workgroups of kRedThreads per chunk
 // of the plan): the vertex-ground TOI directly, and for a PT / EE candidate its
-// coplanarity cubic and bracket test (with its apart_until, from the same vertices, for the
-// line search); the few candidates with a bracketed root in [0, 1] go to a queue (one
-// atomic per wave).  toi_solve_kernel: the full collision_time of each
+// coplanarity cubic and bracket test; the few candidates with a bracketed root in [0, 1] go
+// to a queue (one atomic per wave).  (The native driver's filter of the swept set does this
+// per entry: KeepSweep.)  toi_solve_kernel: the full collision_time of each
 // queued candidate (root searches and validity), its TOI below 1 min-ed into its scene's
 // slot (non-negative doubles order like their bit patterns, so an integer atomic min is
 // exact).  toi_final_kernel: per scene the minimum of its chunks' partials and its slot.
@@ -435,40 +432,30 @@ __global__ __launch_bounds__(kRedThreads, 4) void toi_scan_kernel(AbdScene sc, A
                                                                const double* __restrict__ x1, Lists L, int S,
                                                                const int64_t* __restrict__ seg,
                                                                const int64_t* __restrict__ choff,
-                                                               const uint8_t* __restrict__ active,
                                                                double* __restrict__ part, int32_t* __restrict__ queue,
                                                                int32_t* __restrict__ qcount) {
     __shared__ double sh[kRedThreads / kWave];
     const int64_t c = blockIdx.x;
     if (c >= choff[S]) return;  // uniform over the workgroup
     const ChunkRange r = chunk_range(S, seg, choff, c);
-    const bool on = !active || active[r.s];
     const SceneView V{sc.voff, sc.foff, sc.eoff, sc.tris, sc.edges, sc.x0};
     const ListRef& Lr = L.l[r.l < kLists ? r.l : 0];
     const int kind = Lr.kind, ck = kind == kListPT ? 0 : 1;
     const int64_t i = r.start + (int64_t)blockIdx.y * kRedThreads + threadIdx.x;
-    const double dhat = fmax(P.dhat, sqrt(P.d2hat));  // the boxes' dilation, the barrier's range
     double acc = 1.0;
     bool queued = false;
     int32_t entry = 0;
     if (r.l < kLists && i < r.end) {
-        float apart = 0.0f;
-        if (on) {
-            const int32_t* t = Lr.p + (int64_t)width_of(kind) * i;
-            if (kind == kListVG) {
-                const int64_t vid = sc.voff[t[0]] + t[1];
-                apart = apart_until_vg(x0[3 * vid + 1], x1[3 * vid + 1], P.ground, dhat);
-                const double tv = cand_toi_vg(sc.voff, x0, x1, t, P.ground);
-                if (tv < 1.0) acc = tv;  // `if t < 1: atomic_min`
-            } else {
-                d3 a[4], b[4];
-                cand_verts(ck, V, x0, x1, t, a, b, vids_of(Lr, i));
-                apart = apart_until(ck, a, b, dhat);
-                queued = toi_bracketed(a, b);
-                entry = (int32_t)((i << 1) | (kind == kListEE ? 1 : 0));
-            }
+        const int32_t* t = Lr.p + (int64_t)width_of(kind) * i;
+        if (kind == kListVG) {
+            const double tv = cand_toi_vg(sc.voff, x0, x1, t, P.ground);
+            if (tv < 1.0) acc = tv;  // `if t < 1: atomic_min`
+        } else {
+            d3 a[4], b[4];
+            cand_verts(ck, V, x0, x1, t, a, b, vids_of(Lr, i));
+            queued = toi_bracketed(a, b);
+            entry = (int32_t)((i << 1) | (kind == kListEE ? 1 : 0));
         }
-        if (Lr.apart) Lr.apart[i] = apart;
     }
     // wave-aggregated push of the queued candidates
     const unsigned long long mask = __ballot(queued);
@@ -490,15 +477,67 @@ __global__ __launch_bounds__(kRedThreads, 4) void toi_scan_kernel(AbdScene sc, A
     }
 }
 
+// The reduction plan of the EE, PT and VG lists a sweep wrote (plan_kernel's) from its
+// per-scene counts (S = 1: the lists' sizes dn), by one wave.
+struct SweepPlan {
+    const uint32_t* scnt = nullptr;
+    const int64_t* dn = nullptr;
+    int use[kLists] = {};
+    int64_t* plan = nullptr;  // nullptr: no plan
+};
+__device__ __forceinline__ void sweep_plan(int S, const SweepPlan& Q) {
+    int64_t *seg = Q.plan, *choff = seg + 2 * kLists * (int64_t)S;
+    int64_t carry[kLists + 1] = {};
+    for (int base = 0; base < S; base += kWave) {
+        const int s = base + lane_id();
+        int64_t v[kLists + 1] = {};
+#pragma unroll
+        for (int l = 0; l < kLists; ++l) {
+            if (s < S && Q.use[l])
+                v[l] = S > 1 ? (int64_t)Q.scnt[(int64_t)l * S + s] : Q.dn[l == 0 ? 3 : l == 1 ? 2 : 4];
+            v[kLists] += n_chunks(v[l]);
+        }
+#pragma unroll
+        for (int l = 0; l <= kLists; ++l) {
+            int64_t incl = v[l];
+            for (int o = 1; o < kWave; o <<= 1) {
+                const int64_t u = __shfl_up(incl, o);
+                if (lane_id() >= o) incl += u;
+            }
+            const int64_t e = carry[l] + incl;
+            if (s < S) {
+                if (l < kLists) {
+                    seg[2 * (kLists * (int64_t)s + l)] = e - v[l];
+                    seg[2 * (kLists * (int64_t)s + l) + 1] = e;
+                } else {
+                    choff[s] = e - v[l];
+                }
+            }
+            carry[l] = __shfl(e, kWave - 1);
+        }
+    }
+    if (lane_id() == 0) choff[S] = carry[kLists];
+}
+
 __global__ __launch_bounds__(kToiSolveThreads) void toi_solve_kernel(AbdScene sc, Lists L, int S,
                                                                      const double* __restrict__ x0,
                                                                      const double* __restrict__ x1,
                                                                      const int32_t* __restrict__ queue,
                                                                      const int32_t* __restrict__ qcount,
-                                                                     unsigned long long* __restrict__ slots) {
+                                                                     unsigned long long* __restrict__ slots,
+                                                                     SweepPlan Q) {
+    int block = blockIdx.x, blocks = gridDim.x;
+    if (Q.plan) {  // block 0 makes the plan, the others solve
+        if (block == 0) {
+            sweep_plan(S, Q);
+            return;
+        }
+        --block;
+        --blocks;
+    }
     const int32_t n = *qcount;
     const SceneView V{sc.voff, sc.foff, sc.eoff, sc.tris, sc.edges, sc.x0};
-    for (int32_t q = blockIdx.x * kToiSolveThreads + threadIdx.x; q < n; q += gridDim.x * kToiSolveThreads) {
+    for (int32_t q = block * kToiSolveThreads + threadIdx.x; q < n; q += blocks * kToiSolveThreads) {
         const int32_t e = queue[q];
         const int ee = e & 1;
         const ListRef& Lr = L.l[ee ? 0 : 1];  // the lists' order: EE, PT, VG
@@ -511,8 +550,9 @@ __global__ __launch_bounds__(kToiSolveThreads) void toi_solve_kernel(AbdScene sc
     }
 }
 
-// alpha (nullable): the line search's first step length of each scene from its TOI
-// (first_step_length; -1 for a scene not in `active`)
+// choff (nullable): no partials, the slots hold every list's minima.  alpha (nullable): the
+// line search's first step length of each scene from its TOI (first_step_length; -1 for a
+// scene not in `active`)
 __global__ __launch_bounds__(kRedThreads) void toi_final_kernel(const int64_t* __restrict__ choff,
                                                                 const double* __restrict__ part,
                                                                 const unsigned long long* __restrict__ slots,
@@ -522,11 +562,14 @@ __global__ __launch_bounds__(kRedThreads) void toi_final_kernel(const int64_t* _
     __shared__ double sh[kRedThreads];
     const int s = blockIdx.x;
     double acc = __longlong_as_double((long long)slots[s]);
-    for (int64_t i = choff[s] * kToiSplit + threadIdx.x; i < choff[s + 1] * kToiSplit; i += blockDim.x) {
-        const double v = part[i];
-        acc = v < acc ? v : acc;
+    double r = acc;
+    if (choff) {
+        for (int64_t i = choff[s] * kToiSplit + threadIdx.x; i < choff[s + 1] * kToiSplit; i += blockDim.x) {
+            const double v = part[i];
+            acc = v < acc ? v : acc;
+        }
+        r = block_min(acc, sh);
     }
-    const double r = block_min(acc, sh);
     if (threadIdx.x == 0) {
         out[s] = r;
         if (alpha) alpha[s] = !active || active[s] ? first_step_length(r) : -1.0;
@@ -622,9 +665,9 @@ int get_plan(hipStream_t s, const AbdScene& sc, int S, const Lists& L, const int
     return ABD_OK;
 }
 
-// The arena's scene slots and queue count of the CCD.
-int toi_slots(int S, unsigned long long** slots, int32_t** qcount) {
-    const int rc = arena_get(kSlotToiSlots, sizeof(unsigned long long) * (size_t)(S + 1), (void**)slots);
+int toi_scratch(int S, int64_t nq, unsigned long long** slots, int32_t** qcount, int32_t** queue) {
+    int rc = arena_get(kSlotToiQueue, sizeof(int32_t) * (size_t)(nq + 1), (void**)queue);
+    if (!rc) rc = arena_get(kSlotToiSlots, sizeof(unsigned long long) * (size_t)(S + 1), (void**)slots);
     if (!rc) *qcount = reinterpret_cast<int32_t*>(*slots + S);
     return rc;
 }
@@ -651,17 +694,16 @@ int seg_reduce(hipStream_t s, const AbdScene& sc, const AbdParams& P, int S, con
 
 // Algorithmic bytes of a launch over the plan's scenes: c_ee, c_pt, c_vg per EE, PT and VG
 // candidate of every (trial k, scene s) it evaluates -- K trials with step lengths alpha
-// [K][S] (nullable; a negative step length skips the scene's trial) of the scenes with
-// active[s] set (nullable: all) -- from the plan's per-scene segments.
+// [K][S] (nullable; a negative step length skips the scene's trial) -- from the plan's
+// per-scene segments.
 __global__ __launch_bounds__(kRedThreads) void seg_bytes_kernel(int S, int K, const double* __restrict__ alpha,
-                                                                const uint8_t* __restrict__ active,
                                                                 const int64_t* __restrict__ seg, double c_ee,
                                                                 double c_pt, double c_vg, double* __restrict__ out) {
     __shared__ double sh[kRedThreads];
     double acc = 0.0;
     for (int64_t i = threadIdx.x; i < (int64_t)S * K; i += blockDim.x) {
         const int64_t sc = i % S;
-        if ((alpha && !(alpha[i] >= 0.0)) || (active && !active[sc])) continue;
+        if (alpha && !(alpha[i] >= 0.0)) continue;
         const int64_t* q = seg + 2 * (int64_t)kLists * sc;
         acc += c_ee * (double)(q[1] - q[0]) + c_pt * (double)(q[3] - q[2]) + c_vg * (double)(q[5] - q[4]);
     }
@@ -670,23 +712,36 @@ __global__ __launch_bounds__(kRedThreads) void seg_bytes_kernel(int S, int K, co
 }
 
 // Attaches to `handle` the bytes of seg_bytes_kernel (nothing when the handle is -1).
-int attach_seg_bytes(int handle, hipStream_t s, int S, int K, const double* alpha, const uint8_t* active,
-                     const int64_t* seg, double c_ee, double c_pt, double c_vg) {
+int attach_seg_bytes(int handle, hipStream_t s, int S, int K, const double* alpha, const int64_t* seg, double c_ee,
+                     double c_pt, double c_vg) {
     double* out;
     int rc = prof_byte_slot(handle, &out);
     if (rc || !out) return rc;
-    hipLaunchKernelGGL(seg_bytes_kernel, dim3(1), dim3(kRedThreads), 0, s, S, K, alpha, active, seg, c_ee, c_pt,
-                       c_vg, out);
+    hipLaunchKernelGGL(seg_bytes_kernel, dim3(1), dim3(kRedThreads), 0, s, S, K, alpha, seg, c_ee, c_pt, c_vg,
+                       out);
     ABD_CHECK_LAUNCH();
     prof_stop(handle, s, nullptr, out);
+    return ABD_OK;
+}
+
+// The queued candidates of the EE and PT lists (L.l[0], L.l[1]) solved into the slots.
+int toi_solve(hipStream_t s, const AbdScene& sc, int S, const double* x0, const double* x1, const Lists& L,
+              const int32_t* queue, const int32_t* qcount, unsigned long long* slots, bool prof,
+              const SweepPlan& Q = {}) {
+    const int64_t nq = L.l[0].n + L.l[1].n;
+    const int64_t gmax = tuning().toi_grid > 0 ? tuning().toi_grid : kToiSolveGrid;
+    const unsigned grid = (unsigned)std::min<int64_t>(gmax, std::max<int64_t>(1, ceil_div(nq, 4 * kToiSolveThreads)));
+    const int ph = prof ? prof_start_ext(kProfToiSolve, 0.0) : -1;
+    prof_launch(ph, toi_solve_kernel, dim3(grid + (Q.plan ? 1 : 0)), dim3(kToiSolveThreads), 0, s, sc, L, S, x0, x1,
+                queue, qcount, slots, Q);
+    ABD_CHECK_LAUNCH();
     return ABD_OK;
 }
 
 // Per-scene TOI (toi_scan_kernel, toi_solve_kernel, toi_final_kernel) with scratch from
 // scr (nullable: the arena; then the scan and the solve are timed when profiling).
 int toi_reduce(hipStream_t s, const AbdScene& sc, const AbdParams& P, int S, const double* x0, const double* x1,
-               const Lists& L, const int64_t* plan_in, double* out, const uint8_t* active,
-               const ReduceScratch* scr, double* first_alpha = nullptr, const SceneDots* dots = nullptr) {
+               const Lists& L, double* out, const ReduceScratch* scr) {
     const int64_t bound = chunk_bound(L, S);
     if (bound * kToiSplit > INT32_MAX) return ABD_ERR_ARG;
     const int64_t nq = L.l[0].n + L.l[1].n;  // every PT and EE candidate may queue
@@ -698,29 +753,23 @@ int toi_reduce(hipStream_t s, const AbdScene& sc, const AbdParams& P, int S, con
     } else {
         int rc;
         if ((rc = arena_get(kSlotReduce, sizeof(double) * (size_t)(bound * kToiSplit), (void**)&w.part))) return rc;
-        if ((rc = arena_get(kSlotToiQueue, sizeof(int32_t) * (size_t)(nq + 1), (void**)&w.queue))) return rc;
-        if ((rc = toi_slots(S, &w.slots, &w.qcount))) return rc;
+        if ((rc = toi_scratch(S, nq, &w.slots, &w.qcount, &w.queue))) return rc;
     }
     const int64_t *seg, *choff;
-    // (a plan made by reduce_plan has set the arena's slots)
-    int rc = get_plan(s, sc, S, L, plan_in, &seg, &choff, w.plan, ToiInit{w.slots, w.qcount});
+    int rc = get_plan(s, sc, S, L, nullptr, &seg, &choff, w.plan, ToiInit{w.slots, w.qcount});
     if (rc) return rc;
     // algorithmic bytes of the scan: tuple, indices and four vertices at both ends per PT / EE
     // candidate (224 / 228 B), tuple, offset and a vertex at both ends per VG candidate (56 B),
     // over the scenes it evaluates (counted on the device)
     const int ph = scr ? -1 : prof_start_ext(kProfToi, 1.0);
     prof_launch(ph, toi_scan_kernel, dim3((unsigned)bound, kToiSplit), dim3(kRedThreads), 0, s, sc, P, x0, x1, L, S,
-                seg, choff, active, w.part, w.queue, w.qcount);
+                seg, choff, w.part, w.queue, w.qcount);
     ABD_CHECK_LAUNCH();
-    if ((rc = attach_seg_bytes(ph, s, S, 1, nullptr, active, seg, 228.0, 224.0, 56.0))) return rc;
-    const int64_t gmax = tuning().toi_grid > 0 ? tuning().toi_grid : kToiSolveGrid;
-    const unsigned grid = (unsigned)std::min<int64_t>(gmax, std::max<int64_t>(1, ceil_div(nq, 4 * kToiSolveThreads)));
-    const int ph2 = scr ? -1 : prof_start_ext(kProfToiSolve, 0.0);
-    prof_launch(ph2, toi_solve_kernel, dim3(grid), dim3(kToiSolveThreads), 0, s, sc, L, S, x0, x1,
-                (const int32_t*)w.queue, (const int32_t*)w.qcount, w.slots);
-    ABD_CHECK_LAUNCH();
+    if ((rc = attach_seg_bytes(ph, s, S, 1, nullptr, seg, 228.0, 224.0, 56.0))) return rc;
+    if ((rc = toi_solve(s, sc, S, x0, x1, L, w.queue, w.qcount, w.slots, !scr))) return rc;
     hipLaunchKernelGGL(toi_final_kernel, dim3(S), dim3(kRedThreads), 0, s, choff, (const double*)w.part,
-                       (const unsigned long long*)w.slots, out, active, first_alpha, dots ? *dots : SceneDots{});
+                       (const unsigned long long*)w.slots, out, (const uint8_t*)nullptr, (double*)nullptr,
+                       SceneDots{});
     ABD_CHECK_LAUNCH();
     return ABD_OK;
 }
@@ -740,18 +789,6 @@ Lists contact_lists(const AbdParams& P, const int32_t* pt, int64_t npt, const in
 }
 
 size_t reduce_plan_elems(int S) { return 2 * kLists * (size_t)S + (size_t)S + 1; }
-
-int reduce_plan(hipStream_t s, const AbdScene* sc, const AbdParams* P, int S, const int32_t* pt, int64_t npt,
-                const int32_t* ee, int64_t nee, const int32_t* vg, int64_t nvg, int64_t* plan, const int64_t* dn,
-                int64_t* zero, int nzero) {
-    const Lists L = contact_lists(*P, pt, npt, ee, nee, vg, nvg, dn);
-    ToiInit init{nullptr, nullptr, zero, nzero};
-    if (int rc = toi_slots(S, &init.slots, &init.qcount)) return rc;
-    hipLaunchKernelGGL(plan_kernel, dim3(1), dim3(kPlanThreads), 0, s, S, sc->body_scene, L, plan,
-                       plan + 2 * kLists * (size_t)S, init);
-    ABD_CHECK_LAUNCH();
-    return ABD_OK;
-}
 
 // ---------------------------------------------------------- line-search trials
 // K trial states q - alpha dq evaluated together (alpha: [K][S] on the device; S = 1
@@ -791,7 +828,7 @@ int line_chunks(hipStream_t s, const AbdScene* sc, const AbdParams* P, int S, in
     prof_launch(ph, trial_chunk_kernel, dim3((unsigned)bound, groups), dim3(kRedThreads), 0, s, *sc, *P,
                 TrialArgs{alpha, st}, L, S, K, seg, choff, part, bound);
     ABD_CHECK_LAUNCH();
-    if ((rc = attach_seg_bytes(ph, s, S, K, alpha, nullptr, seg, 132.0, 128.0, 32.0))) return rc;
+    if ((rc = attach_seg_bytes(ph, s, S, K, alpha, seg, 132.0, 128.0, 32.0))) return rc;
     *out = TrialSums{choff, part, bound};
     return ABD_OK;
 }
@@ -817,15 +854,35 @@ int contact_energy(hipStream_t s, const AbdScene* sc, const AbdParams* P, int S,
     return seg_reduce(s, *sc, *P, S, xk, L, E, kProfEnergy);
 }
 
+int sweep_toi(hipStream_t s, const AbdScene* sc, const AbdParams* P, int S, const double* x_t0, const double* x_t1,
+              const int32_t* pt, int64_t npt, const int32_t* ee, int64_t nee, const int64_t* dn, CandSide side,
+              const KeepSweep& W, int64_t* plan, double* toi, double* first_alpha, const SceneDots& dots) {
+    const Lists L = contact_lists(*P, pt, npt, ee, nee, nullptr, 0, nullptr, side);
+    SweepPlan Q;
+    Q.scnt = W.scnt;
+    Q.dn = dn;
+    Q.use[0] = W.use_ee;
+    Q.use[1] = W.use_pt;
+    Q.use[2] = W.use_vg;
+    Q.plan = plan;
+    int rc;
+    if ((rc = toi_solve(s, *sc, S, x_t0, x_t1, L, W.queue, W.qcount, W.slots, true, Q))) return rc;
+    hipLaunchKernelGGL(toi_final_kernel, dim3(S), dim3(kRedThreads), 0, s, (const int64_t*)nullptr,
+                       (const double*)nullptr, (const unsigned long long*)W.slots, toi, W.active, first_alpha, dots);
+    ABD_CHECK_LAUNCH();
+    return ABD_OK;
+}
+
+namespace {
 int scene_toi(hipStream_t s, const AbdScene* sc, const AbdParams* P, int S, const double* x_t0, const double* x_t1,
               const int32_t* pt, int64_t npt, const int32_t* ee, int64_t nee, const int32_t* vg, int64_t nvg,
-              const int64_t* plan, double* toi, const uint8_t* active, const int64_t* dn, double* first_alpha,
-              CandSide vids, const SceneDots* dots) {
+              double* toi) {
     if (!P || !x_t0 || !x_t1 || !toi || npt < 0 || nee < 0 || nvg < 0) return ABD_ERR_ARG;
     if ((npt && !pt) || (nee && !ee) || (nvg && !vg)) return ABD_ERR_ARG;
-    const Lists L = contact_lists(*P, pt, npt, ee, nee, vg, nvg, dn, vids);  // abd.py:288-299
-    return toi_reduce(s, *sc, *P, S, x_t0, x_t1, L, plan, toi, active, nullptr, first_alpha, dots);
+    const Lists L = contact_lists(*P, pt, npt, ee, nee, vg, nvg);  // abd.py:288-299
+    return toi_reduce(s, *sc, *P, S, x_t0, x_t1, L, toi, nullptr);
 }
+}  // namespace
 
 // ------------------------------------------------- allocation-free TOI scratch
 // The fixed scratch of abd_toi_noalloc: the chunk plan (kNoAllocPlanElems int64), the scene
@@ -894,8 +951,7 @@ int abd_toi(abd_stream_t stream, const AbdScene* sc, const AbdParams* P, const d
             const int32_t* pt, int64_t npt, const int32_t* ee, int64_t nee, const int32_t* vg, int64_t nvg,
             double* toi) {
     if (!sc) return ABD_ERR_ARG;
-    return scene_toi(to_stream(stream), sc, P, 1, x_t0, x_t1, pt, npt, ee, nee, vg, nvg, nullptr, toi, nullptr,
-                     nullptr);
+    return scene_toi(to_stream(stream), sc, P, 1, x_t0, x_t1, pt, npt, ee, nee, vg, nvg, toi);
 }
 
 int abd_toi_noalloc(abd_stream_t stream, const AbdScene* sc, const AbdParams* P, const double* x_t0,
@@ -909,15 +965,14 @@ int abd_toi_noalloc(abd_stream_t stream, const AbdScene* sc, const AbdParams* P,
     ReduceScratch scr;
     int rc = noalloc_scratch(&scr);
     if (rc) return rc;
-    return toi_reduce(to_stream(stream), *sc, *P, 1, x_t0, x_t1, L, nullptr, toi, nullptr, &scr);
+    return toi_reduce(to_stream(stream), *sc, *P, 1, x_t0, x_t1, L, toi, &scr);
 }
 
 int abd_scene_toi(abd_stream_t stream, const AbdScene* sc, const AbdParams* P, const double* x_t0,
                   const double* x_t1, const int32_t* pt, int64_t npt, const int32_t* ee, int64_t nee,
                   const int32_t* vg, int64_t nvg, double* toi) {
     if (!scenes_ok(sc)) return ABD_ERR_ARG;
-    return scene_toi(to_stream(stream), sc, P, sc->n_scenes, x_t0, x_t1, pt, npt, ee, nee, vg, nvg, nullptr,
-                     toi, nullptr, nullptr);
+    return scene_toi(to_stream(stream), sc, P, sc->n_scenes, x_t0, x_t1, pt, npt, ee, nee, vg, nvg, toi);
 }
 
 int abd_dot(abd_stream_t stream, const double* a, const double* b, int64_t n, double* out) {

@@ -125,6 +125,10 @@ struct Sim {
     CandSet sup;
     BoxBuf sbody, stri, sedge, spt;  // the superset's boxes
     DevBuf<double> vlo, vhi;         // its vertex ranges
+    DevBuf<uint8_t> body_on;         // body_end's
+    DevBuf<uint32_t> kcnt;           // the filters' counters (sweep_words)
+    unsigned long long* toi_slots = nullptr;  // the CCD's scratch (arena)
+    int32_t *toi_qcount = nullptr, *toi_queue = nullptr;
     DevBuf<double> qref;             // the states they were made around
     DevBuf<double> rest_max, rest_ref;  // the bodies' rest extents and the rest positions then
     bool sup_valid = false;
@@ -335,7 +339,7 @@ int collision_from(hipStream_t s, Sim& S, const CandSet& W, const double* xv) {
                      dh,   0.0,     &W == &S.sw ? S.sv.p + kSvAlpha * S.ns : nullptr,
                      S.ns > 1 ? S.sc.body_scene : nullptr};
     if ((rc = keep_from_superset(s, &S.sc, in, bx, S.P.dhat, S.P.ground, out, S.cnt.p + kCntCol, nullptr, false,
-                                 &at)))
+                                 &at, &W == &S.sw ? S.kcnt.p : nullptr)))
         return rc;
     S.col.nij = W.nij;
     S.col.npt = W.npt;
@@ -404,6 +408,46 @@ int64_t size_bound(int64_t n) {
     return (n + step - 1) / step * step;
 }
 
+// The counters of the filters of an iteration, 0 before it: the collision set's, the swept
+// set's, then its kept entries per list and scene; with the CCD's scratch for the superset.
+int64_t filter_words(const Sim& S) { return (int64_t)keep_counters(S.sup.nij, S.sup.npt, S.sup.nee, S.sup.nvg); }
+int64_t sweep_words(const Sim& S) { return 2 * filter_words(S) + kSweepLists * (int64_t)S.ns; }
+int sweep_buffers(Sim& S) {
+    int rc;
+    if ((rc = S.kcnt.reserve((size_t)sweep_words(S)))) return rc;
+    return toi_scratch(S.ns, S.sup.npt + S.sup.nee, &S.toi_slots, &S.toi_qcount, &S.toi_queue);
+}
+__global__ __launch_bounds__(kBlock) void sweep_reset_kernel(uint32_t* __restrict__ words, int64_t nwords,
+                                                                 unsigned long long* __restrict__ slots, int ns,
+                                                                 int32_t* __restrict__ qcount,
+                                                                 int64_t* __restrict__ counters, int ncounters) {
+    const int64_t i0 = blockIdx.x * (int64_t)kBlock + threadIdx.x, step = gridDim.x * (int64_t)kBlock;
+    for (int64_t i = i0; i < nwords; i += step) words[i] = 0;
+    for (int64_t i = i0; i < ns; i += step) slots[i] = 0x3FF0000000000000ull;  // 1.0
+    if (i0 < ncounters) counters[i0] = 0;
+    if (i0 == 0) *qcount = 0;
+}
+KeepSweep sweep_of(Sim& S) {
+    KeepSweep W{};
+    W.S = S.ns;
+    W.active = S.lsflag.p + (size_t)kLfNewton * S.ns;
+    W.body_on = S.body_on.p;
+    W.body_scene = S.sc.body_scene;
+    W.ground = S.P.ground;
+    W.dhat = std::max(S.P.dhat, sqrt(S.P.d2hat));  // the boxes' dilation, the barrier's range
+    W.queue = S.toi_queue;
+    W.qcount = S.toi_qcount;
+    W.slots = S.toi_slots;
+    W.apt = S.sw.apt.p;
+    W.aee = S.sw.aee.p;
+    W.avg = S.sw.avg.p;
+    W.scnt = S.kcnt.p + 2 * filter_words(S);
+    W.use_pt = S.P.pt != 0;
+    W.use_ee = S.P.ee != 0;
+    W.use_vg = S.P.vg != 0;
+    return W;
+}
+
 // The superset culled anew around the current step (its ends widened by the skin; host
 // synchronizations for the culling counts), then the swept set filtered from it.
 int swept_set_recull(hipStream_t s, Sim& S) {
@@ -445,6 +489,14 @@ int swept_set_recull(hipStream_t s, Sim& S) {
     S.sup.dn = S.cnt.p + kCntSup;
     S.sup.exact = false;
     S.sup_valid = true;
+    // the filters' counters of the new sizes and the CCD's start values (an iteration that
+    // starts with this superset has them from body_start)
+    if ((rc = sweep_buffers(S))) return rc;
+    const int64_t n = std::max<int64_t>(sweep_words(S), S.ns);
+    hipLaunchKernelGGL(sweep_reset_kernel, dim3(grid_for(n, kBlock, 1024)), dim3(kBlock), 0, s, S.kcnt.p,
+                       sweep_words(S), S.toi_slots, S.ns, S.toi_qcount, S.cnt.p + kCntNewton,
+                       kCntSolver - kCntNewton + 1);
+    ABD_CHECK_LAUNCH();
     return swept_set_launch(s, S);
 }
 
@@ -470,7 +522,9 @@ int swept_set_launch(hipStream_t s, Sim& S) {
         o.eev = S.sw.eev.p;
     }
     const KeepAtX at{st.x, st.xk, S.P.dhat, dh, 0.0};
-    if ((rc = keep_from_superset(s, &S.sc, in, bx, S.P.dhat, S.P.ground, o, S.cnt.p + kCntSw, nullptr, false, &at)))
+    const KeepSweep sweep = sweep_of(S);
+    if ((rc = keep_from_superset(s, &S.sc, in, bx, S.P.dhat, S.P.ground, o, S.cnt.p + kCntSw, nullptr, false, &at,
+                                 S.kcnt.p + filter_words(S), &sweep)))
         return rc;
     S.sw.nij = W.nij;
     S.sw.npt = W.npt;
@@ -726,10 +780,11 @@ int step_end_scenes(hipStream_t s, Sim& S, const uint8_t* active) {
     U.skin = skin_of(S);
     U.margin = range_margin(S);
     U.flag = S.cnt.p + kCntRange;
+    U.on = S.body_on.p;
     return body_end(s, &S.sc, U);
 }
 
-// The swept set's TOI, q.g and g.g, and both line-search passes with their decisions, then
+// The swept set's TOI (from its filter's slots and queue), q.g and g.g, and both line-search passes with their decisions, then
 // the counts' read-back (launched; the caller waits).
 int ccd_and_search_scenes(hipStream_t s, Sim& S, const LsDev& L) {
     const AbdSimState& st = S.st;
@@ -737,9 +792,6 @@ int ccd_and_search_scenes(hipStream_t s, Sim& S, const LsDev& L) {
     const int ns = S.ns;
     const CandSet& W = S.sw;
     int rc;
-    if ((rc = reduce_plan(s, &S.sc, &P, ns, W.ptl.p, W.npt, W.eel.p, W.nee, W.vgl.p, W.nvg, S.plan.p, W.counts(),
-                          S.cnt.p + kCntNewton, kCntSolver - kCntNewton + 1)))
-        return rc;
     // the TOI of the scenes still iterating and from it the first trial's step lengths; in the
     // same final pass q.g and g.g of the Armijo and stopping tests (abd.py:148,265: g and dq
     // are final here)
@@ -752,8 +804,8 @@ int ccd_and_search_scenes(hipStream_t s, Sim& S, const LsDev& L) {
     qg.d = st.g;
     qg.out1 = S.sv.p + kSvQtg * ns;
     qg.out2 = S.sv.p + kSvGtg * ns;
-    if ((rc = scene_toi(s, &S.sc, &P, ns, st.x, st.xk, W.ptl.p, W.npt, W.eel.p, W.nee, W.vgl.p, W.nvg, S.plan.p,
-                        S.sv.p + kSvToi * ns, L.newton, W.counts(), S.cand_alpha.p, W.side(), &qg)))
+    if ((rc = sweep_toi(s, &S.sc, &P, ns, st.x, st.xk, W.ptl.p, W.npt, W.eel.p, W.nee, W.counts(), W.side(),
+                        sweep_of(S), S.plan.p, S.sv.p + kSvToi * ns, S.cand_alpha.p, qg)))
         return rc;
     // the line search: the first trial, then every remaining halving of the scenes that
     // rejected it, each decided on the device
@@ -778,7 +830,7 @@ int iteration_scenes(hipStream_t s, Sim& S) {
     // rows committed, x and its body boxes, the inertia terms, the off-diagonal slots zeroed
     const int64_t nij = S.col_fresh ? S.col.nij : S.sw.nij;
     if ((rc = S.blocks.reserve((nb + 2 * (size_t)nij) * 144))) return rc;
-    BodyStart U;
+    BodyStart U{};
     U.alpha = L.dalpha;
     U.A = st.A;
     U.p = st.p;
@@ -797,6 +849,15 @@ int iteration_scenes(hipStream_t s, Sim& S) {
     U.blocks = S.blocks.p;
     U.zero = S.blocks.p + 144 * (int64_t)nb;
     U.nzero = 2 * 144 * nij;
+    if (S.sup_valid) {  // (else the superset's culling sets them)
+        if ((rc = sweep_buffers(S))) return rc;
+        U.zero32 = S.kcnt.p;
+        U.nzero32 = sweep_words(S);
+        U.slots = S.toi_slots;
+        U.qcount = S.toi_qcount;
+    }
+    U.counters = S.cnt.p + kCntNewton;
+    U.ncounters = kCntSolver - kCntNewton + 1;
     U.ns = ns;
     U.newton = S.lsflag.p + (size_t)kLfNewton * ns;
     U.E0 = S.lsval.p + (size_t)kLvE0 * ns;
@@ -1009,6 +1070,7 @@ int abd_sim_create(const AbdScene* scene, const AbdParams* params, const AbdSimS
     if (!rc) rc = S->qref.reserve(24 * nb);
     if (!rc) rc = S->rest_max.reserve(3 * nb);
     if (!rc) rc = S->rest_ref.reserve(3 * (size_t)S->nv + 3);
+    if (!rc) rc = S->body_on.reserve(nb);
     for (CandSet* C : {&S->col, &S->sw, &S->sup}) {
         if (!rc) rc = C->ij.reserve(2 * 256);
         if (!rc) rc = C->ji.reserve(2 * 256);
@@ -1233,6 +1295,8 @@ int abd_sim_destroy(void* sim) {
     S->vlo.release();
     S->vhi.release();
     S->qref.release();
+    S->kcnt.release();
+    S->body_on.release();
     S->rest_max.release();
     S->rest_ref.release();
     S->row_ptr.release();

@@ -1,5 +1,7 @@
 """Kernels at the sizes where their work splits can go wrong (one item, remainders, one more
 than a full grid), against the oracle."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -116,3 +118,67 @@ def test_body_passes_by_mesh_size(mesh):
         body = np.repeat(np.arange(3), np.diff(sp.voff))
         x = np.einsum("vr,vrk->vk", sp.x0, A[body]) + q[body]
         assert np.abs(sim.meshes.x_view.cpu().numpy() - x).max() <= 1e-13
+
+
+@pytest.mark.parametrize("sizes", [(1, 1, 1, 1), (256, 257, 255, 0), (2049, 16385, 16384, 513),
+                                   (65536, 2048, 1, 2047), (65793, 40003, 30001, 3001)])
+@pytest.mark.parametrize("with_ji", [True, False])
+def test_keep_filter_block_edges(sizes, with_ji):
+    """The superset filter (abd_cull_keep) at the edges of its blocks (256 entries), of its
+    super-blocks (64 blocks) and of the pair blocks it sums in LDS (65536 pairs): the kept
+    entries in their order with the kept pairs' indices, exactly."""
+    from abd_hip import _lib, scenes
+    from abd_hip.abd import AffineBodySimulator
+    from abd_hip.const_params import ContactParams
+    nij, npt, nee, nvg = sizes
+    rng = np.random.default_rng(nij)
+    nb = 400
+    spec = scenes.build_scene([scenes.cube_mesh()] * nb, np.stack([np.eye(3)] * nb), np.zeros((nb, 3)),
+                              np.zeros((nb, 3, 3)), np.zeros((nb, 3)), ground=0.0)
+    m = AffineBodySimulator(spec, ContactParams(ground=0.0), native=False).meshes
+
+    def boxes(n):
+        lo = rng.uniform(-1, 1, (n, 3)).astype(np.float32)
+        return lo, lo + rng.uniform(0, 2, (n, 3)).astype(np.float32)
+
+    def hit(a, i, b, j):
+        return ((a[0][i] <= b[1][j]) & (a[1][i] >= b[0][j])).all(1)
+
+    body, pnt, edg, tri = boxes(nb), boxes(8 * nb), boxes(18 * nb), boxes(12 * nb)
+    I, J = np.triu_indices(nb, 1)
+    sel = np.sort(rng.choice(len(I), nij, replace=False))
+    ij = np.stack([I[sel], J[sel]], 1).astype(np.int32)
+    ji = ij[:, ::-1].copy()
+    keep_ij = hit(body, ij[:, 0], body, ij[:, 1])
+    new = np.cumsum(keep_ij) - 1
+
+    def tuples(n, na, nbm, first, A, B):
+        q = np.sort(rng.integers(0, nij, n))
+        t = np.stack([ij[q, 0], ij[q, 1], q, rng.integers(0, na, n), rng.integers(0, nbm, n)], 1).astype(np.int32)
+        k = keep_ij[q] & hit(A, na * t[:, 0] + t[:, 3], B, nbm * t[:, 1] + t[:, 4])
+        out = t[k].copy()
+        out[:, 2] = new[out[:, 2]]
+        return t, out
+
+    pt, pt_ref = tuples(npt, 8, 12, 0, pnt, tri)
+    ee, ee_ref = tuples(nee, 18, 18, 0, edg, edg)
+    vg = np.stack([np.sort(rng.integers(0, nb, nvg)), rng.integers(0, 8, nvg)], 1).astype(np.int32)
+    dhat, ground = 0.01, 0.1
+    v = 8 * vg[:, 0] + vg[:, 1]
+    q = (np.float32([-1e3, -1e3, -1e3]), np.array([1e3, ground, 1e3], np.float32))
+    keep_vg = (body[0][vg[:, 0], 1].astype(np.float64) < 0.5 * dhat + ground) & (
+        (pnt[0][v] <= q[1]) & (pnt[1][v] >= q[0])).all(1)
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    ins = [d(x) for x in (ij, ji, pt, ee, vg)]
+    bx = [d(x) for b in (body, pnt, edg, tri) for x in b]
+    outs = [torch.full_like(x, -7) for x in ins]
+    P = _lib.ptr
+    cnt = (ctypes.c_int64 * 5)()
+    _lib.call("abd_cull_keep", _lib.stream_handle(), m.c, P(ins[0]), P(ins[1]) if with_ji else None, nij, P(ins[2]),
+              npt, P(ins[3]), nee, P(ins[4]), nvg, *[P(b) for b in bx], dhat, ground, P(outs[0]),
+              P(outs[1]) if with_ji else None, P(outs[2]), P(outs[3]), P(outs[4]), cnt)
+    refs = [ij[keep_ij], ji[keep_ij] if with_ji else ji[:0], pt_ref, ee_ref, vg[keep_vg]]
+    assert list(cnt) == [len(r) for r in refs]
+    for o, r in zip(outs, refs):
+        o = o.cpu().numpy()
+        assert np.array_equal(o[:len(r)], r) and (o[len(r):] == -7).all()
