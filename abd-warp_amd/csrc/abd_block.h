@@ -69,59 +69,72 @@ __device__ __forceinline__ float block_maxf(float v, float* sh) {
     return r;
 }
 
-// Sum over the workgroup with two barriers: a fixed shuffle tree inside each
-// wave (lane 0 ends with the wave's sum), wave sums through LDS, then the first
-// wave reduces those in the same fixed order.  Every thread receives the value
-// computed by one lane, so all waves branch alike on it.  blockDim.x must be a
-// multiple of 64 and at most 1024; sh must hold 17 doubles.
-__device__ __forceinline__ double wave_sum_down(double v) {
-#pragma unroll
-    for (int off = kWave / 2; off > 0; off >>= 1) v += __shfl_down(v, off, kWave);
+// Sums across lanes by the vector unit's own lane moves (DPP, and the half and row swaps),
+// about 25 cycles a level where a shuffle through the LDS unit takes over 100.  The pairing
+// is that of a shfl_down tree (lanes 32 apart first), every lane ending with lane 0's value.
+// All lanes must be active.
+template <int CTRL>
+__device__ __forceinline__ double dpp_move(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppRor4 = 0x124, kDppRor8 = 0x128;
+// v summed over each row of 16 lanes (8 apart first; a rotation by 4 is lane ^ 4 once lanes
+// 8 apart hold the same value)
+__device__ __forceinline__ double row_sum(double v) {
+    v += dpp_move<kDppRor8>(v);
+    v += dpp_move<kDppRor4>(v);
+    v += dpp_move<kDppXor2>(v);
+    v += dpp_move<kDppXor1>(v);
     return v;
 }
-__device__ __forceinline__ double block_sum_fast(double v, double* sh) {
-    const int lane = lane_id(), w = wave_id(), nw = n_waves();
-    v = wave_sum_down(v);
-    if (lane == 0) sh[w] = v;
-    __syncthreads();
-    if (w == 0) {
-        double t = lane < nw ? sh[lane] : 0.0;
-#pragma unroll
-        for (int off = 8; off > 0; off >>= 1) t += __shfl_down(t, off, kWave);
-        if (lane == 0) sh[16] = t;
+__device__ __forceinline__ double wave_sum(double v) {
+    {
+        const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(v), __double2loint(v), false, false);
+        const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(v), __double2hiint(v), false, false);
+        v = __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);  // lane i and i ^ 32
     }
+    {
+        const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(v), __double2loint(v), false, false);
+        const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(v), __double2hiint(v), false, false);
+        v = __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);  // i ^ 16
+    }
+    return row_sum(v);
+}
+// The waves' sums (sh: one per wave, at most 16, absent ones 0) in the pairing 8, 4, 2, 1
+// apart, by every wave.
+__device__ __forceinline__ double waves_sum(const double* sh, int nw) {
+    const int i = lane_id() & 15;
+    return row_sum(i < nw ? sh[i] : 0.0);
+}
+
+// Sum over the workgroup with two barriers: wave_sum inside each wave, the wave sums through
+// LDS, reduced in the same fixed order by every wave (alike, so all waves branch alike on
+// it).  blockDim.x must be a multiple of 64 and at most 1024; sh must hold 16 doubles.
+__device__ __forceinline__ double block_sum_fast(double v, double* sh) {
+    v = wave_sum(v);
+    if (lane_id() == 0) sh[wave_id()] = v;
     __syncthreads();
-    return sh[16];
+    const double r = waves_sum(sh, n_waves());
+    __syncthreads();
+    return r;
 }
 
 // Two independent sums with the reduction pattern of block_sum_fast (each result
 // bit-identical to a block_sum_fast of that value alone) and the same two
 // barriers.  sh must hold 34 doubles.
 __device__ __forceinline__ void block_sum2_fast(double& a, double& b, double* sh) {
-    const int lane = lane_id(), w = wave_id(), nw = n_waves();
-    a = wave_sum_down(a);
-    b = wave_sum_down(b);
-    if (lane == 0) {
-        sh[w] = a;
-        sh[17 + w] = b;
+    a = wave_sum(a);
+    b = wave_sum(b);
+    if (lane_id() == 0) {
+        sh[wave_id()] = a;
+        sh[17 + wave_id()] = b;
     }
     __syncthreads();
-    if (w == 0) {
-        double ta = lane < nw ? sh[lane] : 0.0;
-        double tb = lane < nw ? sh[17 + lane] : 0.0;
-#pragma unroll
-        for (int off = 8; off > 0; off >>= 1) {
-            ta += __shfl_down(ta, off, kWave);
-            tb += __shfl_down(tb, off, kWave);
-        }
-        if (lane == 0) {
-            sh[16] = ta;
-            sh[33] = tb;
-        }
-    }
+    a = waves_sum(sh, n_waves());
+    b = waves_sum(sh + 17, n_waves());
     __syncthreads();
-    a = sh[16];
-    b = sh[33];
 }
 
 // Exclusive prefix sum of one int64 per thread (sh: at least n_waves() entries): a

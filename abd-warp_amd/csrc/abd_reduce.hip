@@ -378,7 +378,7 @@ __global__ __launch_bounds__(kRedThreads, 4) void trial_chunk_kernel(AbdScene sc
                 }
             }
             if (whole || k + 1 < k1) {
-                const double v = wave_sum_down(acc);
+                const double v = wave_sum(acc);
                 if (lane == 0) wsum[k][w] = v;
                 acc = 0.0;
             }

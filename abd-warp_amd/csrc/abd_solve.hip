@@ -2,11 +2,10 @@
 // unpreconditioned BiCGSTAB (abd.py:244, warp.optim.linear.bicgstab) and the
 // Jacobi-preconditioned CG of bsr_utils.py:126-235.
 //
-// One workgroup runs the whole Krylov loop for one system: the vectors live in
-// the scratch arena (L2-resident for the scene sizes this path sees), every dot
-// product is a fixed-order LDS reduction, and the stopping test is evaluated
-// inside the kernel every `check_every` iterations, so a solve is one launch
-// with no host round trips.
+// One workgroup runs the whole Krylov loop for one system: matrix and vectors in registers
+// where they fit (RegSystem), else the vectors in LDS or the scratch arena; every dot product
+// is a fixed-order reduction, and the stopping test is evaluated inside the kernel every
+// `check_every` iterations, so a solve is one launch with no host round trips.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -225,6 +224,275 @@ __device__ __forceinline__ double vdot(const double* __restrict__ a, const doubl
     return block_sum_fast(acc, sh);
 }
 
+// The Krylov loops of a system whose rows fit one per thread (n <= T) and whose blocks fit
+// four threads each (entry-parallel mode): the matrix in registers for the whole solve, K
+// rows of one block a thread (K = 1, 2, 3: the least that fits), the vectors too, each thread
+// its row; only the multiplied vector and the block rows' partial products pass through LDS.
+// Every sum is the one of cg_body / bicgstab_body in entry-parallel mode (a thread there owns
+// the same row; absent waves add 0), so the bits are the same.  What bounds these solves is
+// the latency of an iteration's dependent steps: hence no matrix reads from L2, one barrier a
+// sum, lane moves in place of LDS shuffles, and waves without rows taking part in the
+// products only.  Against the memory loops: CG of 61 systems of 2 to 40 bodies 294 -> 116 us,
+// CG of 16 uncoupled bodies 33.5 -> 14.8 us, BiCGSTAB of 2 bodies 98 -> 22 us (of which one wave
+// in place of 16 about a quarter).
+constexpr int kRegRows = 3;
+template <int K, int T>
+struct RegSystem {
+    static constexpr int kPer = 12 / K;  // threads a block
+    double B[K][12];
+    int xo;      // first entry of the column in the multiplied vector (-1: none)
+    int e0, e1;  // the entries of this thread's row
+    bool rows;   // this wave has rows
+    int nw;      // waves with rows
+    double* part;
+    double* sums;  // LDS: [2][2][16], the halves in turn
+    int turn;
+    double one[2];  // the sums of a single wave
+
+    __device__ __forceinline__ RegSystem(const Bsr& M, const Rows& R, int n, double* lds_sums)
+        : xo(-1), e0(0), e1(0), nw((n + kWave - 1) / kWave), part(R.part), sums(lds_sums), turn(0) {
+        const int t = threadIdx.x, e = t / kPer, r0 = K * (t % kPer);
+        rows = T == kWave || __builtin_amdgcn_readfirstlane(wave_id()) < nw;
+#pragma unroll
+        for (int k = 0; k < K; ++k)
+#pragma unroll
+            for (int q = 0; q < 12; ++q) B[k][q] = 0.0;
+        if (e < R.lrp[R.nbs]) {
+            const int2 en = R.ent[e];
+            if (en.x >= 0) {
+                xo = 12 * en.x;
+#pragma unroll
+                for (int k = 0; k < K; ++k) load_block_row(M.blocks, en.y, (r0 + k) / 3, (r0 + k) % 3, B[k]);
+            } else {
+                for (int k = 0; k < K; ++k) part[12 * e + r0 + k] = 0.0;  // outside the system: adds nothing
+            }
+        }
+        if (t < n) {
+            e0 = R.lrp[t / 12];
+            e1 = R.lrp[t / 12 + 1];
+        }
+    }
+    // the block rows' products with `in` (LDS); then a barrier and row()
+    __device__ __forceinline__ void products(const double* __restrict__ in) const {
+        if (xo < 0) return;
+        double y[K];
+#pragma unroll
+        for (int k = 0; k < K; ++k) y[k] = 0.0;
+#pragma unroll
+        for (int q = 0; q < 12; q += 3) {  // block_row_add of every row, the column's entries read once
+            const double x0 = in[xo + q], x1 = in[xo + q + 1], x2 = in[xo + q + 2];
+#pragma unroll
+            for (int k = 0; k < K; ++k) y[k] += B[k][q] * x0 + B[k][q + 1] * x1 + B[k][q + 2] * x2;
+        }
+#pragma unroll
+        for (int k = 0; k < K; ++k) part[K * threadIdx.x + k] = y[k];
+    }
+    // this thread's row of the product: its blocks' in column order, four loads in flight
+    __device__ __forceinline__ double row() const {
+        double acc = 0.0;
+        const double* pr = part + threadIdx.x % 12;
+        for (int e = e0; e < e1; e += 4) {
+            double v[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] = e + j < e1 ? pr[12 * (e + j)] : 0.0;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc += v[j];
+        }
+        return acc;
+    }
+    // block_sum_fast's value in three parts: put (waves with rows), a barrier, get; the
+    // buffers alternate, so the next put needs no barrier of its own
+    __device__ __forceinline__ void put(double v, int which = 0) {
+        v = wave_sum(v);
+        if (T == kWave)
+            one[which] = v + 0.0;
+        else if (lane_id() == 0)
+            sums[32 * turn + 16 * which + wave_id()] = v;
+    }
+    __device__ __forceinline__ double get(int which = 0) const {
+        return T == kWave ? one[which] : waves_sum(sums + 32 * turn + 16 * which, nw);
+    }
+    __device__ __forceinline__ void next() { turn ^= 1; }
+};
+
+template <int K, int T>
+__device__ __forceinline__ void bicgstab_regs(const Bsr& M, const Rows& R, int n, const double* __restrict__ b,
+                                              double* __restrict__ xg, double tol, int maxiter, int check_every,
+                                              double* V, int32_t* __restrict__ iters, double* __restrict__ resid,
+                                              double* sums) {
+    double *pl = V, *rl = V + n;
+    const int i = threadIdx.x;
+    const bool own = i < n;
+    double x = own ? xg[i] : 0.0;
+    const double bi = own ? b[i] : 0.0;
+    if (own) pl[i] = x;
+    RegSystem<K, T> H(M, R, n, sums);
+    const bool rows = H.rows;
+    __syncthreads();
+    H.products(pl);
+    __syncthreads();
+    double r = 0.0;
+    if (rows) {
+        r = bi - H.row();
+        H.put(own ? 0.0 + r * r : 0.0);
+        H.put(own ? 0.0 + bi * bi : 0.0, 1);
+    }
+    __syncthreads();
+    double rr = H.get();
+    const double atol = tol * sqrt(H.get(1));
+    H.next();
+    const double atol_sq = atol * atol;
+    int it = 0;
+    if (rr > atol_sq) {
+        const double r0 = r;
+        double p = r, rho = rr, v = 0.0, t = 0.0, alpha = 0.0, omega = 0.0;
+        if (own) pl[i] = p;
+        __syncthreads();
+        for (;;) {
+            for (int c = 1; c <= check_every; ++c) {
+                H.products(pl);
+                __syncthreads();
+                if (rows) {
+                    v = H.row();
+                    H.put(own ? 0.0 + r0 * v : 0.0);
+                }
+                __syncthreads();
+                if (rows) {
+                    const double r0v = H.get();
+                    alpha = r0v != 0.0 ? rho / r0v : 0.0;
+                    x += alpha * p;
+                    r -= alpha * v;
+                    if (own) rl[i] = r;
+                }
+                H.next();
+                __syncthreads();
+                H.products(rl);
+                __syncthreads();
+                if (rows) {
+                    t = H.row();
+                    H.put(own ? 0.0 + t * r : 0.0);
+                    H.put(own ? 0.0 + t * t : 0.0, 1);
+                }
+                __syncthreads();
+                if (rows) {
+                    const double tr = H.get(), tt = H.get(1);
+                    H.next();
+                    omega = tt != 0.0 ? tr / tt : 0.0;
+                    x += omega * r;
+                    r -= omega * t;
+                    H.put(own ? 0.0 + r * r : 0.0);
+                    H.put(own ? 0.0 + r0 * r : 0.0, 1);
+                } else {
+                    H.next();
+                }
+                __syncthreads();
+                if (rows || c == check_every) rr = H.get();
+                if (rows) {
+                    const double rho_old = rho;
+                    rho = H.get(1);
+                    const double beta = (rho_old != 0.0 && omega != 0.0) ? (rho / rho_old) * (alpha / omega) : 0.0;
+                    p = r + beta * (p - omega * v);
+                    if (own) pl[i] = p;
+                }
+                H.next();
+                __syncthreads();
+            }
+            it += check_every;
+            if (rr <= atol_sq || it >= maxiter) break;
+        }
+    }
+    if (own) xg[i] = x;
+    if (i == 0) {
+        if (iters) *iters = it;
+        if (resid) *resid = rr;
+    }
+}
+
+template <int K, int T>
+__device__ __forceinline__ void cg_regs(const Bsr& M, const Rows& R, int n, const double* __restrict__ b,
+                                        double* __restrict__ xg, double tol, int maxiter, int check_every, double* V,
+                                        int32_t* __restrict__ iters, double* __restrict__ resid, double* sums) {
+    double* pl = V;
+    const int i = threadIdx.x;
+    const bool own = i < n;
+    double x = 0.0, bi = 0.0, da = 0.0;
+    bool plain = true;  // a zero diagonal sub-block, or no row: z = r
+    if (own) {
+        const double* D = M.blocks + 9 * (16 * (int64_t)(R.row0 + i / 12) + 5 * (i % 12 / 3));
+        const double d0 = D[0], d1 = D[4], d2 = D[8];
+        plain = d0 * d0 + d1 * d1 + d2 * d2 == 0.0;
+        da = fabs(i % 3 == 0 ? d0 : i % 3 == 1 ? d1 : d2);
+        x = xg[i];
+        bi = b[i];
+        pl[i] = x;
+    }
+    RegSystem<K, T> H(M, R, n, sums);
+    const bool rows = H.rows;
+    __syncthreads();
+    H.products(pl);
+    __syncthreads();
+    double r = 0.0, z = 0.0, p = 0.0;
+    if (rows) {
+        r = bi - H.row();
+        z = plain ? r : r / da;
+        p = z;
+        H.put(own ? 0.0 + r * z : 0.0);
+        if (own) pl[i] = p;
+    }
+    __syncthreads();
+    double rz_old = H.get(), rz_new = 0.0;
+    H.next();
+    const double tol_sq = tol * tol * (double)n;
+    double err = rz_old;
+    int end_iter = 0;
+    if (err > tol_sq) {
+        end_iter = maxiter;
+        for (int c = 0; c < maxiter; ++c) {
+            const bool check = ((c + 1) % check_every) == 0;
+            double Ap = 0.0;
+            H.products(pl);
+            __syncthreads();
+            if (rows) {
+                Ap = H.row();
+                H.put(own ? 0.0 + p * Ap : 0.0);
+            }
+            __syncthreads();
+            if (rows) {
+                const double pAp = H.get();
+                H.next();
+                const double alpha = pAp != 0.0 ? rz_old / pAp : 0.0;
+                x += alpha * p;
+                r -= alpha * Ap;
+                z = plain ? r : r / da;
+                H.put(own ? 0.0 + r * z : 0.0);
+            } else {
+                H.next();
+            }
+            __syncthreads();
+            if (rows || check) rz_new = H.get();
+            H.next();
+            if (check && rz_new <= tol_sq) {  // uniform: the same sum in every wave
+                end_iter = c;
+                err = rz_new;
+                break;
+            }
+            if (rows) {
+                const double beta = rz_new > tol_sq ? rz_new / rz_old : 0.0;
+                p = z + beta * p;
+                if (own) pl[i] = p;
+            }
+            __syncthreads();
+            rz_old = rz_new;
+            err = rz_old;
+        }
+    }
+    if (own) xg[i] = x;
+    if (i == 0) {
+        if (iters) *iters = end_iter;
+        if (resid) *resid = err;
+    }
+}
+
 // Dynamic LDS of a solve workgroup: the staged structure (lrp, then ent), the six Krylov
 // vectors of the system's n rows when LDS (else in the scratch arena), then the partial
 // products of the entry-parallel SpMV.
@@ -320,9 +588,16 @@ __device__ __forceinline__ void bicgstab_body(const Bsr& M, const Rows& R, int n
     }
 }
 
-// budget: bytes of dynamic LDS (SolveLds; -1: the device holds no staged structure).
-template <bool LDS>
-__global__ __launch_bounds__(kSolveThreads) void bicgstab_kernel(Bsr M, const int32_t* __restrict__ sboff,
+// Whether a system takes the register-resident loops of T threads (12 / kRegRows a block).
+template <int T>
+__device__ __forceinline__ bool regs_fit(const Rows& R, int n) {
+    return n <= T && 4 * R.lrp[R.nbs] <= T;
+}
+
+// budget: bytes of dynamic LDS (SolveLds; -1: the device holds no staged structure).  T: the
+// workgroup's threads (solve_threads).
+template <bool LDS, int T>
+__global__ __launch_bounds__(T) void bicgstab_kernel(Bsr M, const int32_t* __restrict__ sboff,
                                                                   const uint8_t* __restrict__ active,
                                                                   const double* __restrict__ b,
                                                                   double* __restrict__ xg, double tol, int maxiter,
@@ -331,7 +606,7 @@ __global__ __launch_bounds__(kSolveThreads) void bicgstab_kernel(Bsr M, const in
                                                                   int32_t* __restrict__ iters,
                                                                   double* __restrict__ resid) {
     __shared__ double sh[17];
-    __shared__ double sh2[34];
+    __shared__ double sh2[64];
     // one system per workgroup: the bodies of scene blockIdx.x (all bodies without scenes)
     const int sidx = blockIdx.x;
     if (active && !active[sidx]) return;
@@ -349,7 +624,16 @@ __global__ __launch_bounds__(kSolveThreads) void bicgstab_kernel(Bsr M, const in
     if (maxiter <= 0) maxiter = n;  // the system size of this workgroup's system
     Rows R{row0, n / 12, nullptr, nullptr, S.part};
     const int mode = stage_rows(M, R, S.lrp, S.ent, budget);
-    if (mode == kSpmvEntries)
+    if (mode == kSpmvEntries && regs_fit<T>(R, n)) {
+        double* Vr = LDS ? S.V : S.part + 12 * R.lrp[R.nbs];  // two of entries_fit's six vectors
+        const int nnz = R.lrp[R.nbs];
+        if (12 * nnz <= T)
+            bicgstab_regs<1, T>(M, R, n, b, xg, tol, maxiter, check_every, Vr, iters, resid, sh2);
+        else if (6 * nnz <= T)
+            bicgstab_regs<2, T>(M, R, n, b, xg, tol, maxiter, check_every, Vr, iters, resid, sh2);
+        else
+            bicgstab_regs<kRegRows, T>(M, R, n, b, xg, tol, maxiter, check_every, Vr, iters, resid, sh2);
+    } else if (mode == kSpmvEntries)
         bicgstab_body<kSpmvEntries>(M, R, n, b, xg, tol, maxiter, check_every, S.V, iters, resid, sh, sh2);
     else if (mode == kSpmvRowsStaged)
         bicgstab_body<kSpmvRowsStaged>(M, R, n, b, xg, tol, maxiter, check_every, S.V, iters, resid, sh, sh2);
@@ -540,8 +824,8 @@ __device__ __forceinline__ void cg_body(const Bsr& M, const Rows& R, int n, cons
 
 // BJ: the per-body 12x12 block-Jacobi preconditioner (beyond the reference) in place of
 // the diagonal one; dinv: [nb][144] workspace of the inverses.  budget as bicgstab_kernel.
-template <bool LDS, bool BJ>
-__global__ __launch_bounds__(kSolveThreads) void cg_kernel(Bsr M, const int32_t* __restrict__ sboff,
+template <bool LDS, bool BJ, int T>
+__global__ __launch_bounds__(T) void cg_kernel(Bsr M, const int32_t* __restrict__ sboff,
                                                            const uint8_t* __restrict__ active,
                                                            const double* __restrict__ b, double* __restrict__ xg,
                                                            double tol, int maxiter, int check_every, int cap_rows,
@@ -549,7 +833,7 @@ __global__ __launch_bounds__(kSolveThreads) void cg_kernel(Bsr M, const int32_t*
                                                            double* __restrict__ dinv, int32_t* __restrict__ iters,
                                                            double* __restrict__ resid,
                                                            const int32_t* __restrict__ pending) {
-    __shared__ double sh[17];
+    __shared__ double sh[BJ ? 17 : 64];
     // one system per workgroup: the bodies of scene blockIdx.x (all bodies without scenes);
     // pending (nullable): only the systems the direct solve declined
     const int sidx = blockIdx.x;
@@ -569,6 +853,18 @@ __global__ __launch_bounds__(kSolveThreads) void cg_kernel(Bsr M, const int32_t*
     if (maxiter <= 0) maxiter = n;  // the system size of this workgroup's system
     Rows R{row0, n / 12, nullptr, nullptr, S.part};
     const int mode = stage_rows(M, R, S.lrp, S.ent, budget);
+    if constexpr (!BJ)
+        if (mode == kSpmvEntries && regs_fit<T>(R, n)) {
+            double* Vr = LDS ? S.V : S.part + 12 * R.lrp[R.nbs];  // one of entries_fit's six vectors
+            const int nnz = R.lrp[R.nbs];
+            if (12 * nnz <= T)
+                cg_regs<1, T>(M, R, n, b, xg, tol, maxiter, check_every, Vr, iters, resid, sh);
+            else if (6 * nnz <= T)
+                cg_regs<2, T>(M, R, n, b, xg, tol, maxiter, check_every, Vr, iters, resid, sh);
+            else
+                cg_regs<kRegRows, T>(M, R, n, b, xg, tol, maxiter, check_every, Vr, iters, resid, sh);
+            return;
+        }
     if (mode == kSpmvEntries)
         cg_body<BJ, kSpmvEntries>(M, R, n, b, xg, tol, maxiter, check_every, S.V, dinv, iters, resid, sh);
     else if (mode == kSpmvRowsStaged)
@@ -1246,10 +1542,16 @@ using namespace abd;
 extern "C" {
 
 namespace {
-// Workgroup size of a solve.  It must not depend on the other systems of a launch,
-// so that a scene solved on its own or inside a batch reduces in the same order;
-// 16 waves per system keep enough loads in flight for the block SpMV.
-int solve_threads(int) { return kSolveThreads; }
+// Workgroup size of a solve of systems of up to max_bodies bodies: the smallest whose
+// threads hold every row and a matrix with all its max_bodies^2 blocks (regs_fit); else 16 waves, which keep enough loads in flight where a matrix stays in
+// memory.  A system's sums are the same for every size (each thread owns at most the rows
+// it has in the largest; absent waves add 0), so a scene gives the same bits on its own or
+// in a batch.
+int solve_threads(int max_bodies) {
+    for (int t : {kWave, 4 * kWave})
+        if (12 * (int64_t)max_bodies <= t && 4 * (int64_t)max_bodies * max_bodies <= t) return t;
+    return kSolveThreads;
+}
 
 int launch_solve(hipStream_t s, int32_t method, const Bsr& M, int nsys, const int32_t* sboff, const uint8_t* active,
                  int max_rows, const double* b, double* x, double tol, int32_t maxiter, int32_t check_every,
@@ -1291,34 +1593,41 @@ int launch_solve(hipStream_t s, int32_t method, const Bsr& M, int nsys, const in
     std::unique_lock<std::mutex> attr_lock(attr_mu);
     if (!attr_set) {
         const int cap = (int)usable;
-        const void* fns[] = {(const void*)bicgstab_kernel<true>,     (const void*)bicgstab_kernel<false>,
-                             (const void*)cg_kernel<true, false>,    (const void*)cg_kernel<true, true>,
-                             (const void*)cg_kernel<false, false>,   (const void*)cg_kernel<false, true>};
+        const void* fns[] = {(const void*)bicgstab_kernel<true, kWave>,
+                             (const void*)bicgstab_kernel<true, 4 * kWave>,
+                             (const void*)bicgstab_kernel<true, kSolveThreads>,
+                             (const void*)bicgstab_kernel<false, kSolveThreads>,
+                             (const void*)cg_kernel<true, false, kWave>,
+                             (const void*)cg_kernel<true, false, 4 * kWave>,
+                             (const void*)cg_kernel<true, false, kSolveThreads>,
+                             (const void*)cg_kernel<true, true, kSolveThreads>,
+                             (const void*)cg_kernel<false, false, kSolveThreads>,
+                             (const void*)cg_kernel<false, true, kSolveThreads>};
         for (const void* f : fns) ABD_CHECK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, cap));
         attr_set = true;
     }
     attr_lock.unlock();
-    if (lds) {
-        if (method == ABD_SOLVER_BICGSTAB)
-            hipLaunchKernelGGL(bicgstab_kernel<true>, dim3(nsys), dim3(threads), dyn, s, M, sboff, active, b, x, tol,
-                               maxiter, check_every, max_rows, budget, ws, iters, resid);
-        else if (bj)
-            hipLaunchKernelGGL((cg_kernel<true, true>), dim3(nsys), dim3(threads), dyn, s, M, sboff, active, b, x,
-                               tol, maxiter, check_every, max_rows, budget, ws, dinv, iters, resid, pending);
-        else
-            hipLaunchKernelGGL((cg_kernel<true, false>), dim3(nsys), dim3(threads), dyn, s, M, sboff, active, b, x,
-                               tol, maxiter, check_every, max_rows, budget, ws, dinv, iters, resid, pending);
-    } else {
-        if (method == ABD_SOLVER_BICGSTAB)
-            hipLaunchKernelGGL(bicgstab_kernel<false>, dim3(nsys), dim3(threads), dyn, s, M, sboff, active, b, x,
-                               tol, maxiter, check_every, max_rows, budget, ws, iters, resid);
-        else if (bj)
-            hipLaunchKernelGGL((cg_kernel<false, true>), dim3(nsys), dim3(threads), dyn, s, M, sboff, active, b, x,
-                               tol, maxiter, check_every, max_rows, budget, ws, dinv, iters, resid, pending);
-        else
-            hipLaunchKernelGGL((cg_kernel<false, false>), dim3(nsys), dim3(threads), dyn, s, M, sboff, active, b, x,
-                               tol, maxiter, check_every, max_rows, budget, ws, dinv, iters, resid, pending);
+    if (bj || !lds) threads = kSolveThreads;
+    auto bicgstab = bicgstab_kernel<false, kSolveThreads>;
+    auto cg = cg_kernel<false, false, kSolveThreads>;
+    if (lds && threads == kWave) {
+        bicgstab = bicgstab_kernel<true, kWave>;
+        cg = cg_kernel<true, false, kWave>;
+    } else if (lds && threads == 4 * kWave) {
+        bicgstab = bicgstab_kernel<true, 4 * kWave>;
+        cg = cg_kernel<true, false, 4 * kWave>;
+    } else if (lds) {
+        bicgstab = bicgstab_kernel<true, kSolveThreads>;
+        cg = bj ? cg_kernel<true, true, kSolveThreads> : cg_kernel<true, false, kSolveThreads>;
+    } else if (bj) {
+        cg = cg_kernel<false, true, kSolveThreads>;
     }
+    if (method == ABD_SOLVER_BICGSTAB)
+        hipLaunchKernelGGL(bicgstab, dim3(nsys), dim3(threads), dyn, s, M, sboff, active, b, x, tol, maxiter,
+                           check_every, max_rows, budget, ws, iters, resid);
+    else
+        hipLaunchKernelGGL(cg, dim3(nsys), dim3(threads), dyn, s, M, sboff, active, b, x, tol, maxiter, check_every,
+                           max_rows, budget, ws, dinv, iters, resid, pending);
     ABD_CHECK_LAUNCH();
     prof_stop(ph, s);
     if (ph >= 0 && iters) {

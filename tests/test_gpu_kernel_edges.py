@@ -182,3 +182,81 @@ def test_keep_filter_block_edges(sizes, with_ji):
     for o, r in zip(outs, refs):
         o = o.cpu().numpy()
         assert np.array_equal(o[:len(r)], r) and (o[len(r):] == -7).all()
+
+
+@pytest.mark.parametrize("method", [0, 1])
+def test_krylov_in_registers_edges(method):
+    """BiCGSTAB and Jacobi CG where the workgroup's size and the rows kept in registers change
+    (n = 12 bodies <= 64, 256, 1024 threads; 12, 6 or 4 threads a block): a batch of the sizes
+    gives each system the bits of its solve alone, and the dense solution.  The residual is
+    below 1e-10 of b and the matrices' condition below 2: 1e-9."""
+    import abd_hip
+    from abd_hip import _lib
+    from abd_hip.sparse import BsrMatrix, SolveInfo, bicgstab, bsr_cg
+    abd_hip.load()
+    rng = np.random.default_rng(5)
+    sizes = [(1, 0), (4, 6), (5, 3), (8, 28), (9, 0), (21, 32), (22, 32), (42, 64), (43, 64), (64, 96), (65, 96),
+             (85, 20), (86, 20)]
+    boff = np.concatenate([[0], np.cumsum([m for m, _ in sizes])]).astype(np.int32)
+    nb = int(boff[-1])
+    pairs = []
+    for (m, k), r0 in zip(sizes, boff):
+        a, b = np.triu_indices(m, 1)
+        sel = rng.choice(len(a), k, replace=False) if k else []
+        pairs += [(int(a[q] + r0), int(b[q] + r0)) for q in sel]
+    ij = np.array(sorted(pairs), np.int32)
+    nij = len(ij)
+    blocks = np.zeros(((nb + 2 * nij), 16, 3, 3))
+    dense = np.zeros((12 * nb, 12 * nb))
+
+    def put(slot, i, j, M):
+        blocks[slot] = M.reshape(4, 3, 4, 3).transpose(2, 0, 1, 3).reshape(16, 3, 3)
+        dense[12 * i:12 * i + 12, 12 * j:12 * j + 12] = M
+
+    for k, (i, j) in enumerate(ij):
+        M = 0.3 * rng.normal(size=(12, 12))
+        put(nb + k, i, j, M)
+        put(nb + nij + k, j, i, M.T)
+    for i in range(nb):
+        Q = rng.normal(size=(12, 12))
+        put(i, i, i, Q @ Q.T + 600.0 * np.eye(12))
+    rhs, x0 = rng.normal(size=(12 * nb)), 0.01 * rng.normal(size=(12 * nb))
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+    def structure(n, p):
+        q = p[np.lexsort((p[:, 0], p[:, 1]))]
+        out = [torch.empty(s, dtype=torch.int32, device="cuda") for s in (n + 1, n + 2 * len(p), n + 2 * len(p))]
+        tp, tq = d(p.astype(np.int32)), d(q.astype(np.int32))
+        _lib.call("abd_bsr_structure", _lib.stream_handle(), n, _lib.ptr(tp), _lib.ptr(tq), len(p),
+                  *[_lib.ptr(o) for o in out])
+        torch.cuda.synchronize()
+        return out
+
+    rp, cl, sl = structure(nb, ij)
+    tboff, tbs = d(boff), d(np.repeat(np.arange(len(sizes)), [m for m, _ in sizes]).astype(np.int32))
+    sc = _lib.AbdScene()
+    sc.n_bodies, sc.n_scenes = nb, len(sizes)
+    sc.scene_boff, sc.body_scene = tboff.data_ptr(), tbs.data_ptr()
+    tb, tr, x = d(blocks), d(rhs), d(x0)
+    active = torch.ones(len(sizes), dtype=torch.uint8, device="cuda")
+    iters = torch.zeros(len(sizes), dtype=torch.int32, device="cuda")
+    resid = torch.zeros(len(sizes), dtype=torch.float64, device="cuda")
+    tol = 1e-11 if method == 0 else 1e-12
+    _lib.call("abd_bsr_solve_scenes", _lib.stream_handle(), method, ctypes.byref(sc), 86, _lib.ptr(rp), _lib.ptr(cl),
+              _lib.ptr(sl), _lib.ptr(tb), _lib.ptr(tr), _lib.ptr(x), tol, 500, 10, _lib.ptr(active),
+              _lib.ptr(iters), _lib.ptr(resid))
+    xb = x.cpu().numpy()
+    assert rel_err(xb, np.linalg.solve(dense, rhs)) <= 1e-9
+    for s, (m, k) in enumerate(sizes):
+        r0, r1 = boff[s], boff[s + 1]
+        q = np.nonzero((ij[:, 0] >= r0) & (ij[:, 0] < r1))[0]
+        slots = np.concatenate([np.arange(r0, r1), nb + q, nb + nij + q])
+        A = BsrMatrix(m, *structure(m, ij[q] - r0), d(blocks[slots].reshape(-1, 3, 3)))
+        xs, info = d(x0[12 * r0:12 * r1].reshape(-1, 3)), SolveInfo("cuda")
+        bs = d(rhs[12 * r0:12 * r1].reshape(-1, 3))
+        if method == 0:
+            bicgstab(A, bs, xs, tol, 500, 10, info)
+        else:
+            bsr_cg(A, xs, bs, 500, tol, 10, info)
+        assert np.array_equal(xs.cpu().numpy().ravel(), xb[12 * r0:12 * r1]), (m, k)
+        assert int(info.iters[0]) == int(iters[s]) and float(info.resid[0]) == float(resid[s])
