@@ -10,6 +10,7 @@
 
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 
 #include "abd_block.h"
 #include "abd_internal.h"
@@ -881,12 +882,14 @@ __global__ __launch_bounds__(T) void cg_kernel(Bsr M, const int32_t* __restrict_
 // of that order's elimination tree (parent of k: the first body above k coupled to it;
 // level: 0 for a leaf, else one more than the highest child's) -- bodies of one level are
 // never coupled to each other and are eliminated together, level after level, in chunks
-// of at most kLdltCols augmented columns.  The factor's upper blocks live in the system's
+// of at most kLdltCols columns of [A' | I].  The factor's upper blocks live in the system's
 // workspace region (row i's blocks from pos[i], in column order), the chunk's W blocks
 // after them.  Elimination of body k: Gauss-Jordan elimination without row exchanges on
-// [P | A'_k,j1 .. A'_k,jd | I], P = A'_kk, one thread per column (12 doubles in
-// registers; the chunk's pivot columns broadcast through LDS, one barrier per pivot
-// column), leaving W_j = P^-1 A'_kj and P^-1 (which replaces P in the factor).  Each
+// [P | A'_k,j1 .. A'_k,jd | I], P = A'_kk, leaving W_j = P^-1 A'_kj and P^-1.  The pivot
+// columns depend on P alone: pivot_columns() finds them for all bodies of the chunk, 16 lanes
+// a body, and stores each as the columns take it; then every column of A' and I goes through
+// the 12 pivots in registers with no barrier between (64 bodies of one level: 26 k cycles, as
+// with one barrier per pivot pair; a level of one body: 5.3 k + 3.9 k instead of 10 k).  Each
 // Schur target A'_ij (and each forward-solve target y_i) is updated by its chunk's bodies
 // in ascending order, A'_ij -= A'_ki^T W_j, y_i -= W_i^T y_k (12-term sums), by the
 // thread of the lowest of them, so a system gives the same bits whatever else a launch
@@ -898,9 +901,13 @@ __global__ __launch_bounds__(T) void cg_kernel(Bsr M, const int32_t* __restrict_
 // and resid (nullable) = |b - H x|^2.  The factor and the W blocks live in the workgroup's dynamic
 // LDS (dyn_blocks 12x12 blocks) when they fit there -- the factor's upper blocks with fill
 // and at most min(kLdltWBlocks, off-diagonal blocks) W blocks -- else in the system's
-// workspace region; the arithmetic is the same in both places.
-constexpr int kLdltColsPerThread = 2;  // adjacent columns 2t, 2t + 1 of one body
-constexpr int kLdltCols = kLdltColsPerThread * kSolveThreads;
+// workspace region, with each chunk's pivot columns, A' and W blocks staged in the LDS where
+// those fit; the arithmetic is the same in all places.  Latency bounds it: a level's few
+// dependent phases, on one CU.  Against a barrier per pivot pair, one element of a Schur target
+// a thread and nothing staged: 64 bodies of two levels 41 -> 32 us, 256 scenes of 2 to 64 bodies
+// 60 -> 48 us, 64 bodies of 47 levels (11 blocks a row, in memory) 589 -> 413 us, about half of
+// that by the tiles and the staged blocks (12-17 k -> 4.5 k cycles a level).
+constexpr int kLdltCols = kSolveThreads;      // one column a thread
 constexpr int kLdltWBlocks = kLdltCols / 12;  // bound on a chunk's W blocks
 __host__ __device__ inline int64_t ldlt_region(int m) { return 144 * ((int64_t)m * (m + 1) / 2 + kLdltWBlocks); }
 
@@ -920,6 +927,40 @@ __device__ __forceinline__ unsigned long long bits_above(unsigned long long row,
 }
 __device__ __forceinline__ unsigned long long bits_below(int j) { return (1ull << j) - 1ull; }
 
+// v, recomputed where it is used: comparisons and indices derived from it are not kept in
+// registers from an earlier use.
+__device__ __forceinline__ int fresh(int v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
+// The pivot columns of a 12x12 block in 16 lanes (a DPP row), row l in p of lane l (lanes 12
+// to 15: zeros): for pivot C, out[12 C + q], q < 11, the entries of column C below and then
+// above row C (rows C + 1, .., 11, 0, .., C - 1) as pivot C meets them, and out[12 C + 11] the
+// reciprocal pivot.  Only the columns above C are still needed.  write: this block exists;
+// bad: a pivot was not positive.  Unrolled: as a loop that moves rows and columns up one
+// place a pivot it took twice as long (10 k cycles a level, 26 k with 64 bodies).
+template <int C, class Out>
+__device__ __forceinline__ void pivot_columns(double (&p)[12], Out out, bool write, bool& bad) {
+    const int l = fresh(threadIdx.x & 15);
+    const double piv = dpp_move<kDppRowBcast + C>(p[C]), f = p[C];
+    const double inv = 1.0 / piv;
+    bad |= !(piv > 0.0) || !isfinite(piv);
+    if (write && l < 12) out[12 * C + l - C + (l > C ? -1 : 11)] = l == C ? inv : f;
+    if constexpr (C < 11) {
+        double u[12];
+#pragma unroll
+        for (int j = C + 1; j < 12; ++j) u[j] = dpp_move<kDppRowBcast + C>(p[j]) * inv;
+        if (l != C) {
+#pragma unroll
+            for (int j = C + 1; j < 12; ++j) u[j] = p[j] - f * u[j];
+        }
+#pragma unroll
+        for (int j = C + 1; j < 12; ++j) p[j] = u[j];
+        pivot_columns<C + 1>(p, out, write, bad);
+    }
+}
+
 __global__ __launch_bounds__(kSolveThreads) void ldlt_kernel(Bsr M, const int32_t* __restrict__ sboff,
                                                              const uint8_t* __restrict__ active,
                                                              const double* __restrict__ b, double* __restrict__ xg,
@@ -927,24 +968,19 @@ __global__ __launch_bounds__(kSolveThreads) void ldlt_kernel(Bsr M, const int32_
                                                              int32_t* __restrict__ status, double* __restrict__ resid,
                                                              int dyn_blocks) {
     constexpr int MB = kLdltMaxBodies;
-    extern __shared__ double ldlt_dyn[];
+    extern __shared__ __align__(16) double ldlt_dyn[];
     __shared__ unsigned long long adj[MB];   // upper row pattern with fill (bits >= row)
     __shared__ unsigned long long colm[MB];  // colm[i]: the rows k < i whose pattern holds i
     __shared__ unsigned long long levm[MB];  // the bodies of each level
     __shared__ int lvl[MB];                  // the level of each body
     __shared__ unsigned char mlist[MB][MB];  // mlist[k]: the columns above k in row k, ascending
     __shared__ int lrp[MB + 1], pos[MB + 1];
-    // the system's CSR entries (slot, local column: 0xff outside the system; at most m^2), read
-    // only while the factor is filled, share their LDS with the elimination's pivot columns
-    // (two per step, double-buffered) and reciprocal pivots
-    constexpr int kEntryBytes = MB * MB * 5, kPivotBytes = MB * 2 * 2 * 13 * 8;
-    __shared__ __align__(16) unsigned char tables[kEntryBytes > kPivotBytes ? kEntryBytes : kPivotBytes];
-    int* eslot = reinterpret_cast<int*>(tables);
-    unsigned char* ecol = tables + 4 * MB * MB;
-    double(*colc)[2][2][12] = reinterpret_cast<double(*)[2][2][12]>(tables);
-    double(*colinv)[2][2] = reinterpret_cast<double(*)[2][2]>(tables + MB * 2 * 2 * 12 * 8);
+    // the system's CSR entries (at most m^2): slot, and row << 8 | local column, then the
+    // factor's block (0xffff: lower, or outside the system)
+    __shared__ int eslot[MB * MB];
+    __shared__ uint16_t eblk[MB * MB];
     __shared__ int cnode[MB], cstart[MB + 1], sstart[MB + 1], woff[MB];  // the chunk
-    __shared__ int nlev, fail, nchunk;
+    __shared__ int nlev, fail, nchunk, nstage;
     __shared__ unsigned long long chunkmask, restm;  // the chunk; the level's bodies not yet eliminated
     __shared__ double y[12 * MB];  // b, then the forward solve, then x
     __shared__ double z[12 * MB];
@@ -983,10 +1019,20 @@ __global__ __launch_bounds__(kSolveThreads) void ldlt_kernel(Bsr M, const int32_
         const int j = M.cols[e0 + e] - row0;
         const int i = last_le(lrp, m, e);
         eslot[e] = M.slots[e0 + e];
-        ecol[e] = (unsigned)j < (unsigned)m ? (unsigned char)j : 0xff;
+        eblk[e] = j >= i && j < m ? (uint16_t)(i << 8 | j) : (uint16_t)0xffff;
         if (j > i && j < m) atomicOr(&adj[i], 1ull << j);
     }
     __syncthreads();
+    // a thread copies element q of blocks e0, e0 + 7, ...; the first kAhead of them are in
+    // flight while the structure is found
+    constexpr int kAhead = 8, kAtOnce = kSolveThreads / 144;
+    const int q0 = t % 144, e0t = t < 144 * kAtOnce ? t / 144 : MB * MB;
+    double ahead[kAhead];
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+        const int e = e0t + u * kAtOnce;
+        ahead[u] = M.blocks[e < nnz ? 144 * (int64_t)eslot[e] + q0 : 0];
+    }
     if (t < 64) {  // wave 0, lane = row: fill, transposed pattern and tree levels, row by row
         unsigned long long mine = t < m ? adj[t] : 0ull, cm = 0ull;
         int h = 0;
@@ -1041,52 +1087,77 @@ __global__ __launch_bounds__(kSolveThreads) void ldlt_kernel(Bsr M, const int32_
     const bool in_lds = fail == 2;  // uniform
     __syncthreads();
     if (t == 0) fail = 0;
+    for (int e = t; e < nnz; e += nt)
+        if (eblk[e] != 0xffff) {
+            const int i = eblk[e] >> 8, j = eblk[e] & 0xff;
+            eblk[e] = (uint16_t)(pos[i] + __popcll(adj[i] & bits_below(j)));
+        }
     // The factorization and both solves, instantiated for a factor in LDS (its accesses then
     // LDS instructions) and for one in the global workspace; false: a pivot was not positive.
-    auto factor_solve = [&](auto U, auto W) __attribute__((always_inline)) -> bool {
+    typedef __attribute__((address_space(3))) double lds_double;
+    auto factor_solve = [&](auto U, auto W, auto lds_c) __attribute__((always_inline)) -> bool {
         for (int64_t e = t; e < 144 * (int64_t)pos[m]; e += nt) U[e] = 0.0;
         __syncthreads();
-        // the matrix's upper blocks into the factor (row-major 12x12): one wave per block, its
-        // lanes reading the slot's 144 doubles in storage order (16 3x3 sub-blocks, sub-block
-        // (R/3, C/3) at 9 (R/3 + 4 C/3), row-major inside)
+        // the matrix's upper blocks into the factor (row-major 12x12), the lanes reading the
+        // slots' 144 doubles in storage order (16 3x3 sub-blocks, sub-block (R/3, C/3) at
+        // 9 (R/3 + 4 C/3), row-major inside)
         {
-            const int lane = t & (kWave - 1), wv = t / kWave, nwv = nt / kWave;
-            for (int e = wv; e < nnz; e += nwv) {  // uniform over the wave
-                const int j = ecol[e];
-                const int i = last_le(lrp, m, e);
-                if (j < i || j >= m) continue;  // lower, or outside the system (0xff)
-                const double* src = M.blocks + 144 * (int64_t)eslot[e];
-                auto dst = U + 144 * (int64_t)(pos[i] + __popcll(adj[i] & bits_below(j)));
-                for (int q = lane; q < 144; q += kWave) {
-                    const int sb = q / 9, w9 = q % 9;
-                    dst[12 * (3 * (sb % 4) + w9 / 3) + 3 * (sb / 4) + w9 % 3] = src[q];
+            const int sb = q0 / 9, w9 = q0 % 9;
+            auto dst = U + (12 * (3 * (sb & 3) + w9 / 3) + 3 * (sb >> 2) + w9 % 3);
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u) {
+                const int e = e0t + u * kAtOnce;
+                if (e < nnz && eblk[e] != 0xffff) dst[144 * (int)eblk[e]] = ahead[u];
+            }
+            for (int e1 = e0t + kAhead * kAtOnce; e1 < nnz; e1 += 4 * kAtOnce) {
+                double v[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const int e = e1 + u * kAtOnce;
+                    v[u] = M.blocks[e < nnz ? 144 * (int64_t)eslot[e] + q0 : 0];
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const int e = e1 + u * kAtOnce;
+                    if (e < nnz && eblk[e] != 0xffff) dst[144 * (int)eblk[e]] = v[u];
                 }
             }
         }
         const int levels = nlev;
         for (int L = 0; L < levels; ++L) {
             if (t == 0) restm = levm[L];
-            for (;;) {
+            bool more;
+            do {
                 __syncthreads();  // the previous chunk is written back, its tables are free
                 if (t < kWave) {
                     // wave 0, lane = body: the chunk is the lowest bodies of the level not yet
-                    // eliminated whose augmented columns fit kLdltCols (prefix sums in body order;
-                    // a single body always fits)
+                    // eliminated whose columns fit kLdltCols and, for a factor in memory, whose
+                    // pivot, A' and W blocks fit the LDS (prefix sums in body order; a single
+                    // body's columns always fit, one whose blocks do not is a chunk unstaged)
                     const unsigned long long rest = restm;
                     const bool member = t < m && ((rest >> t) & 1ull);
                     const int d = member ? __popcll(bits_above(adj[t], t)) : 0;
-                    const int c0 = member ? 12 * (d + 2) : 0, s0 = member ? 144 * (d * (d + 1) / 2) : 0, w0 = d;
-                    int ic = c0, is = s0, iw = w0;
+                    // columns (16 bits), Schur tiles (24), W blocks (12), bodies
+                    const unsigned long long one =
+                        member ? (unsigned long long)(12 * (d + 1)) | (unsigned long long)(8 * d * (d + 1)) << 16 |
+                                     (unsigned long long)d << 40 | 1ull << 52
+                               : 0ull;
+                    unsigned long long incl = one;
                     for (int off = 1; off < kWave; off <<= 1) {
-                        const int vc = __shfl_up(ic, off, kWave), vs = __shfl_up(is, off, kWave),
-                                  vw = __shfl_up(iw, off, kWave);
-                        if (t >= off) {
-                            ic += vc;
-                            is += vs;
-                            iw += vw;
-                        }
+                        const unsigned long long v = __shfl_up(incl, off, kWave);
+                        if (t >= off) incl += v;
                     }
-                    const bool take = member && ic <= kLdltCols;
+                    const unsigned long long excl = incl - one;
+                    const int ic = (int)(incl & 0xffff), is = (int)(incl >> 16 & 0xffffff), iw = (int)(incl >> 40 & 0xfff);
+                    const int c0 = (int)(one & 0xffff), s0 = (int)(one >> 16 & 0xffffff), w0 = d;
+                    const int need = (int)(incl >> 52) + 2 * iw;
+                    bool take = member && ic <= kLdltCols;
+                    if (!in_lds) {
+                        const bool first = member && excl == 0;
+                        const bool alone = __ballot(first && need > dyn_blocks) != 0;  // unstaged
+                        take = take && (alone ? first : need <= dyn_blocks);
+                        if (t == 0) nstage = alone ? 0 : 1;
+                    }
                     const unsigned long long cmask = __ballot(take);
                     const int nc = __popcll(cmask);
                     if (take) {
@@ -1101,7 +1172,6 @@ __global__ __launch_bounds__(kSolveThreads) void ldlt_kernel(Bsr M, const int32_
                         }
                     }
                     if (t == 0) {
-                        if (nc == 0) cstart[0] = sstart[0] = 0;
                         nchunk = nc;
                         chunkmask = cmask;
                         restm = rest & ~cmask;
@@ -1109,158 +1179,170 @@ __global__ __launch_bounds__(kSolveThreads) void ldlt_kernel(Bsr M, const int32_
                 }
                 __syncthreads();
                 const int nc = nchunk;
-                if (nc == 0) break;  // uniform: the level is done
+                more = restm != 0ull;  // read here: written again only after the chunk's barriers
                 const unsigned long long cmask = chunkmask;
                 const int C = cstart[nc];
-                double a[kLdltColsPerThread][12];
-                int cln[kLdltColsPerThread], cg[kLdltColsPerThread], cc_[kLdltColsPerThread], cd[kLdltColsPerThread];
-    #pragma unroll
-                for (int s = 0; s < kLdltColsPerThread; ++s) {
-                    const int col = kLdltColsPerThread * t + s;
-                    cln[s] = -1;
-                    cg[s] = cc_[s] = cd[s] = 0;
-                    if (col < C) {
-                        const int ln = last_le(cstart, nc, col);
-                        const int k = cnode[ln], within = col - cstart[ln];
-                        const int g = within / 12, c = within % 12, d = (cstart[ln + 1] - cstart[ln]) / 12 - 2;
-                        cln[s] = ln;
-                        cg[s] = g;
-                        cc_[s] = c;
-                        cd[s] = d;
-                        if (g <= d) {
-                            const auto src = U + 144 * (int64_t)(pos[k] + g) + c;
-    #pragma unroll
-                            for (int r = 0; r < 12; ++r) a[s][r] = src[12 * r];
-                        } else {
-    #pragma unroll
-                            for (int r = 0; r < 12; ++r) a[s][r] = r == c ? 1.0 : 0.0;
-                        }
+                // F: the bodies' pivot columns, then P^-1 (over P, or block ln of the stage);
+                // Ab: their A' blocks from aoff; Wb: their W blocks from woff
+                auto eliminate = [&](auto Fb, auto Wb, auto Ab, auto staged_c) __attribute__((always_inline)) -> bool {
+                    constexpr bool staged = decltype(staged_c)::value;
+                    auto foff = [&](int ln, int k) { return 144 * (int64_t)(staged ? ln : pos[k]); };
+                    auto aoff = [&](int k) { return 144 * (int64_t)(staged ? woff[k] : pos[k] + 1); };
+                    if (4 * (t / kWave) < nc) {  // uniform over the wave: its four bodies' pivots
+                        const int q = t >> 4, kq = cnode[q < nc ? q : 0], l = t & 15;
+                        double p[12];
+                        const auto src = U + 144 * (int64_t)pos[kq] + 12 * l;
+#pragma unroll
+                        for (int j = 0; j < 12; ++j) p[j] = q < nc && l < 12 ? src[j] : 0.0;
+                        bool bad = false;
+                        pivot_columns<0>(p, Fb + foff(q, kq), q < nc, bad);
+                        if (bad && q < nc) fail = 1;
                     }
-                }
-                // two pivot columns per barrier.  A thread's columns are adjacent and a body's
-                // column count is a multiple of 12, so both belong to one body and the pivot pair
-                // (cp, cp + 1) of a body is one thread's: it publishes column cp as it stands and
-                // column cp + 1 as pivot cp leaves it (the update every column gets), with both
-                // reciprocal pivots; every column then takes pivot cp, then pivot cp + 1 -- the
-                // arithmetic of one pivot per step
-    #pragma unroll
-                for (int cp = 0; cp < 12; cp += 2) {
-                    const int bf = (cp >> 1) & 1;
-                    if (cln[0] >= 0 && cg[0] == 0 && cc_[0] == cp) {
-                        const double inv0 = 1.0 / a[0][cp];
-                        if (!(a[0][cp] > 0.0) || !isfinite(a[0][cp])) fail = 1;
-                        const double sc1 = a[1][cp] * inv0;
-                        double piv1 = 0.0;
-    #pragma unroll
-                        for (int r = 0; r < 12; ++r) {
-                            const double v = r == cp ? sc1 : a[1][r] - a[0][r] * sc1;
-                            colc[cln[0]][bf][0][r] = a[0][r];
-                            colc[cln[0]][bf][1][r] = v;
-                            if (r == cp + 1) piv1 = v;
+                    double a[12];
+                    const int col = t;
+                    int ln = -1, k = 0, g = 0, c = 0, d = 0;
+                    if (col < C) {
+                        ln = last_le(cstart, nc, col);
+                        k = cnode[ln];
+                        const int within = col - cstart[ln];
+                        g = within / 12;
+                        c = within % 12;
+                        d = (cstart[ln + 1] - cstart[ln]) / 12 - 1;
+                        if (g < d) {
+                            const auto src = U + 144 * (int64_t)(pos[k] + 1 + g) + c;
+#pragma unroll
+                            for (int r = 0; r < 12; ++r) a[r] = src[12 * r];
+                            if (staged) {
+                                auto dst = Ab + aoff(k) + 144 * g + c;
+#pragma unroll
+                                for (int r = 0; r < 12; ++r) dst[12 * r] = a[r];
+                            }
+                        } else {
+#pragma unroll
+                            for (int r = 0; r < 12; ++r) a[r] = r == c ? 1.0 : 0.0;
                         }
-                        if (!(piv1 > 0.0) || !isfinite(piv1)) fail = 1;
-                        colinv[cln[0]][bf][0] = inv0;
-                        colinv[cln[0]][bf][1] = 1.0 / piv1;
                     }
                     __syncthreads();
-                    if (cln[0] >= 0) {
-    #pragma unroll
-                        for (int h = 0; h < 2; ++h) {  // pivot cp + h
-                            const int pc = cp + h;
-                            double f[12];
-    #pragma unroll
-                            for (int r = 0; r < 12; ++r) f[r] = colc[cln[0]][bf][h][r];
-                            const double inv = colinv[cln[0]][bf][h];
-    #pragma unroll
-                            for (int s = 0; s < kLdltColsPerThread; ++s)
-                                if (cln[s] >= 0) {
-                                    const double sc = a[s][pc] * inv;
-    #pragma unroll
-                                    for (int r = 0; r < 12; ++r)
-                                        if (r != pc) a[s][r] -= f[r] * sc;
-                                    a[s][pc] = sc;
-                                }
+                    if (fail) {  // uniform
+                        if (t == 0) status[sidx] = kLdltFailed;
+                        return false;
+                    }
+                    if (ln >= 0) {
+                        // each pivot's entry is first in turn: the others move up one place
+                        auto F = Fb + foff(ln, k);
+                        double f[12];
+#pragma unroll
+                        for (int r = 0; r < 12; ++r) f[r] = F[r];
+#pragma unroll 1
+                        for (int pc = 0; pc < 12; ++pc) {
+                            double next[12];  // the next pivot's column, in flight meanwhile
+                            if (pc < 11) F += 12;
+#pragma unroll
+                            for (int r = 0; r < 12; ++r) next[r] = F[r];
+                            const double sc = a[0] * f[11];
+#pragma unroll
+                            for (int r = 0; r < 11; ++r) a[r] = a[r + 1] - f[r] * sc;
+                            a[11] = sc;
+#pragma unroll
+                            for (int r = 0; r < 12; ++r) f[r] = next[r];
+                        }
+                        if (g < d) {
+                            auto dst = Wb + 144 * (int64_t)(woff[k] + g) + c;
+#pragma unroll
+                            for (int r = 0; r < 12; ++r) dst[12 * r] = a[r];
                         }
                     }
-                }
-                if (fail) {  // uniform: written before the last pivot column's barrier
-                    if (t == 0) status[sidx] = kLdltFailed;
-                    return false;
-                }
-                // W (g = 1..d) to the chunk's area, P^-1 (g = d + 1) over P
-    #pragma unroll
-                for (int s = 0; s < kLdltColsPerThread; ++s)
-                    if (cln[s] >= 0 && cg[s] >= 1) {
-                        const int k = cnode[cln[s]];
-                        auto dst = cg[s] <= cd[s] ? W + 144 * (int64_t)(woff[k] + cg[s] - 1) + cc_[s]
-                                                     : U + 144 * (int64_t)pos[k] + cc_[s];
-    #pragma unroll
-                        for (int r = 0; r < 12; ++r) dst[12 * r] = a[s][r];
+                    __syncthreads();
+                    if (ln >= 0 && g == d) {  // P^-1 over the pivot columns, all read
+                        auto dst = Fb + foff(ln, k) + c;
+#pragma unroll
+                        for (int r = 0; r < 12; ++r) dst[12 * r] = a[r];
                     }
-                __syncthreads();
-                // Schur complement: target (i, j), i <= j, updated by the thread of its lowest
-                // contributor in the chunk, the contributors in ascending order
-                for (int w = t; w < sstart[nc]; w += nt) {
-                    const int ln = last_le(sstart, nc, w);
-                    const int k = cnode[ln], within = w - sstart[ln];
-                    const int pidx = within / 144, q = within % 144;
-                    int v = (int)((sqrt(8.0 * pidx + 1.0) - 1.0) * 0.5);
-                    while (v * (v + 1) / 2 > pidx) --v;
-                    while ((v + 1) * (v + 2) / 2 <= pidx) ++v;
-                    const int u = pidx - v * (v + 1) / 2;
-                    const int i = mlist[k][u], j = mlist[k][v];
-                    const unsigned long long contrib = cmask & colm[i] & colm[j];
-                    if (__builtin_ctzll(contrib) != k) continue;
-                    auto tgt = U + 144 * (int64_t)(pos[i] + __popcll(adj[i] & bits_below(j))) + q;
-                    double val = *tgt;
-                    for (unsigned long long bt = contrib; bt; bt &= bt - 1ull) {
-                        const int k2 = __builtin_ctzll(bt);
-                        const unsigned long long ab = bits_above(adj[k2], k2);
-                        const auto Aki = U + 144 * (int64_t)(pos[k2] + 1 + __popcll(ab & bits_below(i))) + q / 12;
-                        const auto Wj = W + 144 * (int64_t)(woff[k2] + __popcll(ab & bits_below(j))) + q % 12;
+                    // Schur complement: 3x3 tiles of target (i, j), i <= j, updated by the thread of
+                    // its lowest contributor in the chunk, the contributors in ascending order
+                    for (int w = t; w < sstart[nc]; w += nt) {
+                        const int l2 = last_le(sstart, nc, w);
+                        const int k1 = cnode[l2], within = w - sstart[l2];
+                        const int pidx = within >> 4, ta = 3 * (within >> 2 & 3), tb = 3 * (within & 3);
+                        int v = (int)((__builtin_sqrtf(8.0f * pidx + 1.0f) - 1.0f) * 0.5f);
+                        while (v * (v + 1) / 2 > pidx) --v;
+                        while ((v + 1) * (v + 2) / 2 <= pidx) ++v;
+                        const int i = mlist[k1][pidx - v * (v + 1) / 2], j = mlist[k1][v];
+                        const unsigned long long contrib = cmask & colm[i] & colm[j];
+                        if (__builtin_ctzll(contrib) != k1) continue;
+                        auto tgt = U + 144 * (int64_t)(pos[i] + __popcll(adj[i] & bits_below(j))) + 12 * ta + tb;
+                        double val[9];
+#pragma unroll
+                        for (int q = 0; q < 9; ++q) val[q] = tgt[12 * (q / 3) + q % 3];
+                        for (unsigned long long bt = contrib; bt; bt &= bt - 1ull) {
+                            const int k2 = __builtin_ctzll(bt);
+                            const unsigned long long ab = bits_above(adj[k2], k2);
+                            const auto Aki = Ab + aoff(k2) + 144 * __popcll(ab & bits_below(i)) + ta;
+                            const auto Wj = Wb + 144 * (int64_t)(woff[k2] + __popcll(ab & bits_below(j))) + tb;
+                            double acc[9];
+#pragma unroll
+                            for (int q = 0; q < 9; ++q) acc[q] = 0.0;
+#pragma unroll 4
+                            for (int r = 0; r < 12; ++r) {
+                                const double x[3] = {Aki[12 * r], Aki[12 * r + 1], Aki[12 * r + 2]};
+                                const double y3[3] = {Wj[12 * r], Wj[12 * r + 1], Wj[12 * r + 2]};
+#pragma unroll
+                                for (int q = 0; q < 9; ++q) acc[q] += x[q / 3] * y3[q % 3];
+                            }
+#pragma unroll
+                            for (int q = 0; q < 9; ++q) val[q] -= acc[q];
+                        }
+#pragma unroll
+                        for (int q = 0; q < 9; ++q) tgt[12 * (q / 3) + q % 3] = val[q];
+                    }
+                    // forward solve: y_i -= W_i^T y_k over the chunk's bodies k coupled to i, ascending
+                    for (int w = t; w < n; w += nt) {
+                        const int i = w / 12, a2 = w % 12;
+                        unsigned long long bt = cmask & colm[i];
+                        if (!bt) continue;
+                        double val = y[w];
+                        for (; bt; bt &= bt - 1ull) {
+                            const int k2 = __builtin_ctzll(bt);
+                            const unsigned long long ab = bits_above(adj[k2], k2);
+                            const auto Wi = Wb + 144 * (int64_t)(woff[k2] + __popcll(ab & bits_below(i))) + a2;
+                            double acc = 0.0;
+#pragma unroll
+                            for (int r = 0; r < 12; ++r) acc += Wi[12 * r] * y[12 * k2 + r];
+                            val -= acc;
+                        }
+                        y[w] = val;
+                    }
+                    __syncthreads();
+                    // z_k = P^-1 y_k for the chunk's bodies
+                    for (int w = t; w < 12 * nc; w += nt) {
+                        const int kz = cnode[w / 12], a2 = w % 12;
+                        const auto Di = Fb + foff(w / 12, kz) + 12 * a2;
                         double acc = 0.0;
-    #pragma unroll
-                        for (int r = 0; r < 12; ++r) acc += Aki[12 * r] * Wj[12 * r];
-                        val -= acc;
+#pragma unroll
+                        for (int r = 0; r < 12; ++r) acc += Di[r] * y[12 * kz + r];
+                        z[12 * kz + a2] = acc;
                     }
-                    *tgt = val;
-                }
-                // forward solve: y_i -= W_i^T y_k over the chunk's bodies k coupled to i, ascending
-                for (int w = t; w < n; w += nt) {
-                    const int i = w / 12, a2 = w % 12;
-                    unsigned long long bt = cmask & colm[i];
-                    if (!bt) continue;
-                    double val = y[w];
-                    for (; bt; bt &= bt - 1ull) {
-                        const int k2 = __builtin_ctzll(bt);
-                        const unsigned long long ab = bits_above(adj[k2], k2);
-                        const auto Wi = W + 144 * (int64_t)(woff[k2] + __popcll(ab & bits_below(i))) + a2;
-                        double acc = 0.0;
-    #pragma unroll
-                        for (int r = 0; r < 12; ++r) acc += Wi[12 * r] * y[12 * k2 + r];
-                        val -= acc;
+                    // rows of the factor: W (read back: kept in registers over the tiles it spills)
+                    if (ln >= 0 && g < d) {
+                        auto dst = U + 144 * (int64_t)(pos[k] + 1 + g) + c;
+                        const auto src = Wb + 144 * (int64_t)(woff[k] + g) + c;
+#pragma unroll
+                        for (int r = 0; r < 12; ++r) dst[12 * r] = src[12 * r];
                     }
-                    y[w] = val;
+                    return true;
+                };
+                bool ok;
+                if constexpr (decltype(lds_c)::value) {
+                    ok = eliminate(U, W, U, std::false_type{});
+                } else if (nstage) {  // uniform
+                    lds_double* St = (lds_double*)ldlt_dyn;
+                    const int nw = (C / 12 - nc);
+                    ok = eliminate(St, St + 144 * nc, St + 144 * (nc + nw), std::true_type{});
+                } else {
+                    ok = eliminate(U, W, U, std::false_type{});
                 }
-                // z_k = P^-1 y_k for the chunk's bodies
-                for (int w = t; w < 12 * nc; w += nt) {
-                    const int k = cnode[w / 12], a2 = w % 12;
-                    const auto Di = U + 144 * (int64_t)pos[k] + 12 * a2;
-                    double acc = 0.0;
-    #pragma unroll
-                    for (int r = 0; r < 12; ++r) acc += Di[r] * y[12 * k + r];
-                    z[12 * k + a2] = acc;
-                }
-                __syncthreads();
-                // rows of the factor: W
-    #pragma unroll
-                for (int s = 0; s < kLdltColsPerThread; ++s)
-                    if (cln[s] >= 0 && cg[s] >= 1 && cg[s] <= cd[s]) {
-                        auto dst = U + 144 * (int64_t)(pos[cnode[cln[s]]] + cg[s]) + cc_[s];
-    #pragma unroll
-                        for (int r = 0; r < 12; ++r) dst[12 * r] = a[s][r];
-                    }
-            }
+                if (!ok) return false;
+            } while (more);  // uniform; every level has a body
         }
         // backward solve, levels from the top
         for (int L = levels - 1; L >= 0; --L) {
@@ -1285,11 +1367,10 @@ __global__ __launch_bounds__(kSolveThreads) void ldlt_kernel(Bsr M, const int32_
     };
     bool ok;
     if (in_lds) {
-        typedef __attribute__((address_space(3))) double lds_double;
         lds_double* Ul = (lds_double*)ldlt_dyn;
-        ok = factor_solve(Ul, Ul + 144 * (int64_t)pos[m]);
+        ok = factor_solve(Ul, Ul + 144 * (int64_t)pos[m], std::true_type{});
     } else {
-        ok = factor_solve(U, W);
+        ok = factor_solve(U, W, std::false_type{});
     }
     if (!ok) return;
     __syncthreads();

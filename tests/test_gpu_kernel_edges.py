@@ -260,3 +260,38 @@ def test_krylov_in_registers_edges(method):
             bsr_cg(A, xs, bs, 500, tol, 10, info)
         assert np.array_equal(xs.cpu().numpy().ravel(), xb[12 * r0:12 * r1]), (m, k)
         assert int(info.iters[0]) == int(iters[s]) and float(info.resid[0]) == float(resid[s])
+
+
+def _ldlt_pairs(kind, m):
+    if kind == "dense":
+        return [(i, j) for i in range(m) for j in range(i + 1, m)]
+    if kind == "star":  # the last body coupled to all: the others are one level
+        return [(i, m - 1) for i in range(m - 1)]
+    if kind == "pairs":
+        return [(2 * i, 2 * i + 1) for i in range(m // 2)]
+    return [(i, i + w) for i in range(m) for w in (1, 9, 10) if i + w < m]  # "band"
+
+
+@pytest.mark.parametrize("kind,m", [("dense", 3), ("dense", 13), ("dense", 14), ("dense", 15), ("dense", 51),
+                                    ("dense", 52), ("dense", 64), ("star", 43), ("star", 44), ("star", 64),
+                                    ("pairs", 63), ("band", 64)])
+def test_ldlt_chunk_edges(kind, m):
+    """The direct solve where its storage changes (the factor in LDS, in memory with staged
+    chunks, in memory unstaged) and where a level takes several chunks (1024 columns): against
+    the oracle's same sums, 1e-14 (the bound of the batched comparison)."""
+    import abd_hip
+    from abd_hip.sparse import BsrMatrix, SolveInfo, bsr_ldlt
+    from test_gpu_ldlt import _structure, _system
+    lib = abd_hip.load()
+    rng = np.random.default_rng(m)
+    ij = np.array(sorted(_ldlt_pairs(kind, m)), np.int32).reshape(-1, 2)
+    blocks, dense = _system(m, ij, rng)
+    b = rng.normal(size=(4 * m, 3))
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    A = BsrMatrix(m, *_structure(lib, m, ij), d(blocks))
+    x, info = d(np.zeros((4 * m, 3))), SolveInfo("cuda")
+    bsr_ldlt(A, x, d(b), info=info)
+    ref, st = O.bsr_ldlt(m, ij, blocks, b, np.zeros((4 * m, 3)))
+    assert st == 1 and int(info.iters[0]) == 1
+    assert rel_err(x.cpu().numpy(), ref) <= 1e-14
+    assert rel_err(x.cpu().numpy().ravel(), np.linalg.solve(dense, b.ravel())) <= 1e-10
