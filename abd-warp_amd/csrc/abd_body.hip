@@ -66,6 +66,7 @@ __global__ __launch_bounds__(T) void body_start_kernel(AbdScene sc, AbdParams P,
     if (b >= nb) {
         const int64_t i0 = (int64_t)(b - nb) * T + t, step = (int64_t)(gridDim.x - nb) * T;
         for (int64_t i = i0; i < U.nzero; i += step) U.zero[i] = 0;
+        for (int64_t i = i0; i < U.nzero2; i += step) U.zero2[i] = 0;
         for (int64_t i = i0; i < U.nzero32; i += step) U.zero32[i] = 0;
         for (int64_t s = i0; s < U.ns; s += step) {
             U.newton[s] = U.newton[U.ns + s];
@@ -236,7 +237,8 @@ int body_start(hipStream_t s, const AbdScene* sc, const AbdParams* P, const Body
     const bool small = small_bodies(sc);
     const int T = small ? kWave : kBlock;
     // workgroups for the rows and the fill: about 16 words a thread
-    const int64_t extra = std::min<int64_t>(4096, 1 + ceil_div(std::max<int64_t>(U.nzero + U.nzero32 / 2, U.ns), 16 * (int64_t)T));
+    const int64_t words = U.nzero + U.nzero2 + U.nzero32 / 2;
+    const int64_t extra = std::min<int64_t>(4096, 1 + ceil_div(std::max<int64_t>(words, U.ns), 16 * (int64_t)T));
     const dim3 grid((unsigned)(sc->n_bodies + extra));
     if (small)
         hipLaunchKernelGGL(body_start_kernel<kWave>, grid, dim3(T), 0, s, *sc, *P, U);

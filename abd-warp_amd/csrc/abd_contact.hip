@@ -32,7 +32,8 @@
 
 namespace abd {
 
-constexpr int kCItems = 8;          // candidates per thread in the compaction passes
+constexpr int kSuperBlocks = 64;   // blocks (kBlock candidates) per super-block of active counts
+constexpr int kSuperStride = 8;    // words between those: adds to one cache line wait for each other
 constexpr int kGhBoundMib = 8192;  // stored contacts sized by a list bound, at most (default)
 constexpr int kContactStride = 128;  // doubles per stored contact: c[0..4], b', pad, then V[5][24]
 constexpr int kCoefOff = 0;
@@ -149,7 +150,8 @@ __device__ bool contact_terms(int kind, const d3 v[4], const d3 r[4], double d2h
     return true;
 }
 
-// stage A: active flags over [PT | EE], plus ordering checks.
+// stage A: active flags over [PT | EE] and their counts per block of kBlock candidates (bcnt)
+// and per super-block (scnt, 0 before), plus ordering checks.
 // dn (nullable): the list sizes on the device, [nij, nij, npt, nee, nvg] (the arguments are
 // then upper bounds that only size the launch)
 __global__ __launch_bounds__(kBlock) void classify_kernel(AbdScene sc, AbdParams P, const double* __restrict__ x,
@@ -158,20 +160,24 @@ __global__ __launch_bounds__(kBlock) void classify_kernel(AbdScene sc, AbdParams
                                                            const int32_t* __restrict__ vg, int64_t nvg,
                                                            const int64_t* __restrict__ dn,
                                                            uint8_t* __restrict__ flag, int* __restrict__ err,
-                                                           int64_t* __restrict__ bcnt) {
+                                                           uint32_t* __restrict__ bcnt,
+                                                           uint32_t* __restrict__ scnt) {
     const SceneView S = view_of(sc);
     if (dn) {
         npt = dn[2];
         nee = dn[3];
         nvg = dn[4];
     }
-    const int64_t n = npt + nee;
-    for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n + nvg; i += (int64_t)gridDim.x * kBlock) {
+    const int64_t n = npt + nee, nblk = (n + kBlock - 1) / kBlock, nvblk = (nvg + kBlock - 1) / kBlock;
+    for (int64_t blk = blockIdx.x; blk < nblk + nvblk; blk += gridDim.x) {  // uniform over the workgroup
+        if (blk >= nblk) {
+            const int64_t k = (blk - nblk) * kBlock + threadIdx.x;
+            if (k > 0 && k < nvg && vg[2 * k] < vg[2 * (k - 1)]) *err = 1;
+            continue;
+        }
         bool act = false;
-        if (i >= n) {
-            int64_t k = i - n;
-            if (k > 0 && vg[2 * k] < vg[2 * (k - 1)]) *err = 1;
-        } else {
+        const int64_t i = blk * kBlock + threadIdx.x;
+        if (i < n) {
         const bool is_ee = i >= npt;
         const int64_t k = is_ee ? i - npt : i;
         const int32_t* t5 = (is_ee ? ee : pt) + 5 * k;
@@ -196,37 +202,88 @@ __global__ __launch_bounds__(kBlock) void classify_kernel(AbdScene sc, AbdParams
         }
         flag[i] = act ? 1 : 0;
         }
-        if (bcnt) {
-            // stage B's count: the wave's active candidates (its 64 consecutive ones lie in one
-            // compaction block) added to the block's count; lane 0 holds the wave's first one
-            const uint64_t m = __ballot(act);
-            if (lane_id() == 0 && m != 0)
-                atomicAdd(reinterpret_cast<unsigned long long*>(bcnt + i / ((int64_t)kBlock * kCItems)),
-                          (unsigned long long)__popcll(m));
+        const int c = __syncthreads_count(act);
+        if (threadIdx.x == 0) {
+            bcnt[blk] = (uint32_t)c;
+            if (c) atomicAdd(scnt + kSuperStride * (blk / kSuperBlocks), (uint32_t)c);
         }
     }
 }
 
-// stage B: ordered compaction of the flags (count / write passes).
-template <bool WRITE>
-__global__ __launch_bounds__(kBlock) void compact_flags_kernel(const uint8_t* __restrict__ flag, int64_t n,
-                                                                const int64_t* __restrict__ dn,
-                                                                int64_t* __restrict__ bcnt,
-                                                                const int64_t* __restrict__ boff,
-                                                                int32_t* __restrict__ out) {
-    __shared__ int shw[kBlock / kWave];
-    if (dn) n = dn[2] + dn[3];
-    int64_t base = (int64_t)blockIdx.x * kBlock * kCItems;
-    int64_t run = WRITE ? boff[blockIdx.x] : 0;
-    for (int it = 0; it < kCItems; ++it) {
-        int64_t i = base + (int64_t)it * kBlock + threadIdx.x;
-        bool pred = i < n && flag[i];
-        int tot;
-        int r = block_rank(pred, shw, &tot);
-        if (WRITE && pred) out[run + r] = (int32_t)i;
-        run += tot;
+// The active candidates before block blk (its workgroup's threads together; sh: one per wave).
+__device__ __forceinline__ int64_t active_before(const uint32_t* __restrict__ bcnt, const uint32_t* __restrict__ scnt,
+                                                 int64_t blk, int64_t* sh) {
+    const int64_t sb = blk / kSuperBlocks, b = sb * kSuperBlocks + threadIdx.x;
+    int64_t v = b < blk ? (int64_t)bcnt[b] : 0;
+    for (int64_t q = threadIdx.x; q < sb; q += kBlock) v += scnt[kSuperStride * q];
+#pragma unroll
+    for (int o = kWave / 2; o > 0; o >>= 1) v += __shfl_xor(v, o);
+    if (lane_id() == 0) sh[wave_id()] = v;
+    __syncthreads();
+    v = 0;
+    for (int w = 0; w < kBlock / kWave; ++w) v += sh[w];
+    return v;
+}
+
+// The active count (one workgroup), where it is wanted before stage C's sizes.
+__global__ __launch_bounds__(kBlock) void active_total_kernel(const uint32_t* __restrict__ scnt, int64_t nsup,
+                                                              int64_t* __restrict__ total) {
+    __shared__ int64_t sh[kBlock / kWave];
+    const int64_t v = active_before(nullptr, scnt, nsup * kSuperBlocks, sh);
+    if (threadIdx.x == 0) *total = v;
+}
+
+// A block's share of stages B and C: its active candidates in order (their places in the block
+// listed in LDS) and the index of the first among all; the last block writes the total.
+// Returns their number; uniform over the workgroup, whose threads meet before the next block.
+struct ActiveArgs {
+    const uint8_t* flag;
+    int64_t n;            // PT + EE candidates (dn, nullable: counted on the device)
+    const int64_t* dn;
+    const uint32_t *bcnt, *scnt;
+    int64_t *total, *total2;  // total2 nullable
+};
+__device__ __forceinline__ int64_t active_blocks(const ActiveArgs& A, int64_t& n) {
+    n = A.dn ? A.dn[2] + A.dn[3] : A.n;
+    if (n == 0 && blockIdx.x == 0 && threadIdx.x == 0) {
+        *A.total = 0;
+        if (A.total2) *A.total2 = 0;
     }
-    if (!WRITE && threadIdx.x == 0) bcnt[blockIdx.x] = run;
+    return (n + kBlock - 1) / kBlock;
+}
+__device__ __forceinline__ int active_block(const ActiveArgs& A, int64_t n, int64_t blk, int64_t nblk, uint8_t* list,
+                                            int64_t& first) {
+    __shared__ int64_t sh[kBlock / kWave];
+    __shared__ int shw[kBlock / kWave];
+    const int c = (int)A.bcnt[blk];
+    if (c == 0 && blk + 1 < nblk) return 0;
+    __syncthreads();  // the last block's list is read
+    first = active_before(A.bcnt, A.scnt, blk, sh);
+    if (blk + 1 == nblk && threadIdx.x == 0) {
+        *A.total = first + c;
+        if (A.total2) *A.total2 = first + c;
+    }
+    const int64_t i = blk * kBlock + threadIdx.x;
+    const bool pred = i < n && A.flag[i];
+    int tot;
+    const int r = block_rank(pred, shw, &tot);
+    if (pred) list[r] = (uint8_t)threadIdx.x;
+    __syncthreads();
+    return c;
+}
+// workgroups of the kernels over those blocks, at most
+constexpr int64_t kActiveGrid = 4096;
+
+// stage B on its own (the dense modes): the active candidates in order.
+__global__ __launch_bounds__(kBlock) void compact_flags_kernel(ActiveArgs A, int32_t* __restrict__ out) {
+    __shared__ uint8_t list[kBlock];
+    int64_t n;
+    const int64_t nblk = active_blocks(A, n);
+    for (int64_t blk = blockIdx.x; blk < nblk; blk += gridDim.x) {
+        int64_t first;
+        const int c = active_block(A, n, blk, nblk, list, first);
+        if (threadIdx.x < c) out[first + threadIdx.x] = (int32_t)(blk * kBlock + list[threadIdx.x]);
+    }
 }
 
 // sort key of candidate i of [PT | EE]: (type << 32) | body pair
@@ -237,6 +294,14 @@ __device__ __forceinline__ int64_t active_key(const int32_t* __restrict__ pt, in
     return ((int64_t)(is_ee ? 1 : 0) << 32) | (int64_t)t5[2];
 }
 
+// A run of contacts [begin, end) as stored in pseg: (kRunBase - begin, end), each the largest of
+// its writers' (0, 0: empty), so the contacts of a run need not meet in one workgroup.
+constexpr unsigned long long kRunBase = 1ull << 40;
+__device__ __forceinline__ void read_run(const unsigned long long* __restrict__ ps, int64_t& begin, int64_t& end) {
+    begin = ps[0] ? (int64_t)(kRunBase - ps[0]) : 0;
+    end = (int64_t)ps[1];
+}
+
 // Where stage C leaves what stage D needs of the active contacts, beside their terms.
 struct ContactOut {
     double* __restrict__ cbuf;
@@ -245,23 +310,18 @@ struct ContactOut {
     uint8_t* __restrict__ hl_ee;
     uint8_t* __restrict__ pflag;
     int64_t nij;
-    int64_t* __restrict__ pseg;
+    unsigned long long* __restrict__ pseg;
 };
 
-// The pair's flags and run of active contact e = candidate i, tuple t5.
-__device__ __forceinline__ void contact_bookkeeping(const ContactOut& O, const int32_t* __restrict__ pt, int64_t npt,
-                                                    const int32_t* __restrict__ ee,
-                                                    const int32_t* __restrict__ act, int64_t nact, int64_t e,
-                                                    bool is_ee, const int32_t* __restrict__ t5) {
-    const int64_t key = ((int64_t)(is_ee ? 1 : 0) << 32) | (int64_t)t5[2];
+// The pair's flags and run of active contact e, tuple t5, key; kprev, knext: the keys of its
+// neighbours in the sorted active list (-1: none known; the contact then also offers its ends).
+__device__ __forceinline__ void contact_bookkeeping(const ContactOut& O, int64_t e, int64_t key, int64_t kprev,
+                                                    int64_t knext, const int32_t* __restrict__ t5) {
+    const bool is_ee = (key >> 32) != 0;
     O.pflag[t5[2]] = 1;  // the body pair has an active contact (every writer stores 1)
-    // the run of this key in the sorted active list: [begin, end) of (type, pair) from
-    // the neighbours' keys (recomputed here from the lists)
-    const int64_t kprev = e > 0 ? active_key(pt, npt, ee, act[e - 1]) : -1;
-    const int64_t knext = e + 1 < nact ? active_key(pt, npt, ee, act[e + 1]) : -1;
-    int64_t* ps = O.pseg + 2 * ((is_ee ? O.nij : 0) + t5[2]);
-    if (kprev != key) ps[0] = e;
-    if (knext != key) ps[1] = e + 1;
+    unsigned long long* ps = O.pseg + 2 * ((is_ee ? O.nij : 0) + t5[2]);
+    if (kprev != key) atomicMax(ps, kRunBase - (unsigned long long)e);
+    if (knext != key) atomicMax(ps + 1, (unsigned long long)(e + 1));
     O.swap[e] = t5[0] > t5[1] ? 1 : 0;  // body I is ij1 (PT second order)
     if (is_ee)
         O.hl_ee[t5[1]] = 1;
@@ -269,30 +329,43 @@ __device__ __forceinline__ void contact_bookkeeping(const ContactOut& O, const i
         O.hl_pt[t5[1]] = 1;
 }
 
-// stage C: one thread per active contact (the contact-space terms, psd 0 and 1).
+// stages B and C: the active contacts of a block of kBlock candidates, one thread each (the
+// contact-space terms, psd 0 and 1).  As a compaction and a kernel over its list these were
+// two launches, with the scan between them three (4.6 + 8.1 + 16.4 us at 87 k candidates, 2 k
+// active; 12.7 us here).
 __global__ __launch_bounds__(kBlock) void contact_kernel(AbdScene sc, AbdParams P, const double* __restrict__ x,
                                                           const int32_t* __restrict__ pt, int64_t npt,
-                                                          const int32_t* __restrict__ ee,
-                                                          const int32_t* __restrict__ act, int64_t nact,
-                                                          const int64_t* __restrict__ dnact,
-                                                          const int64_t* __restrict__ dn, ContactOut O) {
+                                                          const int32_t* __restrict__ ee, ActiveArgs A,
+                                                          ContactOut O) {
+    __shared__ uint8_t list[kBlock];
+    __shared__ int64_t keys[kBlock];
     const SceneView S = view_of(sc);
-    if (dnact) nact = *dnact;
-    if (dn) npt = dn[2];
-    for (int64_t e = (int64_t)blockIdx.x * kBlock + threadIdx.x; e < nact; e += (int64_t)gridDim.x * kBlock) {
-        const int64_t i = act[e];
-        const bool is_ee = i >= npt;
-        const int32_t* t5 = is_ee ? ee + 5 * (i - npt) : pt + 5 * i;
-        int64_t vi[4];
-        if (is_ee)
-            fetch_ee_idx(S, t5, vi);
-        else
-            fetch_pt_idx(S, t5, vi);
-        d3 v[4], r[4];
-        load4(x, vi, v);
-        load4(sc.x0, vi, r);
-        contact_terms(is_ee ? 1 : 0, v, r, P.d2hat, P.kappa, P.psd, O.cbuf + e * kContactStride);
-        contact_bookkeeping(O, pt, npt, ee, act, nact, e, is_ee, t5);
+    int64_t n;
+    const int64_t nblk = active_blocks(A, n);
+    if (A.dn) npt = A.dn[2];
+    const int t = threadIdx.x;
+    for (int64_t blk = blockIdx.x; blk < nblk; blk += gridDim.x) {
+        int64_t first;
+        const int c = active_block(A, n, blk, nblk, list, first);
+        if (c == 0) continue;  // uniform
+        const int64_t i = blk * kBlock + (t < c ? list[t] : 0);
+        if (t < c) keys[t] = active_key(pt, npt, ee, i);
+        __syncthreads();
+        if (t < c) {
+            const int64_t e = first + t;
+            const bool is_ee = i >= npt;
+            const int32_t* t5 = is_ee ? ee + 5 * (i - npt) : pt + 5 * i;
+            int64_t vi[4];
+            if (is_ee)
+                fetch_ee_idx(S, t5, vi);
+            else
+                fetch_pt_idx(S, t5, vi);
+            d3 v[4], r[4];
+            load4(x, vi, v);
+            load4(sc.x0, vi, r);
+            contact_terms(is_ee ? 1 : 0, v, r, P.d2hat, P.kappa, P.psd, O.cbuf + e * kContactStride);
+            contact_bookkeeping(O, e, keys[t], t > 0 ? keys[t - 1] : -1, t + 1 < c ? keys[t + 1] : -1, t5);
+        }
     }
 }
 
@@ -326,7 +399,9 @@ __global__ __launch_bounds__(kWave) void contact_dense_kernel(AbdScene sc, AbdPa
             wave_contact_full(lane, is_ee ? 1 : 0, v, r, P.d2hat, P.kappa, D, O.cbuf + e * kDenseStride);
         else
             wave_contact_exact(lane, is_ee ? 1 : 0, v, r, P.d2hat, P.kappa, D, O.cbuf + e * kDenseStride);
-        if (lane == 0) contact_bookkeeping(O, pt, npt, ee, act, nact, e, is_ee, t5);
+        if (lane == 0)
+            contact_bookkeeping(O, e, active_key(pt, npt, ee, i), e > 0 ? active_key(pt, npt, ee, act[e - 1]) : -1,
+                                e + 1 < nact ? active_key(pt, npt, ee, act[e + 1]) : -1, t5);
     }
 }
 
@@ -335,60 +410,91 @@ __global__ __launch_bounds__(kWave) void contact_dense_kernel(AbdScene sc, AbdPa
 constexpr int64_t kDenseGrid = 4096;
 
 constexpr int kPairThreads = 576;  // one thread per entry of the 24x24 body-pair block
-constexpr int kPairBufStride = 2 * 144 + 24;  // diag(ij0), diag(ij1), g(ij0), g(ij1)
 constexpr int64_t kPairGrid = 2048;           // workgroups of stage D (grid-stride over pairs)
 
 constexpr int kPairChunk = 64;  // contacts of one stage-D work item
 constexpr int kPartStride = 600;  // one chunk's partial sums: the 24x24 block, then g (24)
 
 // stage D1: the work items of each body pair: its PT run and its EE run cut into chunks of
-// kPairChunk contacts (runs from stage C; empty runs are [0, 0)).  One workgroup scans the pairs'
-// item counts into their first items coff and the total.
-__device__ __forceinline__ int64_t pair_item_count(const int64_t* __restrict__ pseg, int64_t nij, int64_t ii) {
-    const int64_t npt = pseg[2 * ii + 1] - pseg[2 * ii], nee = pseg[2 * (nij + ii) + 1] - pseg[2 * (nij + ii)];
-    return (npt + kPairChunk - 1) / kPairChunk + (nee + kPairChunk - 1) / kPairChunk;
-}
-__global__ __launch_bounds__(kScanThreads) void pair_chunks_scan_kernel(int64_t nij, const int64_t* __restrict__ pseg,
-                                                                        int64_t* __restrict__ coff,
-                                                                        int64_t* __restrict__ total) {
-    scan_block_exclusive_by([=](int64_t ii) { return pair_item_count(pseg, nij, ii); }, coff, nij, total, nullptr);
-}
-
-// stage D's items: pair ii owns the items [coff[ii], coff[ii] + cnt[ii]), its PT run's chunks
-// then its EE run's; item i's descriptor is its first contact | its contact count << 56.
-// The order the rank-one partial sums run them in (slot -> item, odesc / oitem) takes the full
-// chunks first (counted in counters[0], from the front) and the others after them (counters[1],
-// from the back): the longest sums start first.  Where an item lands in it changes no result.
-// One wave per pair, its lanes striding over the pair's items.
+// kPairChunk contacts (runs from stage C).  Pair ii owns the items [pitem[ii].x, + pitem[ii].y),
+// taken from a counter in any order (where a pair's items lie changes no result), its PT run's
+// chunks then its EE run's; item i's descriptor idesc is its first contact | its contact count
+// << 56.  The order the rank-one partial sums run them in takes the full chunks first (odesc /
+// oitem from the front, counters[0] of them) and the others after them (from cap on,
+// counters[1]): the longest sums start first.  counters[2]: all items.  A workgroup takes kBlock
+// pairs and one add per counter (adds to one cache line wait for each other: with three a pair
+// this took 28 us for 700 pairs with contacts; 5 us here), then its threads stride over the items.
 constexpr int kItemShift = 56;
-__global__ __launch_bounds__(kBlock) void pair_items_kernel(int64_t nij, const int64_t* __restrict__ coff,
-                                                            const int64_t* __restrict__ pseg,
-                                                            const int64_t* __restrict__ total,
-                                                            int64_t* __restrict__ idesc, int* __restrict__ counters,
-                                                            int64_t* __restrict__ odesc,
-                                                            int64_t* __restrict__ oitem) {
-    const int64_t ntot = *total;
-    const int lane = threadIdx.x & (kWave - 1);
-    const int64_t nw = (int64_t)gridDim.x * (kBlock / kWave);
-    for (int64_t ii = ((int64_t)blockIdx.x * kBlock + threadIdx.x) / kWave; ii < nij; ii += nw) {
-        const int64_t o = coff[ii];
-        const int64_t p0 = pseg[2 * ii], p1 = pseg[2 * ii + 1];
-        const int64_t e0 = pseg[2 * (nij + ii)], e1 = pseg[2 * (nij + ii) + 1];
-        const int64_t npc = (p1 - p0 + kPairChunk - 1) / kPairChunk;
-        const int64_t n = npc + (e1 - e0 + kPairChunk - 1) / kPairChunk;
-        for (int64_t c = lane; c < n; c += kWave) {
+struct PairItems {
+    int2* pitem;
+    int64_t *idesc, *odesc, *oitem;
+    int64_t cap;
+    int* counters;
+};
+__global__ __launch_bounds__(kBlock) void pair_items_kernel(int64_t nij, const int64_t* __restrict__ dn,
+                                                            const uint8_t* __restrict__ pflag,
+                                                            const unsigned long long* __restrict__ pseg,
+                                                            int64_t nij_cap, PairItems I) {
+    if (dn) nij = dn[0];
+    __shared__ int64_t sh[kBlock / kWave];
+    __shared__ int64_t run[kBlock][4];   // PT and EE runs of the workgroup's pairs
+    __shared__ int ifirst[kBlock], ffirst[kBlock], pfirst[kBlock];  // first item, full and other chunk
+    __shared__ int base[3], nitems;
+    const int t = threadIdx.x;
+    constexpr int kPartialShift = 40;
+    for (int64_t ii0 = (int64_t)blockIdx.x * kBlock; ii0 < nij; ii0 += (int64_t)gridDim.x * kBlock) {
+        const int64_t ii = ii0 + t;
+        int64_t p0 = 0, p1 = 0, e0 = 0, e1 = 0;
+        if (ii < nij && pflag[ii]) {
+            read_run(pseg + 2 * ii, p0, p1);
+            read_run(pseg + 2 * (nij_cap + ii), e0, e1);
+        }
+        const int64_t full = (p1 - p0) / kPairChunk + (e1 - e0) / kPairChunk;
+        const int64_t partial = ((p1 - p0) % kPairChunk != 0) + ((e1 - e0) % kPairChunk != 0);
+        const int64_t mine = full | partial << kPartialShift;
+        const int64_t before = block_exclusive_scan_i64(mine, sh);
+        const int nf = (int)(before & ((int64_t(1) << kPartialShift) - 1)), np = (int)(before >> kPartialShift);
+        run[t][0] = p0;
+        run[t][1] = p1;
+        run[t][2] = e0;
+        run[t][3] = e1;
+        ifirst[t] = nf + np;
+        ffirst[t] = nf;
+        pfirst[t] = np;
+        if (t == kBlock - 1) {
+            const int tf = nf + (int)full, tp = np + (int)partial;
+            nitems = tf + tp;
+            if (tf) base[0] = atomicAdd(I.counters, tf);
+            if (tp) base[1] = atomicAdd(I.counters + 1, tp);
+            if (tf + tp) base[2] = atomicAdd(I.counters + 2, tf + tp);
+        }
+        __syncthreads();
+        if (full + partial) I.pitem[ii] = make_int2(base[2] + ifirst[t], (int)(full + partial));
+        for (int q = t; q < nitems; q += kBlock) {
+            int lo = 0, hi = kBlock - 1;  // the pair: the last whose first item is <= q
+            while (lo < hi) {
+                const int mid = (lo + hi + 1) >> 1;
+                if (ifirst[mid] <= q)
+                    lo = mid;
+                else
+                    hi = mid - 1;
+            }
+            const int64_t a0 = run[lo][0], a1 = run[lo][1], b0 = run[lo][2], b1 = run[lo][3];
+            const int64_t npc = (a1 - a0 + kPairChunk - 1) / kPairChunk, c = q - ifirst[lo];
             const bool pt = c < npc;
-            const int64_t c0 = pt ? p0 + c * kPairChunk : e0 + (c - npc) * kPairChunk;
-            const int64_t end = pt ? p1 : e1;
+            const int64_t c0 = pt ? a0 + c * kPairChunk : b0 + (c - npc) * kPairChunk;
+            const int64_t end = pt ? a1 : b1;
             const int64_t nc = end - c0 < kPairChunk ? end - c0 : kPairChunk;
             const int64_t d = c0 | (nc << kItemShift);
-            idesc[o + c] = d;
-            const bool full = nc == kPairChunk;
-            const int64_t k = atomicAdd(counters + (full ? 0 : 1), 1);
-            const int64_t slot = full ? k : ntot - 1 - k;
-            odesc[slot] = d;
-            oitem[slot] = o + c;
+            I.idesc[base[2] + q] = d;
+            // PT's full chunks come first among the pair's, its partial one (if any) too
+            const bool whole = nc == kPairChunk, pt_rest = (a1 - a0) % kPairChunk != 0;
+            const int64_t slot = whole ? base[0] + ffirst[lo] + c - (!pt && pt_rest ? 1 : 0)
+                                       : I.cap + base[1] + pfirst[lo] + (!pt && pt_rest ? 1 : 0);
+            I.odesc[slot] = d;
+            I.oitem[slot] = base[2] + q;
         }
+        __syncthreads();  // the tables are free for the next pairs
     }
 }
 
@@ -397,18 +503,16 @@ __global__ __launch_bounds__(kBlock) void pair_items_kernel(int64_t nij, const i
 // order [ij0 | ij1], then g), for contacts stored whole by contact_dense_kernel.
 __global__ __launch_bounds__(kPairThreads) void pair_partial_dense_kernel(const double* __restrict__ cbuf,
                                                                            const uint8_t* __restrict__ swap,
-                                                                           const int64_t* __restrict__ idesc,
-                                                                     const int64_t* __restrict__ total,
-                                                                     double* __restrict__ part) {
+                                                                           PairItems I, double* __restrict__ part) {
     constexpr int kStride = kDenseStride;
     constexpr int kBatch = 4;
     __shared__ double sc[kBatch][kStride];
     __shared__ uint8_t ssw[kBatch];
     const int t = threadIdx.x;
     const int R = t / 24, C = t % 24;
-    const int64_t nitem = *total;
+    const int64_t nitem = I.counters[2];
     for (int64_t gc = blockIdx.x; gc < nitem; gc += gridDim.x) {
-        const int64_t d = idesc[gc];
+        const int64_t d = I.idesc[gc];
         const int64_t c0 = d & ((int64_t(1) << kItemShift) - 1);
         const int64_t c1 = c0 + (d >> kItemShift);
         double h = 0.0, gacc = 0.0;
@@ -474,10 +578,7 @@ __device__ __forceinline__ void rank_batch_store(dbl2* dst, int np, int t, const
 
 __global__ __launch_bounds__(kRankThreads, 5) void pair_partial_rank_kernel(const double* __restrict__ cbuf,
                                                                          const uint8_t* __restrict__ swap,
-                                                                         const int64_t* __restrict__ odesc,
-                                                                         const int64_t* __restrict__ oitem,
-                                                                         const int64_t* __restrict__ total,
-                                                                         double* __restrict__ part) {
+                                                                         PairItems I, double* __restrict__ part) {
     // the staged batch, then a 16-byte slot the pieces past the batch are stored to
     __shared__ __align__(16) double st[kRankBatch * kStaged + 2];
     const int t = threadIdx.x, lane = t % kWave;
@@ -493,12 +594,14 @@ __global__ __launch_bounds__(kRankThreads, 5) void pair_partial_rank_kernel(cons
     // V indices in the stored order, without and with the halves swapped (body I is ij1)
     const int tg = t % 24;
     const int rA = r, rB = (r + 12) % 24, cA = c, cB = (c + 12) % 24, gA = tg, gB = (tg + 12) % 24;
-    const int64_t nitem = *total;
-    int64_t gc = blockIdx.x;  // the execution slot (its item: oitem[gc])
+    const int64_t nfull = I.counters[0], nitem = nfull + I.counters[1];
+    const int64_t gap = I.cap - nfull;  // execution slots past the full chunks are stored from cap on
+    int64_t gc = blockIdx.x;  // the execution slot
     if (gc >= nitem) return;  // uniform
     const int64_t kMask = (int64_t(1) << kItemShift) - 1;
-    int64_t c0 = odesc[gc] & kMask;
-    int nc = (int)(odesc[gc] >> kItemShift), b0 = 0;
+    const int64_t d0 = I.odesc[gc < nfull ? gc : gc + gap];
+    int64_t c0 = d0 & kMask;
+    int nc = (int)(d0 >> kItemShift), b0 = 0;
     dbl2 piece[kRankPieces];
     rank_batch_load<0>(reinterpret_cast<const dbl2*>(cbuf + c0 * kContactStride), 63 * min(nc, kRankBatch), t,
                        piece);
@@ -518,7 +621,7 @@ __global__ __launch_bounds__(kRankThreads, 5) void pair_partial_rank_kernel(cons
             gn = gc + gridDim.x;
             bn = 0;
             if (gn < nitem) {
-                const int64_t dn_ = odesc[gn];
+                const int64_t dn_ = I.odesc[gn < nfull ? gn : gn + gap];
                 cn = dn_ & kMask;
                 nn = (int)(dn_ >> kItemShift);
             }
@@ -545,7 +648,7 @@ __global__ __launch_bounds__(kRankThreads, 5) void pair_partial_rank_kernel(cons
             gacc += K[5] * S[6 + 96 + (sw ? gB : gA)];
         }
         if (gn != gc) {  // uniform: the item is summed
-            double* pp = part + oitem[gc] * kPartStride;
+            double* pp = part + I.oitem[gc < nfull ? gc : gc + gap] * kPartStride;
             if (ent) {
                 pp[24 * r + c] = h;
                 pp[24 * c + r] = h;
@@ -559,44 +662,6 @@ __global__ __launch_bounds__(kRankThreads, 5) void pair_partial_rank_kernel(cons
         c0 = cn;
         nc = nn;
         b0 = bn;
-    }
-}
-
-// stage D3: per body pair with active contacts (grid-stride): its chunks' partial sums
-// (items [coff[ii], coff[ii + 1]); coff has nij + 1 entries, the last the total) added in
-// order (PT chunks, then EE), diagonal parts to the pair buffer (stage E adds
-// them per body), the off-diagonal block to the matrix.  nij: pairs of the buffers (an upper
-// bound when dn gives the count of the matrix's pairs, dn[0], which places its lower slots).
-__global__ __launch_bounds__(kPairThreads) void pair_reduce_kernel(int nb, int64_t nij,
-                                                                    const int64_t* __restrict__ dn,
-                                                                    const uint8_t* __restrict__ pflag,
-                                                                    const int64_t* __restrict__ coff,
-                                                                    const double* __restrict__ part,
-                                                                    double* __restrict__ pbuf,
-                                                                    double* __restrict__ blocks) {
-    const int t = threadIdx.x;
-    const int R = t / 24, C = t % 24;
-    const int64_t nij_m = dn ? dn[0] : nij;
-    for (int64_t ii = blockIdx.x; ii < nij; ii += gridDim.x) {
-        if (!pflag[ii]) continue;  // uniform over the workgroup
-        const int64_t c0 = coff[ii], nc = coff[ii + 1] - c0;  // coff[nij] holds the items' total
-        double h = 0.0, gacc = 0.0;
-        for (int64_t c = c0; c < c0 + nc; ++c) {
-            h += part[c * kPartStride + t];
-            if (t < 24) gacc += part[c * kPartStride + 576 + t];
-        }
-        double* pb = pbuf + ii * kPairBufStride;
-        if (R < 12 && C < 12) pb[R * 12 + C] = h;
-        if (R >= 12 && C >= 12) pb[144 + (R - 12) * 12 + (C - 12)] = h;
-        if (t < 24) pb[288 + t] = gacc;
-        // off-diagonal: upper slot nb + ii holds rows ij0 x cols ij1, lower slot its transpose
-        if (R < 12 && C >= 12) {
-            const int c2 = C - 12;
-            const int bi = R / 3, rr = R % 3, bj = c2 / 3, cc = c2 % 3;
-            const int64_t up = nb + ii, lo = nb + nij_m + ii;
-            blocks[9 * (16 * up + bi + 4 * bj) + 3 * rr + cc] += h;
-            blocks[9 * (16 * lo + bj + 4 * bi) + 3 * cc + rr] += h;
-        }
     }
 }
 
@@ -641,19 +706,26 @@ __device__ __forceinline__ void body_vg_range(const int32_t* __restrict__ vg, in
     k1 = lo[1];
 }
 
-// stage E: one workgroup per body (144 Hessian entries + 12 gradient entries).
+// stage E: one workgroup per body: its 144 Hessian and 12 gradient entries, and the off-diagonal
+// blocks of the pairs whose first body it is.  A pair's chunks' partial sums (part, in the
+// pair's body order [ij0 | ij1]) are added in order (PT chunks, then EE), the pairs in row
+// order; nij_cap: pairs of the buffers (a bound when dn counts the matrix's, dn[0], which
+// places the lower slots).  nact (nullable): an active count no stage wrote, zeroed.
 __global__ __launch_bounds__(kBlock) void body_finalize_kernel(AbdScene sc, AbdParams P,
                                                                 const double* __restrict__ x, int64_t nij,
                                                                 const int64_t* __restrict__ dn,
                                                                 const int32_t* __restrict__ row_ptr,
                                                                 const int32_t* __restrict__ slots,
                                                                 const uint8_t* __restrict__ pflag,
-                                                                const double* __restrict__ pbuf,
+                                                                const int2* __restrict__ pitem,
+                                                                const double* __restrict__ part,
                                                                 const int32_t* __restrict__ vg, int64_t nvg,
                                                                 double* __restrict__ g, double* __restrict__ blocks,
                                                                 const uint8_t* __restrict__ hl_pt,
                                                                 const uint8_t* __restrict__ hl_ee,
-                                                                uint8_t* __restrict__ highlight) {
+                                                                uint8_t* __restrict__ highlight,
+                                                                int64_t* __restrict__ nact) {
+    __shared__ int s_item[kBlock], s_n[kBlock], s_slot[kBlock];
     const int b = blockIdx.x;
     const int t = threadIdx.x;
     const int nb = sc.n_bodies;
@@ -661,21 +733,51 @@ __global__ __launch_bounds__(kBlock) void body_finalize_kernel(AbdScene sc, AbdP
         nij = dn[0];
         nvg = dn[4];
     }
+    if (nact && b == 0 && t == 0) *nact = 0;
     // threads 0..143: the entries of the diagonal block; 144..155: the gradient; the rest
     // only help to evaluate the vertex-ground terms
     const bool act = t < 156;
     const bool isg = t >= 144;
     const int R = isg ? t - 144 : t / 12, C = isg ? 0 : t % 12;
     double acc = 0.0;
-    if (act && nij > 0) {
-        for (int e = row_ptr[b]; e < row_ptr[b + 1]; ++e) {
-            const int s = slots[e];
-            if (s < nb) continue;
-            const int64_t ii = s < nb + nij ? s - nb : s - nb - nij;
-            if (!pflag[ii]) continue;  // a pair without active contacts adds nothing
-            const int side = s < nb + nij ? 0 : 1;  // upper slot in row b: b is ij0
-            const double* pb = pbuf + ii * kPairBufStride;
-            acc += isg ? pb[288 + 12 * side + R] : pb[144 * side + R * 12 + C];
+    if (part && nij > 0) {  // uniform
+        const int e1 = row_ptr[b + 1];
+        for (int eb = row_ptr[b]; eb < e1; eb += kBlock) {
+            const int ne = e1 - eb < kBlock ? e1 - eb : kBlock;
+            if (t < ne) {  // the row's pairs with active contacts: their items, side
+                const int s = slots[eb + t];
+                int2 it = make_int2(0, 0);
+                if (s >= nb) {
+                    const int64_t ii = s < nb + nij ? s - nb : s - nb - nij;
+                    if (pflag[ii]) it = pitem[ii];
+                }
+                s_item[t] = it.x;
+                s_n[t] = it.y;
+                s_slot[t] = s;
+            }
+            __syncthreads();
+            if (act)
+                for (int q = 0; q < ne; ++q) {
+                    const int n = s_n[q];
+                    if (n == 0) continue;  // the diagonal, or a pair without active contacts
+                    const int s = s_slot[q];
+                    const int side = s < nb + nij ? 0 : 1;  // upper slot in row b: b is ij0
+                    const double* pp = part + (int64_t)s_item[q] * kPartStride;
+                    const int at = isg ? 576 + 12 * side + R : 24 * (12 * side + R) + 12 * side + C;
+                    double h = 0.0, ho = 0.0;
+                    for (int c = 0; c < n; ++c) {
+                        h += pp[(int64_t)c * kPartStride + at];
+                        if (!isg && side == 0) ho += pp[(int64_t)c * kPartStride + 24 * R + 12 + C];
+                    }
+                    acc += h;
+                    if (!isg && side == 0) {
+                        // upper slot s holds rows ij0 x cols ij1, lower slot its transpose
+                        const int bi = R / 3, rr = R % 3, bj = C / 3, cc = C % 3;
+                        blocks[9 * (16 * (int64_t)s + bi + 4 * bj) + 3 * rr + cc] += ho;
+                        blocks[9 * (16 * (s + nij) + bj + 4 * bi) + 3 * cc + rr] += ho;
+                    }
+                }
+            __syncthreads();
         }
     }
     if (P.vg && nvg > 0) {
@@ -731,20 +833,34 @@ __global__ __launch_bounds__(kBlock) void body_finalize_kernel(AbdScene sc, AbdP
     if (t == 0 && highlight) highlight[b] = (uint8_t)((hl_pt[b] ? 1 : 0) | (hl_ee[b] ? 2 : 0));
 }
 
-// the gh stage's flags and counters: the ordering flag, n8 bytes at a8, n64 int64 at a64
-// (nact_dev, nullable: an active count that no later stage writes)
-__global__ void gh_zero_kernel(int* __restrict__ err, uint8_t* __restrict__ a8, int64_t n8,
-                               int64_t* __restrict__ a64, int64_t n64, int64_t* __restrict__ b64, int64_t nb64,
-                               int64_t* __restrict__ nact_dev) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < nb64) b64[i] = 0;
-    if (i == 0) {
-        if (nact_dev) *nact_dev = 0;
-        err[0] = 0;
-        err[1] = err[2] = 0;  // stage D's counters of full and partial chunks
-    }
-    if (i < n8) a8[i] = 0;
-    if (i < n64) a64[i] = 0;
+// The gh stage's flags and counters, 0 before it: the ordering flag, stage D's counters and the
+// active count (16 words), the active counts of the super-blocks, the pairs' runs, then the
+// bodies' highlight bytes (PT, EE) and the pairs' active flags.
+struct GhScratch {
+    int* err;
+    int* counters;
+    int64_t* total;
+    uint32_t* scnt;
+    unsigned long long* pseg;  // [2][nij][2]
+    uint8_t *hl_pt, *hl_ee, *pflag;
+    int64_t nsup, words;       // 8-byte words in all
+};
+int gh_scratch(int nb, int64_t nij, int64_t n, GhScratch& G) {
+    G.nsup = ceil_div(ceil_div(n, (int64_t)kBlock), (int64_t)kSuperBlocks);
+    const size_t bytes = 2 * (size_t)nb + (size_t)nij;
+    G.words = 8 + kSuperStride * G.nsup / 2 + 4 * nij + (int64_t)((bytes + 7) / 8);
+    uint64_t* p;
+    const int rc = arena_get(kSlotMisc, sizeof(uint64_t) * (size_t)G.words, (void**)&p);
+    if (rc) return rc;
+    G.err = reinterpret_cast<int*>(p);
+    G.counters = G.err + 1;
+    G.total = reinterpret_cast<int64_t*>(p + 4);
+    G.scnt = reinterpret_cast<uint32_t*>(p + 8);
+    G.pseg = reinterpret_cast<unsigned long long*>(p + 8 + kSuperStride * G.nsup / 2);
+    G.hl_pt = reinterpret_cast<uint8_t*>(G.pseg + 4 * nij);
+    G.hl_ee = G.hl_pt + nb;
+    G.pflag = G.hl_ee + nb;
+    return ABD_OK;
 }
 
 // Per-contact entry (tests, microbenchmarks): dense 24x24 and gradient per contact.
@@ -844,7 +960,7 @@ __global__ void inertia_hessian_kernel(int nb, AbdParams P, const double* __rest
 // that are not grouped.
 int contact_gh(hipStream_t s, const AbdScene* sc, const AbdParams* P, const double* x, const GhLists& L,
                const int32_t* row_ptr, const int32_t* slots, double* g, double* blocks, uint8_t* highlight,
-               int64_t* n_active, int64_t* n_active_dev) {
+               int64_t* n_active, int64_t* n_active_dev, bool zeroed) {
     const int nb = sc->n_bodies;
     if (nb == 0) return ABD_OK;
     const int32_t *pt = L.pt, *ee = L.ee, *vg = L.vg;
@@ -853,55 +969,34 @@ int contact_gh(hipStream_t s, const AbdScene* sc, const AbdParams* P, const doub
     const int64_t* dn = L.dn;
     const int64_t n = npt + nee;
     int rc;
-    // misc: err flag, highlight bytes [2 nb], active-pair flags [nij]
-    uint8_t* misc;
-    if ((rc = arena_get(kSlotMisc, 64 + 2 * (size_t)nb + (size_t)nij, (void**)&misc))) return rc;
-    int* err = reinterpret_cast<int*>(misc);
-    uint8_t* hl_pt = misc + 64;
-    uint8_t* hl_ee = hl_pt + nb;
-    uint8_t* pflag = hl_ee + nb;
-    // the pair runs of stage C (empty unless written), zeroed with the flags
-    int64_t* pseg = nullptr;  // [2][nij][2]
-    if (nij > 0 && (rc = arena_get(kSlotPairSeg, sizeof(int64_t) * 4 * (size_t)nij, (void**)&pseg))) return rc;
-    // stage B's per-block counts, added to by stage A (zeroed here with the flags)
-    const int64_t nblk = n > 0 ? ceil_div(n, (int64_t)kBlock * kCItems) : 0;
-    int64_t *bcnt = nullptr, *boff = nullptr;
-    if (n > 0) {
-        if ((rc = arena_get(kSlotScanA, sizeof(int64_t) * (nblk + 1), (void**)&bcnt))) return rc;
-        if ((rc = arena_get(kSlotScanB, sizeof(int64_t) * (nblk + 1), (void**)&boff))) return rc;
-    }
-    {
-        const int64_t n8 = 2 * (int64_t)nb + nij, n64 = 4 * nij;
-        const int64_t nz = std::max(std::max(n8, n64), nblk);
-        hipLaunchKernelGGL(gh_zero_kernel, dim3(grid_for(nz, kBlock, INT32_MAX)), dim3(kBlock), 0, s, err, hl_pt, n8,
-                           pseg, n64, bcnt, nblk, n > 0 ? nullptr : n_active_dev);
-        ABD_CHECK_LAUNCH();
-    }
+    GhScratch G;
+    if ((rc = gh_scratch(nb, nij, n, G))) return rc;
+    if (!zeroed && (rc = zero_fill(s, G.err, sizeof(uint64_t) * (size_t)G.words))) return rc;
     int64_t nact = 0;
-    int32_t* act = nullptr;
-    const int64_t* dev_nact = nullptr;
+    const int64_t nblk = ceil_div(n, (int64_t)kBlock);
+    uint8_t* flag = nullptr;
+    uint32_t* bcnt = nullptr;
     if (n + nvg > 0) {
-        uint8_t* flag;
         if ((rc = arena_get(kSlotFlags, (size_t)n + 1, (void**)&flag))) return rc;
+        if ((rc = arena_get(kSlotScanA, sizeof(uint32_t) * ((size_t)nblk + 1), (void**)&bcnt))) return rc;
         int ph = prof_start(kProfClassify, s, dn ? 1.0 : 129.0 * npt + 133.0 * nee + 8.0 * nvg);
-        hipLaunchKernelGGL(classify_kernel, dim3(grid_for(n + nvg, kBlock, 8192)), dim3(kBlock), 0, s, *sc, *P, x,
-                           pt, npt, ee, nee, vg, nvg, dn, flag, err, bcnt);
+        const int64_t blocks_all = nblk + ceil_div(nvg, (int64_t)kBlock);
+        hipLaunchKernelGGL(classify_kernel, dim3((unsigned)std::min<int64_t>(blocks_all, 8192)), dim3(kBlock), 0, s, *sc, *P, x,
+                           pt, npt, ee, nee, vg, nvg, dn, flag, G.err, bcnt, G.scnt);
         ABD_CHECK_LAUNCH();
         prof_stop(ph, s);
         if ((rc = prof_count_bytes(ph, s, dn, 129.0, 133.0, 8.0, 0.0))) return rc;
-        if (n > 0) {
-            if ((rc = arena_get(kSlotList, sizeof(int32_t) * (size_t)n, (void**)&act))) return rc;
-            if ((rc = scan_exclusive_i64(s, bcnt, boff, nblk, boff + nblk, n_active_dev))) return rc;
-            hipLaunchKernelGGL(compact_flags_kernel<true>, dim3((unsigned)nblk), dim3(kBlock), 0, s,
-                               (const uint8_t*)flag, n, dn, bcnt, (const int64_t*)boff, act);
-            ABD_CHECK_LAUNCH();
-            dev_nact = boff + nblk;
-        }
     }
+    const auto total_now = [&]() -> int {  // the active count for the host
+        hipLaunchKernelGGL(active_total_kernel, dim3(1), dim3(kBlock), 0, s, (const uint32_t*)G.scnt, G.nsup,
+                           G.total);
+        ABD_CHECK_LAUNCH();
+        return ABD_OK;
+    };
     const bool dense = P->psd >= 2;
     const int stride = dense ? kDenseStride : kContactStride;
     if (dn) {
-        nact = dev_nact ? n : 0;  // an upper bound: the stages below read the count on the device
+        nact = n;  // an upper bound: the stages below read the count on the device
         // The bound is the capacity of the candidate lists, which a superset swept by a very
         // long step can make many times the contacts: past the tuning's contact_bound_mib of
         // stored contacts the active count is read back and sizes the buffers instead (never
@@ -911,7 +1006,8 @@ int contact_gh(hipStream_t s, const AbdScene* sc, const AbdParams* P, const doub
             if (capturing()) return ABD_ERR_CAPACITY;
             int64_t* hv;
             if ((rc = arena_host(sizeof(int64_t), (void**)&hv))) return rc;
-            ABD_CHECK(hipMemcpyAsync(hv, dev_nact, sizeof(int64_t), hipMemcpyDeviceToHost, s));
+            if ((rc = total_now())) return rc;
+            ABD_CHECK(hipMemcpyAsync(hv, G.total, sizeof(int64_t), hipMemcpyDeviceToHost, s));
             ABD_CHECK(hipStreamSynchronize(s));
             nact = hv[0];
         }
@@ -920,8 +1016,11 @@ int contact_gh(hipStream_t s, const AbdScene* sc, const AbdParams* P, const doub
         int64_t* hv;
         if ((rc = arena_host(2 * sizeof(int64_t), (void**)&hv))) return rc;
         hv[0] = 0;
-        if (dev_nact) ABD_CHECK(hipMemcpyAsync(hv, dev_nact, sizeof(int64_t), hipMemcpyDeviceToHost, s));
-        ABD_CHECK(hipMemcpyAsync(hv + 1, err, sizeof(int), hipMemcpyDeviceToHost, s));
+        if (n > 0) {
+            if ((rc = total_now())) return rc;
+            ABD_CHECK(hipMemcpyAsync(hv, G.total, sizeof(int64_t), hipMemcpyDeviceToHost, s));
+        }
+        ABD_CHECK(hipMemcpyAsync(hv + 1, G.err, sizeof(int), hipMemcpyDeviceToHost, s));
         ABD_CHECK(hipStreamSynchronize(s));
         nact = hv[0];
         int herr = 0;
@@ -929,10 +1028,10 @@ int contact_gh(hipStream_t s, const AbdScene* sc, const AbdParams* P, const doub
         if (herr) return ABD_ERR_UNSORTED;
         if (n_active) *n_active = nact;
     }
-    double* pbuf = nullptr;
-    if (nij > 0) {
-        if ((rc = arena_get(kSlotPair, sizeof(double) * kPairBufStride * (size_t)nij, (void**)&pbuf))) return rc;
-    }
+    double* part = nullptr;
+    int2* pitem = nullptr;
+    // a count read back is 0: no stage below writes the device's
+    int64_t* const nact_unwritten = nact > 0 ? nullptr : n_active_dev;
     if (nact > 0) {
         double* cbuf;
         uint8_t* swp;
@@ -940,9 +1039,15 @@ int contact_gh(hipStream_t s, const AbdScene* sc, const AbdParams* P, const doub
         swp = reinterpret_cast<uint8_t*>(cbuf + stride * nact);
         const double cbytes = 4.0 + 20 + 16 + 192 + 8.0 * stride + 9;
         int ph = prof_start(kProfContact, s, dn ? 1.0 : cbytes * nact);
-        const int64_t* dnact = dn ? dev_nact : nullptr;
-        const ContactOut O{cbuf, swp, hl_pt, hl_ee, pflag, nij, pseg};
+        const int64_t* dnact = dn ? G.total : nullptr;
+        const ContactOut O{cbuf, swp, G.hl_pt, G.hl_ee, G.pflag, nij, G.pseg};
+        const ActiveArgs A{flag, n, dn, bcnt, G.scnt, G.total, n_active_dev};
         if (dense) {
+            int32_t* act;
+            if ((rc = arena_get(kSlotList, sizeof(int32_t) * (size_t)n, (void**)&act))) return rc;
+            hipLaunchKernelGGL(compact_flags_kernel, dim3((unsigned)std::min(nblk, kActiveGrid)), dim3(kBlock), 0, s, A,
+                               act);
+            ABD_CHECK_LAUNCH();
             const dim3 dgrid((unsigned)std::min<int64_t>(nact, kDenseGrid));
             if (P->psd == 3)
                 hipLaunchKernelGGL(contact_dense_kernel<3>, dgrid, dim3(kWave), 0, s, *sc, *P, x, pt, npt, ee,
@@ -951,8 +1056,8 @@ int contact_gh(hipStream_t s, const AbdScene* sc, const AbdParams* P, const doub
                 hipLaunchKernelGGL(contact_dense_kernel<2>, dgrid, dim3(kWave), 0, s, *sc, *P, x, pt, npt, ee,
                                    (const int32_t*)act, nact, dnact, dn, O);
         } else {
-            hipLaunchKernelGGL(contact_kernel, dim3(grid_for(nact, kBlock, 65535)), dim3(kBlock), 0, s, *sc, *P, x,
-                               pt, npt, ee, (const int32_t*)act, nact, dnact, dn, O);
+            hipLaunchKernelGGL(contact_kernel, dim3((unsigned)std::min(nblk, kActiveGrid)), dim3(kBlock), 0, s, *sc, *P, x,
+                               pt, npt, ee, A, O);
         }
         ABD_CHECK_LAUNCH();
         prof_stop(ph, s);
@@ -962,50 +1067,50 @@ int contact_gh(hipStream_t s, const AbdScene* sc, const AbdParams* P, const doub
         const int64_t pgrid = tuning().pair_grid > 0 ? tuning().pair_grid : kPairGrid;
         const int64_t runs = 2 * nij < nact ? 2 * nij : nact;
         const int64_t cap_items = nact / kPairChunk + runs + 1;
-        int64_t* pcoff;
-        if ((rc = arena_get(kSlotPairChunk, sizeof(int64_t) * ((size_t)nij + 2 + 3 * (size_t)cap_items),
-                            (void**)&pcoff)))
+        PairItems I{};
+        if ((rc = arena_get(kSlotPairChunk, sizeof(int64_t) * ((size_t)nij + 5 * (size_t)cap_items),
+                            (void**)&I.pitem)))
             return rc;
-        int64_t* ptotal = pcoff + nij;
-        int64_t* idesc = ptotal + 2;
-        int64_t* odesc = idesc + cap_items;
-        int64_t* oitem = odesc + cap_items;
-        double* part;
+        I.idesc = reinterpret_cast<int64_t*>(I.pitem + nij);
+        I.odesc = I.idesc + cap_items;
+        I.oitem = I.odesc + 2 * cap_items;
+        I.cap = cap_items;
+        I.counters = G.counters;
+        pitem = I.pitem;
         if ((rc = arena_get(kSlotPairPart, sizeof(double) * kPartStride * (size_t)cap_items, (void**)&part)))
             return rc;
-        hipLaunchKernelGGL(pair_chunks_scan_kernel, dim3(1), dim3(kScanThreads), 0, s, nij, (const int64_t*)pseg,
-                           pcoff, ptotal);
-        ABD_CHECK_LAUNCH();
-        hipLaunchKernelGGL(pair_items_kernel, dim3(grid_for(nij, kBlock / kWave)), dim3(kBlock), 0, s, nij,
-                           (const int64_t*)pcoff, (const int64_t*)pseg, (const int64_t*)ptotal,
-                           idesc, err + 1, odesc, oitem);
+        hipLaunchKernelGGL(pair_items_kernel, dim3(grid_for(nij, kBlock)), dim3(kBlock), 0, s, nij, dn,
+                           (const uint8_t*)G.pflag, (const unsigned long long*)G.pseg, nij, I);
         ABD_CHECK_LAUNCH();
         // timed: the partial sums (each stored contact read once, its body-order flag once)
         ph = prof_start_ext(kProfPairReduce, dn ? 1.0 : (8.0 * stride + 1) * nact);
         if (dense)
             prof_launch(ph, pair_partial_dense_kernel, dim3((unsigned)pgrid), dim3(kPairThreads), 0, s,
-                        (const double*)cbuf, (const uint8_t*)swp, (const int64_t*)idesc, (const int64_t*)ptotal,
-                        part);
+                        (const double*)cbuf, (const uint8_t*)swp, I, part);
         else
             prof_launch(ph, pair_partial_rank_kernel, dim3((unsigned)pgrid), dim3(kRankThreads), 0, s,
-                        (const double*)cbuf, (const uint8_t*)swp, (const int64_t*)odesc, (const int64_t*)oitem,
-                        (const int64_t*)ptotal, part);
+                        (const double*)cbuf, (const uint8_t*)swp, I, part);
         ABD_CHECK_LAUNCH();
         if ((rc = prof_count_bytes(ph, s, dnact, 8.0 * stride + 1, 0.0, 0.0, 0.0, true))) return rc;
-        hipLaunchKernelGGL(pair_reduce_kernel, dim3(grid_for(nij, 1, pgrid)), dim3(kPairThreads), 0, s, nb, nij,
-                           dn, (const uint8_t*)pflag, (const int64_t*)pcoff,
-                           (const double*)part, pbuf, blocks);
-        ABD_CHECK_LAUNCH();
     }
     const double fbytes = 2.0 * 8 * 156 * nb;
-    int phf = prof_start(kProfBodyFinalize, s, dn ? 1.0 : fbytes + 8.0 * kPairBufStride * nij + 40.0 * nvg);
+    const double pbytes = 8.0 * 2 * 312;  // a pair's partial sums, read by both bodies (one chunk)
+    int phf = prof_start(kProfBodyFinalize, s, dn ? 1.0 : fbytes + pbytes * nij + 40.0 * nvg);
     hipLaunchKernelGGL(body_finalize_kernel, dim3(nb), dim3(kBlock), 0, s, *sc, *P, x, nij, dn, row_ptr, slots,
-                       (const uint8_t*)pflag, (const double*)pbuf, vg, nvg, g, blocks, (const uint8_t*)hl_pt,
-                       (const uint8_t*)hl_ee, highlight);
+                       (const uint8_t*)G.pflag, (const int2*)pitem, (const double*)part, vg, nvg, g, blocks,
+                       (const uint8_t*)G.hl_pt, (const uint8_t*)G.hl_ee, highlight, nact_unwritten);
     ABD_CHECK_LAUNCH();
     prof_stop(phf, s);
-    if ((rc = prof_count_bytes(phf, s, dn, 0.0, 0.0, 40.0, 8.0 * kPairBufStride, false, fbytes))) return rc;
+    if ((rc = prof_count_bytes(phf, s, dn, 0.0, 0.0, 40.0, pbytes, false, fbytes))) return rc;
     return ABD_OK;
+}
+
+int gh_zero_region(int nb, int64_t nij, int64_t n, void** p, int64_t* words) {
+    GhScratch G;
+    const int rc = gh_scratch(nb, nij, n, G);
+    *p = G.err;
+    *words = G.words;
+    return rc;
 }
 
 }  // namespace abd

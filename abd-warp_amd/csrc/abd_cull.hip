@@ -352,42 +352,32 @@ __device__ __forceinline__ int64_t lower_bound2(const int32_t* __restrict__ a, i
     return lo;
 }
 
-// dnij (nullable): the pair count on the device (nij is then unused)
-__global__ void rowlen_kernel(int nb, int64_t nij, const int64_t* __restrict__ dnij, const int32_t* __restrict__ ij,
-                              const int32_t* __restrict__ ji, int64_t* __restrict__ len) {
+// The block structure from the sorted pairs, one thread per body row: before row b lie one
+// diagonal entry a body, the pairs whose first body is below b and those whose second is
+// (found in the sorted lists, so no scan of row lengths).  dnij (nullable): the pair count on
+// the device (nij is then unused).
+__global__ void structure_kernel(int nb, int64_t nij, const int64_t* __restrict__ dnij,
+                                 const int32_t* __restrict__ ij, const int32_t* __restrict__ ji,
+                                 int32_t* __restrict__ row_ptr, int32_t* __restrict__ cols,
+                                 int32_t* __restrict__ slots) {
     int b = blockIdx.x * blockDim.x + threadIdx.x;
     if (b >= nb) return;
     if (dnij) nij = *dnij;
-    int64_t nu = lower_bound2(ij, 0, 0, nij, b + 1) - lower_bound2(ij, 0, 0, nij, b);
-    int64_t nl = lower_bound2(ji, 1, 0, nij, b + 1) - lower_bound2(ji, 1, 0, nij, b);
-    len[b] = nl + 1 + nu;
-}
-
-__global__ void rowfill_kernel(int nb, int64_t nij, const int64_t* __restrict__ dnij, const int32_t* __restrict__ ij,
-                               const int32_t* __restrict__ ji, const int64_t* __restrict__ off,
-                               int32_t* __restrict__ row_ptr, int32_t* __restrict__ cols,
-                               int32_t* __restrict__ slots) {
-    int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= nb) return;
-    if (dnij) nij = *dnij;
-    const int64_t total = (int64_t)nb + 2 * nij;
-    int64_t o = off[b];
+    const int64_t l0 = lower_bound2(ji, 1, 0, nij, b), u0 = lower_bound2(ij, 0, 0, nij, b);
+    int64_t o = b + l0 + u0;
     row_ptr[b] = (int32_t)o;
-    if (b == nb - 1) row_ptr[nb] = (int32_t)total;
-    int64_t l0 = lower_bound2(ji, 1, 0, nij, b), l1 = lower_bound2(ji, 1, 0, nij, b + 1);
-    for (int64_t k = l0; k < l1; ++k) {
-        int i = ji[2 * k];
-        int64_t u0 = lower_bound2(ij, 0, 0, nij, i), u1 = lower_bound2(ij, 0, 0, nij, i + 1);
-        int64_t ii = lower_bound2(ij, 1, u0, u1, b);
+    if (b == nb - 1) row_ptr[nb] = (int32_t)(nb + 2 * nij);
+    for (int64_t k = l0; k < nij && ji[2 * k + 1] == b; ++k) {
+        const int i = ji[2 * k];
+        const int64_t v0 = lower_bound2(ij, 0, 0, nij, i), v1 = lower_bound2(ij, 0, v0, nij, i + 1);
         cols[o] = i;
-        slots[o] = (int32_t)(nb + nij + ii);
+        slots[o] = (int32_t)(nb + nij + lower_bound2(ij, 1, v0, v1, b));
         ++o;
     }
     cols[o] = b;
     slots[o] = b;
     ++o;
-    int64_t u0 = lower_bound2(ij, 0, 0, nij, b), u1 = lower_bound2(ij, 0, 0, nij, b + 1);
-    for (int64_t k = u0; k < u1; ++k) {
+    for (int64_t k = u0; k < nij && ij[2 * k] == b; ++k) {
         cols[o] = ij[2 * k + 1];
         slots[o] = (int32_t)(nb + k);
         ++o;
@@ -653,15 +643,8 @@ namespace abd {
 
 int bsr_structure(hipStream_t s, int nb, const int32_t* ij, const int32_t* ji, int64_t nij, const int64_t* dnij,
                   int32_t* row_ptr, int32_t* cols, int32_t* slots) {
-    int64_t *len, *off;
-    int rc;
-    if ((rc = arena_get(kSlotScanA, sizeof(int64_t) * (nb + 1), (void**)&len))) return rc;
-    if ((rc = arena_get(kSlotScanB, sizeof(int64_t) * (nb + 1), (void**)&off))) return rc;
-    hipLaunchKernelGGL(rowlen_kernel, dim3(grid_for(nb)), dim3(kBlock), 0, s, nb, nij, dnij, ij, ji, len);
-    ABD_CHECK_LAUNCH();
-    if ((rc = scan_exclusive_i64(s, len, off, nb, off + nb))) return rc;
-    hipLaunchKernelGGL(rowfill_kernel, dim3(grid_for(nb)), dim3(kBlock), 0, s, nb, nij, dnij, ij, ji,
-                       (const int64_t*)off, row_ptr, cols, slots);
+    hipLaunchKernelGGL(structure_kernel, dim3(grid_for(nb, kWave, INT32_MAX)), dim3(kWave), 0, s, nb, nij, dnij, ij, ji,
+                       row_ptr, cols, slots);
     ABD_CHECK_LAUNCH();
     return ABD_OK;
 }

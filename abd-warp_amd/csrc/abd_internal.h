@@ -39,7 +39,6 @@ enum ArenaSlot {
     kSlotChunk,
     kSlotChunkCount,
     kSlotContact,
-    kSlotPair,
     kSlotMisc,
     kSlotSolver,
     kSlotSpare,
@@ -57,7 +56,6 @@ enum ArenaSlot {
     kSlotChunkB,
     kSlotVgA,
     kSlotVgB,
-    kSlotPairSeg,  // per body pair and contact type: the active contacts' [begin, end)
     kSlotKeep,     // keep_from_superset: block counts and offsets
     kSlotKeepMap,  // keep_from_superset: old -> new pair index
     kSlotKeepCount,
@@ -195,6 +193,8 @@ struct BodyStart {
     double *g, *blocks;
     double* zero;  // nzero words zeroed
     int64_t nzero;
+    double* zero2;  // nzero2 more
+    int64_t nzero2;
     uint32_t* zero32;  // nzero32 more, of 4 bytes
     int64_t nzero32;
     unsigned long long* slots;  // [ns] set to 1.0
@@ -334,7 +334,10 @@ struct GhLists {
 };
 int contact_gh(hipStream_t s, const AbdScene* sc, const AbdParams* P, const double* x, const GhLists& L,
                const int32_t* row_ptr, const int32_t* slots, double* g, double* blocks, uint8_t* highlight,
-               int64_t* n_active, int64_t* n_active_dev);
+               int64_t* n_active, int64_t* n_active_dev, bool zeroed = false);
+// The words (8 bytes) that a contact_gh over these sizes wants 0; with them zeroed before it it
+// runs with zeroed = true.
+int gh_zero_region(int nb, int64_t nij, int64_t n, void** p, int64_t* words);
 // A set of arena buffers.  The stateless entry points share one per device (process-wide);
 // each simulator owns one, made the calling thread's arena by an ArenaScope for the length
 // of a simulator call, so simulators stepped from different threads or streams never share

@@ -849,6 +849,11 @@ int iteration_scenes(hipStream_t s, Sim& S) {
     U.blocks = S.blocks.p;
     U.zero = S.blocks.p + 144 * (int64_t)nb;
     U.nzero = 2 * 144 * nij;
+    // contact_gh's flags and counters, over the collision set it will take
+    const CandSet& Wn = S.col_fresh ? S.col : S.sw;
+    void* ghz;
+    if ((rc = gh_zero_region(nb, nij, Wn.npt + Wn.nee, &ghz, &U.nzero2))) return rc;
+    U.zero2 = static_cast<double*>(ghz);
     if (S.sup_valid) {  // (else the superset's culling sets them)
         if ((rc = sweep_buffers(S))) return rc;
         U.zero32 = S.kcnt.p;
@@ -873,7 +878,7 @@ int iteration_scenes(hipStream_t s, Sim& S) {
     const CandSet& C = S.col;
     const GhLists GL{C.ptl.p, C.npt, C.eel.p, C.nee, C.vgl.p, C.nvg, C.nij, C.counts()};
     if ((rc = contact_gh(s, &S.sc, &P, st.x, GL, S.row_ptr.p, S.slots.p, st.g, S.blocks.p, nullptr, nullptr,
-                         S.cnt.p + kCntNact)))
+                         S.cnt.p + kCntNact, true)))
         return rc;
     if (ns > 1)
         rc = abd_bsr_solve_scenes(s, P.solver, &S.sc, S.max_scene_bodies, S.row_ptr.p, S.cols.p, S.slots.p,

@@ -295,3 +295,44 @@ def test_ldlt_chunk_edges(kind, m):
     assert st == 1 and int(info.iters[0]) == 1
     assert rel_err(x.cpu().numpy(), ref) <= 1e-14
     assert rel_err(x.cpu().numpy().ravel(), np.linalg.solve(dense, b.ravel())) <= 1e-10
+
+
+@pytest.mark.parametrize("psd,total", [(1, 255), (1, 256), (1, 257), (1, 16385), (1, 40000), (3, 600)])
+def test_gh_over_repeated_candidates(psd, total):
+    """The contact gradient and Hessian over lists in which every candidate is repeated until
+    they pass the edges of the active-candidate blocks (256), super-blocks (16384) and the
+    chunks of a pair's sums (64): n times the sums of the list itself.  Sums of n equal terms:
+    relative error below 2 n 2^-53 plus the bound of the sums, 1e-10 for the sizes here."""
+    import abd_hip
+    from abd_hip.ipc import IPCContactEnergy
+    from test_gpu_parity import T, _gpu_scene, _stage_lists, contact_scene
+    abd_hip.load()
+    spec = contact_scene()
+    cp = params(ground=spec.ground, psd=psd)
+    m = _gpu_scene(spec)
+    sc = O.OracleScene(spec)
+    x = O.project(sc, spec.A, spec.p)
+    m.x.copy_(T(x))
+    m.xk.copy_(T(x))
+    G = _stage_lists(m, cp)
+    nij, nb = len(G["pairs"].ij), spec.n_bodies
+    ipc = IPCContactEnergy(cp)
+    vg = G["vg"][:0]
+
+    def gh(pt, ee):
+        g = torch.zeros((4 * nb, 3), dtype=torch.float64, device="cuda")
+        blocks = torch.zeros(((nb + 2 * nij) * 16, 3, 3), dtype=torch.float64, device="cuda")
+        hl, n = ipc.gh([pt.contiguous(), ee.contiguous(), vg, nij, m, g, blocks], return_active=True)
+        return g.cpu().numpy(), blocks.cpu().numpy(), hl.cpu().numpy(), n
+
+    # only the active candidates (found one at a time from their count), then n of each
+    pt, ee = G["pt"], G["ee"]
+    pt = pt[[k for k in range(len(pt)) if gh(pt[k:k + 1], ee[:0])[3]]]
+    ee = ee[[k for k in range(len(ee)) if gh(pt[:0], ee[k:k + 1])[3]]]
+    assert len(pt) + len(ee) > 2
+    g1, b1, h1, n1 = gh(pt, ee)
+    assert n1 == len(pt) + len(ee)
+    k = -(-total // n1)
+    gk, bk, hk, nk = gh(pt.repeat_interleave(k, 0), ee.repeat_interleave(k, 0))
+    assert nk == k * n1 and np.array_equal(h1, hk)
+    assert rel_err(gk, k * g1) <= 1e-10 and rel_err(bk, k * b1) <= 1e-10
