@@ -241,9 +241,9 @@ int body_start(hipStream_t s, const AbdScene* sc, const AbdParams* P, const Body
     const int64_t extra = std::min<int64_t>(4096, 1 + ceil_div(std::max<int64_t>(words, U.ns), 16 * (int64_t)T));
     const dim3 grid((unsigned)(sc->n_bodies + extra));
     if (small)
-        hipLaunchKernelGGL(body_start_kernel<kWave>, grid, dim3(T), 0, s, *sc, *P, U);
+        launch_kernel(body_start_kernel<kWave>, grid, dim3(T), 0, s, *sc, *P, U);
     else
-        hipLaunchKernelGGL(body_start_kernel<kBlock>, grid, dim3(T), 0, s, *sc, *P, U);
+        launch_kernel(body_start_kernel<kBlock>, grid, dim3(T), 0, s, *sc, *P, U);
     ABD_CHECK_LAUNCH();
     return ABD_OK;
 }
@@ -251,16 +251,16 @@ int body_start(hipStream_t s, const AbdScene* sc, const AbdParams* P, const Body
 int body_end(hipStream_t s, const AbdScene* sc, const BodyEnd& U) {
     if (sc->n_bodies == 0) return ABD_OK;
     if (small_bodies(sc))
-        hipLaunchKernelGGL(body_end_kernel<kWave>, dim3(sc->n_bodies), dim3(kWave), 0, s, *sc, U);
+        launch_kernel(body_end_kernel<kWave>, dim3(sc->n_bodies), dim3(kWave), 0, s, *sc, U);
     else
-        hipLaunchKernelGGL(body_end_kernel<kBlock>, dim3(sc->n_bodies), dim3(kBlock), 0, s, *sc, U);
+        launch_kernel(body_end_kernel<kBlock>, dim3(sc->n_bodies), dim3(kBlock), 0, s, *sc, U);
     ABD_CHECK_LAUNCH();
     return ABD_OK;
 }
 
 int rest_max(hipStream_t s, const AbdScene* sc, double* out, double* copy) {
     if (sc->n_bodies == 0) return ABD_OK;
-    hipLaunchKernelGGL(rest_max_kernel, dim3(sc->n_bodies), dim3(kWave), 0, s, *sc, out, copy);
+    launch_kernel(rest_max_kernel, dim3(sc->n_bodies), dim3(kWave), 0, s, *sc, out, copy);
     ABD_CHECK_LAUNCH();
     return ABD_OK;
 }
@@ -268,7 +268,7 @@ int rest_max(hipStream_t s, const AbdScene* sc, double* out, double* copy) {
 int step_states(hipStream_t s, const AbdScene* sc, const double* A, const double* p, const double* dq,
                 const uint8_t* active, double* qref) {
     if (sc->n_bodies == 0) return ABD_OK;
-    hipLaunchKernelGGL(step_states_kernel, dim3(grid_for(12 * (int64_t)sc->n_bodies, kBlock, INT32_MAX)), dim3(kBlock),
+    launch_kernel(step_states_kernel, dim3(grid_for(12 * (int64_t)sc->n_bodies, kBlock, INT32_MAX)), dim3(kBlock),
                        0, s, sc->n_bodies, sc->n_scenes > 1 ? sc->body_scene : nullptr, A, p, dq, active, qref);
     ABD_CHECK_LAUNCH();
     return ABD_OK;

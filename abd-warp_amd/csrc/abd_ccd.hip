@@ -44,7 +44,7 @@ int abd_cubic_roots(abd_stream_t stream, const double* coef, int64_t n, double x
                     double* roots) {
     if (n < 0 || (n && (!coef || !nroots || !roots))) return ABD_ERR_ARG;
     if (n == 0) return ABD_OK;
-    hipLaunchKernelGGL(cubic_roots_kernel, dim3(grid_for(n, kBlock, INT32_MAX)), dim3(kBlock), 0, to_stream(stream),
+    launch_kernel(cubic_roots_kernel, dim3(grid_for(n, kBlock, INT32_MAX)), dim3(kBlock), 0, to_stream(stream),
                        coef, n, x0, x1, nroots, roots);
     ABD_CHECK_LAUNCH();
     return ABD_OK;
@@ -54,7 +54,7 @@ int abd_collision_time(abd_stream_t stream, int32_t kind, const double* p_t0, co
                        double* t) {
     if (n < 0 || (kind != 0 && kind != 1) || (n && (!p_t0 || !p_t1 || !t))) return ABD_ERR_ARG;
     if (n == 0) return ABD_OK;
-    hipLaunchKernelGGL(collision_time_kernel, dim3(grid_for(n, kBlock, INT32_MAX)), dim3(kBlock), 0,
+    launch_kernel(collision_time_kernel, dim3(grid_for(n, kBlock, INT32_MAX)), dim3(kBlock), 0,
                        to_stream(stream), kind, p_t0, p_t1, n, t);
     ABD_CHECK_LAUNCH();
     return ABD_OK;

@@ -17,7 +17,8 @@ constexpr int kMaxDevices = 64;
 Arena g_arena[kMaxDevices];
 std::mutex g_arena_mutex;
 thread_local Arena* t_arena = nullptr;  // a simulator's own arena during its calls
-thread_local bool t_capturing = false;    // this thread is recording a HIP graph
+thread_local hipGraph_t t_graph = nullptr;      // the graph this thread records
+thread_local hipGraphNode_t t_node = nullptr;   // its last node
 std::atomic<uint64_t> g_alloc_gen{1};
 
 int current_device(int* dev) {
@@ -39,8 +40,34 @@ ArenaScope::~ArenaScope() { t_arena = prev_; }
 
 uint64_t alloc_generation() { return g_alloc_gen.load(std::memory_order_relaxed); }
 void note_reallocation() { g_alloc_gen.fetch_add(1, std::memory_order_relaxed); }
-void set_capturing(bool on) { t_capturing = on; }
-bool capturing() { return t_capturing; }
+void graph_record(hipGraph_t g) {
+    t_graph = g;
+    t_node = nullptr;
+}
+bool capturing() { return t_graph != nullptr; }
+int graph_add_kernel(const void* f, dim3 grid, dim3 block, void** args, size_t lds) {
+    hipKernelNodeParams p{};
+    p.func = const_cast<void*>(f);
+    p.gridDim = grid;
+    p.blockDim = block;
+    p.kernelParams = args;
+    p.sharedMemBytes = (unsigned)lds;
+    hipGraphNode_t node = nullptr;
+    ABD_CHECK(hipGraphAddKernelNode(&node, t_graph, t_node ? &t_node : nullptr, t_node ? 1 : 0, &p));
+    t_node = node;
+    return ABD_OK;
+}
+int copy_to_host(hipStream_t s, void* dst, const void* src, size_t bytes) {
+    if (!capturing()) {
+        ABD_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s));
+        return ABD_OK;
+    }
+    hipGraphNode_t node = nullptr;
+    ABD_CHECK(hipGraphAddMemcpyNode1D(&node, t_graph, t_node ? &t_node : nullptr, t_node ? 1 : 0, dst, src, bytes,
+                                      hipMemcpyDeviceToHost));
+    t_node = node;
+    return ABD_OK;
+}
 
 int arena_get(int slot, size_t bytes, void** ptr) {
     int dev;
@@ -51,7 +78,7 @@ int arena_get(int slot, size_t bytes, void** ptr) {
     Arena& A = t_arena ? *t_arena : g_arena[dev];
     if (bytes == 0) bytes = 256;
     if (A.size[slot] < bytes) {
-        if (t_capturing) return ABD_ERR_CAPACITY;  // no allocation inside a recorded graph
+        if (capturing()) return ABD_ERR_CAPACITY;  // no allocation inside a recorded graph
         note_reallocation();
         size_t want = bytes + bytes / 2;
         want = (want + 255) & ~size_t(255);
@@ -82,7 +109,7 @@ int arena_host(size_t bytes, void** ptr) {
     if (!t_arena) lock.lock();
     Arena& A = t_arena ? *t_arena : g_arena[dev];
     if (A.host_size < bytes) {
-        if (t_capturing) return ABD_ERR_CAPACITY;
+        if (capturing()) return ABD_ERR_CAPACITY;
         note_reallocation();
         if (A.host) {
             ABD_CHECK(hipDeviceSynchronize());
@@ -127,7 +154,7 @@ int zero_fill(hipStream_t s, void* p, size_t bytes) {
     if (bytes % 8 || ((uintptr_t)p & 7)) return ABD_ERR_ARG;
     const int64_t n = (int64_t)(bytes / 8);
     if (n == 0) return ABD_OK;
-    hipLaunchKernelGGL(zero_words_kernel, dim3(grid_for(n, kBlock, 1 << 16)), dim3(kBlock), 0, s, (uint64_t*)p, n);
+    launch_kernel(zero_words_kernel, dim3(grid_for(n, kBlock, 1 << 16)), dim3(kBlock), 0, s, (uint64_t*)p, n);
     ABD_CHECK_LAUNCH();
     return ABD_OK;
 }
@@ -160,13 +187,13 @@ int scan_exclusive_i64_multi(hipStream_t s, const ScanSeg* segs, int nseg) {
     if (nseg == 0) return ABD_OK;
     ScanSegs S;
     for (int k = 0; k < nseg; ++k) S.s[k] = segs[k];
-    hipLaunchKernelGGL(scan_i64_multi_kernel, dim3(nseg), dim3(kScanThreads), 0, s, S);
+    launch_kernel(scan_i64_multi_kernel, dim3(nseg), dim3(kScanThreads), 0, s, S);
     ABD_CHECK_LAUNCH();
     return ABD_OK;
 }
 
 int scan_exclusive_i64(hipStream_t s, const int64_t* in, int64_t* out, int64_t n, int64_t* total, int64_t* total2) {
-    hipLaunchKernelGGL(scan_i64_kernel, dim3(1), dim3(kScanThreads), 0, s, in, out, n, total, total2);
+    launch_kernel(scan_i64_kernel, dim3(1), dim3(kScanThreads), 0, s, in, out, n, total, total2);
     ABD_CHECK_LAUNCH();
     return ABD_OK;
 }

@@ -981,14 +981,14 @@ int contact_gh(hipStream_t s, const AbdScene* sc, const AbdParams* P, const doub
         if ((rc = arena_get(kSlotScanA, sizeof(uint32_t) * ((size_t)nblk + 1), (void**)&bcnt))) return rc;
         int ph = prof_start(kProfClassify, s, dn ? 1.0 : 129.0 * npt + 133.0 * nee + 8.0 * nvg);
         const int64_t blocks_all = nblk + ceil_div(nvg, (int64_t)kBlock);
-        hipLaunchKernelGGL(classify_kernel, dim3((unsigned)std::min<int64_t>(blocks_all, 8192)), dim3(kBlock), 0, s, *sc, *P, x,
+        launch_kernel(classify_kernel, dim3((unsigned)std::min<int64_t>(blocks_all, 8192)), dim3(kBlock), 0, s, *sc, *P, x,
                            pt, npt, ee, nee, vg, nvg, dn, flag, G.err, bcnt, G.scnt);
         ABD_CHECK_LAUNCH();
         prof_stop(ph, s);
         if ((rc = prof_count_bytes(ph, s, dn, 129.0, 133.0, 8.0, 0.0))) return rc;
     }
     const auto total_now = [&]() -> int {  // the active count for the host
-        hipLaunchKernelGGL(active_total_kernel, dim3(1), dim3(kBlock), 0, s, (const uint32_t*)G.scnt, G.nsup,
+        launch_kernel(active_total_kernel, dim3(1), dim3(kBlock), 0, s, (const uint32_t*)G.scnt, G.nsup,
                            G.total);
         ABD_CHECK_LAUNCH();
         return ABD_OK;
@@ -1045,18 +1045,18 @@ int contact_gh(hipStream_t s, const AbdScene* sc, const AbdParams* P, const doub
         if (dense) {
             int32_t* act;
             if ((rc = arena_get(kSlotList, sizeof(int32_t) * (size_t)n, (void**)&act))) return rc;
-            hipLaunchKernelGGL(compact_flags_kernel, dim3((unsigned)std::min(nblk, kActiveGrid)), dim3(kBlock), 0, s, A,
+            launch_kernel(compact_flags_kernel, dim3((unsigned)std::min(nblk, kActiveGrid)), dim3(kBlock), 0, s, A,
                                act);
             ABD_CHECK_LAUNCH();
             const dim3 dgrid((unsigned)std::min<int64_t>(nact, kDenseGrid));
             if (P->psd == 3)
-                hipLaunchKernelGGL(contact_dense_kernel<3>, dgrid, dim3(kWave), 0, s, *sc, *P, x, pt, npt, ee,
+                launch_kernel(contact_dense_kernel<3>, dgrid, dim3(kWave), 0, s, *sc, *P, x, pt, npt, ee,
                                    (const int32_t*)act, nact, dnact, dn, O);
             else
-                hipLaunchKernelGGL(contact_dense_kernel<2>, dgrid, dim3(kWave), 0, s, *sc, *P, x, pt, npt, ee,
+                launch_kernel(contact_dense_kernel<2>, dgrid, dim3(kWave), 0, s, *sc, *P, x, pt, npt, ee,
                                    (const int32_t*)act, nact, dnact, dn, O);
         } else {
-            hipLaunchKernelGGL(contact_kernel, dim3((unsigned)std::min(nblk, kActiveGrid)), dim3(kBlock), 0, s, *sc, *P, x,
+            launch_kernel(contact_kernel, dim3((unsigned)std::min(nblk, kActiveGrid)), dim3(kBlock), 0, s, *sc, *P, x,
                                pt, npt, ee, A, O);
         }
         ABD_CHECK_LAUNCH();
@@ -1079,7 +1079,7 @@ int contact_gh(hipStream_t s, const AbdScene* sc, const AbdParams* P, const doub
         pitem = I.pitem;
         if ((rc = arena_get(kSlotPairPart, sizeof(double) * kPartStride * (size_t)cap_items, (void**)&part)))
             return rc;
-        hipLaunchKernelGGL(pair_items_kernel, dim3(grid_for(nij, kBlock)), dim3(kBlock), 0, s, nij, dn,
+        launch_kernel(pair_items_kernel, dim3(grid_for(nij, kBlock)), dim3(kBlock), 0, s, nij, dn,
                            (const uint8_t*)G.pflag, (const unsigned long long*)G.pseg, nij, I);
         ABD_CHECK_LAUNCH();
         // timed: the partial sums (each stored contact read once, its body-order flag once)
@@ -1096,7 +1096,7 @@ int contact_gh(hipStream_t s, const AbdScene* sc, const AbdParams* P, const doub
     const double fbytes = 2.0 * 8 * 156 * nb;
     const double pbytes = 8.0 * 2 * 312;  // a pair's partial sums, read by both bodies (one chunk)
     int phf = prof_start(kProfBodyFinalize, s, dn ? 1.0 : fbytes + pbytes * nij + 40.0 * nvg);
-    hipLaunchKernelGGL(body_finalize_kernel, dim3(nb), dim3(kBlock), 0, s, *sc, *P, x, nij, dn, row_ptr, slots,
+    launch_kernel(body_finalize_kernel, dim3(nb), dim3(kBlock), 0, s, *sc, *P, x, nij, dn, row_ptr, slots,
                        (const uint8_t*)G.pflag, (const int2*)pitem, (const double*)part, vg, nvg, g, blocks,
                        (const uint8_t*)G.hl_pt, (const uint8_t*)G.hl_ee, highlight, nact_unwritten);
     ABD_CHECK_LAUNCH();
@@ -1142,10 +1142,10 @@ int abd_pair_gh(abd_stream_t stream, int32_t kind, const AbdParams* P, const dou
     int rc = arena_get(kSlotContact, sizeof(double) * stride * (size_t)n, (void**)&scratch);
     if (rc) return rc;
     if (P->psd >= 2)
-        hipLaunchKernelGGL(pair_gh_dense_kernel, dim3((unsigned)std::min<int64_t>(n, kDenseGrid)), dim3(kWave), 0,
+        launch_kernel(pair_gh_dense_kernel, dim3((unsigned)std::min<int64_t>(n, kDenseGrid)), dim3(kWave), 0,
                            to_stream(stream), kind, *P, x4, r4, n, active, g24, H24, scratch);
     else
-        hipLaunchKernelGGL(pair_gh_kernel, dim3(grid_for(n)), dim3(kBlock), 0, to_stream(stream), kind, *P, x4, r4, n,
+        launch_kernel(pair_gh_kernel, dim3(grid_for(n)), dim3(kBlock), 0, to_stream(stream), kind, *P, x4, r4, n,
                            active, g24, H24, scratch);
     ABD_CHECK_LAUNCH();
     return ABD_OK;
@@ -1156,7 +1156,7 @@ int abd_inertia_gradient(abd_stream_t stream, const AbdScene* sc, const AbdParam
     if (!sc || !P || !A || !p || !A0 || !p0 || !Adot || !pdot || !g) return ABD_ERR_ARG;
     const int nb = sc->n_bodies;
     if (!nb) return ABD_OK;
-    hipLaunchKernelGGL(inertia_gradient_kernel, dim3(grid_for(nb)), dim3(kBlock), 0, to_stream(stream), nb, *P,
+    launch_kernel(inertia_gradient_kernel, dim3(grid_for(nb)), dim3(kBlock), 0, to_stream(stream), nb, *P,
                        sc->mass, sc->I0, A, p, A0, p0, Adot, pdot, g);
     ABD_CHECK_LAUNCH();
     return ABD_OK;
@@ -1167,7 +1167,7 @@ int abd_inertia_hessian(abd_stream_t stream, const AbdScene* sc, const AbdParams
     if (!sc || !P || !A || !blocks) return ABD_ERR_ARG;
     const int nb = sc->n_bodies;
     if (!nb) return ABD_OK;
-    hipLaunchKernelGGL(inertia_hessian_kernel, dim3(grid_for(16 * (int64_t)nb)), dim3(kBlock), 0, to_stream(stream),
+    launch_kernel(inertia_hessian_kernel, dim3(grid_for(16 * (int64_t)nb)), dim3(kBlock), 0, to_stream(stream),
                        nb, *P, sc->mass, sc->I0, A, blocks);
     ABD_CHECK_LAUNCH();
     return ABD_OK;

@@ -432,7 +432,7 @@ int prim_cull_begin(hipStream_t s, const AbdScene* sc, int mode, const int32_t* 
     }
     if (nb > 0) {
         const HullSet H1{S.off1, lo1, hi1, h1, h1 + 3 * nb}, H2{S.off2, lo2, hi2, h2, h2 + 3 * nb};
-        hipLaunchKernelGGL(hull_kernel, dim3((unsigned)ceil_div(nb, kBlock / kWave), same ? 1 : 2), dim3(kBlock), 0,
+        launch_kernel(hull_kernel, dim3((unsigned)ceil_div(nb, kBlock / kWave), same ? 1 : 2), dim3(kBlock), 0,
                            s, nb, H1, H2);
         ABD_CHECK_LAUNCH();
     }
@@ -441,12 +441,12 @@ int prim_cull_begin(hipStream_t s, const AbdScene* sc, int mode, const int32_t* 
     if ((rc = arena_get(slot[4], sizeof(int64_t) * (size_t)(C.nunits + 1), (void**)&C.nchunk))) return rc;
     if ((rc = arena_get(slot[5], sizeof(int64_t) * (size_t)(C.nunits + 1), (void**)&C.choff))) return rc;
     int ph = prof_start(kProfFilter, s, 0.0);
-    hipLaunchKernelGGL(filter_kernel, dim3((unsigned)(2 * C.nunits)), dim3(kBlock), 0, s, C.pt, ij, S, C.maxs,
+    launch_kernel(filter_kernel, dim3((unsigned)(2 * C.nunits)), dim3(kBlock), 0, s, C.pt, ij, S, C.maxs,
                        C.flist, C.fcnt);
     ABD_CHECK_LAUNCH();
     prof_stop(ph, s);
     C.tune = tuning();
-    hipLaunchKernelGGL(unit_chunks_kernel, dim3(grid_for(C.nunits)), dim3(kBlock), 0, s, C.nunits, C.tune.cull_chunk,
+    launch_kernel(unit_chunks_kernel, dim3(grid_for(C.nunits)), dim3(kBlock), 0, s, C.nunits, C.tune.cull_chunk,
                        C.fcnt, C.nchunk);
     ABD_CHECK_LAUNCH();
     if ((rc = scan_exclusive_i64(s, C.nchunk, C.choff, C.nunits, C.choff + C.nunits, total_copy))) return rc;
@@ -464,7 +464,7 @@ int prim_cull_count(hipStream_t s, PrimCull& C, int64_t T, int64_t* total_copy) 
     if ((rc = arena_get(slot[7], sizeof(int64_t) * (size_t)(T + 1), (void**)&C.ccoff))) return rc;
     C.grid = (unsigned)(T < C.tune.cull_grid ? T : C.tune.cull_grid);
     int ph = prof_start(kProfPrimCount, s, 0.0);
-    hipLaunchKernelGGL(prim_pairs_kernel<false>, dim3(C.grid), dim3(kBlock), 0, s, C.pt, C.tune.cull_chunk, C.ij, C.S,
+    launch_kernel(prim_pairs_kernel<false>, dim3(C.grid), dim3(kBlock), 0, s, C.pt, C.tune.cull_chunk, C.ij, C.S,
                        C.maxs, (const int32_t*)C.flist, (const int64_t*)C.fcnt, (const int64_t*)C.choff, C.nunits,
                        (const int64_t*)C.total_chunks, C.ccnt, (const int64_t*)nullptr, (int32_t*)nullptr, (int64_t)0);
     ABD_CHECK_LAUNCH();
@@ -477,7 +477,7 @@ int prim_cull_count(hipStream_t s, PrimCull& C, int64_t T, int64_t* total_copy) 
 int prim_cull_fill(hipStream_t s, PrimCull& C, int32_t* out, int64_t cap, int64_t n) {
     if (C.T == 0 || n == 0) return ABD_OK;
     int ph = prof_start(kProfPrimFill, s, 20.0 * n);
-    hipLaunchKernelGGL(prim_pairs_kernel<true>, dim3(C.grid), dim3(kBlock), 0, s, C.pt, C.tune.cull_chunk, C.ij, C.S,
+    launch_kernel(prim_pairs_kernel<true>, dim3(C.grid), dim3(kBlock), 0, s, C.pt, C.tune.cull_chunk, C.ij, C.S,
                        C.maxs, (const int32_t*)C.flist, (const int64_t*)C.fcnt, (const int64_t*)C.choff, C.nunits,
                        (const int64_t*)C.total_chunks, C.ccnt, (const int64_t*)C.ccoff, out, cap);
     ABD_CHECK_LAUNCH();
@@ -502,7 +502,7 @@ int vg_cull_begin(hipStream_t s, const AbdScene* sc, const float* blo, const flo
     if ((rc = arena_get(kSlotVgA, sizeof(int64_t) * (C.nblk + 1), (void**)&C.bcnt))) return rc;
     if ((rc = arena_get(kSlotVgB, sizeof(int64_t) * (C.nblk + 1), (void**)&C.boff))) return rc;
     int ph = prof_start(kProfVg, s, 28.0 * nv);
-    hipLaunchKernelGGL(vg_kernel<false>, dim3((unsigned)C.nblk), dim3(kBlock), 0, s, nv, sc->vert_body, sc->voff, blo,
+    launch_kernel(vg_kernel<false>, dim3((unsigned)C.nblk), dim3(kBlock), 0, s, nv, sc->vert_body, sc->voff, blo,
                        plo, phi, C.yth, C.fg, C.bcnt, (const int64_t*)nullptr, (int32_t*)nullptr, (int64_t)0);
     ABD_CHECK_LAUNCH();
     prof_stop(ph, s);
@@ -514,7 +514,7 @@ int vg_cull_begin(hipStream_t s, const AbdScene* sc, const float* blo, const flo
 int vg_cull_fill(hipStream_t s, VgCull& C, int32_t* out, int64_t cap, int64_t n) {
     if (n == 0 || !C.total) return ABD_OK;
     const AbdScene* sc = C.sc;
-    hipLaunchKernelGGL(vg_kernel<true>, dim3((unsigned)C.nblk), dim3(kBlock), 0, s, (int64_t)sc->n_verts,
+    launch_kernel(vg_kernel<true>, dim3((unsigned)C.nblk), dim3(kBlock), 0, s, (int64_t)sc->n_verts,
                        sc->vert_body, sc->voff, C.blo, C.plo, C.phi, C.yth, C.fg, C.bcnt, (const int64_t*)C.boff, out,
                        cap);
     ABD_CHECK_LAUNCH();
@@ -541,7 +541,7 @@ int cull_bodies(hipStream_t s, const AbdScene* sc, const float* lo, const float*
     rc = arena_get(kSlotScanB, sizeof(int64_t) * (nblk + 1), (void**)&boff);
     if (rc) return rc;
     int ph = prof_start(kProfBodyPairs, s, 24.0 * nb);
-    hipLaunchKernelGGL(body_pairs_kernel<false>, dim3((unsigned)nblk), dim3(kBlock), 0, s, nb, npairs, 0, sg,
+    launch_kernel(body_pairs_kernel<false>, dim3((unsigned)nblk), dim3(kBlock), 0, s, nb, npairs, 0, sg,
                        sc->body_scene, lo, hi, bcnt, (const int64_t*)nullptr, (int32_t*)nullptr, (int64_t)0);
     ABD_CHECK_LAUNCH();
     prof_stop(ph, s);
@@ -551,16 +551,16 @@ int cull_bodies(hipStream_t s, const AbdScene* sc, const float* lo, const float*
     *count = n;
     if (n > cap) return ABD_ERR_OVERFLOW;
     if (n == 0) return ABD_OK;
-    hipLaunchKernelGGL(body_pairs_kernel<true>, dim3((unsigned)nblk), dim3(kBlock), 0, s, nb, npairs, 0, sg,
+    launch_kernel(body_pairs_kernel<true>, dim3((unsigned)nblk), dim3(kBlock), 0, s, nb, npairs, 0, sg,
                        sc->body_scene, lo, hi, bcnt, (const int64_t*)boff, ij, cap);
     ABD_CHECK_LAUNCH();
     if (!ji) return ABD_OK;
     // (j, i) order: same predicate, second enumeration
-    hipLaunchKernelGGL(body_pairs_kernel<false>, dim3((unsigned)nblk), dim3(kBlock), 0, s, nb, npairs, 1, sg,
+    launch_kernel(body_pairs_kernel<false>, dim3((unsigned)nblk), dim3(kBlock), 0, s, nb, npairs, 1, sg,
                        sc->body_scene, lo, hi, bcnt, (const int64_t*)nullptr, (int32_t*)nullptr, (int64_t)0);
     ABD_CHECK_LAUNCH();
     if ((rc = scan_exclusive_i64(s, bcnt, boff, nblk, boff + nblk))) return rc;
-    hipLaunchKernelGGL(body_pairs_kernel<true>, dim3((unsigned)nblk), dim3(kBlock), 0, s, nb, npairs, 1, sg,
+    launch_kernel(body_pairs_kernel<true>, dim3((unsigned)nblk), dim3(kBlock), 0, s, nb, npairs, 1, sg,
                        sc->body_scene, lo, hi, bcnt, (const int64_t*)boff, ji, cap);
     ABD_CHECK_LAUNCH();
     return ABD_OK;
@@ -625,7 +625,7 @@ int abd_set_triplets(abd_stream_t stream, int32_t nb, const int32_t* ij, int64_t
     if (nb < 0 || nij < 0 || (nij > 0 && !ij) || !rows || !cols) return ABD_ERR_ARG;
     int64_t n = 16 * ((int64_t)nb + 2 * nij);
     if (n == 0) return ABD_OK;
-    hipLaunchKernelGGL(triplets_kernel, dim3(grid_for(n, kBlock, INT32_MAX)), dim3(kBlock), 0, to_stream(stream), nb,
+    launch_kernel(triplets_kernel, dim3(grid_for(n, kBlock, INT32_MAX)), dim3(kBlock), 0, to_stream(stream), nb,
                        nij, ij, rows, cols);
     ABD_CHECK_LAUNCH();
     return ABD_OK;
@@ -643,7 +643,7 @@ namespace abd {
 
 int bsr_structure(hipStream_t s, int nb, const int32_t* ij, const int32_t* ji, int64_t nij, const int64_t* dnij,
                   int32_t* row_ptr, int32_t* cols, int32_t* slots) {
-    hipLaunchKernelGGL(structure_kernel, dim3(grid_for(nb, kWave, INT32_MAX)), dim3(kWave), 0, s, nb, nij, dnij, ij, ji,
+    launch_kernel(structure_kernel, dim3(grid_for(nb, kWave, INT32_MAX)), dim3(kWave), 0, s, nb, nij, dnij, ij, ji,
                        row_ptr, cols, slots);
     ABD_CHECK_LAUNCH();
     return ABD_OK;
@@ -1152,7 +1152,7 @@ __global__ __launch_bounds__(kBlock) void cand_vid_kernel(SceneView V, int kind,
 int cand_vertex_ids(hipStream_t s, const AbdScene* sc, int kind, const int32_t* tuples, int64_t n, int32_t* vid) {
     if (n <= 0) return ABD_OK;
     const SceneView V{sc->voff, sc->foff, sc->eoff, sc->tris, sc->edges, sc->x0};
-    hipLaunchKernelGGL(cand_vid_kernel, dim3(grid_for(n, kBlock, 1 << 16)), dim3(kBlock), 0, s, V, kind, tuples, n, vid);
+    launch_kernel(cand_vid_kernel, dim3(grid_for(n, kBlock, 1 << 16)), dim3(kBlock), 0, s, V, kind, tuples, n, vid);
     ABD_CHECK_LAUNCH();
     return ABD_OK;
 }
@@ -1223,11 +1223,11 @@ int keep_from_superset(hipStream_t s, const AbdScene* sc, const KeepInput& in, c
     if ((rc = arena_get(kSlotKeepFlags, (size_t)nflag + 1, (void**)&A.flag))) return rc;
     const int ph = prof_start(kProfKeep, s, 0.0);
     if (nall > 0) {
-        hipLaunchKernelGGL(keep_count_kernel, dim3((unsigned)nall), dim3(kBlock), 0, s, A);
+        launch_kernel(keep_count_kernel, dim3((unsigned)nall), dim3(kBlock), 0, s, A);
         ABD_CHECK_LAUNCH();
     }
     if (scan) {
-        hipLaunchKernelGGL(keep_pair_scan_kernel, dim3(1), dim3(kScanThreads), 0, s, (const uint32_t*)A.bcnt[0],
+        launch_kernel(keep_pair_scan_kernel, dim3(1), dim3(kScanThreads), 0, s, (const uint32_t*)A.bcnt[0],
                            nblk[0], pair_off);
         ABD_CHECK_LAUNCH();
     }
@@ -1240,13 +1240,13 @@ int keep_from_superset(hipStream_t s, const AbdScene* sc, const KeepInput& in, c
         // bytes: per superset entry (an upper bound of the kept ones) the CCD's tuple, ids and
         // vertices at both ends
         const int phw = prof_start(kProfToi, s, 228.0 * in.nee + 224.0 * in.npt + 56.0 * in.nvg);
-        hipLaunchKernelGGL(sweep_write_kernel, dim3((unsigned)std::max<int64_t>(A.grp0[kKeepLists], 1)),
+        launch_kernel(sweep_write_kernel, dim3((unsigned)std::max<int64_t>(A.grp0[kKeepLists], 1)),
                            dim3(kBlock), 0, s, A);
         ABD_CHECK_LAUNCH();
         prof_stop(phw, s);
     } else {
         const int phw = prof_start(kProfKeep, s, 0.0);
-        hipLaunchKernelGGL(keep_write_kernel, dim3((unsigned)std::max<int64_t>(nall, 1)), dim3(kBlock), 0, s, A);
+        launch_kernel(keep_write_kernel, dim3((unsigned)std::max<int64_t>(nall, 1)), dim3(kBlock), 0, s, A);
         ABD_CHECK_LAUNCH();
         prof_stop(phw, s);
     }

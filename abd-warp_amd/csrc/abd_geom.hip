@@ -272,7 +272,7 @@ __global__ void update_q_scenes_kernel(int nb, const int32_t* __restrict__ body_
 int update_q_dual(hipStream_t s, int nb, const double* A, const double* p, const double* dq, double alpha,
                   double* A_out, double* p_out, double* A_out2, double* p_out2) {
     if (nb == 0) return ABD_OK;
-    hipLaunchKernelGGL(update_q_kernel, dim3(grid_for(12 * (int64_t)nb)), dim3(kBlock), 0, s, nb, A, p, dq, alpha,
+    launch_kernel(update_q_kernel, dim3(grid_for(12 * (int64_t)nb)), dim3(kBlock), 0, s, nb, A, p, dq, alpha,
                        A_out, p_out, A_out2, p_out2);
     ABD_CHECK_LAUNCH();
     return ABD_OK;
@@ -282,7 +282,7 @@ int update_q_scenes_dual(hipStream_t s, const AbdScene* sc, const double* A, con
                          const double* alpha, double* A_out, double* p_out, double* A_out2, double* p_out2) {
     const int nb = sc->n_bodies;
     if (nb == 0) return ABD_OK;
-    hipLaunchKernelGGL(update_q_scenes_kernel, dim3(grid_for(12 * (int64_t)nb)), dim3(kBlock), 0, s, nb,
+    launch_kernel(update_q_scenes_kernel, dim3(grid_for(12 * (int64_t)nb)), dim3(kBlock), 0, s, nb,
                        sc->n_scenes > 1 ? sc->body_scene : nullptr, A, p, dq, alpha, A_out, p_out, A_out2, p_out2);
     ABD_CHECK_LAUNCH();
     return ABD_OK;
@@ -313,7 +313,7 @@ __global__ __launch_bounds__(kBlock) void within_ranges_kernel(int64_t n3, const
 int vertex_ranges(hipStream_t s, int64_t n3, const double* x0, const double* x1, double skin, double* lo,
                   double* hi) {
     if (n3 <= 0) return ABD_OK;
-    hipLaunchKernelGGL(vertex_ranges_kernel, dim3(grid_for(n3)), dim3(kBlock), 0, s, n3, x0, x1, skin, lo, hi);
+    launch_kernel(vertex_ranges_kernel, dim3(grid_for(n3)), dim3(kBlock), 0, s, n3, x0, x1, skin, lo, hi);
     ABD_CHECK_LAUNCH();
     return ABD_OK;
 }
@@ -321,7 +321,7 @@ int vertex_ranges(hipStream_t s, int64_t n3, const double* x0, const double* x1,
 int within_ranges(hipStream_t s, int64_t n3, const double* x, const double* lo, const double* hi, double margin,
                   const double* r, const double* r0, int64_t* flag) {
     if (n3 <= 0) return ABD_OK;
-    hipLaunchKernelGGL(within_ranges_kernel, dim3(grid_for(n3, kBlock, 4096)), dim3(kBlock), 0, s, n3, x, lo, hi,
+    launch_kernel(within_ranges_kernel, dim3(grid_for(n3, kBlock, 4096)), dim3(kBlock), 0, s, n3, x, lo, hi,
                        margin, r, r0, flag);
     ABD_CHECK_LAUNCH();
     return ABD_OK;
@@ -331,19 +331,19 @@ int swept_boxes(hipStream_t s, const AbdScene* sc, int kind, const double* x0, c
                 float* lo, float* hi) {
     if (kind == ABD_KIND_POINT) {
         if (!sc->n_verts) return ABD_OK;
-        hipLaunchKernelGGL(swept_point_boxes_kernel, dim3(grid_for(3 * (int64_t)sc->n_verts)), dim3(kBlock), 0, s, x0,
+        launch_kernel(swept_point_boxes_kernel, dim3(grid_for(3 * (int64_t)sc->n_verts)), dim3(kBlock), 0, s, x0,
                            x1, (int64_t)sc->n_verts, (float)dil, lo, hi);
     } else if (kind == ABD_KIND_EDGE) {
         if (!sc->n_edges) return ABD_OK;
-        hipLaunchKernelGGL(swept_prim_boxes_kernel<2>, dim3(grid_for(sc->n_edges)), dim3(kBlock), 0, s,
+        launch_kernel(swept_prim_boxes_kernel<2>, dim3(grid_for(sc->n_edges)), dim3(kBlock), 0, s,
                            sc->edge_body, sc->voff, sc->edges, x0, x1, (int64_t)sc->n_edges, dil, lo, hi);
     } else if (kind == ABD_KIND_TRI) {
         if (!sc->n_tris) return ABD_OK;
-        hipLaunchKernelGGL(swept_prim_boxes_kernel<3>, dim3(grid_for(sc->n_tris)), dim3(kBlock), 0, s, sc->tri_body,
+        launch_kernel(swept_prim_boxes_kernel<3>, dim3(grid_for(sc->n_tris)), dim3(kBlock), 0, s, sc->tri_body,
                            sc->voff, sc->tris, x0, x1, (int64_t)sc->n_tris, dil, lo, hi);
     } else if (kind == -1) {
         if (!sc->n_bodies) return ABD_OK;
-        hipLaunchKernelGGL(swept_body_boxes_kernel, dim3((unsigned)ceil_div(sc->n_bodies, kBlock / kWave)),
+        launch_kernel(swept_body_boxes_kernel, dim3((unsigned)ceil_div(sc->n_bodies, kBlock / kWave)),
                            dim3(kBlock), 0, s, sc->n_bodies, sc->voff, x0, x1, dil, lo, hi);
     } else {
         return ABD_ERR_ARG;
@@ -362,7 +362,7 @@ int abd_project_vertices(abd_stream_t stream, const AbdScene* sc, const double* 
     if (!sc || !A || !p || !x) return ABD_ERR_ARG;
     if (sc->n_verts == 0) return ABD_OK;
     int ph = prof_start(kProfProject, to_stream(stream), 52.0 * sc->n_verts + 96.0 * sc->n_bodies);
-    hipLaunchKernelGGL(project_kernel, dim3(grid_for(sc->n_verts)), dim3(kBlock), 0, to_stream(stream),
+    launch_kernel(project_kernel, dim3(grid_for(sc->n_verts)), dim3(kBlock), 0, to_stream(stream),
                        sc->vert_body, sc->x0, A, p, x, (int64_t)sc->n_verts);
     ABD_CHECK_LAUNCH();
     prof_stop(ph, to_stream(stream));
@@ -380,7 +380,7 @@ int abd_update_q0qdot(abd_stream_t stream, int32_t nb, double dt, const double* 
                       double* p0, double* Adot, double* pdot) {
     if (nb < 0 || !A || !p || !A0 || !p0 || !Adot || !pdot) return ABD_ERR_ARG;
     if (nb == 0) return ABD_OK;
-    hipLaunchKernelGGL(update_q0qdot_kernel, dim3(grid_for(12 * (int64_t)nb)), dim3(kBlock), 0, to_stream(stream),
+    launch_kernel(update_q0qdot_kernel, dim3(grid_for(12 * (int64_t)nb)), dim3(kBlock), 0, to_stream(stream),
                        nb, dt, A, p, A0, p0, Adot, pdot);
     ABD_CHECK_LAUNCH();
     return ABD_OK;
@@ -400,13 +400,13 @@ int abd_prim_boxes(abd_stream_t stream, const AbdScene* sc, int32_t kind, const 
     if (nprim == 0) return ABD_OK;
     int ph = prof_start(kProfBoxes, s, bytes);
     if (kind == ABD_KIND_POINT) {
-        hipLaunchKernelGGL(point_boxes_kernel, dim3(grid_for(3 * (int64_t)sc->n_verts)), dim3(kBlock), 0, s, x,
+        launch_kernel(point_boxes_kernel, dim3(grid_for(3 * (int64_t)sc->n_verts)), dim3(kBlock), 0, s, x,
                            (int64_t)sc->n_verts, (float)dil, lo, hi);
     } else if (kind == ABD_KIND_EDGE) {
-        hipLaunchKernelGGL(prim_boxes_kernel<2>, dim3(grid_for(sc->n_edges)), dim3(kBlock), 0, s, sc->edge_body,
+        launch_kernel(prim_boxes_kernel<2>, dim3(grid_for(sc->n_edges)), dim3(kBlock), 0, s, sc->edge_body,
                            sc->voff, sc->edges, x, (int64_t)sc->n_edges, dil, lo, hi);
     } else {
-        hipLaunchKernelGGL(prim_boxes_kernel<3>, dim3(grid_for(sc->n_tris)), dim3(kBlock), 0, s, sc->tri_body,
+        launch_kernel(prim_boxes_kernel<3>, dim3(grid_for(sc->n_tris)), dim3(kBlock), 0, s, sc->tri_body,
                            sc->voff, sc->tris, x, (int64_t)sc->n_tris, dil, lo, hi);
     }
     ABD_CHECK_LAUNCH();
@@ -420,15 +420,15 @@ int abd_prim_boxes_traj(abd_stream_t stream, const AbdScene* sc, int32_t kind, c
     hipStream_t s = to_stream(stream);
     if (kind == ABD_KIND_POINT) {
         if (!sc->n_verts) return ABD_OK;
-        hipLaunchKernelGGL(point_traj_kernel, dim3(grid_for(3 * (int64_t)sc->n_verts)), dim3(kBlock), 0, s, x_end,
+        launch_kernel(point_traj_kernel, dim3(grid_for(3 * (int64_t)sc->n_verts)), dim3(kBlock), 0, s, x_end,
                            (int64_t)sc->n_verts, lo, hi);
     } else if (kind == ABD_KIND_EDGE) {
         if (!sc->n_edges) return ABD_OK;
-        hipLaunchKernelGGL(prim_traj_kernel<2>, dim3(grid_for(sc->n_edges)), dim3(kBlock), 0, s, sc->edge_body,
+        launch_kernel(prim_traj_kernel<2>, dim3(grid_for(sc->n_edges)), dim3(kBlock), 0, s, sc->edge_body,
                            sc->voff, sc->edges, x_end, (int64_t)sc->n_edges, lo, hi);
     } else if (kind == ABD_KIND_TRI) {
         if (!sc->n_tris) return ABD_OK;
-        hipLaunchKernelGGL(prim_traj_kernel<3>, dim3(grid_for(sc->n_tris)), dim3(kBlock), 0, s, sc->tri_body,
+        launch_kernel(prim_traj_kernel<3>, dim3(grid_for(sc->n_tris)), dim3(kBlock), 0, s, sc->tri_body,
                            sc->voff, sc->tris, x_end, (int64_t)sc->n_tris, lo, hi);
     } else {
         return ABD_ERR_ARG;
@@ -440,7 +440,7 @@ int abd_prim_boxes_traj(abd_stream_t stream, const AbdScene* sc, int32_t kind, c
 int abd_body_boxes(abd_stream_t stream, const AbdScene* sc, const double* x, double dil, float* lo, float* hi) {
     if (!sc || !x || !lo || !hi) return ABD_ERR_ARG;
     if (!sc->n_bodies) return ABD_OK;
-    hipLaunchKernelGGL(body_boxes_kernel, dim3((unsigned)ceil_div(sc->n_bodies, kBlock / kWave)), dim3(kBlock), 0,
+    launch_kernel(body_boxes_kernel, dim3((unsigned)ceil_div(sc->n_bodies, kBlock / kWave)), dim3(kBlock), 0,
                        to_stream(stream), sc->n_bodies, sc->voff, x, dil, 0, lo, hi);
     ABD_CHECK_LAUNCH();
     return ABD_OK;
@@ -449,7 +449,7 @@ int abd_body_boxes(abd_stream_t stream, const AbdScene* sc, const double* x, dou
 int abd_body_boxes_traj(abd_stream_t stream, const AbdScene* sc, const double* x_end, float* lo, float* hi) {
     if (!sc || !x_end || !lo || !hi) return ABD_ERR_ARG;
     if (!sc->n_bodies) return ABD_OK;
-    hipLaunchKernelGGL(body_boxes_kernel, dim3((unsigned)ceil_div(sc->n_bodies, kBlock / kWave)), dim3(kBlock), 0,
+    launch_kernel(body_boxes_kernel, dim3((unsigned)ceil_div(sc->n_bodies, kBlock / kWave)), dim3(kBlock), 0,
                        to_stream(stream), sc->n_bodies, sc->voff, x_end, 0.0, 1, lo, hi);
     ABD_CHECK_LAUNCH();
     return ABD_OK;

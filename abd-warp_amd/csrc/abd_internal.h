@@ -6,6 +6,8 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include <tuple>
+
 #include "../../include/abd_hip.h"
 
 namespace abd {
@@ -19,6 +21,30 @@ int hip_failure(hipError_t e, const char* file, int line, const char* expr);
         if (_e != hipSuccess) return ::abd::hip_failure(_e, __FILE__, __LINE__, #expr); \
     } while (0)
 #define ABD_CHECK_LAUNCH() ABD_CHECK(hipGetLastError())
+
+// A graph recorded by this thread: between graph_record(g) and graph_record(nullptr) every
+// launch_kernel and copy_to_host of the thread becomes the next node of g, one after the other,
+// and nothing runs.  (Not a stream capture: while a stream of the process is captured the
+// runtime refuses device synchronization, which any other thread may be doing.)
+void graph_record(hipGraph_t g);
+bool capturing();
+int graph_add_kernel(const void* f, dim3 grid, dim3 block, void** args, size_t lds);
+int copy_to_host(hipStream_t s, void* dst, const void* src, size_t bytes);
+
+// Launches f on s, or records the launch.
+template <typename... P, typename... A>
+inline void launch_kernel(void (*f)(P...), dim3 grid, dim3 block, size_t lds, hipStream_t s, A&&... a) {
+    std::tuple<P...> vals(static_cast<P>(a)...);
+    std::apply(
+        [&](P&... v) {
+            void* args[] = {(void*)&v...};
+            if (capturing())
+                (void)graph_add_kernel((const void*)f, grid, block, args, lds);
+            else
+                (void)hipLaunchKernel((const void*)f, grid, block, args, lds, s);
+        },
+        vals);
+}
 
 inline hipStream_t to_stream(abd_stream_t s) { return reinterpret_cast<hipStream_t>(s); }
 
@@ -366,10 +392,8 @@ int arena_free(Arena& a);  // synchronizes the device, then releases every buffe
 // a recorded HIP graph stay valid while it is unchanged.
 uint64_t alloc_generation();
 void note_reallocation();
-// While set on this thread (graph capture), scratch that would have to grow returns
-// ABD_ERR_CAPACITY instead of allocating.
-void set_capturing(bool on);
-bool capturing();
+// (While this thread records a graph, scratch that would have to grow returns
+// ABD_ERR_CAPACITY instead of allocating.)
 // Zeroes `bytes` (a multiple of 8, 8-byte aligned) with a kernel: a fill that may be recorded in
 // a HIP graph (memset nodes are avoided there).
 int zero_fill(hipStream_t s, void* p, size_t bytes);

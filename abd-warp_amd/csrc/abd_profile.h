@@ -68,7 +68,7 @@ template <typename F, typename... Args>
 inline void prof_launch(int handle, F kernel, const dim3& grid, const dim3& block, uint32_t shm, hipStream_t s,
                         Args... args) {
     if (handle < 0) {  // an ordinary launch (also the form a recorded graph takes)
-        hipLaunchKernelGGL(kernel, grid, block, shm, s, args...);
+        launch_kernel(kernel, grid, block, shm, s, args...);
         return;
     }
     hipEvent_t a = nullptr, b = nullptr;

@@ -117,7 +117,7 @@ int prof_count_bytes(int handle, hipStream_t s, const int64_t* dn, double c_pt, 
     double* out;
     int rc = prof_byte_slot(handle, &out);
     if (rc) return rc;
-    hipLaunchKernelGGL(prof_bytes_kernel, dim3(1), dim3(1), 0, s, dn, c_pt, c_ee, c_vg, c_nij, single ? 1 : 0, base,
+    launch_kernel(prof_bytes_kernel, dim3(1), dim3(1), 0, s, dn, c_pt, c_ee, c_vg, c_nij, single ? 1 : 0, base,
                        out);
     ABD_CHECK_LAUNCH();
     prof_stop(handle, s, nullptr, out);

@@ -657,7 +657,7 @@ int get_plan(hipStream_t s, const AbdScene& sc, int S, const Lists& L, const int
     int64_t* plan = plan_buf;
     int rc = plan ? ABD_OK : arena_get(kSlotPlan, sizeof(int64_t) * reduce_plan_elems(S), (void**)&plan);
     if (rc) return rc;
-    hipLaunchKernelGGL(plan_kernel, dim3(1), dim3(kPlanThreads), 0, s, S, sc.body_scene, L, plan,
+    launch_kernel(plan_kernel, dim3(1), dim3(kPlanThreads), 0, s, S, sc.body_scene, L, plan,
                        plan + 2 * kLists * (size_t)S, init);
     ABD_CHECK_LAUNCH();
     *seg = plan;
@@ -687,7 +687,7 @@ int seg_reduce(hipStream_t s, const AbdScene& sc, const AbdParams& P, int S, con
     prof_launch(ph, chunk_kernel, dim3((unsigned)bound), dim3(kRedThreads), 0, s, sc, P, x, L, S, seg, choff, part);
     ABD_CHECK_LAUNCH();
     if ((rc = prof_count_bytes(ph, s, L.dn, 128.0, 132.0, 32.0, 0.0))) return rc;
-    hipLaunchKernelGGL(scene_final_kernel, dim3(S), dim3(kRedThreads), 0, s, choff, (const double*)part, out);
+    launch_kernel(scene_final_kernel, dim3(S), dim3(kRedThreads), 0, s, choff, (const double*)part, out);
     ABD_CHECK_LAUNCH();
     return ABD_OK;
 }
@@ -717,7 +717,7 @@ int attach_seg_bytes(int handle, hipStream_t s, int S, int K, const double* alph
     double* out;
     int rc = prof_byte_slot(handle, &out);
     if (rc || !out) return rc;
-    hipLaunchKernelGGL(seg_bytes_kernel, dim3(1), dim3(kRedThreads), 0, s, S, K, alpha, seg, c_ee, c_pt, c_vg,
+    launch_kernel(seg_bytes_kernel, dim3(1), dim3(kRedThreads), 0, s, S, K, alpha, seg, c_ee, c_pt, c_vg,
                        out);
     ABD_CHECK_LAUNCH();
     prof_stop(handle, s, nullptr, out);
@@ -767,7 +767,7 @@ int toi_reduce(hipStream_t s, const AbdScene& sc, const AbdParams& P, int S, con
     ABD_CHECK_LAUNCH();
     if ((rc = attach_seg_bytes(ph, s, S, 1, nullptr, seg, 228.0, 224.0, 56.0))) return rc;
     if ((rc = toi_solve(s, sc, S, x0, x1, L, w.queue, w.qcount, w.slots, !scr))) return rc;
-    hipLaunchKernelGGL(toi_final_kernel, dim3(S), dim3(kRedThreads), 0, s, choff, (const double*)w.part,
+    launch_kernel(toi_final_kernel, dim3(S), dim3(kRedThreads), 0, s, choff, (const double*)w.part,
                        (const unsigned long long*)w.slots, out, (const uint8_t*)nullptr, (double*)nullptr,
                        SceneDots{});
     ABD_CHECK_LAUNCH();
@@ -800,7 +800,7 @@ int trial_states(hipStream_t s, const AbdScene* sc, const AbdParams* P, int S, i
                  const double* Adot, const double* pdot, double* st, double* e) {
     const int64_t n = (int64_t)sc->n_bodies * K;
     if (n <= 0) return ABD_OK;
-    hipLaunchKernelGGL(trial_states_kernel, dim3(grid_for(n, kRedThreads, INT32_MAX)), dim3(kRedThreads), 0, s, *sc,
+    launch_kernel(trial_states_kernel, dim3(grid_for(n, kRedThreads, INT32_MAX)), dim3(kRedThreads), 0, s, *sc,
                        *P, S, K, alpha, halve ? 1 : 0, A, p, dq, A0, p0, Adot, pdot, st, e);
     ABD_CHECK_LAUNCH();
     return ABD_OK;
@@ -867,7 +867,7 @@ int sweep_toi(hipStream_t s, const AbdScene* sc, const AbdParams* P, int S, cons
     Q.plan = plan;
     int rc;
     if ((rc = toi_solve(s, *sc, S, x_t0, x_t1, L, W.queue, W.qcount, W.slots, true, Q))) return rc;
-    hipLaunchKernelGGL(toi_final_kernel, dim3(S), dim3(kRedThreads), 0, s, (const int64_t*)nullptr,
+    launch_kernel(toi_final_kernel, dim3(S), dim3(kRedThreads), 0, s, (const int64_t*)nullptr,
                        (const double*)nullptr, (const unsigned long long*)W.slots, toi, W.active, first_alpha, dots);
     ABD_CHECK_LAUNCH();
     return ABD_OK;
@@ -977,14 +977,14 @@ int abd_scene_toi(abd_stream_t stream, const AbdScene* sc, const AbdParams* P, c
 
 int abd_dot(abd_stream_t stream, const double* a, const double* b, int64_t n, double* out) {
     if (n < 0 || (!a && n) || (!b && n) || !out) return ABD_ERR_ARG;
-    hipLaunchKernelGGL(seg_dot_kernel, dim3(1), dim3(kRedThreads), 0, to_stream(stream), nullptr, n, a, b, out);
+    launch_kernel(seg_dot_kernel, dim3(1), dim3(kRedThreads), 0, to_stream(stream), nullptr, n, a, b, out);
     ABD_CHECK_LAUNCH();
     return ABD_OK;
 }
 
 int abd_scene_dot(abd_stream_t stream, const AbdScene* sc, const double* a, const double* b, double* out) {
     if (!scenes_ok(sc) || !a || !b || !out) return ABD_ERR_ARG;
-    hipLaunchKernelGGL(seg_dot_kernel, dim3(sc->n_scenes), dim3(kRedThreads), 0, to_stream(stream), sc->scene_boff,
+    launch_kernel(seg_dot_kernel, dim3(sc->n_scenes), dim3(kRedThreads), 0, to_stream(stream), sc->scene_boff,
                        (int64_t)0, a, b, out);
     ABD_CHECK_LAUNCH();
     return ABD_OK;
@@ -993,7 +993,7 @@ int abd_scene_dot(abd_stream_t stream, const AbdScene* sc, const double* a, cons
 int abd_inertia_energy(abd_stream_t stream, const AbdScene* sc, const AbdParams* P, const double* Ak, const double* pk,
                        const double* A0, const double* p0, const double* Adot, const double* pdot, double* E) {
     if (!sc || !P || !Ak || !pk || !A0 || !p0 || !Adot || !pdot || !E) return ABD_ERR_ARG;
-    hipLaunchKernelGGL(seg_inertia_kernel, dim3(1), dim3(kRedThreads), 0, to_stream(stream), nullptr, sc->n_bodies,
+    launch_kernel(seg_inertia_kernel, dim3(1), dim3(kRedThreads), 0, to_stream(stream), nullptr, sc->n_bodies,
                        *P, sc->mass, sc->I0, Ak, pk, A0, p0, Adot, pdot, E);
     ABD_CHECK_LAUNCH();
     return ABD_OK;
@@ -1003,7 +1003,7 @@ int abd_scene_inertia_energy(abd_stream_t stream, const AbdScene* sc, const AbdP
                              const double* pk, const double* A0, const double* p0, const double* Adot,
                              const double* pdot, double* E) {
     if (!scenes_ok(sc) || !P || !Ak || !pk || !A0 || !p0 || !Adot || !pdot || !E) return ABD_ERR_ARG;
-    hipLaunchKernelGGL(seg_inertia_kernel, dim3(sc->n_scenes), dim3(kRedThreads), 0, to_stream(stream),
+    launch_kernel(seg_inertia_kernel, dim3(sc->n_scenes), dim3(kRedThreads), 0, to_stream(stream),
                        sc->scene_boff, sc->n_bodies, *P, sc->mass, sc->I0, Ak, pk, A0, p0, Adot, pdot, E);
     ABD_CHECK_LAUNCH();
     return ABD_OK;

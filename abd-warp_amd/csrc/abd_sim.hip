@@ -158,7 +158,6 @@ struct Sim {
     bool solve_waits = false;  // the solver reads back between its launches: never recorded
     int64_t gcount[3] = {};  // iterations replayed, recorded (then replayed), launched eagerly
     hipGraphExec_t gexec = nullptr;
-    hipStream_t cap_stream = nullptr;  // the recording stream (the caller's may be the null stream)
     uint64_t gkey[kKeyWords] = {}, gseen[kKeyWords] = {}, gfailed[kKeyWords] = {};
     int32_t* hiters = nullptr;  // pinned [ns]: the iteration counts read back at a frame's end
     std::vector<int32_t> scene_it;  // Newton iterations of each scene in the last frame
@@ -493,7 +492,7 @@ int swept_set_recull(hipStream_t s, Sim& S) {
     // starts with this superset has them from body_start)
     if ((rc = sweep_buffers(S))) return rc;
     const int64_t n = std::max<int64_t>(sweep_words(S), S.ns);
-    hipLaunchKernelGGL(sweep_reset_kernel, dim3(grid_for(n, kBlock, 1024)), dim3(kBlock), 0, s, S.kcnt.p,
+    launch_kernel(sweep_reset_kernel, dim3(grid_for(n, kBlock, 1024)), dim3(kBlock), 0, s, S.kcnt.p,
                        sweep_words(S), S.toi_slots, S.ns, S.toi_qcount, S.cnt.p + kCntNewton,
                        kCntSolver - kCntNewton + 1);
     ABD_CHECK_LAUNCH();
@@ -701,7 +700,7 @@ int frame_start_scenes(hipStream_t s, Sim& S) {
     int rc;
     const AbdSimState& st = S.st;
     const int ns = S.ns;
-    hipLaunchKernelGGL(frame_state_kernel, dim3(grid_for(std::max(9 * (int64_t)S.nb, (int64_t)ns), kLsThreads, INT32_MAX)),
+    launch_kernel(frame_state_kernel, dim3(grid_for(std::max(9 * (int64_t)S.nb, (int64_t)ns), kLsThreads, INT32_MAX)),
                        dim3(kLsThreads), 0, s, S.nb, ns, st.A0, st.p0, st.A, st.p, st.Ak, st.pk,
                        S.sv.p + kSvAlpha * ns);
     ABD_CHECK_LAUNCH();
@@ -733,7 +732,7 @@ int line_pass(hipStream_t s, Sim& S, const LsDev& L, bool first, int K, int k0) 
     if ((rc = line_chunks(s, &S.sc, &S.P, S.ns, K, S.cand_alpha.p, S.trial_st.p + 12 * nb * k0, S.sw.ptl.p, S.sw.npt,
                           S.sw.eel.p, S.sw.nee, S.sw.vgl.p, S.sw.nvg, S.plan.p, S.sw.counts(), S.sw.side(), &C)))
         return rc;
-    hipLaunchKernelGGL(ls_pass_kernel, dim3(S.ns), dim3(kLsThreads), 0, s, L, S.P.c1, S.P.alpha_min, S.P.tol,
+    launch_kernel(ls_pass_kernel, dim3(S.ns), dim3(kLsThreads), 0, s, L, S.P.c1, S.P.alpha_min, S.P.tol,
                        (int)S.P.max_iter, first ? 1 : 0, K, S.cand_alpha.p, C,
                        (const double*)(S.trial_e.p + nb * k0), S.ns > 1 ? S.sc.scene_boff : nullptr, S.nb);
     ABD_CHECK_LAUNCH();
@@ -812,8 +811,7 @@ int ccd_and_search_scenes(hipStream_t s, Sim& S, const LsDev& L) {
     if ((rc = pass_states(s, S, 1 + kLsSpec, true, 0))) return rc;
     if ((rc = line_pass(s, S, L, true, 1, 0))) return rc;
     if ((rc = line_pass(s, S, L, false, kLsSpec, 1))) return rc;
-    ABD_CHECK(hipMemcpyAsync(S.hcnt, S.cnt.p, kCntLen * sizeof(int64_t), hipMemcpyDeviceToHost, s));
-    return ABD_OK;
+    return copy_to_host(s, S.hcnt, S.cnt.p, kCntLen * sizeof(int64_t));
 }
 
 // One Newton iteration of every scene up to the read-back of its counts (abd.py:224-271): the last
@@ -908,33 +906,22 @@ bool same_key(const uint64_t a[kKeyWords], const uint64_t b[kKeyWords]) {
     return !memcmp(a, b, kKeyWords * sizeof(uint64_t));
 }
 
-// Records iteration_scenes into S.gexec (updated in place when the topology allows), on a
-// stream of the simulator's own (the legacy null stream cannot record); nothing runs.  A
-// failure leaves no error state behind, and the caller launches the iteration instead.
-int record_iteration(Sim& S) {
-    if (!S.cap_stream) {
-        const hipError_t ce = hipStreamCreateWithFlags(&S.cap_stream, hipStreamNonBlocking);
-        if (ce != hipSuccess) {
-            S.cap_stream = nullptr;
-            (void)hipGetLastError();
-            return -static_cast<int>(ce);
-        }
-    }
-    hipStream_t s = S.cap_stream;
+// Records iteration_scenes into S.gexec (updated in place when the topology allows); nothing
+// runs.  A failure leaves no error state behind, and the caller launches the iteration instead.
+int record_iteration(hipStream_t s, Sim& S) {
     hipGraph_t g = nullptr;
-    const hipError_t be = hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal);
-    if (be != hipSuccess) {
+    const hipError_t ce = hipGraphCreate(&g, 0);
+    if (ce != hipSuccess) {
         (void)hipGetLastError();
-        return -static_cast<int>(be);
+        return -static_cast<int>(ce);
     }
-    set_capturing(true);
-    int rc = iteration_scenes(s, S);
-    set_capturing(false);
-    const hipError_t e = hipStreamEndCapture(s, &g);
-    if (rc || e != hipSuccess || !g) {
-        if (g) (void)hipGraphDestroy(g);
+    graph_record(g);
+    const int rc = iteration_scenes(s, S);
+    graph_record(nullptr);
+    if (rc) {
+        (void)hipGraphDestroy(g);
         (void)hipGetLastError();
-        return rc ? rc : -static_cast<int>(e == hipSuccess ? hipErrorUnknown : e);
+        return rc;
     }
     if (S.gexec) {
         hipGraphNode_t err_node = nullptr;
@@ -967,7 +954,7 @@ int step_scenes(hipStream_t s, Sim& S) {
     {
         // the first iteration's rows, taken over by its body_start_kernel
         const LsDev L = ls_dev(S);
-        hipLaunchKernelGGL(ls_frame_start_kernel, dim3((unsigned)ceil_div(ns, kLsThreads)), dim3(kLsThreads), 0, s,
+        launch_kernel(ls_frame_start_kernel, dim3((unsigned)ceil_div(ns, kLsThreads)), dim3(kLsThreads), 0, s,
                            ns, (const double*)(S.sv.p + kSvEc * ns), (const double*)(S.sv.p + kSvEi * ns), L.E0_nxt,
                            L.newton_nxt, L.it_nxt);
         ABD_CHECK_LAUNCH();
@@ -988,7 +975,7 @@ int step_scenes(hipStream_t s, Sim& S) {
             ran = true;
             ++S.gcount[0];
         } else if (steady && same_key(key, S.gseen) && !same_key(key, S.gfailed)) {
-            if (record_iteration(S) == ABD_OK) {
+            if (record_iteration(s, S) == ABD_OK) {
                 ABD_CHECK(hipGraphLaunch(S.gexec, s));
                 memcpy(S.gkey, key, sizeof(key));
                 ran = true;
@@ -1287,7 +1274,6 @@ int abd_sim_destroy(void* sim) {
     Sim* S = static_cast<Sim*>(sim);
     (void)hipDeviceSynchronize();  // queued work may still use the buffers released below
     if (S->gexec) (void)hipGraphExecDestroy(S->gexec);
-    if (S->cap_stream) (void)hipStreamDestroy(S->cap_stream);
     (void)arena_free(S->arena);
     for (BoxBuf* b : {&S->body, &S->tri, &S->edge, &S->pt, &S->tbody, &S->sbody,
                       &S->stri, &S->sedge, &S->spt}) {

@@ -1649,7 +1649,7 @@ int launch_solve(hipStream_t s, int32_t method, const Bsr& M, int nsys, const in
         if (M.nb > 0) {
             // algorithmic bytes: each diagonal block read, its inverse written
             const int ph_inv = pending ? -1 : prof_start(kProfPrecond, s, 2304.0 * M.nb);
-            hipLaunchKernelGGL(invert_blocks_kernel, dim3(M.nb), dim3(kInvThreads), 0, s, M, dinv, pending, sboff,
+            launch_kernel(invert_blocks_kernel, dim3(M.nb), dim3(kInvThreads), 0, s, M, dinv, pending, sboff,
                                nsys);
             ABD_CHECK_LAUNCH();
             prof_stop(ph_inv, s);
@@ -1704,10 +1704,10 @@ int launch_solve(hipStream_t s, int32_t method, const Bsr& M, int nsys, const in
         cg = cg_kernel<false, true, kSolveThreads>;
     }
     if (method == ABD_SOLVER_BICGSTAB)
-        hipLaunchKernelGGL(bicgstab, dim3(nsys), dim3(threads), dyn, s, M, sboff, active, b, x, tol, maxiter,
+        launch_kernel(bicgstab, dim3(nsys), dim3(threads), dyn, s, M, sboff, active, b, x, tol, maxiter,
                            check_every, max_rows, budget, ws, iters, resid);
     else
-        hipLaunchKernelGGL(cg, dim3(nsys), dim3(threads), dyn, s, M, sboff, active, b, x, tol, maxiter, check_every,
+        launch_kernel(cg, dim3(nsys), dim3(threads), dyn, s, M, sboff, active, b, x, tol, maxiter, check_every,
                            max_rows, budget, ws, dinv, iters, resid, pending);
     ABD_CHECK_LAUNCH();
     prof_stop(ph, s);
@@ -1715,7 +1715,7 @@ int launch_solve(hipStream_t s, int32_t method, const Bsr& M, int nsys, const in
         // the byte count needs the iteration counts: computed behind the solve, on its stream
         double* dbytes;
         if ((rc = arena_get(kSlotSolveBytes, sizeof(double), (void**)&dbytes))) return rc;
-        hipLaunchKernelGGL(solve_bytes_kernel, dim3(1), dim3(256), 0, s, M.row_ptr, M.nb, sboff, active, nsys, iters,
+        launch_kernel(solve_bytes_kernel, dim3(1), dim3(256), 0, s, M.row_ptr, M.nb, sboff, active, nsys, iters,
                            method == ABD_SOLVER_BICGSTAB ? 2 : 1, lds ? 1 : 0, bj ? 1152.0 : 0.0, dbytes);
         ABD_CHECK_LAUNCH();
         prof_stop(ph, s, nullptr, dbytes);
@@ -1761,7 +1761,7 @@ int launch_ldlt(hipStream_t s, const Bsr& M, int nsys, const int32_t* sboff, con
         // algorithmic bytes of the systems solved directly: each block, b and x once
         double* dbytes;
         if ((rc = arena_get(kSlotSolveBytes, sizeof(double), (void**)&dbytes))) return rc;
-        hipLaunchKernelGGL(solve_bytes_kernel, dim3(1), dim3(256), 0, s, M.row_ptr, M.nb, sboff, active, nsys,
+        launch_kernel(solve_bytes_kernel, dim3(1), dim3(256), 0, s, M.row_ptr, M.nb, sboff, active, nsys,
                            (const int32_t*)status, 1, 1, 192.0, dbytes);
         ABD_CHECK_LAUNCH();
         prof_stop(ph, s, nullptr, dbytes);
@@ -1804,7 +1804,7 @@ int solve_cg_multi(hipStream_t s, const Bsr& M, const double* b, double* x, doub
     if (bj) {
         if ((rc = arena_get(kSlotPrecond, sizeof(double) * 144 * (size_t)M.nb, (void**)&dinv))) return rc;
         const int ph_inv = prof_start(kProfPrecond, s, 2304.0 * M.nb);
-        hipLaunchKernelGGL(invert_blocks_kernel, dim3(M.nb), dim3(kInvThreads), 0, s, M, dinv,
+        launch_kernel(invert_blocks_kernel, dim3(M.nb), dim3(kInvThreads), 0, s, M, dinv,
                            (const int32_t*)nullptr, (const int32_t*)nullptr, 1);
         ABD_CHECK_LAUNCH();
         prof_stop(ph_inv, s);
@@ -1812,25 +1812,25 @@ int solve_cg_multi(hipStream_t s, const Bsr& M, const double* b, double* x, doub
     const double tol_sq = tol * tol * (double)n;
     int ph = prof_start(kProfSolve, s, 0.0);
     if (bj)
-        hipLaunchKernelGGL(mw_init_kernel<true>, dim3(nblk), dim3(threads), 0, s, M, b, (const double*)x, W,
+        launch_kernel(mw_init_kernel<true>, dim3(nblk), dim3(threads), 0, s, M, b, (const double*)x, W,
                            (const double*)dinv);
     else
-        hipLaunchKernelGGL(mw_init_kernel<false>, dim3(nblk), dim3(threads), 0, s, M, b, (const double*)x, W,
+        launch_kernel(mw_init_kernel<false>, dim3(nblk), dim3(threads), 0, s, M, b, (const double*)x, W,
                            (const double*)dinv);
     ABD_CHECK_LAUNCH();
-    hipLaunchKernelGGL(mw_start_kernel, dim3(1), dim3(kMwThreads), 0, s, nblk, tol_sq, maxiter, W);
+    launch_kernel(mw_start_kernel, dim3(1), dim3(kMwThreads), 0, s, nblk, tol_sq, maxiter, W);
     ABD_CHECK_LAUNCH();
     for (int i0 = 0; i0 < maxiter; i0 += check_every) {
         const int i1 = i0 + check_every < maxiter ? i0 + check_every : maxiter;
         for (int i = i0; i < i1; ++i) {
-            hipLaunchKernelGGL(mw_spmv_kernel, dim3(nblk), dim3(threads), 0, s, M, W);
+            launch_kernel(mw_spmv_kernel, dim3(nblk), dim3(threads), 0, s, M, W);
             if (bj)
-                hipLaunchKernelGGL(mw_update_kernel<true>, dim3(nblk), dim3(threads), 0, s, n, i, W,
+                launch_kernel(mw_update_kernel<true>, dim3(nblk), dim3(threads), 0, s, n, i, W,
                                    (const double*)dinv);
             else
-                hipLaunchKernelGGL(mw_update_kernel<false>, dim3(nblk), dim3(threads), 0, s, n, i, W,
+                launch_kernel(mw_update_kernel<false>, dim3(nblk), dim3(threads), 0, s, n, i, W,
                                    (const double*)dinv);
-            hipLaunchKernelGGL(mw_direction_kernel, dim3(nblk), dim3(threads), 0, s, n, i, (int)check_every,
+            launch_kernel(mw_direction_kernel, dim3(nblk), dim3(threads), 0, s, n, i, (int)check_every,
                                tol_sq, W);
         }
         ABD_CHECK_LAUNCH();
@@ -1838,7 +1838,7 @@ int solve_cg_multi(hipStream_t s, const Bsr& M, const double* b, double* x, doub
         ABD_CHECK(hipStreamSynchronize(s));
         if (*hdone) break;
     }
-    hipLaunchKernelGGL(mw_finish_kernel, dim3(nblk), dim3(kMwThreads), 0, s, n, W, x, iters, resid);
+    launch_kernel(mw_finish_kernel, dim3(nblk), dim3(kMwThreads), 0, s, n, W, x, iters, resid);
     ABD_CHECK_LAUNCH();
     prof_stop(ph, s);
     return ABD_OK;

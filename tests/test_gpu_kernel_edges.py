@@ -336,3 +336,44 @@ def test_gh_over_repeated_candidates(psd, total):
     gk, bk, hk, nk = gh(pt.repeat_interleave(k, 0), ee.repeat_interleave(k, 0))
     assert nk == k * n1 and np.array_equal(h1, hk)
     assert rel_err(gk, k * g1) <= 1e-10 and rel_err(bk, k * b1) <= 1e-10
+
+
+def test_recording_leaves_other_threads_alone():
+    """A driver records its iteration for replay while another thread synchronizes the device
+    and allocates: neither is refused (a captured stream would make the runtime refuse both)."""
+    import threading
+    from abd_hip import scenes
+    from abd_hip.abd import AffineBodySimulator
+    from abd_hip.const_params import ContactParams
+    m = scenes.cube_mesh()
+    specs = []
+    for k in range(6):
+        p = np.array([[0.0, 0.5005 + j * 1.001, 0.002 * j] for j in range(2 + k)])
+        n = len(p)
+        specs.append(scenes.build_scene([m] * n, np.stack([np.eye(3)] * n), p, np.zeros((n, 3, 3)),
+                                        np.zeros((n, 3)), ground=0.0))
+    done, errors, rounds = threading.Event(), [], [0]
+
+    def other():
+        try:
+            while not done.is_set():
+                torch.cuda.synchronize()
+                t = torch.empty(1 << (12 + rounds[0] % 12), device="cuda")
+                del t
+                torch.cuda.empty_cache()
+                rounds[0] += 1
+        except Exception as e:  # noqa: BLE001 - reported below
+            errors.append(e)
+
+    th = threading.Thread(target=other)
+    th.start()
+    try:
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for spec in specs:
+                sim = AffineBodySimulator(spec, ContactParams(ground=0.0, psd=1, solver=3), native=True)
+                for f in range(4):
+                    sim.step(f)
+    finally:
+        done.set()
+        th.join()
+    assert not errors and rounds[0] > 0
