@@ -138,6 +138,34 @@ __device__ __forceinline__ void block_sum2_fast(double& a, double& b, double* sh
     __syncthreads();
 }
 
+// The extrema of a body's vertices over the T threads of its workgroup, valid in thread 0.
+template <int T>
+__device__ __forceinline__ void body_extrema(double (&mn)[3], double (&mx)[3], double* sh) {
+#pragma unroll
+    for (int off = kWave / 2; off > 0; off >>= 1)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const double a = __shfl_xor(mn[k], off, kWave), b = __shfl_xor(mx[k], off, kWave);
+            mn[k] = a < mn[k] ? a : mn[k];
+            mx[k] = b > mx[k] ? b : mx[k];
+        }
+    if (T > kWave) {
+        if (lane_id() == 0)
+            for (int k = 0; k < 3; ++k) {
+                sh[6 * wave_id() + k] = mn[k];
+                sh[6 * wave_id() + 3 + k] = mx[k];
+            }
+        __syncthreads();
+        if (threadIdx.x == 0)
+            for (int w = 1; w < T / kWave; ++w)
+                for (int k = 0; k < 3; ++k) {
+                    const double a = sh[6 * w + k], b = sh[6 * w + 3 + k];
+                    mn[k] = a < mn[k] ? a : mn[k];
+                    mx[k] = b > mx[k] ? b : mx[k];
+                }
+    }
+}
+
 // Exclusive prefix sum of one int64 per thread (sh: at least n_waves() entries): a
 // shuffle scan inside each wave, then the totals of the waves before it (two barriers).
 __device__ __forceinline__ int64_t block_exclusive_scan_i64(int64_t v, int64_t* sh) {

@@ -27,8 +27,11 @@ namespace abd {
 
 __device__ __forceinline__ bool overlap(const float* __restrict__ alo, const float* __restrict__ ahi,
                                         const float* __restrict__ blo, const float* __restrict__ bhi) {
-    return !(alo[0] > bhi[0] || ahi[0] < blo[0] || alo[1] > bhi[1] || ahi[1] < blo[1] || alo[2] > bhi[2] ||
-             ahi[2] < blo[2]);
+    // every bound is loaded before any is compared: as one condition after the other the six
+    // loads waited for each other
+    const float a0 = alo[0], a1 = alo[1], a2 = alo[2], A0 = ahi[0], A1 = ahi[1], A2 = ahi[2];
+    const float b0 = blo[0], b1 = blo[1], b2 = blo[2], B0 = bhi[0], B1 = bhi[1], B2 = bhi[2];
+    return !((a0 > B0) | (A0 < b0) | (a1 > B1) | (A1 < b1) | (a2 > B2) | (A2 < b2));
 }
 
 // ---------------------------------------------------------------- bodies
@@ -89,14 +92,19 @@ __device__ __forceinline__ void seg_pair_of(int64_t k, int nb, int order, const 
     j += b0;
 }
 
+// blockIdx.y: the order of the enumeration, its counts and offsets nblk + 1 apart.
 template <bool WRITE>
-__global__ __launch_bounds__(kBlock) void body_pairs_kernel(int nb, int64_t npairs, int order, SceneSeg sg,
+__global__ __launch_bounds__(kBlock) void body_pairs_kernel(int nb, int64_t npairs, SceneSeg sg,
                                                              const int32_t* __restrict__ scene,
                                                              const float* __restrict__ lo,
                                                              const float* __restrict__ hi, int64_t* __restrict__ bcnt,
-                                                             const int64_t* __restrict__ boff, int32_t* out,
-                                                             int64_t cap) {
+                                                             const int64_t* __restrict__ boff, int32_t* out_ij,
+                                                             int32_t* out_ji, int64_t cap) {
     __shared__ int shw[kBlock / kWave];
+    const int order = blockIdx.y;
+    int32_t* out = order ? out_ji : out_ij;
+    bcnt += order * ((int64_t)gridDim.x + 1);
+    if (WRITE) boff += order * ((int64_t)gridDim.x + 1);
     int64_t base = (int64_t)blockIdx.x * kBlock * kPairItems;
     int64_t run = WRITE ? boff[blockIdx.x] : 0;
     for (int it = 0; it < kPairItems; ++it) {
@@ -123,42 +131,6 @@ __global__ __launch_bounds__(kBlock) void body_pairs_kernel(int nb, int64_t npai
 
 // ------------------------------------------------------------- primitives
 
-// Hull of the FP32 boxes of each body's primitives: one wave per body (kBlock / 64 bodies
-// per workgroup), the six extrema reduced by lane shuffles (a minimum or maximum does not
-// depend on the order).  blockIdx.y selects one of two primitive sets (set 1 only when
-// nsets == 1).
-struct HullSet {
-    const int32_t* offs;
-    const float *lo, *hi;
-    float *hlo, *hhi;
-};
-__global__ __launch_bounds__(kBlock) void hull_kernel(int nb, HullSet H1, HullSet H2) {
-    const HullSet& H = blockIdx.y ? H2 : H1;
-    const int b = blockIdx.x * (kBlock / kWave) + wave_id();
-    if (b >= nb) return;  // the whole wave (no barrier below)
-    const int p0 = H.offs[b], p1 = H.offs[b + 1];
-    float mn[3] = {INFINITY, INFINITY, INFINITY}, mx[3] = {-INFINITY, -INFINITY, -INFINITY};
-    for (int p = p0 + lane_id(); p < p1; p += kWave) {
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            mn[k] = fminf(mn[k], H.lo[3 * (int64_t)p + k]);
-            mx[k] = fmaxf(mx[k], H.hi[3 * (int64_t)p + k]);
-        }
-    }
-#pragma unroll
-    for (int off = kWave / 2; off > 0; off >>= 1)
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            mn[k] = fminf(mn[k], __shfl_xor(mn[k], off, kWave));
-            mx[k] = fmaxf(mx[k], __shfl_xor(mx[k], off, kWave));
-        }
-    if (lane_id() < 3) {
-        const int k = lane_id();
-        H.hlo[3 * b + k] = k == 0 ? mn[0] : (k == 1 ? mn[1] : mn[2]);
-        H.hhi[3 * b + k] = k == 0 ? mx[0] : (k == 1 ? mx[1] : mx[2]);
-    }
-}
-
 // unit -> (ii, I (set-1 body), J (set-2 body))
 __device__ __forceinline__ void unit_bodies(int pt, int64_t u, const int32_t* __restrict__ ij, int64_t& ii, int& I,
                                             int& J) {
@@ -174,44 +146,132 @@ __device__ __forceinline__ void unit_bodies(int pt, int64_t u, const int32_t* __
     }
 }
 
-// One workgroup per (unit, side): side 0 keeps set-1 prims of I overlapping hull2[J],
-// side 1 keeps set-2 prims of J overlapping hull1[I]; local ids in ascending order.
-__global__ __launch_bounds__(kBlock) void filter_kernel(int pt, const int32_t* __restrict__ ij, PrimSets S,
-                                                         int64_t maxs, int32_t* __restrict__ flist,
+constexpr int kXcds = 8;
+// Which of n blocks the workgroup `loc` of a list takes (-1: none): the workgroups of one XCD
+// (they are dealt to the XCDs in turn) take a contiguous run of blocks, whose entries share
+// vertices in its L2.  n: the blocks in use, of a launch over at least as many rounded up.
+__device__ __forceinline__ int64_t xcd_block(int64_t loc, int64_t n) {
+    const int64_t run = (n + kXcds - 1) / kXcds, y = loc / kXcds, b = loc % kXcds * run + y;
+    return y < run && b < n ? b : -1;
+}
+
+// The hull of the boxes of primitives [p0, p1) over the workgroup (four loads in flight a
+// thread, past the end the last primitive again; sh: 6 floats a wave).
+__device__ __forceinline__ void prims_hull(const float* __restrict__ lo, const float* __restrict__ hi, int p0, int p1,
+                                           float* sh, float (&mn)[3], float (&mx)[3]) {
+    constexpr int kAtOnce = 4;
+    for (int k = 0; k < 3; ++k) {
+        mn[k] = INFINITY;
+        mx[k] = -INFINITY;
+    }
+    for (int p = p0 + threadIdx.x; p < p1; p += kAtOnce * kBlock) {
+        float l[kAtOnce][3], h[kAtOnce][3];
+#pragma unroll
+        for (int j = 0; j < kAtOnce; ++j) {
+            const int64_t q = 3 * (int64_t)min(p + j * kBlock, p1 - 1);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                l[j][k] = lo[q + k];
+                h[j][k] = hi[q + k];
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < kAtOnce; ++j)
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                mn[k] = fminf(mn[k], l[j][k]);
+                mx[k] = fmaxf(mx[k], h[j][k]);
+            }
+    }
+#pragma unroll
+    for (int off = kWave / 2; off > 0; off >>= 1)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            mn[k] = fminf(mn[k], __shfl_xor(mn[k], off, kWave));
+            mx[k] = fmaxf(mx[k], __shfl_xor(mx[k], off, kWave));
+        }
+    if (lane_id() == 0)
+        for (int k = 0; k < 3; ++k) {
+            sh[6 * wave_id() + k] = mn[k];
+            sh[6 * wave_id() + 3 + k] = mx[k];
+        }
+    __syncthreads();
+    for (int w = 0; w < kBlock / kWave; ++w)
+        for (int k = 0; k < 3; ++k) {
+            mn[k] = fminf(mn[k], sh[6 * w + k]);
+            mx[k] = fmaxf(mx[k], sh[6 * w + 3 + k]);
+        }
+}
+
+// One workgroup per (unit, side): side 0 keeps the set-1 prims of I whose box overlaps the hull
+// of J's set-2 prims, side 1 the set-2 prims of J against the hull of I's set-1 prims; local
+// ids in ascending order.  Four primitives a thread and one barrier a pass.  (With the hulls
+// of all bodies in a kernel before it, one wave a body, and one primitive a thread here, 634
+// pairs of bodies of 3200 edges took 43 + 46 us; 33 here: the XCD order gives about 8 of that
+// and overlap() loading all its bounds at once 30.)
+__global__ __launch_bounds__(kBlock) void filter_kernel(int pt, const int32_t* __restrict__ ij, int64_t ntasks,
+                                                         PrimSets S, int64_t maxs, int32_t* __restrict__ flist,
                                                          int64_t* __restrict__ fcnt) {
-    __shared__ int shw[kBlock / kWave];
-    const int64_t u = blockIdx.x >> 1;
-    const int side = blockIdx.x & 1;
+    constexpr int kWaves = kBlock / kWave, kPer = 4;
+    __shared__ float sh[6 * kWaves];
+    __shared__ int cnt[2][kWaves];
+    // neighbouring units share bodies: the workgroups of one XCD take them in runs
+    const int64_t task = xcd_block(blockIdx.x, ntasks);
+    if (task < 0) return;  // uniform
+    const int64_t u = task >> 1;
+    const bool side = task & 1;
     int64_t ii;
     int I, J;
     unit_bodies(pt, u, ij, ii, I, J);
-    const int32_t* offs = side ? S.off2 : S.off1;
-    const float* lo = side ? S.lo2 : S.lo1;
-    const float* hi = side ? S.hi2 : S.hi1;
-    const int body = side ? J : I;
-    const int other = side ? I : J;
-    const float* hlo = side ? S.hlo1 + 3 * other : S.hlo2 + 3 * other;
-    const float* hhi = side ? S.hhi1 + 3 * other : S.hhi2 + 3 * other;
+    const int32_t *offs = side ? S.off2 : S.off1, *offs_h = side ? S.off1 : S.off2;
+    const float *lo = side ? S.lo2 : S.lo1, *hi = side ? S.hi2 : S.hi1;
+    const int body = side ? J : I, other = side ? I : J;
+    float mn[3], mx[3];
+    prims_hull(side ? S.lo1 : S.lo2, side ? S.hi1 : S.hi2, offs_h[other], offs_h[other + 1], sh, mn, mx);
     const int p0 = offs[body], p1 = offs[body + 1];
-    int32_t* dst = flist + blockIdx.x * maxs;
+    int32_t* dst = flist + task * maxs;
     int64_t run = 0;
-    for (int base = p0; base < p1; base += kBlock) {
-        int p = base + threadIdx.x;
-        bool pred = p < p1 && overlap(lo + 3 * (int64_t)p, hi + 3 * (int64_t)p, hlo, hhi);
-        int tot;
-        int r = block_rank(pred, shw, &tot);
-        if (pred) dst[run + r] = p - p0;
+    int turn = 0;
+    for (int base = p0; base < p1; base += kPer * kBlock, turn ^= 1) {
+        const int p = base + kPer * threadIdx.x;
+        bool pred[kPer];
+        int before = 0, mine = 0;
+        const unsigned long long below = (1ull << lane_id()) - 1ull;
+#pragma unroll
+        for (int j = 0; j < kPer; ++j) {
+            const int64_t q = 3 * (int64_t)min(p + j, p1 - 1);
+            pred[j] = overlap(lo + q, hi + q, mn, mx) && p + j < p1;
+        }
+#pragma unroll
+        for (int j = 0; j < kPer; ++j) {
+            const unsigned long long m = __ballot(pred[j]);
+            before += __popcll(m & below);
+            mine += __popcll(m);
+        }
+        if (lane_id() == 0) cnt[turn][wave_id()] = mine;  // (buffers in turn: one barrier a pass)
+        __syncthreads();
+        int tot = 0;
+        for (int w = 0; w < kWaves; ++w) {
+            if (w < wave_id()) before += cnt[turn][w];
+            tot += cnt[turn][w];
+        }
+        int64_t o = run + before;
+#pragma unroll
+        for (int j = 0; j < kPer; ++j)
+            if (pred[j]) dst[o++] = p + j - p0;
         run += tot;
     }
-    if (threadIdx.x == 0) fcnt[blockIdx.x] = run;
+    if (threadIdx.x == 0) fcnt[task] = run;
 }
 
-__global__ void unit_chunks_kernel(int64_t nunits, int chunk, const int64_t* __restrict__ fcnt,
-                                   int64_t* __restrict__ nchunk) {
-    int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (u >= nunits) return;
-    int64_t nt = fcnt[2 * u] * fcnt[2 * u + 1];
-    nchunk[u] = (nt + chunk - 1) / chunk;
+// The units' chunks of `chunk` primitive tests, scanned into their first chunks choff.
+__global__ __launch_bounds__(kScanThreads) void unit_chunks_kernel(int64_t nunits, int chunk,
+                                                                   const int64_t* __restrict__ fcnt,
+                                                                   int64_t* __restrict__ choff,
+                                                                   int64_t* __restrict__ total,
+                                                                   int64_t* __restrict__ total2) {
+    scan_block_exclusive_by(
+        [=](int64_t u) { return (fcnt[2 * u] * fcnt[2 * u + 1] + chunk - 1) / chunk; }, choff, nunits, total, total2);
 }
 
 // last u with choff[u] <= c (choff non-decreasing, choff[0] = 0)
@@ -289,31 +349,45 @@ __global__ __launch_bounds__(kBlock) void vg_kernel(int64_t nv, const int32_t* _
                                                      double ythresh, float fground, int64_t* __restrict__ bcnt,
                                                      const int64_t* __restrict__ boff, int32_t* __restrict__ out,
                                                      int64_t cap) {
-    __shared__ int shw[kBlock / kWave];
+    constexpr int kWaves = kBlock / kWave;
+    __shared__ int cnt[kItems * kWaves];
     const float qlo[3] = {-1e3f, -1e3f, -1e3f};
     const float qhi[3] = {1e3f, fground, 1e3f};
-    int64_t base = (int64_t)blockIdx.x * kBlock * kItems;
-    int64_t run = WRITE ? boff[blockIdx.x] : 0;
+    const int64_t base = (int64_t)blockIdx.x * kBlock * kItems;
+    // all of a thread's items first (their loads in flight together), then one ranking
+    bool pred[kItems];
+    int32_t body[kItems];
+#pragma unroll
     for (int it = 0; it < kItems; ++it) {
-        int64_t v = base + (int64_t)it * kBlock + threadIdx.x;
-        bool pred = false;
-        int b = 0;
-        if (v < nv) {
-            b = vert_body[v];
-            // culling.py:67: lowers[i][1] < 0.5 * dhat + ground (FP64)
-            pred = (double)blo[3 * b + 1] < ythresh && overlap(plo + 3 * v, phi + 3 * v, qlo, qhi);
-        }
-        int tot;
-        int r = block_rank(pred, shw, &tot);
-        if (WRITE && pred) {
-            int64_t o = run + r;
-            if (o < cap) {
-                out[2 * o] = b;
-                out[2 * o + 1] = (int32_t)(v - voff[b]);
-            }
-        }
-        run += tot;
+        const int64_t v = base + (int64_t)it * kBlock + threadIdx.x, u = v < nv ? v : nv - 1;
+        body[it] = vert_body[u];
+        // culling.py:67: lowers[i][1] < 0.5 * dhat + ground (FP64)
+        pred[it] = overlap(plo + 3 * u, phi + 3 * u, qlo, qhi) && v < nv;
     }
+#pragma unroll
+    for (int it = 0; it < kItems; ++it) pred[it] = pred[it] && (double)blo[3 * body[it] + 1] < ythresh;
+    int rank[kItems];
+#pragma unroll
+    for (int it = 0; it < kItems; ++it) {
+        const unsigned long long m = __ballot(pred[it]);
+        rank[it] = __popcll(m & ((1ull << lane_id()) - 1ull));
+        if (lane_id() == 0) cnt[it * kWaves + wave_id()] = __popcll(m);
+    }
+    __syncthreads();
+    int64_t run = WRITE ? boff[blockIdx.x] : 0;
+#pragma unroll
+    for (int it = 0; it < kItems; ++it)
+        for (int w = 0; w < kWaves; ++w) {
+            if (WRITE && pred[it] && w == wave_id()) {
+                const int64_t o = run + rank[it];
+                if (o < cap) {
+                    const int64_t v = base + (int64_t)it * kBlock + threadIdx.x;
+                    out[2 * o] = body[it];
+                    out[2 * o + 1] = (int32_t)(v - voff[body[it]]);
+                }
+            }
+            run += cnt[it * kWaves + w];
+        }
     if (!WRITE && threadIdx.x == 0) bcnt[blockIdx.x] = run;
 }
 
@@ -389,10 +463,9 @@ __global__ void structure_kernel(int nb, int64_t nij, const int64_t* __restrict_
 // so that a caller can run several cullings side by side and read all their counts in
 // one host synchronization.  `set` selects one of two independent workspaces.
 namespace {
-const int kCullSlots[2][8] = {
-    {kSlotHull1, kSlotHull2, kSlotFilter, kSlotFilterCount, kSlotScanA, kSlotScanB, kSlotChunkCount, kSlotChunk},
-    {kSlotHull1B, kSlotHull2B, kSlotFilterB, kSlotFilterCountB, kSlotScanAB, kSlotScanBB, kSlotChunkCountB,
-     kSlotChunkB}};
+const int kCullSlots[2][5] = {
+    {kSlotFilter, kSlotFilterCount, kSlotScanB, kSlotChunkCount, kSlotChunk},
+    {kSlotFilterB, kSlotFilterCountB, kSlotScanBB, kSlotChunkCountB, kSlotChunkB}};
 }  // namespace
 
 int prim_cull_begin(hipStream_t s, const AbdScene* sc, int mode, const int32_t* ij, int64_t nij, const float* lo1,
@@ -402,7 +475,6 @@ int prim_cull_begin(hipStream_t s, const AbdScene* sc, int mode, const int32_t* 
     C.set = set;
     C.pt = mode == ABD_CULL_PT;
     C.ij = ij;
-    const int nb = sc->n_bodies;
     PrimSets& S = C.S;
     S.off1 = C.pt ? sc->voff : sc->eoff;
     S.off2 = C.pt ? sc->foff : sc->eoff;
@@ -417,39 +489,19 @@ int prim_cull_begin(hipStream_t s, const AbdScene* sc, int mode, const int32_t* 
     C.nunits = C.pt ? 2 * nij : nij;
     if (2 * C.nunits > INT32_MAX) return ABD_ERR_ARG;
     int rc;
-    float *h1, *h2;
-    if ((rc = arena_get(slot[0], sizeof(float) * 6 * (size_t)nb, (void**)&h1))) return rc;
-    if ((rc = arena_get(slot[1], sizeof(float) * 6 * (size_t)nb, (void**)&h2))) return rc;
-    S.hlo1 = h1;
-    S.hhi1 = h1 + 3 * nb;
-    S.hlo2 = h2;
-    S.hhi2 = h2 + 3 * nb;
-    // both hulls in one launch; the EE culling compares one set of boxes with itself
-    const bool same = S.off1 == S.off2 && lo1 == lo2 && hi1 == hi2;
-    if (same) {
-        S.hlo2 = S.hlo1;
-        S.hhi2 = S.hhi1;
-    }
-    if (nb > 0) {
-        const HullSet H1{S.off1, lo1, hi1, h1, h1 + 3 * nb}, H2{S.off2, lo2, hi2, h2, h2 + 3 * nb};
-        launch_kernel(hull_kernel, dim3((unsigned)ceil_div(nb, kBlock / kWave), same ? 1 : 2), dim3(kBlock), 0,
-                           s, nb, H1, H2);
-        ABD_CHECK_LAUNCH();
-    }
-    if ((rc = arena_get(slot[2], sizeof(int32_t) * (size_t)(2 * C.nunits * C.maxs), (void**)&C.flist))) return rc;
-    if ((rc = arena_get(slot[3], sizeof(int64_t) * (size_t)(2 * C.nunits), (void**)&C.fcnt))) return rc;
-    if ((rc = arena_get(slot[4], sizeof(int64_t) * (size_t)(C.nunits + 1), (void**)&C.nchunk))) return rc;
-    if ((rc = arena_get(slot[5], sizeof(int64_t) * (size_t)(C.nunits + 1), (void**)&C.choff))) return rc;
+    if ((rc = arena_get(slot[0], sizeof(int32_t) * (size_t)(2 * C.nunits * C.maxs), (void**)&C.flist))) return rc;
+    if ((rc = arena_get(slot[1], sizeof(int64_t) * (size_t)(2 * C.nunits), (void**)&C.fcnt))) return rc;
+    if ((rc = arena_get(slot[2], sizeof(int64_t) * (size_t)(C.nunits + 1), (void**)&C.choff))) return rc;
     int ph = prof_start(kProfFilter, s, 0.0);
-    launch_kernel(filter_kernel, dim3((unsigned)(2 * C.nunits)), dim3(kBlock), 0, s, C.pt, ij, S, C.maxs,
+    launch_kernel(filter_kernel, dim3((unsigned)(ceil_div(2 * C.nunits, (int64_t)kXcds) * kXcds)), dim3(kBlock), 0, s,
+                  C.pt, ij, 2 * C.nunits, S, C.maxs,
                        C.flist, C.fcnt);
     ABD_CHECK_LAUNCH();
     prof_stop(ph, s);
     C.tune = tuning();
-    launch_kernel(unit_chunks_kernel, dim3(grid_for(C.nunits)), dim3(kBlock), 0, s, C.nunits, C.tune.cull_chunk,
-                       C.fcnt, C.nchunk);
+    launch_kernel(unit_chunks_kernel, dim3(1), dim3(kScanThreads), 0, s, C.nunits, C.tune.cull_chunk,
+                       (const int64_t*)C.fcnt, C.choff, C.choff + C.nunits, total_copy);
     ABD_CHECK_LAUNCH();
-    if ((rc = scan_exclusive_i64(s, C.nchunk, C.choff, C.nunits, C.choff + C.nunits, total_copy))) return rc;
     C.total_chunks = C.choff + C.nunits;
     C.total_pairs = nullptr;
     return ABD_OK;
@@ -460,8 +512,8 @@ int prim_cull_count(hipStream_t s, PrimCull& C, int64_t T, int64_t* total_copy) 
     C.T = T;
     if (T == 0) return ABD_OK;
     int rc;
-    if ((rc = arena_get(slot[6], sizeof(int64_t) * (size_t)(T + 1), (void**)&C.ccnt))) return rc;
-    if ((rc = arena_get(slot[7], sizeof(int64_t) * (size_t)(T + 1), (void**)&C.ccoff))) return rc;
+    if ((rc = arena_get(slot[3], sizeof(int64_t) * (size_t)(T + 1), (void**)&C.ccnt))) return rc;
+    if ((rc = arena_get(slot[4], sizeof(int64_t) * (size_t)(T + 1), (void**)&C.ccoff))) return rc;
     C.grid = (unsigned)(T < C.tune.cull_grid ? T : C.tune.cull_grid);
     int ph = prof_start(kProfPrimCount, s, 0.0);
     launch_kernel(prim_pairs_kernel<false>, dim3(C.grid), dim3(kBlock), 0, s, C.pt, C.tune.cull_chunk, C.ij, C.S,
@@ -535,33 +587,32 @@ int cull_bodies(hipStream_t s, const AbdScene* sc, const float* lo, const float*
     if (npairs <= 0) return ABD_OK;
     const int64_t nblk = ceil_div(npairs, (int64_t)kBlock * kPairItems);
     if (nblk > INT32_MAX) return ABD_ERR_ARG;
+    // both orders at once: counts, scans (the totals are equal), then the lists
+    const int orders = ji ? 2 : 1;
     int64_t *bcnt, *boff;
-    int rc = arena_get(kSlotScanA, sizeof(int64_t) * (nblk + 1), (void**)&bcnt);
+    int rc = arena_get(kSlotScanA, sizeof(int64_t) * orders * (nblk + 1), (void**)&bcnt);
     if (rc) return rc;
-    rc = arena_get(kSlotScanB, sizeof(int64_t) * (nblk + 1), (void**)&boff);
+    rc = arena_get(kSlotScanB, sizeof(int64_t) * orders * (nblk + 1), (void**)&boff);
     if (rc) return rc;
     int ph = prof_start(kProfBodyPairs, s, 24.0 * nb);
-    launch_kernel(body_pairs_kernel<false>, dim3((unsigned)nblk), dim3(kBlock), 0, s, nb, npairs, 0, sg,
-                       sc->body_scene, lo, hi, bcnt, (const int64_t*)nullptr, (int32_t*)nullptr, (int64_t)0);
+    launch_kernel(body_pairs_kernel<false>, dim3((unsigned)nblk, orders), dim3(kBlock), 0, s, nb, npairs, sg,
+                       sc->body_scene, lo, hi, bcnt, (const int64_t*)nullptr, (int32_t*)nullptr, (int32_t*)nullptr,
+                       (int64_t)0);
     ABD_CHECK_LAUNCH();
     prof_stop(ph, s);
-    if ((rc = scan_exclusive_i64(s, bcnt, boff, nblk, boff + nblk))) return rc;
+    ScanSeg sg2[2];
+    for (int k = 0; k < orders; ++k) {
+        const int64_t o = k * (nblk + 1);
+        sg2[k] = ScanSeg{bcnt + o, boff + o, nblk, boff + o + nblk, nullptr};
+    }
+    if ((rc = scan_exclusive_i64_multi(s, sg2, orders))) return rc;
     int64_t n;
     if ((rc = read_i64(s, boff + nblk, &n))) return rc;
     *count = n;
     if (n > cap) return ABD_ERR_OVERFLOW;
     if (n == 0) return ABD_OK;
-    launch_kernel(body_pairs_kernel<true>, dim3((unsigned)nblk), dim3(kBlock), 0, s, nb, npairs, 0, sg,
-                       sc->body_scene, lo, hi, bcnt, (const int64_t*)boff, ij, cap);
-    ABD_CHECK_LAUNCH();
-    if (!ji) return ABD_OK;
-    // (j, i) order: same predicate, second enumeration
-    launch_kernel(body_pairs_kernel<false>, dim3((unsigned)nblk), dim3(kBlock), 0, s, nb, npairs, 1, sg,
-                       sc->body_scene, lo, hi, bcnt, (const int64_t*)nullptr, (int32_t*)nullptr, (int64_t)0);
-    ABD_CHECK_LAUNCH();
-    if ((rc = scan_exclusive_i64(s, bcnt, boff, nblk, boff + nblk))) return rc;
-    launch_kernel(body_pairs_kernel<true>, dim3((unsigned)nblk), dim3(kBlock), 0, s, nb, npairs, 1, sg,
-                       sc->body_scene, lo, hi, bcnt, (const int64_t*)boff, ji, cap);
+    launch_kernel(body_pairs_kernel<true>, dim3((unsigned)nblk, orders), dim3(kBlock), 0, s, nb, npairs, sg,
+                       sc->body_scene, lo, hi, bcnt, (const int64_t*)boff, ij, ji, cap);
     ABD_CHECK_LAUNCH();
     return ABD_OK;
 }
@@ -663,7 +714,6 @@ constexpr int kKeepLists = 5;
 // blocks of a super-block: a block's offset is the sum of the super-blocks' counts before its
 // own (added to by the count pass: integers, any order) and of the blocks' before it inside
 constexpr int kSuper = 64;
-constexpr int kXcds = 8;
 // words between super-block counts: adds to one cache line wait for each other (about 10 ns
 // each: packed, a count pass of 18 k blocks took 108 us instead of 87)
 constexpr int kSuperStride = 8;
@@ -865,13 +915,6 @@ __device__ __forceinline__ int64_t keep_n(const KeepArgs& A, int k) {
     return A.in.dn ? (k == 1 && !A.in.ji ? 0 : A.in.dn[k]) : A.n[k];
 }
 
-// Which of n blocks the workgroup `loc` of a list takes (-1: none): the workgroups of one XCD
-// (they are dealt to the XCDs in turn) take a contiguous run of blocks, whose entries share
-// vertices in its L2.  n: the blocks in use, of a launch over at least as many rounded up.
-__device__ __forceinline__ int64_t xcd_block(int64_t loc, int64_t n) {
-    const int64_t run = (n + kXcds - 1) / kXcds, y = loc / kXcds, b = loc % kXcds * run + y;
-    return y < run && b < n ? b : -1;
-}
 __device__ __forceinline__ int64_t blocks_of(int64_t n) { return (n + kBlock - 1) / kBlock; }
 
 __global__ __launch_bounds__(kBlock) void keep_count_kernel(KeepArgs A) {

@@ -164,17 +164,30 @@ __device__ __forceinline__ void wave_extrema(const double* __restrict__ x, int v
         }
 }
 
-// culling2.py:171-210: the FP64 extrema of each body's vertices, one wave per body
-// (kBlock / 64 bodies per workgroup).  traj = 0: lo/hi = f32(min/max -+ dil);
-// traj = 1: lo/hi = min/max(lo/hi, f32(min/max)).
-__global__ __launch_bounds__(kBlock) void body_boxes_kernel(int nb, const int32_t* __restrict__ voff,
-                                                             const double* __restrict__ x, double dil, int traj,
-                                                             float* __restrict__ lo, float* __restrict__ hi) {
-    const int b = blockIdx.x * (kBlock / kWave) + wave_id();
-    if (b >= nb) return;  // the whole wave (no barrier)
+// culling2.py:171-210: the FP64 extrema of each body's vertices, one workgroup per body: one
+// wave, or four above 256 vertices (1024 bodies of 1072 vertices 17 us with one wave each, 10 here).
+// traj = 0: lo/hi = f32(min/max -+ dil); traj = 1: lo/hi = min/max(lo/hi, f32(min/max)).
+template <int T>
+__global__ __launch_bounds__(T) void body_boxes_kernel(const int32_t* __restrict__ voff,
+                                                        const double* __restrict__ x, double dil, int traj,
+                                                        float* __restrict__ lo, float* __restrict__ hi) {
+    __shared__ double sh[6 * (T / kWave)];
+    const int b = blockIdx.x;
     double mn[3], mx[3];
-    wave_extrema(x, voff[b], voff[b + 1], mn, mx);
-    if (lane_id() == 0)
+    for (int k = 0; k < 3; ++k) {
+        mn[k] = 1.0 / 0.0;
+        mx[k] = -1.0 / 0.0;
+    }
+    const int v1 = voff[b + 1];
+    for (int v = voff[b] + threadIdx.x; v < v1; v += T)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const double c = x[3 * (int64_t)v + k];
+            mn[k] = c < mn[k] ? c : mn[k];
+            mx[k] = c > mx[k] ? c : mx[k];
+        }
+    body_extrema<T>(mn, mx, sh);
+    if (threadIdx.x == 0)
         for (int k = 0; k < 3; ++k) {
             if (traj) {
                 hi[3 * b + k] = fmaxf(hi[3 * b + k], (float)mx[k]);
@@ -352,6 +365,19 @@ int swept_boxes(hipStream_t s, const AbdScene* sc, int kind, const double* x0, c
     return ABD_OK;
 }
 
+namespace {
+int body_boxes(hipStream_t s, const AbdScene* sc, const double* x, double dil, int traj, float* lo, float* hi) {
+    if (small_bodies(sc))
+        launch_kernel(body_boxes_kernel<kWave>, dim3(sc->n_bodies), dim3(kWave), 0, s, sc->voff, x, dil, traj, lo,
+                           hi);
+    else
+        launch_kernel(body_boxes_kernel<kBlock>, dim3(sc->n_bodies), dim3(kBlock), 0, s, sc->voff, x, dil, traj,
+                           lo, hi);
+    ABD_CHECK_LAUNCH();
+    return ABD_OK;
+}
+}  // namespace
+
 }  // namespace abd
 
 using namespace abd;
@@ -440,19 +466,13 @@ int abd_prim_boxes_traj(abd_stream_t stream, const AbdScene* sc, int32_t kind, c
 int abd_body_boxes(abd_stream_t stream, const AbdScene* sc, const double* x, double dil, float* lo, float* hi) {
     if (!sc || !x || !lo || !hi) return ABD_ERR_ARG;
     if (!sc->n_bodies) return ABD_OK;
-    launch_kernel(body_boxes_kernel, dim3((unsigned)ceil_div(sc->n_bodies, kBlock / kWave)), dim3(kBlock), 0,
-                       to_stream(stream), sc->n_bodies, sc->voff, x, dil, 0, lo, hi);
-    ABD_CHECK_LAUNCH();
-    return ABD_OK;
+    return body_boxes(to_stream(stream), sc, x, dil, 0, lo, hi);
 }
 
 int abd_body_boxes_traj(abd_stream_t stream, const AbdScene* sc, const double* x_end, float* lo, float* hi) {
     if (!sc || !x_end || !lo || !hi) return ABD_ERR_ARG;
     if (!sc->n_bodies) return ABD_OK;
-    launch_kernel(body_boxes_kernel, dim3((unsigned)ceil_div(sc->n_bodies, kBlock / kWave)), dim3(kBlock), 0,
-                       to_stream(stream), sc->n_bodies, sc->voff, x_end, 0.0, 1, lo, hi);
-    ABD_CHECK_LAUNCH();
-    return ABD_OK;
+    return body_boxes(to_stream(stream), sc, x_end, 0.0, 1, lo, hi);
 }
 
 int abd_update_q_scenes(abd_stream_t stream, const AbdScene* sc, const double* A, const double* p, const double* dq,

@@ -58,8 +58,6 @@ enum ArenaSlot {
     kSlotReduce,
     kSlotFlags,
     kSlotList,
-    kSlotHull1,
-    kSlotHull2,
     kSlotFilter,
     kSlotFilterCount,
     kSlotChunk,
@@ -72,11 +70,8 @@ enum ArenaSlot {
     kSlotPlan,
     kSlotPrecond,
     // a second primitive-culling workspace (culls run side by side) and the VG culling's
-    kSlotHull1B,
-    kSlotHull2B,
     kSlotFilterB,
     kSlotFilterCountB,
-    kSlotScanAB,
     kSlotScanBB,
     kSlotChunkCountB,
     kSlotChunkB,
@@ -103,7 +98,6 @@ struct PrimSets {
     const int32_t* off1;  // per-body offsets of set 1 (PT points / EE edges)
     const int32_t* off2;  // set 2 (PT triangles / EE edges)
     const float *lo1, *hi1, *lo2, *hi2;
-    const float *hlo1, *hhi1, *hlo2, *hhi2;  // per-body hulls
 };
 struct PrimCull {
     int set = 0, pt = 0;
@@ -111,7 +105,7 @@ struct PrimCull {
     PrimSets S{};
     int64_t nunits = 0, maxs = 0, T = 0;
     int32_t* flist = nullptr;
-    int64_t *fcnt = nullptr, *nchunk = nullptr, *choff = nullptr, *ccnt = nullptr, *ccoff = nullptr;
+    int64_t *fcnt = nullptr, *choff = nullptr, *ccnt = nullptr, *ccoff = nullptr;
     const int64_t* total_chunks = nullptr;  // device, after begin
     const int64_t* total_pairs = nullptr;   // device, after count
     AbdTuning tune{};
@@ -233,6 +227,8 @@ struct BodyStart {
     int32_t* it;
     int64_t* range_flag;
 };
+// Whether a body's workgroup is one wave (abd_body.hip).
+bool small_bodies(const AbdScene* sc);
 int body_start(hipStream_t s, const AbdScene* sc, const AbdParams* P, const BodyStart& U);
 // body_end: x = x(q - dq) of the scenes in active (x(q) of the others), the union (slo, shi)
 // of the body boxes there and blo, bhi; with lo, hi the range test (margin inside them) into

@@ -377,3 +377,33 @@ def test_recording_leaves_other_threads_alone():
         done.set()
         th.join()
     assert not errors and rounds[0] > 0
+
+
+@pytest.mark.parametrize("nb", [2, 3, 6])
+@pytest.mark.parametrize("mesh", ["cube", "ico3"])
+def test_culling_pass_edges(nb, mesh):
+    """The collision set of overlapping bodies below one pass of the primitive filter (a cube's
+    8, 18 and 12) and above it (642 points, 1920 edges, 1280 triangles; 1024 a pass), with
+    fewer and more tasks than XCDs: the oracle's lists, exactly."""
+    import abd_hip
+    from abd_hip import scenes
+    from test_gpu_parity import T, _gpu_scene, _stage_lists, oracle_lists
+    abd_hip.load()
+    m = scenes.cube_mesh() if mesh == "cube" else scenes.icosphere_mesh(3, 0.5)
+    h = m[0][:, 1].max() - m[0][:, 1].min()
+    rng = np.random.default_rng(nb)
+    p = np.array([[0.02 * k, 0.45 * h + 0.97 * h * k, 0.01 * k] for k in range(nb)])
+    A = np.stack([np.linalg.qr(np.eye(3) + 0.05 * rng.normal(size=(3, 3)))[0] for _ in range(nb)])
+    spec = scenes.build_scene([m] * nb, A, p, np.zeros((nb, 3, 3)), np.zeros((nb, 3)), ground=0.0)
+    cp = params(ground=0.0)
+    g = _gpu_scene(spec)
+    sc = O.OracleScene(spec)
+    x = O.project(sc, spec.A, spec.p)
+    g.x.copy_(T(x))
+    g.xk.copy_(T(x))
+    G = _stage_lists(g, cp)
+    R = oracle_lists(sc, x, cp.dhat, cp.ground)
+    assert len(R["ij"]) == nb - 1 and len(R["ee"]) and len(R["vg"])
+    assert np.array_equal(G["pairs"].ij.cpu().numpy(), R["ij"])
+    for k in ("pt", "ee", "vg"):
+        assert np.array_equal(G[k].cpu().numpy(), R[k]), k
