@@ -162,8 +162,7 @@ struct CandSide {
 };
 // Line-search trials q - alpha dq of at most kMaxTrials lengths at once (S = 1: the whole
 // system as one scene).  trial_states: the bodies' states st [K][nb][12] (16-byte aligned)
-// and inertia energies e [K][nb] at alpha [K][S] (device), or with `halve` at alpha[s] / 2^k;
-// a negative length is skipped.  line_chunks: the chunks' contact energies at alpha [K][S]
+// and inertia energies e [K][nb] at alpha [K][S] (device); a negative length is skipped.  line_chunks: the chunks' contact energies at alpha [K][S]
 // (negative: 0) over a planned set, scene s's at trial k part[stride k + choff[s] ..
 // choff[s + 1]) in the order their sum is taken.
 constexpr int kMaxTrials = 12;
@@ -172,7 +171,7 @@ struct TrialSums {
     const double* part;
     int64_t stride;
 };
-int trial_states(hipStream_t s, const AbdScene* sc, const AbdParams* P, int S, int K, const double* alpha, bool halve,
+int trial_states(hipStream_t s, const AbdScene* sc, const AbdParams* P, int S, int K, const double* alpha,
                  const double* A, const double* p, const double* dq, const double* A0, const double* p0,
                  const double* Adot, const double* pdot, double* st, double* e);
 int line_chunks(hipStream_t s, const AbdScene* sc, const AbdParams* P, int S, int K, const double* alpha,
@@ -325,10 +324,13 @@ size_t keep_counters(int64_t nij, int64_t npt, int64_t nee, int64_t nvg);
 int toi_scratch(int S, int64_t nq, unsigned long long** slots, int32_t** qcount, int32_t** queue);
 // The reduction plan (int64 [reduce_plan_elems(S)]) of the lists a sweep wrote (dn: their
 // sizes on the device in the keep layout; npt, nee bound them), the scene minima from the
-// queued candidates, the first step lengths and the scenes' dots.
+// queued candidates, the first step lengths, the scenes' dots, and the states and inertia
+// energies (trial_states') of K trials of the first lengths halved k times.
 int sweep_toi(hipStream_t s, const AbdScene* sc, const AbdParams* P, int S, const double* x_t0, const double* x_t1,
               const int32_t* pt, int64_t npt, const int32_t* ee, int64_t nee, const int64_t* dn, CandSide side,
-              const KeepSweep& W, int64_t* plan, double* toi, double* first_alpha, const SceneDots& dots);
+              const KeepSweep& W, int64_t* plan, double* toi, double* first_alpha, const SceneDots& dots, int K,
+              const double* A, const double* p, const double* dq, const double* A0, const double* p0,
+              const double* Adot, const double* pdot, double* st, double* e);
 // sync false: the totals reach hcount with the stream's next synchronization (the caller's);
 // hcount null: they stay on the device.
 // counters (nullable): keep_counters words zeroed before (else the call zeroes its own).

@@ -171,38 +171,86 @@ struct VertsTrial {
     }
 };
 
-// The bodies' trial states q - alpha dq (st [K][nb][12]) and inertia energies there (e
-// [K][nb]) of K trials.  halve: trial k has the length alpha[scene] / 2^k (the halvings of a
-// line search are known with its first length), else alpha[k][scene]; a negative length
-// leaves its trial unwritten.  One thread per (body, trial): the energies' kernels and
-// every candidate evaluated then read 96 bytes of a body instead of forming its state.
-__global__ __launch_bounds__(kRedThreads) void trial_states_kernel(AbdScene sc, AbdParams P, int S, int K,
-                                                                   const double* __restrict__ alpha, int halve,
-                                                                   const double* __restrict__ A,
-                                                                   const double* __restrict__ p,
-                                                                   const double* __restrict__ dq,
-                                                                   const double* __restrict__ A0,
-                                                                   const double* __restrict__ p0,
-                                                                   const double* __restrict__ Adot,
-                                                                   const double* __restrict__ pdot,
-                                                                   double* __restrict__ st, double* __restrict__ e) {
-    const int64_t i = (int64_t)blockIdx.x * kRedThreads + threadIdx.x;
-    const int nb = sc.n_bodies;
-    if (i >= (int64_t)nb * K) return;
-    const int b = (int)(i % nb), k = (int)(i / nb);
-    const int s = S > 1 ? sc.body_scene[b] : 0;
-    double al = halve ? alpha[s] : alpha[(int64_t)k * S + s];
+// Trial i = k nb + b of the bodies' states q - alpha dq and inertia energies: its state st[i]
+// (12) and energy e[i] at length al; a negative length leaves it unwritten.
+struct StateArgs {
+    const double *A, *p, *dq, *A0, *p0, *Adot, *pdot;
+    double *st, *e;
+};
+__device__ __forceinline__ void trial_state_of(const AbdScene& sc, const AbdParams& P, const StateArgs& Q, int64_t i,
+                                               int b, double al) {
     if (al < 0.0) return;
-    if (halve)
-        for (int q = 0; q < k; ++q) al *= 0.5;
     double Ab[9], pb[3];
-    trial_state(b, al, A, p, dq, Ab, pb);
-    double* o = st + 12 * i;
+    trial_state(b, al, Q.A, Q.p, Q.dq, Ab, pb);
+    double* o = Q.st + 12 * i;
 #pragma unroll
     for (int q = 0; q < 9; ++q) o[q] = Ab[q];
 #pragma unroll
     for (int q = 0; q < 3; ++q) o[9 + q] = pb[q];
-    e[i] = inertia_energy_q(P, sc.mass, sc.I0, b, Ab, pb, A0, p0, Adot, pdot);
+    Q.e[i] = inertia_energy_q(P, sc.mass, sc.I0, b, Ab, pb, Q.A0, Q.p0, Q.Adot, Q.pdot);
+}
+// The states of K trials of lengths alpha [K][S].  One thread per (body, trial): the energies'
+// kernels and every candidate evaluated then read 96 bytes of a body instead of forming its
+// state.
+__global__ __launch_bounds__(kRedThreads) void trial_states_kernel(AbdScene sc, AbdParams P, int S, int K,
+                                                                   const double* __restrict__ alpha, StateArgs Q) {
+    const int64_t i = (int64_t)blockIdx.x * kRedThreads + threadIdx.x;
+    const int nb = sc.n_bodies;
+    if (i >= (int64_t)nb * K) return;
+    const int b = (int)(i % nb), k = (int)(i / nb);
+    trial_state_of(sc, P, Q, i, b, alpha[(int64_t)k * S + (S > 1 ? sc.body_scene[b] : 0)]);
+}
+
+// The line search's start: workgroup s < S takes scene s's TOI from its slot to out and the
+// first step length to alpha (first_step_length; -1 for a scene not in `active`) with the
+// scene's dots (seg_dot_kernel's sums); the others form the states of K trials, the first
+// lengths and their halvings (known with the TOI).
+__global__ __launch_bounds__(kRedThreads) void search_start_kernel(AbdScene sc, AbdParams P, int S, int K,
+                                                                   const unsigned long long* __restrict__ slots,
+                                                                   const uint8_t* __restrict__ active,
+                                                                   double* __restrict__ out,
+                                                                   double* __restrict__ alpha, SceneDots D,
+                                                                   StateArgs Q) {
+    __shared__ double sh[34];
+    if ((int)blockIdx.x >= S) {
+        const int64_t i = (int64_t)(blockIdx.x - S) * kRedThreads + threadIdx.x;
+        const int nb = sc.n_bodies;
+        if (i >= (int64_t)nb * K) return;
+        const int b = (int)(i % nb), s = S > 1 ? sc.body_scene[b] : 0;
+        double al = active[s] ? first_step_length(__longlong_as_double((long long)slots[s])) : -1.0;
+        for (int q = (int)(i / nb); q > 0; --q) al *= 0.5;
+        trial_state_of(sc, P, Q, i, b, al);
+        return;
+    }
+    const int s = blockIdx.x;
+    if (threadIdx.x == 0) {
+        const double r = __longlong_as_double((long long)slots[s]);
+        out[s] = r;
+        alpha[s] = active[s] ? first_step_length(r) : -1.0;
+    }
+    const int64_t i0 = D.sboff ? 12 * (int64_t)D.sboff[s] : 0, i1 = D.sboff ? 12 * (int64_t)D.sboff[s + 1] : D.n;
+    double acc1 = 0.0, acc2 = 0.0;
+    constexpr int kAtOnce = 4;  // terms whose loads are in flight together
+    for (int64_t i = i0 + threadIdx.x; i < i1; i += kAtOnce * kRedThreads) {
+        double v1[kAtOnce], v2[kAtOnce];
+#pragma unroll
+        for (int j = 0; j < kAtOnce; ++j) {
+            const int64_t q = i + j * kRedThreads < i1 ? i + j * kRedThreads : i;
+            v1[j] = D.a[q] * D.b[q];
+            v2[j] = D.c[q] * D.d[q];
+        }
+#pragma unroll
+        for (int j = 0; j < kAtOnce; ++j)
+            if (i + j * kRedThreads < i1) {
+                acc1 += v1[j];
+                acc2 += v2[j];
+            }
+    }
+    block_sum2_fast(acc1, acc2, sh);
+    if (threadIdx.x == 0) {
+        D.out1[s] = acc1;
+        D.out2[s] = acc2;
+    }
 }
 
 // ipcsk/energy.py:10-48 per candidate
@@ -550,43 +598,19 @@ __global__ __launch_bounds__(kToiSolveThreads) void toi_solve_kernel(AbdScene sc
     }
 }
 
-// choff (nullable): no partials, the slots hold every list's minima.  alpha (nullable): the
-// line search's first step length of each scene from its TOI (first_step_length; -1 for a
-// scene not in `active`)
 __global__ __launch_bounds__(kRedThreads) void toi_final_kernel(const int64_t* __restrict__ choff,
                                                                 const double* __restrict__ part,
                                                                 const unsigned long long* __restrict__ slots,
-                                                                double* __restrict__ out,
-                                                                const uint8_t* __restrict__ active,
-                                                                double* __restrict__ alpha, SceneDots D) {
-    __shared__ double sh[kRedThreads];
+                                                                double* __restrict__ out) {
+    __shared__ double sh[kRedThreads / kWave];
     const int s = blockIdx.x;
     double acc = __longlong_as_double((long long)slots[s]);
-    double r = acc;
-    if (choff) {
-        for (int64_t i = choff[s] * kToiSplit + threadIdx.x; i < choff[s + 1] * kToiSplit; i += blockDim.x) {
-            const double v = part[i];
-            acc = v < acc ? v : acc;
-        }
-        r = block_min(acc, sh);
+    for (int64_t i = choff[s] * kToiSplit + threadIdx.x; i < choff[s + 1] * kToiSplit; i += blockDim.x) {
+        const double v = part[i];
+        acc = v < acc ? v : acc;
     }
-    if (threadIdx.x == 0) {
-        out[s] = r;
-        if (alpha) alpha[s] = !active || active[s] ? first_step_length(r) : -1.0;
-    }
-    if (D.out1) {  // uniform: seg_dot_kernel's sums of this scene
-        const int64_t i0 = D.sboff ? 12 * (int64_t)D.sboff[s] : 0, i1 = D.sboff ? 12 * (int64_t)D.sboff[s + 1] : D.n;
-        double acc1 = 0.0, acc2 = 0.0;
-        for (int64_t i = i0 + threadIdx.x; i < i1; i += blockDim.x) {
-            acc1 += D.a[i] * D.b[i];
-            acc2 += D.c[i] * D.d[i];
-        }
-        block_sum2_fast(acc1, acc2, sh);
-        if (threadIdx.x == 0) {
-            D.out1[s] = acc1;
-            D.out2[s] = acc2;
-        }
-    }
+    const double r = block_min(acc, sh);
+    if (threadIdx.x == 0) out[s] = r;
 }
 
 // out[s] = sum over the rows [12 sboff[s], 12 sboff[s + 1]) of a * b (one workgroup per scene;
@@ -768,8 +792,7 @@ int toi_reduce(hipStream_t s, const AbdScene& sc, const AbdParams& P, int S, con
     if ((rc = attach_seg_bytes(ph, s, S, 1, nullptr, seg, 228.0, 224.0, 56.0))) return rc;
     if ((rc = toi_solve(s, sc, S, x0, x1, L, w.queue, w.qcount, w.slots, !scr))) return rc;
     launch_kernel(toi_final_kernel, dim3(S), dim3(kRedThreads), 0, s, choff, (const double*)w.part,
-                       (const unsigned long long*)w.slots, out, (const uint8_t*)nullptr, (double*)nullptr,
-                       SceneDots{});
+                       (const unsigned long long*)w.slots, out);
     ABD_CHECK_LAUNCH();
     return ABD_OK;
 }
@@ -795,13 +818,13 @@ size_t reduce_plan_elems(int S) { return 2 * kLists * (size_t)S + (size_t)S + 1;
 // treats the scene as one): per scene the chunks' contact energies of every trial, each
 // bit-identical to the chunk sums at that state.
 
-int trial_states(hipStream_t s, const AbdScene* sc, const AbdParams* P, int S, int K, const double* alpha, bool halve,
+int trial_states(hipStream_t s, const AbdScene* sc, const AbdParams* P, int S, int K, const double* alpha,
                  const double* A, const double* p, const double* dq, const double* A0, const double* p0,
                  const double* Adot, const double* pdot, double* st, double* e) {
     const int64_t n = (int64_t)sc->n_bodies * K;
     if (n <= 0) return ABD_OK;
-    launch_kernel(trial_states_kernel, dim3(grid_for(n, kRedThreads, INT32_MAX)), dim3(kRedThreads), 0, s, *sc,
-                       *P, S, K, alpha, halve ? 1 : 0, A, p, dq, A0, p0, Adot, pdot, st, e);
+    launch_kernel(trial_states_kernel, dim3(grid_for(n, kRedThreads, INT32_MAX)), dim3(kRedThreads), 0, s, *sc, *P, S,
+                  K, alpha, StateArgs{A, p, dq, A0, p0, Adot, pdot, st, e});
     ABD_CHECK_LAUNCH();
     return ABD_OK;
 }
@@ -856,7 +879,9 @@ int contact_energy(hipStream_t s, const AbdScene* sc, const AbdParams* P, int S,
 
 int sweep_toi(hipStream_t s, const AbdScene* sc, const AbdParams* P, int S, const double* x_t0, const double* x_t1,
               const int32_t* pt, int64_t npt, const int32_t* ee, int64_t nee, const int64_t* dn, CandSide side,
-              const KeepSweep& W, int64_t* plan, double* toi, double* first_alpha, const SceneDots& dots) {
+              const KeepSweep& W, int64_t* plan, double* toi, double* first_alpha, const SceneDots& dots, int K,
+              const double* A, const double* p, const double* dq, const double* A0, const double* p0,
+              const double* Adot, const double* pdot, double* st, double* e) {
     const Lists L = contact_lists(*P, pt, npt, ee, nee, nullptr, 0, nullptr, side);
     SweepPlan Q;
     Q.scnt = W.scnt;
@@ -867,8 +892,11 @@ int sweep_toi(hipStream_t s, const AbdScene* sc, const AbdParams* P, int S, cons
     Q.plan = plan;
     int rc;
     if ((rc = toi_solve(s, *sc, S, x_t0, x_t1, L, W.queue, W.qcount, W.slots, true, Q))) return rc;
-    launch_kernel(toi_final_kernel, dim3(S), dim3(kRedThreads), 0, s, (const int64_t*)nullptr,
-                       (const double*)nullptr, (const unsigned long long*)W.slots, toi, W.active, first_alpha, dots);
+    const int64_t blocks = S + ceil_div((int64_t)sc->n_bodies * K, (int64_t)kRedThreads);
+    if (blocks > INT32_MAX) return ABD_ERR_ARG;
+    launch_kernel(search_start_kernel, dim3((unsigned)blocks), dim3(kRedThreads), 0, s, *sc, *P, S, K,
+                  (const unsigned long long*)W.slots, W.active, toi, first_alpha, dots,
+                  StateArgs{A, p, dq, A0, p0, Adot, pdot, st, e});
     ABD_CHECK_LAUNCH();
     return ABD_OK;
 }

@@ -604,12 +604,14 @@ constexpr int kLsThreads = 256;
 // alpha_min (trials_to_floor), -1 past them and for the scenes not searching.  One workgroup
 // per scene; the totals over the scenes are integers, added by atomics (zeroed before the
 // first pass).
+// M: trials of the pass at most (1 for the first).
+template <int M>
 __global__ __launch_bounds__(kLsThreads) void ls_pass_kernel(LsDev L, double c1, double alpha_min, double tol,
                                                               int max_iter, int first, int K,
                                                               double* __restrict__ alpha, TrialSums C,
                                                               const double* __restrict__ e,
                                                               const int32_t* __restrict__ sboff, int nb) {
-    __shared__ double sh[34];
+    __shared__ double sh[M][2][kLsThreads / kWave];
     const int s = blockIdx.x, ns = L.ns, t = threadIdx.x;
     const bool searching = first ? L.newton[s] != 0 : L.search[s] != 0;  // uniform
     if (!searching) {
@@ -628,21 +630,54 @@ __global__ __launch_bounds__(kLsThreads) void ls_pass_kernel(LsDev L, double c1,
     const int b0 = sboff ? sboff[s] : 0, b1 = sboff ? sboff[s + 1] : nb;
     const int64_t c0 = C.choff[s], c1_ = C.choff[s + 1];
     const double e0 = L.E0[s], qtg = L.qtg[s];
+    // the trials' sums side by side, then one barrier for all (one trial after the other, with
+    // its loads' latency and two barriers each, the second pass of 1024 bodies took 20 us; 10.5
+    // here)
+    double al[M], ec[M], ei[M];
+#pragma unroll
+    for (int k = 0; k < M; ++k) {
+        al[k] = k < K ? alpha[(int64_t)k * ns + s] : -1.0;
+        ec[k] = ei[k] = 0.0;
+    }
+    int nk = 0;  // this scene's trials
+#pragma unroll
+    for (int k = 0; k < M; ++k)
+        if (nk == k && al[k] >= 0.0) nk = k + 1;
+    // (a trial past nk reads the first one's: the loads have no branch and issue together)
+    for (int64_t i = c0 + t; i < c1_; i += kLsThreads) {
+        double v[M];
+#pragma unroll
+        for (int k = 0; k < M; ++k) v[k] = C.part[k < nk ? C.stride * k + i : i];
+#pragma unroll
+        for (int k = 0; k < M; ++k) ec[k] += v[k];
+    }
+    for (int b = b0 + t; b < b1; b += kLsThreads) {
+        double v[M];
+#pragma unroll
+        for (int k = 0; k < M; ++k) v[k] = e[k < nk ? (int64_t)nb * k + b : b];
+#pragma unroll
+        for (int k = 0; k < M; ++k) ei[k] += v[k];
+    }
+#pragma unroll
+    for (int k = 0; k < M; ++k)
+        if (k < nk) {  // uniform
+            const double wc = wave_sum(ec[k]), wi = wave_sum(ei[k]);
+            if (lane_id() == 0) {
+                sh[k][0][wave_id()] = wc;
+                sh[k][1][wave_id()] = wi;
+            }
+        }
+    __syncthreads();  // (and every thread has read this pass's trials)
     double last = 0.0, e1 = 0.0;
     bool acc = false;
-    for (int k = 0; k < K && !acc; ++k) {
-        const double a = alpha[(int64_t)k * ns + s];
-        if (a < 0.0) break;  // past this scene's trials
-        last = a;
-        double ec = 0.0, ei = 0.0;
-        for (int64_t i = c0 + t; i < c1_; i += kLsThreads) ec += C.part[C.stride * k + i];
-        for (int b = b0 + t; b < b1; b += kLsThreads) ei += e[(int64_t)nb * k + b];
-        block_sum2_fast(ec, ei, sh);
-        e1 = ec + ei;
-        const bool wolfe = e1 < e0 + c1 * a * qtg;
-        acc = wolfe || a < alpha_min;
-    }
-    __syncthreads();  // every thread has read this pass's trials
+#pragma unroll
+    for (int k = 0; k < M; ++k)
+        if (k < nk && !acc) {
+            last = al[k];
+            e1 = waves_sum(sh[k][0], kLsThreads / kWave) + waves_sum(sh[k][1], kLsThreads / kWave);
+            const bool wolfe = e1 < e0 + c1 * last * qtg;
+            acc = wolfe || last < alpha_min;
+        }
     const double a0 = last * 0.5;  // the next pass's first trial
     const int need = acc ? 0 : trials_to_floor(a0, alpha_min);
     if (t < kLsSpec) {
@@ -732,18 +767,18 @@ int line_pass(hipStream_t s, Sim& S, const LsDev& L, bool first, int K, int k0) 
     if ((rc = line_chunks(s, &S.sc, &S.P, S.ns, K, S.cand_alpha.p, S.trial_st.p + 12 * nb * k0, S.sw.ptl.p, S.sw.npt,
                           S.sw.eel.p, S.sw.nee, S.sw.vgl.p, S.sw.nvg, S.plan.p, S.sw.counts(), S.sw.side(), &C)))
         return rc;
-    launch_kernel(ls_pass_kernel, dim3(S.ns), dim3(kLsThreads), 0, s, L, S.P.c1, S.P.alpha_min, S.P.tol,
-                       (int)S.P.max_iter, first ? 1 : 0, K, S.cand_alpha.p, C,
+    launch_kernel(K == 1 ? ls_pass_kernel<1> : ls_pass_kernel<kLsSpec>, dim3(S.ns), dim3(kLsThreads), 0, s, L, S.P.c1,
+                  S.P.alpha_min, S.P.tol, (int)S.P.max_iter, first ? 1 : 0, K, S.cand_alpha.p, C,
                        (const double*)(S.trial_e.p + nb * k0), S.ns > 1 ? S.sc.scene_boff : nullptr, S.nb);
     ABD_CHECK_LAUNCH();
     return ABD_OK;
 }
 
 // The trial states of K trials into trial_st from trial k0 on
-int pass_states(hipStream_t s, Sim& S, int K, bool halve, int k0) {
+int pass_states(hipStream_t s, Sim& S, int K, int k0) {
     const AbdSimState& st = S.st;
     const int64_t nb = S.nb;
-    return trial_states(s, &S.sc, &S.P, S.ns, K, S.cand_alpha.p, halve, st.A, st.p, st.dq, st.A0, st.p0, st.Adot,
+    return trial_states(s, &S.sc, &S.P, S.ns, K, S.cand_alpha.p, st.A, st.p, st.dq, st.A0, st.p0, st.Adot,
                         st.pdot, S.trial_st.p + 12 * nb * k0, S.trial_e.p + nb * k0);
 }
 
@@ -804,11 +839,11 @@ int ccd_and_search_scenes(hipStream_t s, Sim& S, const LsDev& L) {
     qg.out1 = S.sv.p + kSvQtg * ns;
     qg.out2 = S.sv.p + kSvGtg * ns;
     if ((rc = sweep_toi(s, &S.sc, &P, ns, st.x, st.xk, W.ptl.p, W.npt, W.eel.p, W.nee, W.counts(), W.side(),
-                        sweep_of(S), S.plan.p, S.sv.p + kSvToi * ns, S.cand_alpha.p, qg)))
+                        sweep_of(S), S.plan.p, S.sv.p + kSvToi * ns, S.cand_alpha.p, qg,
+                        1 + kLsSpec, st.A, st.p, st.dq, st.A0, st.p0, st.Adot, st.pdot, S.trial_st.p, S.trial_e.p)))
         return rc;
     // the line search: the first trial, then every remaining halving of the scenes that
     // rejected it, each decided on the device
-    if ((rc = pass_states(s, S, 1 + kLsSpec, true, 0))) return rc;
     if ((rc = line_pass(s, S, L, true, 1, 0))) return rc;
     if ((rc = line_pass(s, S, L, false, kLsSpec, 1))) return rc;
     return copy_to_host(s, S.hcnt, S.cnt.p, kCntLen * sizeof(int64_t));
@@ -1006,7 +1041,7 @@ int step_scenes(hipStream_t s, Sim& S) {
         while (S.hcnt[kCntSearch] > 0) {
             const int64_t K = S.hcnt[kCntK2];
             if ((rc = zero_fill(s, S.cnt.p + kCntK2, sizeof(int64_t)))) return rc;
-            if ((rc = pass_states(s, S, kLsSpec, false, 1))) return rc;
+            if ((rc = pass_states(s, S, kLsSpec, 1))) return rc;
             if ((rc = line_pass(s, S, L, false, kLsSpec, 1))) return rc;
             if ((rc = read_counts(s, S))) return rc;
             S.stats[5] += K;
