@@ -407,3 +407,29 @@ def test_culling_pass_edges(nb, mesh):
     assert np.array_equal(G["pairs"].ij.cpu().numpy(), R["ij"])
     for k in ("pt", "ee", "vg"):
         assert np.array_equal(G[k].cpu().numpy(), R[k]), k
+
+
+@pytest.mark.parametrize("block", [False, True])
+@pytest.mark.parametrize("maxiter,check", [(1, 10), (7, 10), (10, 10), (11, 5), (40, 4)])
+def test_large_cg_batches(block, maxiter, check):
+    """CG over several workgroups (171 bodies) cut off and checked at the ends of its batches:
+    the oracle's iterate and count.  Both run the same recurrence in double; after at most 40
+    iterations of a system of condition below 3 they agree to 1e-9."""
+    import abd_hip
+    from abd_hip.sparse import BsrMatrix, SolveInfo, bsr_cg
+    from test_gpu_ldlt import _structure, _system
+    lib = abd_hip.load()
+    m = 171
+    rng = np.random.default_rng(8)
+    ij = np.array(sorted({tuple(sorted(rng.choice(m, 2, replace=False).tolist())) for _ in range(200)}), np.int32)
+    blocks, _ = _system(m, ij, rng)
+    b = rng.normal(size=(4 * m, 3))
+    x0 = 0.01 * rng.normal(size=(4 * m, 3))
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    A = BsrMatrix(m, *_structure(lib, m, ij), d(blocks))
+    x, info = d(x0), SolveInfo("cuda")
+    tol = 1e-6
+    bsr_cg(A, x, d(b), maxiter, tol, check, info, block_precond=block)
+    ref, it, _ = (O.bsr_cg_block if block else O.bsr_cg)(m, ij, blocks, b, x0, tol, maxiter, check)
+    assert int(info.iters[0]) == it
+    assert rel_err(x.cpu().numpy(), ref) <= 1e-9
