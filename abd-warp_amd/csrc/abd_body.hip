@@ -6,7 +6,8 @@
 // (update_q, the rows' commit, projection, body boxes, fills, inertia terms) and the step's end
 // (projection with the range test, swept body boxes) took 8 launches and read the vertices
 // again for the boxes and, for the range test, 72 bytes of ranges and start positions: 108 us
-// an iteration for 1.06M vertices of 8217 bodies, against 48 us here (29 + 19).
+// an iteration for 1.06M vertices of 8217 bodies, against 48 us here (29 + 19; 59 where the
+// step's end also writes the vertices' swept boxes for the filter after it).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -109,7 +110,7 @@ __global__ __launch_bounds__(T) void body_start_kernel(AbdScene sc, AbdParams P,
 // skin, far above the rounding of positions.)
 template <int T>
 __global__ __launch_bounds__(T) void body_end_kernel(AbdScene sc, BodyEnd U) {
-    __shared__ double q[12];
+    __shared__ double q[12], q0[12];
     __shared__ double sh[6 * (T / kWave)];
     const int b = blockIdx.x, t = threadIdx.x;
     const double al = U.active[U.ns > 1 ? sc.body_scene[b] : 0] ? 1.0 : 0.0;
@@ -117,6 +118,7 @@ __global__ __launch_bounds__(T) void body_end_kernel(AbdScene sc, BodyEnd U) {
         const double v = t < 9 ? U.A[9 * b + t] : U.p[3 * b + t - 9];
         const double d = t < 9 ? U.dq[3 * (4 * b + 1 + t / 3) + t % 3] : U.dq[12 * b + t - 9];
         q[t] = al == 0.0 ? v : v - d * al;
+        q0[t] = v;
     }
     __syncthreads();
     bool test = U.lo != nullptr;
@@ -143,14 +145,25 @@ __global__ __launch_bounds__(T) void body_end_kernel(AbdScene sc, BodyEnd U) {
     const int v1 = sc.voff[b + 1];
     for (int64_t v = sc.voff[b] + t; v < v1; v += T) {
         const double r[3] = {sc.x0[3 * v], sc.x0[3 * v + 1], sc.x0[3 * v + 2]};
+        float e[6];
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
-            const double c = place(q, r, k);
+            const double c = place(q, r, k), c0 = place(q0, r, k);
             U.x[3 * v + k] = c;
+            e[k] = fminf((float)(c0 - U.dil), (float)(c - U.dil));
+            e[3 + k] = fmaxf((float)(c0 + U.dil), (float)(c + U.dil));
+            if (!(c - c0 == c - c0)) {  // not finite: a box that overlaps every other
+                e[k] = -INFINITY;
+                e[3 + k] = INFINITY;
+            }
             mn[k] = c < mn[k] ? c : mn[k];
             mx[k] = c > mx[k] ? c : mx[k];
             if (test)
                 out |= !(c - U.margin >= U.lo[3 * v + k] && c + U.margin <= U.hi[3 * v + k]);  // NaN: outside
+        }
+        if (U.ebox) {
+            U.ebox[2 * v] = make_float4(e[0], e[1], e[2], e[3]);
+            U.ebox[2 * v + 1] = make_float4(e[4], e[5], 0.0f, 0.0f);
         }
     }
     if (__any(out) && lane_id() == 0) *U.flag = 1;  // every writer stores 1

@@ -981,8 +981,8 @@ int contact_gh(hipStream_t s, const AbdScene* sc, const AbdParams* P, const doub
         if ((rc = arena_get(kSlotScanA, sizeof(uint32_t) * ((size_t)nblk + 1), (void**)&bcnt))) return rc;
         int ph = prof_start(kProfClassify, s, dn ? 1.0 : 129.0 * npt + 133.0 * nee + 8.0 * nvg);
         const int64_t blocks_all = nblk + ceil_div(nvg, (int64_t)kBlock);
-        launch_kernel(classify_kernel, dim3((unsigned)std::min<int64_t>(blocks_all, 8192)), dim3(kBlock), 0, s, *sc, *P, x,
-                           pt, npt, ee, nee, vg, nvg, dn, flag, G.err, bcnt, G.scnt);
+        launch_kernel(classify_kernel, dim3((unsigned)std::min<int64_t>(blocks_all, 8192)), dim3(kBlock), 0, s, *sc,
+                      *P, x, pt, npt, ee, nee, vg, nvg, dn, flag, G.err, bcnt, G.scnt);
         ABD_CHECK_LAUNCH();
         prof_stop(ph, s);
         if ((rc = prof_count_bytes(ph, s, dn, 129.0, 133.0, 8.0, 0.0))) return rc;

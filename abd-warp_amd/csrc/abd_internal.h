@@ -245,6 +245,7 @@ struct BodyEnd {
     double skin, margin;
     int64_t* flag;
     uint8_t* on;  // [nb] active of the body's scene
+    float4* ebox;  // nullable: [nv][2] the vertices' boxes at both ends dilated by dil in FP64: lo, hi, 0, 0
 };
 int body_end(hipStream_t s, const AbdScene* sc, const BodyEnd& U);
 // each body's largest |rest coordinate| per axis (out [nb][3]) and a copy of the rest positions
@@ -298,6 +299,9 @@ struct KeepAtX {
     double pdil, edil, tdil;
     const double* alpha = nullptr;
     const int32_t* body_scene = nullptr;
+    // swept (x1): the vertices' edge boxes at both ends (body_end's ebox), read for the EE
+    // entries of an input with vertex ids in place of the positions (nullable)
+    const float4* ebox = nullptr;
 };
 // The CCD of a step taken while its swept set is written (x, x1: the step's ends), over the
 // scenes with active[s]: each kept PT / EE / VG entry's apart_until, the PT / EE entries whose
