@@ -1299,13 +1299,14 @@ int keep_from_superset(hipStream_t s, const AbdScene* sc, const KeepInput& in, c
         for (int k = 0; k < kKeepLists; ++k)
             A.grp0[k + 1] = A.grp0[k] +
                             ceil_div(nblk[k], (int64_t)kXcds * (k == 2 || k == 3 ? kSweepBlocks : 1)) * kXcds;
-        // bytes: per superset entry (an upper bound of the kept ones) the CCD's tuple, ids and
-        // vertices at both ends
-        const int phw = prof_start(kProfToi, s, 228.0 * in.nee + 224.0 * in.npt + 56.0 * in.nvg);
+        // bytes: the CCD's tuple, ids and vertices at both ends of each kept entry, counted on the
+        // device (the host knows only the superset's bounds, many times the kept entries)
+        const int phw = prof_start(kProfToi, s, 1.0);
         launch_kernel(sweep_write_kernel, dim3((unsigned)std::max<int64_t>(A.grp0[kKeepLists], 1)),
                            dim3(kBlock), 0, s, A);
         ABD_CHECK_LAUNCH();
         prof_stop(phw, s);
+        if ((rc = prof_count_bytes(phw, s, dcount, 224.0, 228.0, 56.0, 0.0))) return rc;
     } else {
         const int phw = prof_start(kProfKeep, s, 0.0);
         launch_kernel(keep_write_kernel, dim3((unsigned)std::max<int64_t>(nall, 1)), dim3(kBlock), 0, s, A);

@@ -717,18 +717,13 @@ int seg_reduce(hipStream_t s, const AbdScene& sc, const AbdParams& P, int S, con
 }
 
 // Algorithmic bytes of a launch over the plan's scenes: c_ee, c_pt, c_vg per EE, PT and VG
-// candidate of every (trial k, scene s) it evaluates -- K trials with step lengths alpha
-// [K][S] (nullable; a negative step length skips the scene's trial) -- from the plan's
-// per-scene segments.
-__global__ __launch_bounds__(kRedThreads) void seg_bytes_kernel(int S, int K, const double* __restrict__ alpha,
-                                                                const int64_t* __restrict__ seg, double c_ee,
+// candidate of the plan's per-scene segments.
+__global__ __launch_bounds__(kRedThreads) void seg_bytes_kernel(int S, const int64_t* __restrict__ seg, double c_ee,
                                                                 double c_pt, double c_vg, double* __restrict__ out) {
     __shared__ double sh[kRedThreads];
     double acc = 0.0;
-    for (int64_t i = threadIdx.x; i < (int64_t)S * K; i += blockDim.x) {
-        const int64_t sc = i % S;
-        if (alpha && !(alpha[i] >= 0.0)) continue;
-        const int64_t* q = seg + 2 * (int64_t)kLists * sc;
+    for (int64_t i = threadIdx.x; i < S; i += blockDim.x) {
+        const int64_t* q = seg + 2 * (int64_t)kLists * i;
         acc += c_ee * (double)(q[1] - q[0]) + c_pt * (double)(q[3] - q[2]) + c_vg * (double)(q[5] - q[4]);
     }
     acc = block_sum(acc, sh);
@@ -736,13 +731,55 @@ __global__ __launch_bounds__(kRedThreads) void seg_bytes_kernel(int S, int K, co
 }
 
 // Attaches to `handle` the bytes of seg_bytes_kernel (nothing when the handle is -1).
-int attach_seg_bytes(int handle, hipStream_t s, int S, int K, const double* alpha, const int64_t* seg, double c_ee,
-                     double c_pt, double c_vg) {
+int attach_seg_bytes(int handle, hipStream_t s, int S, const int64_t* seg, double c_ee, double c_pt, double c_vg) {
     double* out;
     int rc = prof_byte_slot(handle, &out);
     if (rc || !out) return rc;
-    launch_kernel(seg_bytes_kernel, dim3(1), dim3(kRedThreads), 0, s, S, K, alpha, seg, c_ee, c_pt, c_vg,
-                       out);
+    launch_kernel(seg_bytes_kernel, dim3(1), dim3(kRedThreads), 0, s, S, seg, c_ee, c_pt, c_vg, out);
+    ABD_CHECK_LAUNCH();
+    prof_stop(handle, s, nullptr, out);
+    return ABD_OK;
+}
+
+// Algorithmic bytes of trial_chunk_kernel, one workgroup per chunk: each candidate's apart_until
+// where a trial of its scene is wanted, and 132, 128 or 32 bytes per EE, PT or VG pair that the
+// kernel lists (the rest it does not read).  Sums of whole numbers: their order is free.
+__global__ __launch_bounds__(kRedThreads) void trial_bytes_kernel(Lists L, int S, int K,
+                                                                  const double* __restrict__ alpha,
+                                                                  const int64_t* __restrict__ seg,
+                                                                  const int64_t* __restrict__ choff,
+                                                                  double* __restrict__ out) {
+    __shared__ double sh[kRedThreads];
+    const int64_t c = blockIdx.x;
+    if (c >= choff[S]) return;
+    const ChunkRange r = chunk_range(S, seg, choff, c);
+    const ListRef& Lr = L.l[r.l < kLists ? r.l : 0];
+    const double each = Lr.kind == kListEE ? 132.0 : Lr.kind == kListPT ? 128.0 : 32.0;
+    double acc = 0.0;
+    for (int64_t i = r.start + threadIdx.x; i < r.end; i += blockDim.x) {
+        const double apart = Lr.apart ? (double)Lr.apart[i] : 0.0;
+        bool wanted = false;
+        for (int k = 0; k < K; ++k) {
+            const double al = alpha[(int64_t)S * k + r.s];
+            if (al < 0.0) continue;
+            wanted = true;
+            if (!(al < apart)) acc += each;
+        }
+        if (wanted && Lr.apart) acc += 4.0;
+    }
+    acc = block_sum(acc, sh);
+    if (threadIdx.x == 0) atomicAdd(out, acc);
+}
+
+// Attaches to `handle` the bytes of trial_bytes_kernel (nothing when the handle is -1).
+int attach_trial_bytes(int handle, hipStream_t s, const Lists& L, int S, int K, const double* alpha,
+                       const int64_t* seg, const int64_t* choff, int64_t chunks) {
+    double* out;
+    int rc = prof_byte_slot(handle, &out);
+    if (rc || !out) return rc;
+    if ((rc = zero_fill(s, out, sizeof(double)))) return rc;
+    launch_kernel(trial_bytes_kernel, dim3((unsigned)chunks), dim3(kRedThreads), 0, s, L, S, K, alpha, seg, choff,
+                  out);
     ABD_CHECK_LAUNCH();
     prof_stop(handle, s, nullptr, out);
     return ABD_OK;
@@ -789,7 +826,7 @@ int toi_reduce(hipStream_t s, const AbdScene& sc, const AbdParams& P, int S, con
     prof_launch(ph, toi_scan_kernel, dim3((unsigned)bound, kToiSplit), dim3(kRedThreads), 0, s, sc, P, x0, x1, L, S,
                 seg, choff, w.part, w.queue, w.qcount);
     ABD_CHECK_LAUNCH();
-    if ((rc = attach_seg_bytes(ph, s, S, 1, nullptr, seg, 228.0, 224.0, 56.0))) return rc;
+    if ((rc = attach_seg_bytes(ph, s, S, seg, 228.0, 224.0, 56.0))) return rc;
     if ((rc = toi_solve(s, sc, S, x0, x1, L, w.queue, w.qcount, w.slots, !scr))) return rc;
     launch_kernel(toi_final_kernel, dim3(S), dim3(kRedThreads), 0, s, choff, (const double*)w.part,
                        (const unsigned long long*)w.slots, out);
@@ -842,7 +879,7 @@ int line_chunks(hipStream_t s, const AbdScene* sc, const AbdParams* P, int S, in
     double* part;
     if ((rc = get_plan(s, *sc, S, L, plan, &seg, &choff))) return rc;
     if ((rc = arena_get(kSlotReduce, sizeof(double) * (size_t)bound * K, (void**)&part))) return rc;
-    // bytes: those of the (trial, scene) pairs evaluated, counted on the device
+    // bytes: those of the (trial, candidate) pairs evaluated, counted on the device
     int ph = prof_start_ext(kProfEnergy, 1.0);
     // a workgroup's trials share its listing and fill its batches; a third of them each, or
     // as many as leave the device kTrialGrid workgroups
@@ -851,7 +888,7 @@ int line_chunks(hipStream_t s, const AbdScene* sc, const AbdParams* P, int S, in
     prof_launch(ph, trial_chunk_kernel, dim3((unsigned)bound, groups), dim3(kRedThreads), 0, s, *sc, *P,
                 TrialArgs{alpha, st}, L, S, K, seg, choff, part, bound);
     ABD_CHECK_LAUNCH();
-    if ((rc = attach_seg_bytes(ph, s, S, K, alpha, seg, 132.0, 128.0, 32.0))) return rc;
+    if ((rc = attach_trial_bytes(ph, s, L, S, K, alpha, seg, choff, bound))) return rc;
     *out = TrialSums{choff, part, bound};
     return ABD_OK;
 }
