@@ -323,7 +323,9 @@ struct TrialArgs {
 // place plus its rank among the wave's ballots, so that the owner finds it again.  Bound by
 // the latency of a workgroup's few dependent gathers: evaluating every candidate at every
 // trial took 60 us for a pass of one trial and 130 us for one of twelve over 1.3M
-// candidates (256 scenes), this 39 and 74 us (0.35M and 1.1M pairs evaluated).
+// candidates (256 scenes), this 39 and 74 us (0.35M and 1.1M pairs evaluated).  Where most
+// candidates are near and listed all the same (256 scenes of 2 to 64 bodies, 0.8 of the bytes),
+// the listing is not repaid: 30 and 58 us against 19 and 44.
 constexpr int kTrialItems = kChunkItems / kRedThreads;
 constexpr int kTrialBatch = 1024;  // pairs listed at a time
 __global__ __launch_bounds__(kRedThreads, 4) void trial_chunk_kernel(AbdScene sc, AbdParams P, TrialArgs T, Lists L,
@@ -881,9 +883,13 @@ int line_chunks(hipStream_t s, const AbdScene* sc, const AbdParams* P, int S, in
     if ((rc = arena_get(kSlotReduce, sizeof(double) * (size_t)bound * K, (void**)&part))) return rc;
     // bytes: those of the (trial, candidate) pairs evaluated, counted on the device
     int ph = prof_start_ext(kProfEnergy, 1.0);
-    // a workgroup's trials share its listing and fill its batches; a third of them each, or
-    // as many as leave the device kTrialGrid workgroups
-    const int64_t most = std::max<int64_t>(3, kTrialGrid / bound);
+    // a workgroup's trials share its listing and fill its batches, but its threads evaluate
+    // them in turn: two trials each, or one where the chunks leave the device fewer than
+    // kTrialGrid workgroups.  The pass of twelve trials in 3, 4, 6 and 12 groups: 78, 67, 58
+    // and 58 us for 256 scenes with most candidates near; three frames of 256 scenes with few
+    // near 18.6, 18.6, 18.65 and 19.2 ms (the listing repeated); a 1024-body pile's 7.87,
+    // 7.85, 7.80 and 7.82 ms
+    const int64_t most = std::max<int64_t>(6, kTrialGrid / bound);
     const unsigned groups = (unsigned)std::min<int64_t>(K, most);
     prof_launch(ph, trial_chunk_kernel, dim3((unsigned)bound, groups), dim3(kRedThreads), 0, s, *sc, *P,
                 TrialArgs{alpha, st}, L, S, K, seg, choff, part, bound);
