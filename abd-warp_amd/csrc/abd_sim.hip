@@ -127,7 +127,7 @@ struct Sim {
     DevBuf<double> vlo, vhi;         // its vertex ranges
     DevBuf<uint8_t> body_on;         // body_end's
     DevBuf<float> ebox;              // body_end's, 8 per vertex
-    bool ebox_ready = false;         // written by the last step end
+    bool ebox_ready = false;         // written by this iteration's step end (writes_ebox)
     DevBuf<uint32_t> kcnt;           // the filters' counters (sweep_words)
     unsigned long long* toi_slots = nullptr;  // the CCD's scratch (arena)
     int32_t *toi_qcount = nullptr, *toi_queue = nullptr;
@@ -791,6 +791,12 @@ int read_counts(hipStream_t s, Sim& S) {
     return ABD_OK;
 }
 
+// Whether an iteration's step end writes the vertices' boxes: they cost 10 ns per 1000 vertices
+// there and save the swept filter 6 ns per 1000 EE entries of the superset.  A function of the
+// size bounds that a recorded iteration is replayed for, so the same for its replays; a step
+// that leaves the ranges is filtered again from what its own iteration wrote.
+bool writes_ebox(const Sim& S) { return S.sup_valid && S.sup.nee >= 2 * (int64_t)S.nv; }
+
 // The end of the step (xk = x(q - dq) for the scenes in `active`), the swept body boxes and
 // the range test against the superset's ranges when there is a superset (a vertex outside
 // writes 1 over the 0 of body_start).
@@ -818,9 +824,6 @@ int step_end_scenes(hipStream_t s, Sim& S, const uint8_t* active) {
     U.margin = range_margin(S);
     U.flag = S.cnt.p + kCntRange;
     U.on = S.body_on.p;
-    // the vertices' boxes cost 10 ns per 1000 vertices here and save the swept filter 6 ns per
-    // 1000 EE entries of the superset
-    S.ebox_ready = S.sup_valid && S.sup.nee >= 2 * (int64_t)S.nv;
     U.ebox = S.ebox_ready ? reinterpret_cast<float4*>(S.ebox.p) : nullptr;
     return body_end(s, &S.sc, U);
 }
@@ -1004,6 +1007,7 @@ int step_scenes(hipStream_t s, Sim& S) {
     int64_t n_active = ns;
     while (n_active > 0) {
         const LsDev L = ls_dev(S);
+        S.ebox_ready = writes_ebox(S);  // launched or replayed
         // a steady iteration (collision set from the last swept set, superset kept) replays
         // its recorded graph; the first time a key is met the iteration runs eagerly, the
         // second time it is recorded (every buffer then holds its size for these launches)
