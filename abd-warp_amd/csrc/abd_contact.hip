@@ -706,11 +706,31 @@ __device__ __forceinline__ void body_vg_range(const int32_t* __restrict__ vg, in
     k1 = lo[1];
 }
 
-// stage E: one workgroup per body: its 144 Hessian and 12 gradient entries, and the off-diagonal
-// blocks of the pairs whose first body it is.  A pair's chunks' partial sums (part, in the
-// pair's body order [ij0 | ij1]) are added in order (PT chunks, then EE), the pairs in row
-// order; nij_cap: pairs of the buffers (a bound when dn counts the matrix's, dn[0], which
-// places the lower slots).  nact (nullable): an active count no stage wrote, zeroed.
+// stage E: one workgroup per body: its 144 Hessian and 12 gradient entries; and the off-diagonal
+// block of every pair.  A pair's chunks' partial sums (part, in the pair's body order [ij0 |
+// ij1]) are added in order (PT chunks, then EE), the pairs in row order; nij: the pairs, or with
+// dn a bound of dn[0] that only sizes the launch.  nact (nullable): an active count no stage
+// wrote, zeroed.
+// Without LONG a row's pairs are taken one after the other, each with its off-diagonal block where
+// the row's body is its first: a few load latencies, hidden by the other bodies' workgroups (59
+// VGPRs, eight waves a SIMD).  A long row makes that a chain with nothing beside it: with LONG
+// its pairs with active contacts are listed, kPairsAtOnce of them have their loads in flight, and
+// the workgroups past the bodies add the off-diagonal blocks.  A plate under 400 cubes takes 93 us
+// with it and 392 without, 8217 bodies in 256 scenes 23.8 and 19.0.  Hence the line at kLongRow
+// bodies to a scene, which bound a row.
+constexpr int kLongRow = 64;
+constexpr int kPairsAtOnce = 8;
+constexpr int64_t kOffGrid = 4096;  // workgroups of the off-diagonal blocks, at most
+
+// the off-diagonal block of pair ii (threads 0..143, one an entry): the upper slot holds rows ij0
+// x cols ij1, the lower one its transpose
+__device__ __forceinline__ void add_off_diagonal(int R, int C, int64_t up, int64_t lo, double h,
+                                                 double* __restrict__ blocks) {
+    const int bi = R / 3, rr = R % 3, bj = C / 3, cc = C % 3;
+    blocks[9 * (16 * up + bi + 4 * bj) + 3 * rr + cc] += h;
+    blocks[9 * (16 * lo + bj + 4 * bi) + 3 * cc + rr] += h;
+}
+template <bool LONG>
 __global__ __launch_bounds__(kBlock) void body_finalize_kernel(AbdScene sc, AbdParams P,
                                                                 const double* __restrict__ x, int64_t nij,
                                                                 const int64_t* __restrict__ dn,
@@ -733,6 +753,18 @@ __global__ __launch_bounds__(kBlock) void body_finalize_kernel(AbdScene sc, AbdP
         nij = dn[0];
         nvg = dn[4];
     }
+    if (LONG && b >= nb) {  // off-diagonal blocks (part is not null), grid-stride over the pairs
+        if (t >= 144) return;
+        const double* off = part + 24 * (t / 12) + 12 + t % 12;
+        for (int64_t ii = b - nb; ii < nij; ii += gridDim.x - nb) {
+            if (!pflag[ii]) continue;  // uniform
+            const int2 it = pitem[ii];
+            double h = 0.0;
+            for (int c = 0; c < it.y; ++c) h += off[(int64_t)(it.x + c) * kPartStride];
+            add_off_diagonal(t / 12, t % 12, nb + ii, nb + nij + ii, h, blocks);
+        }
+        return;
+    }
     if (nact && b == 0 && t == 0) *nact = 0;
     // threads 0..143: the entries of the diagonal block; 144..155: the gradient; the rest
     // only help to evaluate the vertex-ground terms
@@ -743,40 +775,76 @@ __global__ __launch_bounds__(kBlock) void body_finalize_kernel(AbdScene sc, AbdP
     if (part && nij > 0) {  // uniform
         const int e1 = row_ptr[b + 1];
         for (int eb = row_ptr[b]; eb < e1; eb += kBlock) {
-            const int ne = e1 - eb < kBlock ? e1 - eb : kBlock;
+            int ne = e1 - eb < kBlock ? e1 - eb : kBlock, s = 0;
+            int2 it = make_int2(0, 0);
             if (t < ne) {  // the row's pairs with active contacts: their items, side
-                const int s = slots[eb + t];
-                int2 it = make_int2(0, 0);
+                s = slots[eb + t];
                 if (s >= nb) {
                     const int64_t ii = s < nb + nij ? s - nb : s - nb - nij;
                     if (pflag[ii]) it = pitem[ii];
                 }
-                s_item[t] = it.x;
-                s_n[t] = it.y;
-                s_slot[t] = s;
             }
-            __syncthreads();
-            if (act)
-                for (int q = 0; q < ne; ++q) {
-                    const int n = s_n[q];
-                    if (n == 0) continue;  // the diagonal, or a pair without active contacts
-                    const int s = s_slot[q];
-                    const int side = s < nb + nij ? 0 : 1;  // upper slot in row b: b is ij0
-                    const double* pp = part + (int64_t)s_item[q] * kPartStride;
-                    const int at = isg ? 576 + 12 * side + R : 24 * (12 * side + R) + 12 * side + C;
-                    double h = 0.0, ho = 0.0;
-                    for (int c = 0; c < n; ++c) {
-                        h += pp[(int64_t)c * kPartStride + at];
-                        if (!isg && side == 0) ho += pp[(int64_t)c * kPartStride + 24 * R + 12 + C];
-                    }
-                    acc += h;
-                    if (!isg && side == 0) {
-                        // upper slot s holds rows ij0 x cols ij1, lower slot its transpose
-                        const int bi = R / 3, rr = R % 3, bj = C / 3, cc = C % 3;
-                        blocks[9 * (16 * (int64_t)s + bi + 4 * bj) + 3 * rr + cc] += ho;
-                        blocks[9 * (16 * (s + nij) + bj + 4 * bi) + 3 * cc + rr] += ho;
-                    }
+            if constexpr (!LONG) {
+                if (t < ne) {
+                    s_item[t] = it.x;
+                    s_n[t] = it.y;
+                    s_slot[t] = s;
                 }
+                __syncthreads();
+                if (act)
+                    for (int q = 0; q < ne; ++q) {
+                        const int n = s_n[q];
+                        if (n == 0) continue;  // the diagonal, or a pair without active contacts
+                        const int s = s_slot[q];
+                        const int side = s < nb + nij ? 0 : 1;  // upper slot in row b: b is ij0
+                        const double* pp = part + (int64_t)s_item[q] * kPartStride;
+                        const int at = isg ? 576 + 12 * side + R : 24 * (12 * side + R) + 12 * side + C;
+                        double h = 0.0, ho = 0.0;
+                        for (int c = 0; c < n; ++c) {
+                            h += pp[(int64_t)c * kPartStride + at];
+                            if (!isg && side == 0) ho += pp[(int64_t)c * kPartStride + 24 * R + 12 + C];
+                        }
+                        acc += h;
+                        if (!isg && side == 0) add_off_diagonal(R, C, s, s + nij, ho, blocks);
+                    }
+            } else {
+                __shared__ int shw[kBlock / kWave];
+                const int r = block_rank(it.y > 0, shw, &ne);
+                if (it.y > 0) {
+                    s_item[r] = it.x;
+                    s_n[r] = it.y;
+                    s_slot[r] = s;
+                }
+                __syncthreads();
+                if (act)
+                    for (int q = 0; q < ne; q += kPairsAtOnce) {
+                        const double* src[kPairsAtOnce];
+                        int n[kPairsAtOnce], most = 0;
+                        double h[kPairsAtOnce];
+#pragma unroll
+                        for (int j = 0; j < kPairsAtOnce; ++j) {
+                            const int u = q + j < ne ? q + j : q;  // past the end: read, not added
+                            const int side = s_slot[u] < nb + nij ? 0 : 1;
+                            src[j] = part + (int64_t)s_item[u] * kPartStride +
+                                     (isg ? 576 + 12 * side + R : 24 * (12 * side + R) + 12 * side + C);
+                            n[j] = q + j < ne ? s_n[u] : 0;
+                            most = n[j] > most ? n[j] : most;
+                            h[j] = 0.0;
+                        }
+                        for (int c = 0; c < most; ++c) {  // uniform
+                            double v[kPairsAtOnce];
+#pragma unroll
+                            for (int j = 0; j < kPairsAtOnce; ++j)
+                                v[j] = src[j][c < n[j] ? (int64_t)c * kPartStride : 0];
+#pragma unroll
+                            for (int j = 0; j < kPairsAtOnce; ++j)
+                                if (c < n[j]) h[j] += v[j];
+                        }
+#pragma unroll
+                        for (int j = 0; j < kPairsAtOnce; ++j)
+                            if (n[j] > 0) acc += h[j];
+                    }
+            }
             __syncthreads();
         }
     }
@@ -960,9 +1028,10 @@ __global__ void inertia_hessian_kernel(int nb, AbdParams P, const double* __rest
 // that are not grouped.
 int contact_gh(hipStream_t s, const AbdScene* sc, const AbdParams* P, const double* x, const GhLists& L,
                const int32_t* row_ptr, const int32_t* slots, double* g, double* blocks, uint8_t* highlight,
-               int64_t* n_active, int64_t* n_active_dev, bool zeroed) {
+               int64_t* n_active, int64_t* n_active_dev, bool zeroed, int row_bodies) {
     const int nb = sc->n_bodies;
     if (nb == 0) return ABD_OK;
+    if (row_bodies <= 0) row_bodies = nb;
     const int32_t *pt = L.pt, *ee = L.ee, *vg = L.vg;
     const int64_t npt = L.npt, nee = L.nee, nij = L.nij;
     const int64_t nvg = P->vg ? L.nvg : 0;
@@ -1096,7 +1165,10 @@ int contact_gh(hipStream_t s, const AbdScene* sc, const AbdParams* P, const doub
     const double fbytes = 2.0 * 8 * 156 * nb;
     const double pbytes = 8.0 * 2 * 312;  // a pair's partial sums, read by both bodies (one chunk)
     int phf = prof_start(kProfBodyFinalize, s, dn ? 1.0 : fbytes + pbytes * nij + 40.0 * nvg);
-    launch_kernel(body_finalize_kernel, dim3(nb), dim3(kBlock), 0, s, *sc, *P, x, nij, dn, row_ptr, slots,
+    const bool rows = row_bodies > kLongRow;  // that can be long
+    const int64_t off = rows && part ? std::min(nij, kOffGrid) : 0;
+    launch_kernel(rows ? body_finalize_kernel<true> : body_finalize_kernel<false>, dim3((unsigned)(nb + off)),
+                       dim3(kBlock), 0, s, *sc, *P, x, nij, dn, row_ptr, slots,
                        (const uint8_t*)G.pflag, (const int2*)pitem, (const double*)part, vg, nvg, g, blocks,
                        (const uint8_t*)G.hl_pt, (const uint8_t*)G.hl_ee, highlight, nact_unwritten);
     ABD_CHECK_LAUNCH();

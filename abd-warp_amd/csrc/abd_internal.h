@@ -360,9 +360,10 @@ struct GhLists {
     int64_t nij;
     const int64_t* dn;
 };
+// row_bodies: the bodies of the largest scene (0: not known, all bodies), which bound a row's pairs.
 int contact_gh(hipStream_t s, const AbdScene* sc, const AbdParams* P, const double* x, const GhLists& L,
                const int32_t* row_ptr, const int32_t* slots, double* g, double* blocks, uint8_t* highlight,
-               int64_t* n_active, int64_t* n_active_dev, bool zeroed = false);
+               int64_t* n_active, int64_t* n_active_dev, bool zeroed = false, int row_bodies = 0);
 // The words (8 bytes) that a contact_gh over these sizes wants 0; with them zeroed before it it
 // runs with zeroed = true.
 int gh_zero_region(int nb, int64_t nij, int64_t n, void** p, int64_t* words);

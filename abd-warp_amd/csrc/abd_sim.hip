@@ -921,7 +921,7 @@ int iteration_scenes(hipStream_t s, Sim& S) {
     const CandSet& C = S.col;
     const GhLists GL{C.ptl.p, C.npt, C.eel.p, C.nee, C.vgl.p, C.nvg, C.nij, C.counts()};
     if ((rc = contact_gh(s, &S.sc, &P, st.x, GL, S.row_ptr.p, S.slots.p, st.g, S.blocks.p, nullptr, nullptr,
-                         S.cnt.p + kCntNact, true)))
+                         S.cnt.p + kCntNact, true, ns > 1 ? S.max_scene_bodies : 0)))
         return rc;
     if (ns > 1)
         rc = abd_bsr_solve_scenes(s, P.solver, &S.sc, S.max_scene_bodies, S.row_ptr.p, S.cols.p, S.slots.p,
