@@ -1425,8 +1425,8 @@ __global__ void solve_bytes_kernel(const int32_t* __restrict__ row_ptr, int nb, 
 // ten such solves 4.05 -> 3.95 ms).
 // Every workgroup reduces the per-workgroup partials itself, in workgroup order,
 // so all of them hold the same scalars and the sequence is deterministic.  The
-// stopping test (every check_every iterations) sets a device flag that ends the
-// remaining launches of the batch; the host reads it once per batch.
+// stopping test (every check_every iterations) is a launch of its own at a batch's
+// end; the host reads its flag once per batch.
 constexpr int kMwThreads = 256;
 constexpr int kMwBjThreads = 192;  // 16 bodies of 12 rows
 static_assert(kMwBjThreads % 12 == 0 && kMwBjThreads <= kMwThreads, "whole bodies per block-Jacobi workgroup");
@@ -1552,21 +1552,9 @@ __device__ __forceinline__ double mw_row_next(const Bsr& M, const double* __rest
     return acc;
 }
 
-// The stopping test of iteration it (every check_every iterations), alike in every workgroup.
-__device__ __forceinline__ bool mw_stops(int it, int check_every, double tol_sq, double rz_new, const MwState& W) {
-    if (((it + 1) % check_every) != 0 || !(rz_new <= tol_sq)) return false;
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        *W.done = 1;
-        *W.it = it;
-        *W.err = rz_new;
-    }
-    return true;
-}
-
-// iteration i, part 1: the stopping test of iteration i - 1, its beta, this iteration's
-// direction (the first one's is z already), its SpMV and partial p.Ap
-__global__ __launch_bounds__(kMwThreads) void mw_spmv_kernel(Bsr M, int iter, int check_every, double tol_sq,
-                                                             MwState W) {
+// iteration i, part 1: the beta of iteration i - 1, this iteration's direction (the first one's
+// is z already), its SpMV and partial p.Ap
+__global__ __launch_bounds__(kMwThreads) void mw_spmv_kernel(Bsr M, int iter, double tol_sq, MwState W) {
     __shared__ double sh[17];
     if (*W.done) return;
     const int n = 12 * M.nb, nblk = gridDim.x;
@@ -1580,7 +1568,6 @@ __global__ __launch_bounds__(kMwThreads) void mw_spmv_kernel(Bsr M, int iter, in
         }
     } else {
         const double rz_new = mw_sum(W.part + nblk, nblk, sh);
-        if (mw_stops(iter - 1, check_every, tol_sq, rz_new, W)) return;  // uniform over the grid
         const double beta = rz_new > tol_sq ? rz_new / W.rz[(iter - 1) & 1] : 0.0;
         const double* p_old = W.p[(iter - 1) & 1];
         if (i < n) {
@@ -1632,13 +1619,20 @@ __global__ __launch_bounds__(kMwThreads) void mw_update_kernel(int n, int iter, 
     if (threadIdx.x == 0) W.part[nblk + blockIdx.x] = t;
 }
 
-// the end of a batch, whose last iteration is `iter`: its stopping test, for the host
+// the end of a batch, whose last iteration is `iter`: its stopping test (every check_every
+// iterations), for the host.  One workgroup of the iterations' own size, so that the sum it
+// decides by is the one they take; no launch that reads *W.done across workgroups writes it.
 __global__ __launch_bounds__(kMwThreads) void mw_check_kernel(int nblk, int iter, int check_every, double tol_sq,
                                                               MwState W) {
     __shared__ double sh[17];
     if (*W.done) return;
     const double rz_new = mw_sum(W.part + nblk, nblk, sh);
-    if (!mw_stops(iter, check_every, tol_sq, rz_new, W) && threadIdx.x == 0) *W.err = rz_new;
+    if (threadIdx.x != 0) return;
+    *W.err = rz_new;
+    if ((iter + 1) % check_every == 0 && rz_new <= tol_sq) {
+        *W.done = 1;
+        *W.it = iter;
+    }
 }
 
 __global__ void mw_finish_kernel(int n, MwState W, double* __restrict__ xg, int32_t* __restrict__ iters,
@@ -1863,13 +1857,13 @@ int solve_cg_multi(hipStream_t s, const Bsr& M, const double* b, double* x, doub
     for (int i0 = 0; i0 < maxiter; i0 += check_every) {
         const int i1 = i0 + check_every < maxiter ? i0 + check_every : maxiter;
         for (int i = i0; i < i1; ++i) {
-            launch_kernel(mw_spmv_kernel, dim3(nblk), dim3(threads), 0, s, M, i, (int)check_every, tol_sq, W);
+            launch_kernel(mw_spmv_kernel, dim3(nblk), dim3(threads), 0, s, M, i, tol_sq, W);
             if (bj)
                 launch_kernel(mw_update_kernel<true>, dim3(nblk), dim3(threads), 0, s, n, i, W, (const double*)dinv);
             else
                 launch_kernel(mw_update_kernel<false>, dim3(nblk), dim3(threads), 0, s, n, i, W, (const double*)dinv);
         }
-        launch_kernel(mw_check_kernel, dim3(1), dim3(kMwThreads), 0, s, nblk, i1 - 1, (int)check_every, tol_sq, W);
+        launch_kernel(mw_check_kernel, dim3(1), dim3(threads), 0, s, nblk, i1 - 1, (int)check_every, tol_sq, W);
         ABD_CHECK_LAUNCH();
         ABD_CHECK(hipMemcpyAsync(hdone, W.done, sizeof(int32_t), hipMemcpyDeviceToHost, s));
         ABD_CHECK(hipStreamSynchronize(s));

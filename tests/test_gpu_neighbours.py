@@ -72,3 +72,53 @@ def test_gh_of_a_plate_under_cubes(n, last):
             assert np.array_equal(b.reshape(-1, 16, 9)[s], b0.reshape(-1, 16, 9)[s])
     assert rel_err(g.cpu().numpy() - g0, g_ref - g0) <= 1e-9
     assert rel_err(b - b0.reshape(b.shape), b_ref - b0.reshape(b.shape)) <= 1e-9
+
+
+def _cg_system(kind, m, rng):
+    """Blocks of a system of m bodies: 50 on the diagonal, coupling blocks of normal entries times
+    0.1, whose norm is below 10 for the kinds here (condition below 1.5)."""
+    if kind == "dense":
+        ij = np.stack(np.triu_indices(m, 1), 1)
+    elif kind == "first":  # body 0 coupled to all
+        ij = np.stack([np.zeros(m - 1, int), np.arange(1, m)], 1)
+    elif kind == "last":
+        ij = np.stack([np.arange(m - 1), np.full(m - 1, m - 1)], 1)
+    else:  # "sparse": rows of 1 to about 10 entries
+        ij = rng.integers(0, m, (2 * m, 2))
+        ij = np.unique(np.sort(ij[ij[:, 0] != ij[:, 1]], axis=1), axis=0)
+    n = len(ij)
+    B = np.zeros((m + 2 * n, 12, 12))
+    Q = rng.normal(size=(m, 12, 12))
+    B[:m] = 50.0 * np.eye(12) + 0.02 * (Q + Q.transpose(0, 2, 1))
+    B[m:m + n] = 0.1 * rng.normal(size=(n, 12, 12))
+    B[m + n:] = B[m:m + n].transpose(0, 2, 1)
+    blocks = B.reshape(-1, 4, 3, 4, 3).transpose(0, 3, 1, 2, 4).reshape(-1, 3, 3)
+    return ij.astype(np.int32), np.ascontiguousarray(blocks)
+
+
+@pytest.mark.parametrize("block", [False, True])
+@pytest.mark.parametrize("kind,m", [("dense", 171), ("first", 172), ("last", 400), ("sparse", 513),
+                                    ("sparse", 3100)])
+def test_large_cg_long_rows(kind, m, block):
+    """CG over several workgroups with rows of one entry to hundreds, up to more workgroups (194)
+    than one has threads for their partial sums in the block form (192): stopped by its test and
+    cut off, the oracle's iterate, count and residual.  Both run the same recurrence in double;
+    after at most 40 iterations of a system of condition below 1.5 they agree to 1e-9.  The
+    residual r.z is off by 2 |r0| / |r| roundings an iteration, below 1e-9 at the sizes of r
+    here (the smallest is 1e-6 of r0): 1e-8."""
+    import abd_hip
+    from abd_hip.sparse import BsrMatrix, SolveInfo, bsr_cg
+    from test_gpu_ldlt import _structure
+    lib = abd_hip.load()
+    rng = np.random.default_rng(m)
+    ij, blocks = _cg_system(kind, m, rng)
+    b, x0 = rng.normal(size=(4 * m, 3)), 0.01 * rng.normal(size=(4 * m, 3))
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()  # noqa: E731
+    A = BsrMatrix(m, *_structure(lib, m, ij), d(blocks))
+    for tol, maxiter, check in ((1e-5, 40, 3), (0.0, 2, 4)):
+        x, info = d(x0), SolveInfo("cuda")
+        bsr_cg(A, x, d(b), maxiter, tol, check, info, block_precond=block)
+        ref, it, err = (O.bsr_cg_block if block else O.bsr_cg)(m, ij, blocks, b, x0, tol, maxiter, check)
+        assert int(info.iters[0]) == it and (it < 40)
+        assert rel_err(x.cpu().numpy(), ref) <= 1e-9
+        assert abs(float(info.resid[0]) - err) <= 1e-8 * abs(err)
