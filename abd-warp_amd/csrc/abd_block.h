@@ -80,6 +80,7 @@ __device__ __forceinline__ double dpp_move(double v) {
     return __hiloint2double(hi, lo);
 }
 constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppRor4 = 0x124, kDppRor8 = 0x128;
+constexpr int kDppPair0 = 0xA0, kDppPair1 = 0xF5;  // lane k of a pair to both
 constexpr int kDppRowBcast = 0x150;  // + i: lane i of each row of 16 lanes to all of it
 // v summed over each row of 16 lanes (8 apart first; a rotation by 4 is lane ^ 4 once lanes
 // 8 apart hold the same value)

@@ -1421,8 +1421,8 @@ __global__ void solve_bytes_kernel(const int32_t* __restrict__ row_ptr, int nb, 
 // [beta, p = z + beta p and its SpMV, partial p.Ap], [alpha, x / r / z update + partial r.z]:
 // a workgroup forms the directions of the bodies its rows couple to itself (the same
 // arithmetic in every workgroup), so the SpMV needs no launch between (1024 bodies, ten
-// iterations: 30 launches of 2.2 to 3 us became 20 of 2.9 and 3.7 us and a check; a frame of
-// ten such solves 4.05 -> 3.95 ms).
+// iterations: 30 launches of 2.2 to 3 us became 20 of 2.9 and 3.3 us and a check; a frame of
+// ten such solves 4.05 -> 3.91 ms).
 // Every workgroup reduces the per-workgroup partials itself, in workgroup order,
 // so all of them hold the same scalars and the sequence is deterministic.  The
 // stopping test (every check_every iterations) is a launch of its own at a batch's
@@ -1446,9 +1446,11 @@ struct MwState {
     int32_t* it;    // end_iter
 };
 
-__device__ __forceinline__ double mw_sum(const double* __restrict__ part, int nblk, double* sh) {
+// the workgroups' partials as a workgroup of `rows` threads adds them (waves past those add 0)
+__device__ __forceinline__ double mw_sum(const double* __restrict__ part, int nblk, double* sh, int rows) {
     double acc = 0.0;
-    for (int k = threadIdx.x; k < nblk; k += blockDim.x) acc += part[k];
+    if ((int)threadIdx.x < rows)
+        for (int k = threadIdx.x; k < nblk; k += rows) acc += part[k];
     return block_sum_fast(acc, sh);
 }
 
@@ -1523,7 +1525,7 @@ __global__ __launch_bounds__(kMwThreads) void mw_init_kernel(Bsr M, const double
 
 __global__ __launch_bounds__(kMwThreads) void mw_start_kernel(int nblk, double tol_sq, int maxiter, MwState W) {
     __shared__ double sh[17];
-    const double rz = mw_sum(W.part + nblk, nblk, sh);
+    const double rz = mw_sum(W.part + nblk, nblk, sh, blockDim.x);
     if (threadIdx.x == 0) {
         W.rz[0] = rz;
         *W.err = rz;
@@ -1532,58 +1534,104 @@ __global__ __launch_bounds__(kMwThreads) void mw_start_kernel(int nblk, double t
     }
 }
 
-// (H p)[row idx] with p = z + beta p_old formed entry by entry (mw_row's sums)
-__device__ __forceinline__ double mw_row_next(const Bsr& M, const double* __restrict__ z,
-                                              const double* __restrict__ p_old, double beta, int idx) {
-    const int b = idx / 12, lr = idx % 12, ii = lr / 3, k = lr % 3;
-    double acc = 0.0;
-    for (int e = M.row_ptr[b]; e < M.row_ptr[b + 1]; ++e) {
-        const double* zin = z + 12 * (int64_t)M.cols[e];
-        const double* pin = p_old + 12 * (int64_t)M.cols[e];
-        const double* base = M.blocks + 9 * 16 * (int64_t)M.slots[e] + 3 * k;
+// What one of a row's two lanes takes of kMwEntries entries from e on: six of the multiplied
+// vector's values, from q0 on (as it stands, or z and p_old), and the rows of their sub-blocks.
+constexpr int kMwLanes = 2, kMwEntries = 3;
+struct MwPart {
+    double z[6], p[6], B[6];
+};
+template <bool STORED>
+__device__ __forceinline__ void mw_load(const Bsr& M, const double* __restrict__ z, const double* __restrict__ p_old,
+                                        int e, int e1, int at, int q0, MwPart (&E)[kMwEntries]) {
+    if (e >= e1) return;
+    int col[kMwEntries], slot[kMwEntries];
 #pragma unroll
-        for (int jj = 0; jj < 4; ++jj) {
-            const double* B = base + 9 * (ii + 4 * jj);
-            const double x0 = zin[3 * jj] + beta * pin[3 * jj], x1 = zin[3 * jj + 1] + beta * pin[3 * jj + 1],
-                         x2 = zin[3 * jj + 2] + beta * pin[3 * jj + 2];
-            acc += B[0] * x0 + B[1] * x1 + B[2] * x2;
-        }
+    for (int u = 0; u < kMwEntries; ++u) {
+        const int q = e + u < e1 ? e + u : e;
+        col[u] = M.cols[q];
+        slot[u] = M.slots[q];
     }
-    return acc;
+#pragma unroll
+    for (int u = 0; u < kMwEntries; ++u)
+        if (e + u < e1) {
+            const int64_t c = 12 * (int64_t)col[u] + q0;
+            const double* B = M.blocks + 144 * (int64_t)slot[u] + at;
+#pragma unroll
+            for (int q = 0; q < 6; ++q) {
+                E[u].z[q] = z[c + q];
+                if (!STORED) E[u].p[q] = p_old[c + q];
+                E[u].B[q] = B[36 * (q / 3) + q % 3];
+            }
+        }
 }
 
-// iteration i, part 1: the beta of iteration i - 1, this iteration's direction (the first one's
-// is z already), its SpMV and partial p.Ap
-__global__ __launch_bounds__(kMwThreads) void mw_spmv_kernel(Bsr M, int iter, double tol_sq, MwState W) {
+// iteration i, part 1: the beta of iteration i - 1, this iteration's direction (FIRST: z
+// already), its SpMV (mw_row's sums) and partial p.Ap.  Two lanes a row, each with two of an
+// entry's four 3x3 sub-blocks, whose parts both add in order; kRows rows a workgroup: those of
+// the other launches, whose sums it shares.
+// Bound by the latency of a row's entries: three are in flight (242 VGPRs: a workgroup a CU is
+// all there is to run), the first three while the partials of r.z are summed.  An iteration of
+// 600 bodies with 4, 24 and 100 couplings each (block form) 17, 31 and 84 us, the product of a
+// plate under 400 cubes 91.  One thread a row with an entry at a time took 20, 43, 184 and 157;
+// four lanes a row with four entries 17, 34, 93 and 71, but 8 to 28 % more in the Jacobi form,
+// whose registers hold two; a direction kernel before a product that then reads one vector for
+// two 19, 33, 104 and 90.
+template <int kRows, bool FIRST>
+__global__ __launch_bounds__(kMwLanes * kRows) void mw_spmv_kernel(Bsr M, int iter, double tol_sq, MwState W) {
     __shared__ double sh[17];
+    __shared__ double parts[kRows];
     if (*W.done) return;
-    const int n = 12 * M.nb, nblk = gridDim.x;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    double part = 0.0;
-    if (iter == 0) {
-        if (i < n) {
-            const double a = mw_row(M, W.p[0], i);
-            W.Ap[i] = a;
-            part = W.p[0][i] * a;
-        }
-    } else {
-        const double rz_new = mw_sum(W.part + nblk, nblk, sh);
-        const double beta = rz_new > tol_sq ? rz_new / W.rz[(iter - 1) & 1] : 0.0;
-        const double* p_old = W.p[(iter - 1) & 1];
-        if (i < n) {
-            const double p = W.z[i] + beta * p_old[i];
-            W.p[iter & 1][i] = p;
-            const double a = mw_row_next(M, W.z, p_old, beta, i);
-            W.Ap[i] = a;
-            part = p * a;
-        }
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
+    const int n = 12 * M.nb, nblk = gridDim.x, t = threadIdx.x;
+    const int row = t / kMwLanes, l = t % kMwLanes, i = blockIdx.x * kRows + row, b = i / 12, lr = i % 12;
+    const int q0 = 6 * l, at = 9 * (lr / 3) + 3 * (lr % 3) + 12 * q0;
+    const double* z = FIRST ? W.p[0] : W.z;
+    const double* p_old = W.p[(iter - 1) & 1];
+    const int e0 = i < n ? M.row_ptr[b] : 0, e1 = i < n ? M.row_ptr[b + 1] : 0;
+    MwPart E[kMwEntries];
+    mw_load<FIRST>(M, z, p_old, e0, e1, at, q0, E);
+    double beta = 0.0;
+    if (!FIRST) {
+        const double rz_new = mw_sum(W.part + nblk, nblk, sh, kRows);
+        beta = rz_new > tol_sq ? rz_new / W.rz[(iter - 1) & 1] : 0.0;
+        if (blockIdx.x == 0 && t == 0) {
             W.rz[iter & 1] = rz_new;
             *W.err = rz_new;
         }
     }
-    const double t = block_sum_fast(part, sh);
-    if (threadIdx.x == 0) W.part[blockIdx.x] = t;
+    double acc = 0.0;
+    for (int e = e0; e < e1; e += kMwEntries) {
+        if (e != e0) mw_load<FIRST>(M, z, p_old, e, e1, at, q0, E);
+#pragma unroll
+        for (int u = 0; u < kMwEntries; ++u)
+            if (e + u < e1) {
+                double v[2];
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    double x[3];
+#pragma unroll
+                    for (int q = 0; q < 3; ++q)
+                        x[q] = FIRST ? E[u].z[3 * k + q] : E[u].z[3 * k + q] + beta * E[u].p[3 * k + q];
+                    v[k] = E[u].B[3 * k] * x[0] + E[u].B[3 * k + 1] * x[1] + E[u].B[3 * k + 2] * x[2];
+                }
+                acc += dpp_move<kDppPair0>(v[0]);
+                acc += dpp_move<kDppPair0>(v[1]);
+                acc += dpp_move<kDppPair1>(v[0]);
+                acc += dpp_move<kDppPair1>(v[1]);
+            }
+    }
+    if (l == 0) {
+        double part = 0.0;
+        if (i < n) {
+            const double p = FIRST ? z[i] : z[i] + beta * p_old[i];
+            if (!FIRST) W.p[iter & 1][i] = p;
+            W.Ap[i] = acc;
+            part = p * acc;
+        }
+        parts[row] = part;
+    }
+    __syncthreads();
+    const double sum = block_sum_fast(t < kRows ? parts[t] : 0.0, sh);
+    if (t == 0) W.part[blockIdx.x] = sum;
 }
 
 // part 2: alpha, x / r / z update, partial r.z
@@ -1594,7 +1642,7 @@ __global__ __launch_bounds__(kMwThreads) void mw_update_kernel(int n, int iter, 
     __shared__ double rs[BJ ? kMwThreads : 1];
     if (*W.done) return;  // uniform over the grid
     const int nblk = gridDim.x;
-    const double pAp = mw_sum(W.part, nblk, sh);
+    const double pAp = mw_sum(W.part, nblk, sh, blockDim.x);
     const double rz_old = W.rz[iter & 1];
     // unguarded in the reference: p = 0 once the residual vanishes exactly between checks
     const double alpha = pAp != 0.0 ? rz_old / pAp : 0.0;
@@ -1626,7 +1674,7 @@ __global__ __launch_bounds__(kMwThreads) void mw_check_kernel(int nblk, int iter
                                                               MwState W) {
     __shared__ double sh[17];
     if (*W.done) return;
-    const double rz_new = mw_sum(W.part + nblk, nblk, sh);
+    const double rz_new = mw_sum(W.part + nblk, nblk, sh, blockDim.x);
     if (threadIdx.x != 0) return;
     *W.err = rz_new;
     if ((iter + 1) % check_every == 0 && rz_new <= tol_sq) {
@@ -1854,10 +1902,12 @@ int solve_cg_multi(hipStream_t s, const Bsr& M, const double* b, double* x, doub
     ABD_CHECK_LAUNCH();
     launch_kernel(mw_start_kernel, dim3(1), dim3(kMwThreads), 0, s, nblk, tol_sq, maxiter, W);
     ABD_CHECK_LAUNCH();
+    const auto first = bj ? mw_spmv_kernel<kMwBjThreads, true> : mw_spmv_kernel<kMwThreads, true>;
+    const auto next = bj ? mw_spmv_kernel<kMwBjThreads, false> : mw_spmv_kernel<kMwThreads, false>;
     for (int i0 = 0; i0 < maxiter; i0 += check_every) {
         const int i1 = i0 + check_every < maxiter ? i0 + check_every : maxiter;
         for (int i = i0; i < i1; ++i) {
-            launch_kernel(mw_spmv_kernel, dim3(nblk), dim3(threads), 0, s, M, i, tol_sq, W);
+            launch_kernel(i == 0 ? first : next, dim3(nblk), dim3(kMwLanes * threads), 0, s, M, i, tol_sq, W);
             if (bj)
                 launch_kernel(mw_update_kernel<true>, dim3(nblk), dim3(threads), 0, s, n, i, W, (const double*)dinv);
             else
