@@ -1269,7 +1269,33 @@ __global__ __launch_bounds__(kSolveThreads) void ldlt_kernel(Bsr M, const int32_
                         while ((v + 1) * (v + 2) / 2 <= pidx) ++v;
                         const int i = mlist[k1][pidx - v * (v + 1) / 2], j = mlist[k1][v];
                         const unsigned long long contrib = cmask & colm[i] & colm[j];
-                        if (__builtin_ctzll(contrib) != k1) continue;
+                        const int rank = __popcll(contrib & bits_below(k1));
+                        if (__popcll(contrib) >= 3) {
+                            // a row of the tile each for the threads of the three lowest: one
+                            // thread's nine sums over many contributors would be the level's
+                            // chain (20 bodies coupled to one: 53 us, 41 here)
+                            if (rank >= 3) continue;
+                            auto tgt = U + 144 * (int64_t)(pos[i] + __popcll(adj[i] & bits_below(j))) +
+                                       12 * (ta + rank) + tb;
+                            double val[3] = {tgt[0], tgt[1], tgt[2]};
+                            for (unsigned long long bt = contrib; bt; bt &= bt - 1ull) {
+                                const int k2 = __builtin_ctzll(bt);
+                                const unsigned long long ab = bits_above(adj[k2], k2);
+                                const auto Aki = Ab + aoff(k2) + 144 * __popcll(ab & bits_below(i)) + ta + rank;
+                                const auto Wj = Wb + 144 * (int64_t)(woff[k2] + __popcll(ab & bits_below(j))) + tb;
+                                double acc[3] = {0.0, 0.0, 0.0};
+#pragma unroll 4
+                                for (int r = 0; r < 12; ++r)
+#pragma unroll
+                                    for (int q = 0; q < 3; ++q) acc[q] += Aki[12 * r] * Wj[12 * r + q];
+#pragma unroll
+                                for (int q = 0; q < 3; ++q) val[q] -= acc[q];
+                            }
+#pragma unroll
+                            for (int q = 0; q < 3; ++q) tgt[q] = val[q];
+                            continue;
+                        }
+                        if (rank) continue;
                         auto tgt = U + 144 * (int64_t)(pos[i] + __popcll(adj[i] & bits_below(j))) + 12 * ta + tb;
                         double val[9];
 #pragma unroll

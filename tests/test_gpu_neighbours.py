@@ -122,3 +122,26 @@ def test_large_cg_long_rows(kind, m, block):
         assert int(info.iters[0]) == it and (it < 40)
         assert rel_err(x.cpu().numpy(), ref) <= 1e-9
         assert abs(float(info.resid[0]) - err) <= 1e-8 * abs(err)
+
+
+@pytest.mark.parametrize("m", [3, 4, 5, 20, 33])
+def test_ldlt_of_a_body_coupled_to_all(m):
+    """The direct solve where one block is updated by all other bodies at once: by two (one
+    thread takes a tile), three (a row each) and many.  The oracle's same sums, 1e-14 (the bound
+    of the other comparisons of this solve)."""
+    import abd_hip
+    from abd_hip.sparse import BsrMatrix, SolveInfo, bsr_ldlt
+    from test_gpu_ldlt import _structure, _system
+    lib = abd_hip.load()
+    rng = np.random.default_rng(m)
+    ij = np.stack([np.arange(m - 1), np.full(m - 1, m - 1)], 1).astype(np.int32)
+    blocks, dense = _system(m, ij, rng)
+    b = rng.normal(size=(4 * m, 3))
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()  # noqa: E731
+    A = BsrMatrix(m, *_structure(lib, m, ij), d(blocks))
+    x, info = d(np.zeros((4 * m, 3))), SolveInfo("cuda")
+    bsr_ldlt(A, x, d(b), info=info)
+    ref, st = O.bsr_ldlt(m, ij, blocks, b, np.zeros((4 * m, 3)))
+    assert st == 1 and int(info.iters[0]) == 1
+    assert rel_err(x.cpu().numpy(), ref) <= 1e-14
+    assert rel_err(x.cpu().numpy().ravel(), np.linalg.solve(dense, b.ravel())) <= 1e-10
