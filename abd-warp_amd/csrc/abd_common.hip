@@ -19,6 +19,7 @@ std::mutex g_arena_mutex;
 thread_local Arena* t_arena = nullptr;  // a simulator's own arena during its calls
 thread_local hipGraph_t t_graph = nullptr;      // the graph this thread records
 thread_local hipGraphNode_t t_node = nullptr;   // its last node
+thread_local int t_graph_rc = ABD_OK;           // the first node that could not be added
 std::atomic<uint64_t> g_alloc_gen{1};
 
 int current_device(int* dev) {
@@ -43,9 +44,15 @@ void note_reallocation() { g_alloc_gen.fetch_add(1, std::memory_order_relaxed); 
 void graph_record(hipGraph_t g) {
     t_graph = g;
     t_node = nullptr;
+    t_graph_rc = ABD_OK;
+}
+int graph_record_end() {
+    t_graph = nullptr;
+    return t_graph_rc;
 }
 bool capturing() { return t_graph != nullptr; }
-int graph_add_kernel(const void* f, dim3 grid, dim3 block, void** args, size_t lds) {
+void graph_add_kernel(const void* f, dim3 grid, dim3 block, void** args, size_t lds) {
+    if (t_graph_rc) return;
     hipKernelNodeParams p{};
     p.func = const_cast<void*>(f);
     p.gridDim = grid;
@@ -53,15 +60,18 @@ int graph_add_kernel(const void* f, dim3 grid, dim3 block, void** args, size_t l
     p.kernelParams = args;
     p.sharedMemBytes = (unsigned)lds;
     hipGraphNode_t node = nullptr;
-    ABD_CHECK(hipGraphAddKernelNode(&node, t_graph, t_node ? &t_node : nullptr, t_node ? 1 : 0, &p));
-    t_node = node;
-    return ABD_OK;
+    const hipError_t e = hipGraphAddKernelNode(&node, t_graph, t_node ? &t_node : nullptr, t_node ? 1 : 0, &p);
+    if (e != hipSuccess)
+        t_graph_rc = hip_failure(e, __FILE__, __LINE__, "hipGraphAddKernelNode");
+    else
+        t_node = node;
 }
 int copy_to_host(hipStream_t s, void* dst, const void* src, size_t bytes) {
     if (!capturing()) {
         ABD_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s));
         return ABD_OK;
     }
+    if (t_graph_rc) return t_graph_rc;
     hipGraphNode_t node = nullptr;
     ABD_CHECK(hipGraphAddMemcpyNode1D(&node, t_graph, t_node ? &t_node : nullptr, t_node ? 1 : 0, dst, src, bytes,
                                       hipMemcpyDeviceToHost));

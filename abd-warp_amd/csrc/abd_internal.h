@@ -22,16 +22,19 @@ int hip_failure(hipError_t e, const char* file, int line, const char* expr);
     } while (0)
 #define ABD_CHECK_LAUNCH() ABD_CHECK(hipGetLastError())
 
-// A graph recorded by this thread: between graph_record(g) and graph_record(nullptr) every
+// A graph recorded by this thread: between graph_record(g) and graph_record_end() every
 // launch_kernel and copy_to_host of the thread becomes the next node of g, one after the other,
 // and nothing runs.  (Not a stream capture: while a stream of the process is captured the
 // runtime refuses device synchronization, which any other thread may be doing.)
+// graph_record_end: ABD_OK, or why a node could not be added; the graph then lacks it and all
+// that followed, and must not run.
 void graph_record(hipGraph_t g);
+int graph_record_end();
 bool capturing();
-int graph_add_kernel(const void* f, dim3 grid, dim3 block, void** args, size_t lds);
+void graph_add_kernel(const void* f, dim3 grid, dim3 block, void** args, size_t lds);
 int copy_to_host(hipStream_t s, void* dst, const void* src, size_t bytes);
 
-// Launches f on s, or records the launch.
+// Launches f on s (a failure is hipGetLastError's), or records the launch (graph_record_end's).
 template <typename... P, typename... A>
 inline void launch_kernel(void (*f)(P...), dim3 grid, dim3 block, size_t lds, hipStream_t s, A&&... a) {
     std::tuple<P...> vals(static_cast<P>(a)...);
@@ -39,7 +42,7 @@ inline void launch_kernel(void (*f)(P...), dim3 grid, dim3 block, size_t lds, hi
         [&](P&... v) {
             void* args[] = {(void*)&v...};
             if (capturing())
-                (void)graph_add_kernel((const void*)f, grid, block, args, lds);
+                graph_add_kernel((const void*)f, grid, block, args, lds);
             else
                 (void)hipLaunchKernel((const void*)f, grid, block, args, lds, s);
         },

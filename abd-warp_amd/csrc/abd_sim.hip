@@ -961,8 +961,9 @@ int record_iteration(hipStream_t s, Sim& S) {
         return -static_cast<int>(ce);
     }
     graph_record(g);
-    const int rc = iteration_scenes(s, S);
-    graph_record(nullptr);
+    int rc = iteration_scenes(s, S);
+    const int node_rc = graph_record_end();
+    if (!rc) rc = node_rc;
     if (rc) {
         (void)hipGraphDestroy(g);
         (void)hipGetLastError();
