@@ -7,12 +7,6 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-def _same(a, b):
-    return (dict(a.stats) == dict(b.stats) and torch.equal(a.states.A0, b.states.A0) and
-            torch.equal(a.states.p0, b.states.p0) and torch.equal(a.states.Adot, b.states.Adot) and
-            torch.equal(a.states.pdot, b.states.pdot))
-
-
 def test_replay_between_supersets():
     """A graph recorded for a superset of few edge pairs (below two a vertex) replayed after an
     iteration with many (above), in a step that leaves its ranges and is filtered anew: the
@@ -69,3 +63,57 @@ def test_replay_between_supersets():
     for k, (a, b) in enumerate(zip(got, ref)):
         assert a[0] == b[0] and a[1] == b[1], (k, a[:2], b[:2])
         assert torch.equal(a[2], b[2]) and torch.equal(a[3], b[3]), k
+
+
+@pytest.mark.parametrize("solver,psd", [(3, 1), (0, 0)])
+def test_one_scene_replay_equals_launches(solver, psd):
+    """One scene's iterations recorded and replayed while another thread synchronizes the device
+    and allocates: taken, and the states, iterations and statistics of the same iterations
+    launched kernel by kernel."""
+    import threading
+    from abd_hip import scenes
+    from abd_hip.abd import AffineBodySimulator
+    from abd_hip.const_params import ContactParams
+    m = scenes.cube_mesh()
+    n = 5
+    p = np.array([[0.0, 0.5005 + k * 1.001, 0.002 * k] for k in range(n)])
+    spec = scenes.build_scene([m] * n, np.stack([np.eye(3)] * n), p, np.zeros((n, 3, 3)), np.zeros((n, 3)),
+                              ground=0.0)
+    cp = ContactParams(ground=0.0, psd=psd, solver=solver)
+
+    def run(graphs):
+        sim, out = AffineBodySimulator(spec, cp, native=True), []
+        sim.set_graphs(graphs)
+        for f in range(6):
+            it = sim.step(f)
+            out.append((it, dict(sim.stats), sim.states.A0.clone(), sim.states.p0.clone()))
+        return out, sim.graph_counts()
+
+    done, errors, rounds = threading.Event(), [], [0]
+
+    def other():
+        try:
+            while not done.is_set():
+                torch.cuda.synchronize()
+                t = torch.empty(1 << (12 + rounds[0] % 12), device="cuda")
+                del t
+                torch.cuda.empty_cache()
+                rounds[0] += 1
+        except Exception as e:  # noqa: BLE001 - reported below
+            errors.append(e)
+
+    th = threading.Thread(target=other)
+    th.start()
+    try:
+        with torch.cuda.stream(torch.cuda.Stream()):
+            got, gc = run(True)
+    finally:
+        done.set()
+        th.join()
+    assert not errors and rounds[0] > 0
+    assert gc["recorded"] >= 1 and gc["replayed"] >= 5, gc
+    ref, none = run(False)
+    assert none["recorded"] == none["replayed"] == 0
+    for f, (a, b) in enumerate(zip(got, ref)):
+        assert a[0] == b[0] and a[1] == b[1], f
+        assert torch.equal(a[2], b[2]) and torch.equal(a[3], b[3]), f
