@@ -44,30 +44,6 @@ __device__ __forceinline__ double block_min(double v, double* sh) {
     __syncthreads();
     return r;
 }
-__device__ __forceinline__ float block_minf(float v, float* sh) {
-    const int t = threadIdx.x;
-    sh[t] = v;
-    __syncthreads();
-    for (int s = (int)blockDim.x / 2; s > 0; s >>= 1) {
-        if (t < s) sh[t] = fminf(sh[t], sh[t + s]);
-        __syncthreads();
-    }
-    float r = sh[0];
-    __syncthreads();
-    return r;
-}
-__device__ __forceinline__ float block_maxf(float v, float* sh) {
-    const int t = threadIdx.x;
-    sh[t] = v;
-    __syncthreads();
-    for (int s = (int)blockDim.x / 2; s > 0; s >>= 1) {
-        if (t < s) sh[t] = fmaxf(sh[t], sh[t + s]);
-        __syncthreads();
-    }
-    float r = sh[0];
-    __syncthreads();
-    return r;
-}
 
 // Sums across lanes by the vector unit's own lane moves (DPP, and the half and row swaps),
 // about 25 cycles a level where a shuffle through the LDS unit takes over 100.  The pairing

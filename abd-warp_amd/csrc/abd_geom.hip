@@ -33,20 +33,15 @@ __global__ __launch_bounds__(kBlock) void project_kernel(const int32_t* __restri
 
 // abd.py:337-353
 __global__ void update_q_kernel(int nb, const double* __restrict__ A, const double* __restrict__ p,
-                                const double* __restrict__ dq, double alpha, double* A_out, double* p_out,
-                                double* A_out2, double* p_out2) {
+                                const double* __restrict__ dq, double alpha, double* A_out, double* p_out) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= 12 * nb) return;
     int b = i / 12, r = i % 12;
     if (r < 3) {
-        const double v = p[3 * b + r] - dq[3 * (4 * b) + r] * alpha;
-        p_out[3 * b + r] = v;
-        if (p_out2) p_out2[3 * b + r] = v;
+        p_out[3 * b + r] = p[3 * b + r] - dq[3 * (4 * b) + r] * alpha;
     } else {
         int row = (r - 3) / 3, k = (r - 3) % 3;
-        const double v = A[9 * b + 3 * row + k] - dq[3 * (4 * b + 1 + row) + k] * alpha;
-        A_out[9 * b + 3 * row + k] = v;
-        if (A_out2) A_out2[9 * b + 3 * row + k] = v;
+        A_out[9 * b + 3 * row + k] = A[9 * b + 3 * row + k] - dq[3 * (4 * b + 1 + row) + k] * alpha;
     }
 }
 
@@ -281,16 +276,6 @@ __global__ void update_q_scenes_kernel(int nb, const int32_t* __restrict__ body_
     if (out2) *out2 = v;
 }
 
-// q_out = q - alpha dq, also written to (A_out2, p_out2) when they are given
-int update_q_dual(hipStream_t s, int nb, const double* A, const double* p, const double* dq, double alpha,
-                  double* A_out, double* p_out, double* A_out2, double* p_out2) {
-    if (nb == 0) return ABD_OK;
-    launch_kernel(update_q_kernel, dim3(grid_for(12 * (int64_t)nb)), dim3(kBlock), 0, s, nb, A, p, dq, alpha,
-                       A_out, p_out, A_out2, p_out2);
-    ABD_CHECK_LAUNCH();
-    return ABD_OK;
-}
-
 int update_q_scenes_dual(hipStream_t s, const AbdScene* sc, const double* A, const double* p, const double* dq,
                          const double* alpha, double* A_out, double* p_out, double* A_out2, double* p_out2) {
     const int nb = sc->n_bodies;
@@ -399,7 +384,10 @@ int abd_update_q(abd_stream_t stream, int32_t nb, const double* A, const double*
                  double* A_out, double* p_out) {
     if (nb < 0 || !A || !p || !dq || !A_out || !p_out) return ABD_ERR_ARG;
     if (nb == 0) return ABD_OK;
-    return update_q_dual(to_stream(stream), nb, A, p, dq, alpha, A_out, p_out, nullptr, nullptr);
+    launch_kernel(update_q_kernel, dim3(grid_for(12 * (int64_t)nb)), dim3(kBlock), 0, to_stream(stream), nb, A, p, dq,
+                  alpha, A_out, p_out);
+    ABD_CHECK_LAUNCH();
+    return ABD_OK;
 }
 
 int abd_update_q0qdot(abd_stream_t stream, int32_t nb, double dt, const double* A, const double* p, double* A0,

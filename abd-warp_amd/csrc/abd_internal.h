@@ -259,12 +259,9 @@ int step_states(hipStream_t s, const AbdScene* sc, const double* A, const double
 int contact_energy(hipStream_t s, const AbdScene* sc, const AbdParams* P, int S, const double* xk, const int32_t* pt,
                    int64_t npt, const int32_t* ee, int64_t nee, const int32_t* vg, int64_t nvg, const int64_t* dn,
                    double* E);
-// abd_update_q / abd_update_q_scenes writing the result to a second state as well (when
-// A_out2, p_out2 are given).
-int update_q_dual(hipStream_t s, int nb, const double* A, const double* p, const double* dq, double alpha,
-                  double* A_out, double* p_out, double* A_out2, double* p_out2);
 // Whether abd_bsr_solve of nb bodies waits for the device between its launches.
 bool solve_waits(int32_t method, int nb);
+// abd_update_q_scenes writing the result to a second state as well (when A_out2, p_out2 are given).
 int update_q_scenes_dual(hipStream_t s, const AbdScene* sc, const double* A, const double* p, const double* dq,
                          const double* alpha, double* A_out, double* p_out, double* A_out2, double* p_out2);
 // Collision set from a superset of it (keep_from_superset, abd_cull.hip): the superset's
@@ -418,7 +415,6 @@ struct ScanSeg {
 };
 constexpr int kMaxScanSegs = 8;
 int scan_exclusive_i64_multi(hipStream_t s, const ScanSeg* segs, int nseg);
-// Deterministic sum of n doubles: *out (device) = sum, fixed order.
 // Copies one int64 from device to host (synchronizes `s`).
 int read_i64(hipStream_t s, const int64_t* dev, int64_t* host);
 
