@@ -743,45 +743,53 @@ int attach_seg_bytes(int handle, hipStream_t s, int S, const int64_t* seg, doubl
     return ABD_OK;
 }
 
-// Algorithmic bytes of trial_chunk_kernel, one workgroup per chunk: each candidate's apart_until
-// where a trial of its scene is wanted, and 132, 128 or 32 bytes per EE, PT or VG pair that the
-// kernel lists (the rest it does not read).  Sums of whole numbers: their order is free.
-__global__ __launch_bounds__(kRedThreads) void trial_bytes_kernel(Lists L, int S, int K,
+// Algorithmic bytes of trial_chunk_kernel, one workgroup per chunk.  Per candidate, once a launch
+// however many of its trials take it: its apart_until where a trial of its scene is wanted, and
+// 132, 128 or 32 bytes (EE, PT, VG: tuple, indices and rest vertices) where one lists it; per
+// wanted trial of a scene, the states of the scene's bodies (96 bytes each; workgroup 0).  Sums
+// of whole numbers: their order is free.
+__global__ __launch_bounds__(kRedThreads) void trial_bytes_kernel(Lists L, int S, int K, int nb,
+                                                                  const int32_t* __restrict__ scene_boff,
                                                                   const double* __restrict__ alpha,
                                                                   const int64_t* __restrict__ seg,
                                                                   const int64_t* __restrict__ choff,
                                                                   double* __restrict__ out) {
     __shared__ double sh[kRedThreads];
     const int64_t c = blockIdx.x;
-    if (c >= choff[S]) return;
-    const ChunkRange r = chunk_range(S, seg, choff, c);
-    const ListRef& Lr = L.l[r.l < kLists ? r.l : 0];
-    const double each = Lr.kind == kListEE ? 132.0 : Lr.kind == kListPT ? 128.0 : 32.0;
     double acc = 0.0;
-    for (int64_t i = r.start + threadIdx.x; i < r.end; i += blockDim.x) {
-        const double apart = Lr.apart ? (double)Lr.apart[i] : 0.0;
-        bool wanted = false;
-        for (int k = 0; k < K; ++k) {
-            const double al = alpha[(int64_t)S * k + r.s];
-            if (al < 0.0) continue;
-            wanted = true;
-            if (!(al < apart)) acc += each;
+    if (c == 0)
+        for (int i = threadIdx.x; i < S * K; i += blockDim.x)
+            if (!(alpha[i] < 0.0)) acc += 96.0 * (S > 1 ? scene_boff[i % S + 1] - scene_boff[i % S] : nb);
+    if (c < choff[S]) {
+        const ChunkRange r = chunk_range(S, seg, choff, c);
+        const ListRef& Lr = L.l[r.l < kLists ? r.l : 0];
+        const double each = Lr.kind == kListEE ? 132.0 : Lr.kind == kListPT ? 128.0 : 32.0;
+        for (int64_t i = r.start + threadIdx.x; i < r.end; i += blockDim.x) {
+            const double apart = Lr.apart ? (double)Lr.apart[i] : 0.0;
+            bool wanted = false, listed = false;
+            for (int k = 0; k < K; ++k) {
+                const double al = alpha[(int64_t)S * k + r.s];
+                if (al < 0.0) continue;
+                wanted = true;
+                if (!(al < apart)) listed = true;
+            }
+            if (wanted && Lr.apart) acc += 4.0;
+            if (listed) acc += each;
         }
-        if (wanted && Lr.apart) acc += 4.0;
     }
     acc = block_sum(acc, sh);
     if (threadIdx.x == 0) atomicAdd(out, acc);
 }
 
 // Attaches to `handle` the bytes of trial_bytes_kernel (nothing when the handle is -1).
-int attach_trial_bytes(int handle, hipStream_t s, const Lists& L, int S, int K, const double* alpha,
-                       const int64_t* seg, const int64_t* choff, int64_t chunks) {
+int attach_trial_bytes(int handle, hipStream_t s, const AbdScene& sc, const Lists& L, int S, int K,
+                       const double* alpha, const int64_t* seg, const int64_t* choff, int64_t chunks) {
     double* out;
     int rc = prof_byte_slot(handle, &out);
     if (rc || !out) return rc;
     if ((rc = zero_fill(s, out, sizeof(double)))) return rc;
-    launch_kernel(trial_bytes_kernel, dim3((unsigned)chunks), dim3(kRedThreads), 0, s, L, S, K, alpha, seg, choff,
-                  out);
+    launch_kernel(trial_bytes_kernel, dim3((unsigned)chunks), dim3(kRedThreads), 0, s, L, S, K, sc.n_bodies,
+                  sc.scene_boff, alpha, seg, choff, out);
     ABD_CHECK_LAUNCH();
     prof_stop(handle, s, nullptr, out);
     return ABD_OK;
@@ -881,7 +889,7 @@ int line_chunks(hipStream_t s, const AbdScene* sc, const AbdParams* P, int S, in
     double* part;
     if ((rc = get_plan(s, *sc, S, L, plan, &seg, &choff))) return rc;
     if ((rc = arena_get(kSlotReduce, sizeof(double) * (size_t)bound * K, (void**)&part))) return rc;
-    // bytes: those of the (trial, candidate) pairs evaluated, counted on the device
+    // bytes: those of the candidates that some trial lists, counted on the device
     int ph = prof_start_ext(kProfEnergy, 1.0);
     // a workgroup's trials share its listing and fill its batches, but its threads evaluate
     // them in turn: two trials each, or one where the chunks leave the device fewer than
@@ -894,7 +902,7 @@ int line_chunks(hipStream_t s, const AbdScene* sc, const AbdParams* P, int S, in
     prof_launch(ph, trial_chunk_kernel, dim3((unsigned)bound, groups), dim3(kRedThreads), 0, s, *sc, *P,
                 TrialArgs{alpha, st}, L, S, K, seg, choff, part, bound);
     ABD_CHECK_LAUNCH();
-    if ((rc = attach_trial_bytes(ph, s, L, S, K, alpha, seg, choff, bound))) return rc;
+    if ((rc = attach_trial_bytes(ph, s, *sc, L, S, K, alpha, seg, choff, bound))) return rc;
     *out = TrialSums{choff, part, bound};
     return ABD_OK;
 }

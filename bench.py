@@ -447,8 +447,12 @@ def main():
         def roofline_of(k):
             ms, n, byts = prof[k]
             achieved = byts / (ms * 1e-3) / 1e9
-            return dict(kernel=k, bound="hbm", achieved=round(achieved, 3), peak=HBM_PEAK_GBS, unit="GB/s",
-                        frac=achieved / HBM_PEAK_GBS, traffic=measured_traffic(k, a.workload, a.solver), launches=n,
+            # priced against the HBM peak; one that reaches less than half of it is held by the
+            # latency of its dependent steps (no kernel here comes near the FP64 peak)
+            frac = achieved / HBM_PEAK_GBS
+            return dict(kernel=k, bound="hbm" if frac >= 0.5 else "latency", achieved=round(achieved, 3),
+                        peak=HBM_PEAK_GBS, peak_of="hbm", unit="GB/s", frac=frac,
+                        traffic=measured_traffic(k, a.workload, a.solver), launches=n,
                         avg_us=round(1e3 * ms / n, 3), bytes_per_launch=byts / n)
         roof = roofline_of(dom)
         rooflines = {k: roofline_of(k) for k in timed_kernels}
