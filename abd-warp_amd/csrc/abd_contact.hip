@@ -405,8 +405,9 @@ __global__ __launch_bounds__(kWave) void contact_dense_kernel(AbdScene sc, AbdPa
     }
 }
 
-// workgroups of the dense modes' stage C, at most: one wave each, at 8 KB of LDS the 16 or so
-// a CU holds at once fill the device's 256 CUs
+// workgroups of the dense modes' stage C, at most: one wave each, 16 a CU, as many as the exact
+// mode's registers let a CU hold (127 of them: four waves a SIMD; full IPC's 162: three).  Each
+// takes 4 KB of the CU's LDS.
 constexpr int64_t kDenseGrid = 4096;
 
 constexpr int kPairThreads = 576;  // one thread per entry of the 24x24 body-pair block

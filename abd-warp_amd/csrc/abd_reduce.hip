@@ -323,7 +323,7 @@ struct TrialArgs {
 // place plus its rank among the wave's ballots, so that the owner finds it again.  Bound by
 // the latency of a workgroup's few dependent gathers: evaluating every candidate at every
 // trial took 60 us for a pass of one trial and 130 us for one of twelve over 1.3M
-// candidates (256 scenes), this 39 and 74 us (0.35M and 1.1M pairs evaluated).  Where most
+// candidates (256 scenes), this 32 and 73 us (0.35M and 1.1M pairs evaluated).  Where most
 // candidates are near and listed all the same (256 scenes of 2 to 64 bodies, 0.8 of the bytes),
 // the listing is not repaid: 30 and 58 us against 19 and 44.
 constexpr int kTrialItems = kChunkItems / kRedThreads;

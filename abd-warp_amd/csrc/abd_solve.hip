@@ -1752,7 +1752,8 @@ int launch_solve(hipStream_t s, int32_t method, const Bsr& M, int nsys, const in
     double* dinv = nullptr;
     if (bj && (rc = arena_get(kSlotPrecond, sizeof(double) * 144 * (size_t)M.nb, (void**)&dinv))) return rc;
     if (bj) {
-        // every body's diagonal-block inverse, one thread per body (inactive scenes included: cheap)
+        // every body's diagonal-block inverse, one 64-thread workgroup per body (inactive scenes
+        // included: cheap)
         if (M.nb > 0) {
             // algorithmic bytes: each diagonal block read, its inverse written
             const int ph_inv = pending ? -1 : prof_start(kProfPrecond, s, 2304.0 * M.nb);
