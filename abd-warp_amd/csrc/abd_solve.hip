@@ -1270,10 +1270,13 @@ __global__ __launch_bounds__(kSolveThreads) void ldlt_kernel(Bsr M, const int32_
                         const int i = mlist[k1][pidx - v * (v + 1) / 2], j = mlist[k1][v];
                         const unsigned long long contrib = cmask & colm[i] & colm[j];
                         const int rank = __popcll(contrib & bits_below(k1));
-                        if (__popcll(contrib) >= 3) {
+                        if (decltype(lds_c)::value && __popcll(contrib) >= 3) {
                             // a row of the tile each for the threads of the three lowest: one
                             // thread's nine sums over many contributors would be the level's
-                            // chain (20 bodies coupled to one: 53 us, 41 here)
+                            // chain (20 bodies coupled to one: 53 us, 40 here).  Only where the
+                            // factor is in LDS: the other two instances too would take 40 bodies
+                            // coupled so from 95 to 80 us, but every solve 1 us more, in code
+                            // and spilled registers (256 scenes 51 to 52)
                             if (rank >= 3) continue;
                             auto tgt = U + 144 * (int64_t)(pos[i] + __popcll(adj[i] & bits_below(j))) +
                                        12 * (ta + rank) + tb;
